@@ -447,58 +447,89 @@ def wigner_rotate_backward(x: Tensor, grad_out: Tensor, sincos, layout: Rotation
 
 # ---- specialised uvu ----------------------------------------------------------------------------------------
 # How the sorted edge list is cut into one range per wavefront: "aligned" (at segment boundaries, no partial rows),
-# "balanced" (after equal numbers of steps), "positions" (after equal numbers of positions), or "auto": measured on the
-# lmax = 2, C = 64 edge workload, the forward is fastest on aligned ranges (0.061 ms against 0.071 / 0.066) and the
-# backward, whose steps are three times as long, on balanced ones (0.115 ms against 0.122 / 0.118).
+# "balanced" (after equal numbers of steps), "positions" (after equal numbers of positions), or "auto": the rule of
+# SegIndex.prefers_aligned.
 _RANGE_MODE = __import__("os").environ.get("CGTP_RANGE_MODE", "auto")
+_RESIDENT_WAVES = 2048      # wavefronts of the segment kernels the chip holds at once (two per SIMD)
 
 
 class SegIndex:
     """Per-sorted-position index arrays of the segment mode (all int64, same device), and the tables that cut the
-    sorted list into one range per wavefront."""
+    sorted list into one range per wavefront.
+
+    A wavefront walks its range step by step, one memory round trip and the product's arithmetic each (about 1 us at
+    lmax = 2, 4 us at lmax = 3), so a launch lasts at least as long as its longest range.  Short lists are therefore
+    cut as finely as the chip has wavefronts for, down to one step per range, and long ones into a whole number of
+    rounds of resident wavefronts (``balanced_positions``).  Kernel times at C = 64, average degree 14-20, forward |
+    backward in us, with 32 positions per range as for every list before and with this rule:
+
+        lmax 2:   420 edges 19.9 | 36.7 -> 10.1 | 14.6    8192: 28.3 | 44.1 -> 15.6 | 25.3    32768: 31.6 | 53.3 -> 28.9 | 53.2
+        lmax 3:   420 edges 73.5 | 196  -> 19.0 | 43.8    8192: 78.1 | 202  -> 27.7 | 58.2    32768: 88.8 | 210  -> 64.6 | 144
+
+    ``positions_per_wave``: a fixed number of positions per range instead of the rule (both kinds of range)."""
 
     def __init__(self, ptr: Tensor, perm: Optional[Tensor], seg_ids: Tensor, gather: Tensor,
-                 positions_per_wave: int = int(__import__("os").environ.get("CGTP_POSITIONS_PER_WAVE", "32"))):
+                 positions_per_wave: int = int(__import__("os").environ.get("CGTP_POSITIONS_PER_WAVE", "0"))):
         self.ptr, self.perm, self.seg_ids, self.gather = ptr, perm, seg_ids, gather
         self.positions_per_wave = positions_per_wave
-        self.wave_seg = self.aligned_ranges(ptr, positions_per_wave)
+        self.wave_seg = self.aligned_ranges(ptr, positions_per_wave or self.ALIGNED_POSITIONS)
         # the step-balanced cuts for every slot count a launch can have (64 / lanes per edge), built here, where a host
         # sync is expected, and not on the first backward (inside autograd, possibly under graph capture)
         self._wave_pos = {}
         self._build_balanced(self.SLOT_COUNTS)
 
     SLOT_COUNTS = (1, 2, 4, 8, 16, 32, 64)
+    # Positions of a segment-aligned range: about one node's edges each.  A range of a few nodes saves nothing, and the
+    # short ones fill the last round of wavefronts better (lmax 2, C = 64, forward: 200 000 edges 160.9 us at 32 positions,
+    # 152.6 at 8, 174 at 4; 65 536 edges 54.4 at both).
+    ALIGNED_POSITIONS = 8
+    HUB_POSITIONS = 256     # positions from which a segment counts as a hub node's
 
     def _build_balanced(self, slot_counts) -> None:
         import numpy as np
         ptr = self.ptr.detach().cpu().numpy()
         n_pos = int(ptr[-1]) if ptr.shape[0] else 0
+        degrees = np.diff(ptr)
+        self.n_positions, self.longest = n_pos, int(degrees.max()) if degrees.shape[0] else 0
         for slots in slot_counts:
             if n_pos == 0:
                 self._wave_pos[slots] = None
                 continue
-            steps = (np.diff(ptr) + slots - 1) // slots
+            steps = (degrees + slots - 1) // slots
             last = np.cumsum(steps)                            # steps up to and including each segment
             first = last - steps
-            # as many ranges as equal cuts by position would give (a launch sized for that many wavefronts stays
-            # resident in one round)
-            n_ranges = max(1, n_pos // self.positions_per_wave)
+            # whole rounds of resident wavefronts, up to 48 positions per range; a list with a hub node keeps 32
+            # positions per range, since the fix-up adds the partial rows of a segment one after the other
+            per = self.positions_per_wave or (32 if self.longest > self.HUB_POSITIONS else 0)
+            n_ranges = max(1, n_pos // per) if per else _RESIDENT_WAVES * -(-n_pos // (_RESIDENT_WAVES * 48))
             per_wave = max(1, -(-int(last[-1]) // n_ranges))
+            if not per:                        # and no other segment is cut into more than 32 ranges
+                per_wave = max(per_wave, -(-int(steps.max()) // 32))
             targets = np.arange(0, int(last[-1]), per_wave, dtype=np.int64)
             seg = np.searchsorted(last, targets, side="right")
             pos = ptr[:-1][seg] + (targets - first[seg]) * slots
             self._wave_pos[slots] = torch.from_numpy(np.concatenate([pos, [n_pos]]).astype(np.int64)).to(self.ptr.device)
 
+    def prefers_aligned(self, slots: int, backward: bool) -> bool:
+        """Whether a launch with ``slots`` edges per step runs on the segment-aligned ranges.  The backward, with its
+        long steps, never does (lmax 2, C = 64, 65 536 edges: 94.4 us balanced, 102 aligned); neither does a forward
+        with one or two edges per step (lmax 3: 114.6 against 123.4 us), one whose steps do not fill the chip, where a
+        node's edges in one wavefront would take longer than the launch (8192 edges: 15.6 against 17.4 us at lmax 2,
+        27.7 against 48.9 at lmax 3), or one with a node of far more edges than the average wavefront takes.  Otherwise
+        aligned ranges save the partial rows and the fix-up (54.4 against 55.1 us; lmax 1, 200 000 edges: 61.9 against 70)."""
+        return (not backward and slots > 2 and self.wave_seg is not None and self.n_positions > _RESIDENT_WAVES * slots
+                and self.longest <= max(48, self.n_positions >> 10))
+
     @staticmethod
     def aligned_ranges(ptr: Tensor, positions_per_wave: int) -> Optional[Tensor]:
         """Cut the sorted list at segment boundaries into ranges of about ``positions_per_wave`` positions:
         int32 ``[n_ranges + 1]`` segment indices (first 0, last n_seg).  Range k starts at the first segment
-        whose first position is >= k * positions_per_wave.  Returns None (ranges by position are used instead)
-        when a segment is so large that aligned ranges would be badly unbalanced."""
+        whose first position is >= k * positions_per_wave.  Returns None when a segment is a hub node's
+        (aligned ranges would be badly unbalanced)."""
         n_seg, n_pos = ptr.shape[0] - 1, int(ptr[-1])
         if n_seg == 0:
             return None
-        if n_pos and int((ptr[1:] - ptr[:-1]).max()) > 8 * positions_per_wave:
+        if n_pos and int((ptr[1:] - ptr[:-1]).max()) > SegIndex.HUB_POSITIONS:
             return None
         targets = torch.arange(0, max(n_pos, 1), positions_per_wave, device=ptr.device, dtype=ptr.dtype)
         cuts = torch.searchsorted(ptr[:-1].contiguous(), targets)
@@ -509,9 +540,8 @@ class SegIndex:
         """Cut the sorted list after equal numbers of steps: a wavefront takes up to ``slots`` positions of one segment
         per step, so a segment of n positions costs ceil(n / slots) steps wherever it lies, and a range that holds
         whole steps only costs exactly its share.  int64 ``[n_ranges + 1]`` positions (first 0, last n_pos), cuts on
-        step boundaries; as many ranges as ``positions_per_wave`` positions each would give.  The time of a wavefront follows its number of
-        steps, and ranges cut at segment boundaries differ in it by a factor of up to five on a graph of average
-        degree 16."""
+        step boundaries.  The time of a wavefront follows its number of steps, and ranges cut at segment boundaries
+        differ in it by a factor of up to five on a graph of average degree 16."""
         if slots <= 0:
             return None
         if slots not in self._wave_pos:      # a slot count outside SLOT_COUNTS: built now (reads ptr back: a host sync)
@@ -519,17 +549,17 @@ class SegIndex:
         return self._wave_pos[slots]
 
 
-def seg_ranges(cfg: int, seg: SegIndex, dtype_code: int, channels: int, backward: bool):
+def seg_ranges(cfg: int, seg: SegIndex, dtype_code: int, channels: int, backward: bool, long_steps: bool = False):
     """``(wave_seg, wave_pos)``, at most one of them a tensor: how a segment-mode launch of ``cfg`` cuts the sorted list
     into one range per wavefront (``_RANGE_MODE``); both None = ranges of equal numbers of positions, which is also all
-    the block-wise kernels of the large tables take."""
+    the block-wise kernels of the large tables take.  ``long_steps``: a forward whose steps are as long as a backward's."""
     if _lib.lib.cgtp_uvu_blockwise_only(int(cfg)):
         return None, None
-    wave_pos = None
-    if _RANGE_MODE == "balanced" or (_RANGE_MODE == "auto" and (backward or seg.wave_seg is None)):
-        wave_pos = seg.balanced_positions(int(_lib.lib.cgtp_uvu_slots(int(cfg), dtype_code, channels, int(backward))))
-    if wave_pos is not None:
-        return None, wave_pos
+    slots = int(_lib.lib.cgtp_uvu_slots(int(cfg), dtype_code, channels, int(backward)))
+    if _RANGE_MODE == "balanced" or (_RANGE_MODE == "auto" and not seg.prefers_aligned(slots, backward or long_steps)):
+        wave_pos = seg.balanced_positions(slots)
+        if wave_pos is not None:
+            return None, wave_pos
     if seg.wave_seg is not None and _RANGE_MODE != "positions":
         return seg.wave_seg, None
     return None, None
@@ -560,7 +590,7 @@ def identity_segments(n: int, device) -> IdentitySegments:
 
 
 def _uvu_args(cfg: int, x: Tensor, y: Tensor, w: Tensor, seg: Optional[SegIndex], gather: Optional[Tensor],
-              pos_per_wave: int = 0, y_vec: int = 0, backward: bool = False) -> UvuArgs:
+              pos_per_wave: int = 0, y_vec: int = 0, backward: bool = False, long_steps: bool = False) -> UvuArgs:
     a = UvuArgs()
     a.y_vec = y_vec
     a.y_channels = int(y.ndim == 3)
@@ -573,7 +603,7 @@ def _uvu_args(cfg: int, x: Tensor, y: Tensor, w: Tensor, seg: Optional[SegIndex]
             seg.gather.data_ptr()
         a.pos_per_wave = pos_per_wave
         if pos_per_wave == 0:
-            wave_seg, wave_pos = seg_ranges(cfg, seg, a.dtype, a.C, backward)
+            wave_seg, wave_pos = seg_ranges(cfg, seg, a.dtype, a.C, backward, long_steps)
             if wave_pos is not None:
                 a.wave_pos, a.n_waves = wave_pos.data_ptr(), wave_pos.shape[0] - 1
             elif wave_seg is not None:
@@ -732,8 +762,9 @@ def uvu_radial_supported(cfg: int, x: Tensor, h: Tensor, w_last: Tensor) -> bool
 def uvu_radial_forward(cfg: int, dims, x: Tensor, y: Tensor, h: Tensor, w_eff: Tensor, seg: SegIndex,
                        y_vec: int = 0) -> Tensor:
     """Segment-mode forward with the per-edge weights ``h @ w_eff`` formed inside the kernel (``w_eff`` from
-    :func:`radial_effective_weight`)."""
-    a = _uvu_args(Cfg(int(cfg)), x, y, h, seg, None, 0, y_vec)
+    :func:`radial_effective_weight`).  Its steps, which form the weights first, are as long as a backward's: step-balanced
+    ranges (65 536 edges: 77.6 us, on aligned ranges 96-107; 8192: 26 against 40)."""
+    a = _uvu_args(Cfg(int(cfg)), x, y, h, seg, None, 0, y_vec, long_steps=True)
     a.w, a.w_shared, a.path_scale = None, 0, None
     a.radial_h, a.radial_w, a.radial_r = h.data_ptr(), w_eff.data_ptr(), h.shape[1]
     out = torch.empty((a.n_seg, dims[2], x.shape[-1]), dtype=x.dtype, device=x.device)

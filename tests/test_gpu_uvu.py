@@ -489,3 +489,36 @@ def test_edge_fused_ranges_balanced_by_steps(device, hub):
     for name, a, b in zip(("out", "grad_x", "grad_sh", "grad_w"), results["balanced"], results["aligned"]):
         # per-edge results are the same numbers; node rows cut by a range boundary are summed in another order
         assert_close(a, b, 1e-5, f"balanced vs aligned hub={hub} {name}")
+
+
+@pytest.mark.parametrize("n_nodes,n_edges,longest", [(3, 1, 0), (5, 7, 0), (200, 2049, 0), (1100, 8193, 0), (40, 600, 256),
+                                                     (40, 600, 257)])
+@pytest.mark.parametrize("lmax,ch", [(1, 64), (2, 32), (3, 48)])
+def test_edge_fused_on_short_lists(device, n_nodes, n_edges, longest, lmax, ch):
+    """The ranges chosen for short edge lists, one step and up (one edge, fewer steps than wavefronts, just past the
+    sizes at which the forward changes to segment-aligned ranges), and on either side of the length from which a
+    segment counts as a hub node's: output and all gradients against the dense float64 oracle."""
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    mod = _module(SH[lmax], SH[lmax], SH[lmax]).to(device)
+    d = (lmax + 1) ** 2
+    gen = torch.Generator().manual_seed(31)
+    src = torch.randint(0, n_nodes, (n_edges,), generator=gen)
+    dst = torch.randint(0, n_nodes, (n_edges,), generator=gen)
+    if longest:
+        src[src == 7], dst[dst == 7] = 8, 8
+        src[:longest], dst[n_edges - longest:] = 7, 7
+    x, sh, w = tp_inputs(max(n_edges, n_nodes), d, lmax, mod.num_paths, ch, False, seed=32)
+    x, sh, w = x[:n_nodes].contiguous(), sh[:n_edges].contiguous(), w[:n_edges].contiguous()
+    ct = torch.randn(n_nodes, d, ch, generator=gen)
+    plan = EdgePlan(src.to(device), dst.to(device), n_nodes)
+    wrt = [t.to(device).requires_grad_(True) for t in (x, sh, w)]
+    out = edge_tensor_product_uu(*wrt, plan, mod.tp_info_forward)
+    got = (out, *torch.autograd.grad(out, wrt, ct.to(device)))
+
+    def ref_fn(T, x, sh, w):
+        return ref_ops.scatter_sum(ref_ops.dense_u1u(T, x.index_select(0, src), sh, w), dst, n_nodes)
+    T = ref_ops.dense_coupling(SH[lmax], SH[lmax], SH[lmax])
+    ref_out, ref_grads = ref_ops.dense_grads(ref_fn, T, (x, sh, w), ct)
+    for name, a, b in zip(("out", "grad_x", "grad_sh", "grad_w"), got, (ref_out, *ref_grads)):
+        # node rows are sums over up to 257 edges, whose rounding follows the largest term: norm-wise
+        assert_close(a, b, 1e-5, f"{n_edges} edges lmax={lmax} {name}", norm="max" if name in ("out", "grad_x") else "element")
