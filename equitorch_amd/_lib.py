@@ -68,6 +68,13 @@ class UvuTab(C.Structure):
                 ("D1", C.c_int32), ("D2", C.c_int32), ("DO", C.c_int32), ("P", C.c_int32)]
 
 
+class UvuMx(C.Structure):
+    _fields_ = [("fwd", C.c_void_p), ("bwd", C.c_void_p),
+                ("fwd_records", C.c_int32), ("fwd_entries", C.c_int32), ("bwd_records", C.c_int32),
+                ("bwd_entries", C.c_int32), ("row_tiles", C.c_int32), ("rounds", C.c_int32), ("lanes_log2", C.c_int32),
+                ("tiles", C.c_int32)]
+
+
 class PswTable(C.Structure):
     _fields_ = [("entries", C.c_void_p), ("coef", C.c_void_p), ("slots", C.c_void_p), ("blocks", C.c_void_p),
                 ("n_entries", C.c_int32), ("n_slots", C.c_int32), ("n_blocks", C.c_int32), ("max_rows", C.c_int32),
@@ -158,6 +165,11 @@ def _load():
     lib.cgtp_uvu_tab_validate.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.c_int]
     lib.cgtp_uvu_tab_fwd.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.c_void_p]
     lib.cgtp_uvu_tab_bwd.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.c_void_p]
+    lib.cgtp_uvu_mx_workspace_bytes.restype = C.c_int64
+    lib.cgtp_uvu_mx_workspace_bytes.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]
+    lib.cgtp_uvu_mx_validate.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]
+    lib.cgtp_uvu_mx_fwd.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_void_p]
+    lib.cgtp_uvu_mx_bwd.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_void_p]
     lib.cgtp_bessel.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_double, C.c_int32, C.c_void_p]
     lib.cgtp_bessel_grad.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32,
                                      C.c_double, C.c_int32, C.c_void_p]

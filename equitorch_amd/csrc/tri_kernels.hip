@@ -633,14 +633,19 @@ int cgtp_abi_layout(int which, int64_t* out, int capacity) {
                                      CGTP_OFF(cgtp_psw_args, n_rows), CGTP_OFF(cgtp_psw_args, cx),
                                      CGTP_OFF(cgtp_psw_args, cy), CGTP_OFF(cgtp_psw_args, cout),
                                      CGTP_OFF(cgtp_psw_args, dtype)};
+  static const int64_t uvu_mx[] = {sizeof(cgtp_uvu_mx), CGTP_OFF(cgtp_uvu_mx, fwd), CGTP_OFF(cgtp_uvu_mx, bwd),
+                                   CGTP_OFF(cgtp_uvu_mx, fwd_records), CGTP_OFF(cgtp_uvu_mx, fwd_entries),
+                                   CGTP_OFF(cgtp_uvu_mx, bwd_records), CGTP_OFF(cgtp_uvu_mx, bwd_entries),
+                                   CGTP_OFF(cgtp_uvu_mx, row_tiles), CGTP_OFF(cgtp_uvu_mx, rounds),
+                                   CGTP_OFF(cgtp_uvu_mx, lanes_log2), CGTP_OFF(cgtp_uvu_mx, tiles)};
 #undef CGTP_OFF
   const int64_t* tabs[] = {operand, tri, gen_operand, gen, uvu, uvt_item, uvt, uvt_gw, uvt_gy, uvu_tab, psw_table,
-                           psw_args};
+                           psw_args, uvu_mx};
   const int counts[] = {(int)(sizeof(operand) / 8), (int)(sizeof(tri) / 8), (int)(sizeof(gen_operand) / 8),
                         (int)(sizeof(gen) / 8), (int)(sizeof(uvu) / 8), (int)(sizeof(uvt_item) / 8),
                         (int)(sizeof(uvt) / 8), (int)(sizeof(uvt_gw) / 8), (int)(sizeof(uvt_gy) / 8),
-                        (int)(sizeof(uvu_tab) / 8), (int)(sizeof(psw_table) / 8), (int)(sizeof(psw_args) / 8)};
-  if (which < 0 || which >= 12) return -1;
+                        (int)(sizeof(uvu_tab) / 8), (int)(sizeof(psw_table) / 8), (int)(sizeof(psw_args) / 8), (int)(sizeof(uvu_mx) / 8)};
+  if (which < 0 || which >= 13) return -1;
   for (int i = 0; out && i < counts[which] && i < capacity; ++i) out[i] = tabs[which][i];
   return counts[which];
 }

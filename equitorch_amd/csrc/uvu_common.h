@@ -103,6 +103,11 @@ constexpr int kRadialC = 64;
 int uvu_fixup_rows_f32(float* rows, const float* ws, const int64_t* ptr, int64_t n_seg, int64_t row_len, int per_range,
                        int64_t n_ranges, int64_t n_rows, hipStream_t stream);
 
+// Launches the table-driven segment kernel (no fix-up) over ranges of `per_range` sorted positions, of which only those
+// whose word in `flags` is set are computed: for kernels that leave ranges they cannot answer to it.  Status code.
+int uvu_tab_redo_flagged(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backward, int per_range, const int32_t* flags,
+                         int64_t n_flags, hipStream_t stream);
+
 const UvuBigEntry* uvu_big_entries(int* count);
 const UvuBigEntry* uvu_big_entries_scaled(int* count);  // the same kernels applying UvuDev::ps
 

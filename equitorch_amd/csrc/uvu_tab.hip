@@ -29,6 +29,8 @@ struct TabDev {
   const uint32_t* idx;      // (NZ64 + 64) entry words (see kTabEndSeg), padding entries 0
   const uint32_t* paths;   // (paths in walk order + 2) the weight path of every run of entries, then 0xffff twice
   int nnz, nseg, D1, D2, DO, P;   // NZ64 = nnz rounded up to a multiple of 64
+  const int32_t* flags;     // optional: only the ranges whose word is set are computed (uvu_tab_redo_flagged)
+  int64_t n_flags;
 };
 
 // The table is read-only for the whole launch and indexed by values every lane agrees on: through the constant
@@ -229,13 +231,20 @@ struct TabPaths {
   }
 };
 
+// With flags (one word per range), a wavefront none of whose ranges is flagged has nothing to do.
+__device__ __forceinline__ bool tab_wanted(const TabDev& t, int64_t wave, const Lanes& L) {
+  if (!t.flags) return true;
+  const int64_t range = wave * L.slots + L.lane;
+  return __any(L.lane < L.slots && range < t.n_flags && t.flags[range] != 0);
+}
+
 template <int V>
 __global__ void __launch_bounds__(256) uvu_tab_seg_fwd_kernel(const UvuDev<float> a, const TabDev t, int64_t n_waves) {
   extern __shared__ __align__(16) float tab_lds[];
   const Lanes L(a.lpe_log2);
   const int wv = threadIdx.x / kWave;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / kWave) + wv;
-  if (wave >= n_waves) return;
+  if (wave >= n_waves || !tab_wanted(t, wave, L)) return;
   const TabLayout Y(L.lpe, V, t.D1, t.D2, t.DO, t.nnz, false);
   float* wave_lds = tab_lds + (int64_t)wv * L.slots * Y.slot_floats;
   float* mine = wave_lds + L.slot * Y.slot_floats;
@@ -342,7 +351,7 @@ __global__ void __launch_bounds__(256) uvu_tab_seg_bwd_kernel(const UvuDev<float
   const Lanes L(a.lpe_log2);
   const int wv = threadIdx.x / kWave;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / kWave) + wv;
-  if (wave >= n_waves) return;
+  if (wave >= n_waves || !tab_wanted(t, wave, L)) return;
   const TabLayout Y(L.lpe, V, t.D1, t.D2, t.DO, t.nnz, true);
   float* wave_lds = tab_lds + (int64_t)wv * L.slots * Y.slot_floats;
   float* mine = wave_lds + L.slot * Y.slot_floats;
@@ -568,13 +577,11 @@ static UvuDev<float> tab_dev(const cgtp_uvu_args* a, const TabPlan& plan) {
   return d;
 }
 
-static int tab_launch(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backward, hipStream_t stream) {
-  TabPlan plan;
-  const int rc = tab_plan(a, t, backward, &plan);
-  if (rc != CGTP_OK) return rc;
-  if (plan.ws_elems > 0 && !a->workspace) return CGTP_ERR_WORKSPACE;
+// The launch over the ranges alone; segments cut by a range boundary are left to the fix-up pass.
+static int tab_launch_ranges(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backward, const TabPlan& plan,
+                             const int32_t* flags, int64_t n_flags, hipStream_t stream) {
   const UvuDev<float> d = tab_dev(a, plan);
-  const TabDev td = {t->coef, t->idx, t->paths, t->nnz, t->n_segments, t->D1, t->D2, t->DO, t->P};
+  const TabDev td = {t->coef, t->idx, t->paths, t->nnz, t->n_segments, t->D1, t->D2, t->DO, t->P, flags, n_flags};
   if (plan.n_waves > 0) {
     void (*fn)(const UvuDev<float>, const TabDev, int64_t) =
         backward ? (plan.V == 4 ? uvu_tab_seg_bwd_kernel<4> : uvu_tab_seg_bwd_kernel<1>)
@@ -587,11 +594,29 @@ static int tab_launch(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backwar
                        d, td, plan.n_waves);
     if (hipGetLastError() != hipSuccess) return CGTP_ERR_LAUNCH;
   }
-  float* rows = backward ? d.gx : d.out;
-  if (!rows) return CGTP_OK;
+  return CGTP_OK;
+}
+
+int uvu_tab_redo_flagged(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backward, int per_range, const int32_t* flags,
+                         int64_t n_flags, hipStream_t stream) {
+  cgtp_uvu_args args = *a;
+  args.pos_per_wave = per_range;
+  TabPlan plan;
+  const int rc = tab_plan(&args, t, backward, &plan);
+  return rc != CGTP_OK ? rc : tab_launch_ranges(&args, t, backward, plan, flags, n_flags, stream);
+}
+
+static int tab_launch(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int backward, hipStream_t stream) {
+  TabPlan plan;
+  int rc = tab_plan(a, t, backward, &plan);
+  if (rc != CGTP_OK) return rc;
+  if (plan.ws_elems > 0 && !a->workspace) return CGTP_ERR_WORKSPACE;
+  rc = tab_launch_ranges(a, t, backward, plan, nullptr, 0, stream);
+  float* rows = backward ? (float*)a->grad_x : (float*)a->out;
+  if (rc != CGTP_OK || !rows) return rc;
   // every range is one "wavefront" of the fix-up pass; it also writes the zero rows of empty segments
-  return uvu_fixup_rows_f32(rows, d.ws, d.ptr, d.n_seg, (backward ? t->D1 : t->DO) * (int64_t)a->C, plan.per,
-                            plan.n_waves * plan.slots, d.n_rows, stream);
+  return uvu_fixup_rows_f32(rows, (const float*)a->workspace, a->ptr, a->n_seg, (backward ? t->D1 : t->DO) * (int64_t)a->C, plan.per,
+                            plan.n_waves * plan.slots, a->n_rows, stream);
 }
 
 }  // namespace cgtp

@@ -303,6 +303,29 @@ int cgtp_uvu_tab_validate(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, int bac
 int cgtp_uvu_tab_fwd(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, void* stream);
 int cgtp_uvu_tab_bwd(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, void* stream);
 
+/* The same launches on the matrix cores for small tables (D1, DO <= 16, D2 <= 32, P <= 32, every path with a
+ * coefficient) and C <= 64 channels, C a multiple of 1 / 2 / 4 up to 16 / 32 / 64 and the operands aligned to as many
+ * floats; everything else is as above (`t` serves the ranges in which a result is not finite).  The walk is two device
+ * arrays of 32-bit words, an "element" being the place (entry * 64 + step row * 16 + row) of one entry of the coupling
+ * matrix:
+ *   fwd, bwd: records (coef, coef, b | b' << 8 | element << 16): element = coef y[b] + coef' y[b'];
+ *             entries path | first row << 8: four consecutive rows of x (fwd) or grad_out (bwd) of one path;
+ *   bwd also: 16 * row_tiles words path | row of grad_out << 8, one per (path, output row);
+ *             64 * rounds pairs (coef, place in the matrix (path, output row) x 16 rows of x): lane l adds up component
+ *             l >> lanes_log2 of grad_y;
+ *             5 words per tile of the weight gradient: first row of grad_out | steps << 8, then four chunks of up to
+ *             four rows of x of one path: element | path << 16 | 1 << 24 if the path has an earlier chunk | rows << 25. */
+typedef struct cgtp_uvu_mx {
+  const uint32_t* fwd;
+  const uint32_t* bwd;
+  int32_t fwd_records, fwd_entries, bwd_records, bwd_entries;   /* entries <= 64                                    */
+  int32_t row_tiles, rounds, lanes_log2, tiles;
+} cgtp_uvu_mx;
+int64_t cgtp_uvu_mx_workspace_bytes(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, int backward);
+int cgtp_uvu_mx_validate(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, int backward);
+int cgtp_uvu_mx_fwd(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, void* stream);
+int cgtp_uvu_mx_bwd(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, void* stream);
+
 /* Positions of one segment a wavefront takes per step (64 / lanes per edge) in a segment-mode launch of config
  * `cfg` with C channels and aligned operands; 0 if there is no such launch.  Host only. */
 int cgtp_uvu_slots(int cfg, int dtype, int C, int backward);

@@ -1,0 +1,187 @@
+"""The matrix-core segment kernels of small tables that are not compiled in (``cgtp_uvu_mx_fwd`` / ``_bwd``): the walk
+the host builds for them, read back word by word on the CPU, and the kernels at the edges of their range."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_close, stable_seed
+from oracle import ref_ops
+
+# (out, in1, in2): several multiplicities, one row only, 16 rows on either side, 32 rows of y, an uncoupled middle
+TABLES = [
+    ("1o+2e+1e", "0e+1o+2e", "0e+1o"),
+    ("0e+1o+2e+3o", "1o+2e+3o", "0e+1o+2e"),
+    ("2x0e+1o+1e", "0e+2x1o", "0e+1o+1e"),
+    ("0e", "0e", "0e+0e"),
+    ("0e+1e+2e+3e", "0e+1o+2e+3o", "0e+1o"),
+    ("1o+3o", "0e+3o", "0e+1o+2e+3o+4e"),
+]
+
+
+def _info(irreps):
+    from equitorch_amd.nn import SO3Linear
+    io, i1, i2 = irreps
+    return SO3Linear(i1, i2, io, 4, 4, internal_weights=False, feature_mode="uu").tp_info_forward
+
+
+@pytest.mark.parametrize("irreps", TABLES)
+def test_the_walk_covers_the_table(irreps):
+    """Forward and the three gradients of one edge, computed from the words alone with the kernels' index arithmetic,
+    against the table's entries."""
+    from equitorch_amd.ops import kernels
+    coo = kernels.coo_of(_info(irreps))
+    m = kernels.uvu_mx_words(coo)
+    assert m is not None
+    rng = np.random.default_rng(stable_seed("mx walk", irreps))
+    D1, D2, DO, P, C = coo.D1, coo.D2, coo.DO, coo.P, 3
+    x, y, w, g = (rng.standard_normal(s) for s in ((D1, C), (D2,), (P, C), (DO, C)))
+    want = {"out": np.zeros((DO, C)), "gx": np.zeros((D1, C)), "gy": np.zeros(D2), "gw": np.zeros((P, C))}
+    for c, M, a, b, p in zip(coo.coef, coo.M, coo.M1, coo.M2, coo.p):
+        c = float(np.float32(c))
+        want["out"][M] += c * x[a] * y[b] * w[p]
+        want["gx"][a] += c * g[M] * y[b] * w[p]
+        want["gy"][b] += c * (g[M] * x[a] * w[p]).sum()
+        want["gw"][p] += c * g[M] * x[a] * y[b]
+
+    def f32(v):
+        return float(np.uint32(v).view(np.float32))
+
+    def couple(words, n_rec, n_ent):
+        A = np.zeros(64 * n_ent + 4)
+        for c0, c1, k in words[:3 * n_rec].reshape(-1, 3):
+            A[k >> 16] = f32(c0) * y[k & 255] + f32(c1) * y[(k >> 8) & 255]
+        return A, words[3 * n_rec:3 * n_rec + n_ent]
+
+    def contract(A, entries, rows):
+        rows = np.concatenate([rows, np.zeros((3, C))])
+        acc = np.zeros((16, C))
+        for e, k in enumerate(entries):
+            b = w[k & 255] * rows[(k >> 8):(k >> 8) + 4]
+            acc += A[64 * e:64 * e + 64].reshape(4, 16).T @ b
+        return acc
+    A, entries = couple(m["fwd"], m["fwd_records"], m["fwd_entries"])
+    got = {"out": contract(A, entries, x)[:DO]}
+    A, entries = couple(m["bwd"], m["bwd_records"], m["bwd_entries"])
+    got["gx"] = contract(A, entries, g)[:D1]
+    at = 3 * m["bwd_records"] + m["bwd_entries"]
+    rows = m["bwd"][at:at + 16 * m["row_tiles"]]
+    at += 16 * m["row_tiles"]
+    xz = np.concatenate([x, np.zeros((16 - D1, C))])
+    G = np.concatenate([(w[k & 255] * g[k >> 8]) @ xz.T for k in rows])
+    terms = m["bwd"][at:at + 128 * m["rounds"]].reshape(-1, 64, 2)
+    at += 128 * m["rounds"]
+    lanes = np.array([sum(f32(t[lane, 0]) * G[t[lane, 1]] for t in terms) for lane in range(64)])
+    assert D2 << m["lanes_log2"] <= 64
+    got["gy"] = lanes.reshape(-1, 1 << m["lanes_log2"]).sum(1)[:D2]
+    gw = np.full((P, C), np.nan)
+    gz = np.concatenate([g, np.zeros((3, C))])
+    for tile in m["bwd"][at:at + 5 * m["tiles"]].reshape(-1, 5):
+        seen = set()
+        for k in tile[1:]:
+            n, p = int(k >> 25), int((k >> 16) & 255)
+            if n == 0:
+                continue
+            assert p not in seen
+            seen.add(p)
+            v = np.zeros(C)
+            for i in range(n):
+                r0 = int(tile[0] & 255)
+                D = sum(A[(k & 0xffff) + 64 * s + 16 * q + i] * gz[r0 + 4 * s + q]
+                        for s in range(int(tile[0] >> 8)) for q in range(4))
+                v += x[(k & 15) + i] * D
+            gw[p] = v + gw[p] if k & (1 << 24) else v
+    got["gw"] = gw
+    for name in want:
+        np.testing.assert_allclose(got[name], want[name], rtol=0, atol=1e-12 * max(1, np.abs(want[name]).max()), err_msg=name)
+
+
+def test_tables_that_do_not_fit_are_left_to_the_general_walk():
+    from equitorch_amd.ops import kernels
+    assert kernels.uvu_mx_words(kernels.coo_of(_info(("0e+1e+2e+4e", "0e+1o+2e", "0e+1o+2e")))) is None      # 18 rows
+    assert kernels.uvu_mx_words(kernels.coo_of(_info(("0e+2e", "0e+4e+2e+3o", "0e+2e")))) is None             # 22 rows
+
+
+def test_struct_layout():
+    import ctypes as C
+    from equitorch_amd import _lib
+    n = _lib.lib.cgtp_abi_layout(12, None, 0)
+    buf = (C.c_int64 * n)()
+    assert _lib.lib.cgtp_abi_layout(12, buf, n) == n == 1 + len(_lib.UvuMx._fields_)
+    assert buf[0] == C.sizeof(_lib.UvuMx)
+    assert list(buf)[1:] == [getattr(_lib.UvuMx, name).offset for name, _ in _lib.UvuMx._fields_]
+
+
+def _edge_case(irreps, channels, n_nodes, n_edges, hub, seed):
+    from equitorch_amd.irreps import Irreps
+    io, i1, i2 = irreps
+    gen = torch.Generator().manual_seed(seed)
+    src = torch.randint(0, n_nodes, (n_edges,), generator=gen)
+    dst = torch.randint(0, n_nodes, (n_edges,), generator=gen)
+    if hub:
+        dst[torch.rand(n_edges, generator=gen) < 0.4] = 1
+        src[src == 2], dst[dst == 2] = 0, 0
+    P = len(set(_paths(irreps)))
+    return (src, dst, torch.randn(n_nodes, Irreps(i1).dim, channels, generator=gen),
+            torch.randn(n_edges, Irreps(i2).dim, generator=gen), torch.randn(n_edges, P, channels, generator=gen),
+            torch.randn(n_nodes, Irreps(io).dim, channels, generator=gen))
+
+
+def _paths(irreps):
+    from equitorch_amd.ops import kernels
+    return kernels.coo_of(_info(irreps)).p.tolist()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("irreps", TABLES)
+@pytest.mark.parametrize("channels,n_nodes,n_edges,hub", [(64, 5, 1, False), (60, 40, 700, True), (48, 3, 9000, False),
+                                                          (32, 300, 2049, True), (18, 50, 600, False), (16, 70, 900, False),
+                                                          (5, 30, 400, True), (36, 3000, 2500, False)])
+def test_product_and_gradients(device, irreps, channels, n_nodes, n_edges, hub):
+    """One, two and four channels per lane with and without idle lanes; one edge, ranges of more than 64 positions,
+    nodes without edges, a node whose edges span many ranges; every subset of gradients the kernels tell apart."""
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    info = _info(irreps).to(device)
+    src, dst, x, y, w, ct = _edge_case(irreps, channels, n_nodes, n_edges, hub, stable_seed("mx", irreps, channels))
+    plan = EdgePlan(src.to(device), dst.to(device), n_nodes)
+    T = ref_ops.dense_coupling(*irreps).float().double()
+
+    def ref_fn(T, x, sh, w):
+        return ref_ops.scatter_sum(ref_ops.dense_u1u(T, x.index_select(0, src), sh, w), dst, n_nodes)
+    ref_out, ref_grads = ref_ops.dense_grads(ref_fn, T, (x, y, w), ct)
+    for need in ((True, True, True), (False, True, False), (True, False, False), (False, False, True)):
+        wrt = [t.to(device).requires_grad_(n) for t, n in zip((x, y, w), need)]
+        out = edge_tensor_product_uu(*wrt, plan, info)
+        grads = torch.autograd.grad(out, [t for t, n in zip(wrt, need) if n], ct.to(device))
+        assert_close(out, ref_out, 1e-5, f"{irreps} C={channels} out", norm="max")
+        for name, got, want in zip([k for k, n in zip("xyw", need) if n], grads, [r for r, n in zip(ref_grads, need) if n]):
+            assert_close(got, want, 1e-5, f"{irreps} C={channels} grad {name} of {need}", norm="max")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["x", "y", "w", "ct"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 1e38])
+def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, where, value):
+    """An infinity, a NaN or a product that overflows: the results are those of the entry-by-entry kernels, in which a row
+    reaches only the rows it couples to."""
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    from equitorch_amd.ops import kernels
+    irreps = TABLES[1]
+    src, dst, x, y, w, ct = _edge_case(irreps, 32, 40, 500, False, 7)
+    {"x": x, "y": y, "w": w, "ct": ct}[where].view(-1)[123] = value
+    if value == 1e38:
+        {"x": x, "y": y, "w": w, "ct": ct}[where].mul_(10)
+    plan = EdgePlan(src.to(device), dst.to(device), 40)
+    results = {}
+    for route in ("matrix", "entries"):
+        info = _info(irreps).to(device)
+        if route == "entries":
+            monkeypatch.setattr(kernels, "uvu_mx_words", lambda coo: None)
+        wrt = [t.to(device).requires_grad_(True) for t in (x, y, w)]
+        out = edge_tensor_product_uu(*wrt, plan, info)
+        assert (kernels.uvu_table_of(info, wrt[0].device).mx is None) == (route == "entries")
+        results[route] = (out, *torch.autograd.grad(out, wrt, ct.to(device)))
+    for a, b in zip(results["matrix"], results["entries"]):
+        fin = torch.isfinite(b)
+        assert torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
+        # in a range without a value that is not finite the sums run in another order: norm-wise
+        assert float((a[fin] - b[fin]).detach().abs().max()) <= 1e-5 * float(b[fin].abs().max())
