@@ -33,10 +33,15 @@ CONFIGS = OrderedDict([
 ])
 
 
-def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = False) -> str:
+# Tables of the single-precision product on the half-precision matrix cores (uv_split.hip).
+SPLIT_CONFIGS = ("sh1", "sh2", "sh3")
+
+
+def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = False, split: bool = False) -> str:
     """Body of one configuration.  ``gy``: instead of accumulating output rows, contract every tile with the rows of
     a second channelled operand ``g`` (the output gradient) into the gradient w.r.t. the harmonics,
-    ``gy[b] += coef * sum_w g[m, w] * Z[w]`` (forward tables only)."""
+    ``gy[b] += coef * sum_w g[m, w] * Z[w]`` (forward tables only).  ``split``: the body for single precision, in which
+    the operands' fragments and the contraction are the caller's (``Ops``) and every tile comes with a factor per lane."""
     if direction == 0:
         out_idx, in_idx, blocks, din, dout = coo.M, coo.M1, seg_out, coo.D1, coo.DO
     else:
@@ -68,11 +73,18 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
             run_of_tile[k] = j
     L = []
     a = L.append
-    a(f"struct UV_{name}_{'gy' if gy else 'd' + str(direction)} {{")
+    store, load_g, load_a = ("sink", "sink", "ops.load_a") if split else ("store", "load_g", "load_a")
+    a(f"struct UV{'S' if split else ''}_{name}_{'gy' if gy else 'd' + str(direction)} {{")
     a(f"  static constexpr int DIN = {din}, DOUT = {dout}, D2 = {coo.D2}, P = {coo.P};")
-    a("  // xs: this lane's base into the staged input tile (row a of the sample at byte a * CIN * 2);")
-    a("  // load_a(p, frag): fetch the weight fragments of path p;")
-    if gy:
+    if not split:
+        a("  // xs: this lane's base into the staged input tile (row a of the sample at byte a * CIN * 2);")
+        a("  // load_a(p, frag): fetch the weight fragments of path p;")
+    if split:
+        a("  // ops: load_a(p, A&), load_b(row, B&), chain(A, B, z0, z1), scale(p, row): the factor of the tile;")
+        a("  // sink: store(row, t0, t1) emits a finished output row / load_g(row, t0, t1) this lane's channels of g")
+        a("  template <class Ops, class Sink>")
+        a(f"  __device__ __forceinline__ static void run(const Ops& ops, {'' if gy else 'const '}float (&y)[D2], Sink&& sink) {{")
+    elif gy:
         a("  // load_g(row, t0, t1): this lane's 8 channels of row `row` of g; y receives this lane's partial sums.")
         a("  template <int CIN, class LoadA, class LoadG>")
         a("  __device__ __forceinline__ static void run(const unsigned char* xs, LoadA&& load_a, float (&y)[D2],")
@@ -82,8 +94,13 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         a("  template <int CIN, class LoadA, class Store>")
         a("  __device__ __forceinline__ static void run(const unsigned char* xs, LoadA&& load_a, const float (&y)[D2],")
         a("                                             Store&& store) {")
-    a("    constexpr int KS = CIN / 32;")
-    a("    bf16x8 w0[2][KS], w1[2][KS], w2[2][KS], b0[KS], b1[KS];")
+    if split:
+        a("    typename Ops::A w0, w1, w2;")
+        a("    typename Ops::B b0, b1;")
+        a("    float fa = 0.f, fb = 0.f;")
+    else:
+        a("    constexpr int KS = CIN / 32;")
+        a("    bf16x8 w0[2][KS], w1[2][KS], w2[2][KS], b0[KS], b1[KS];")
     a("    floatx4 za0, za1, zb0, zb1;")
     a("    float yy[D2];")
     a("    for (int j = 0; j < D2; ++j) yy[j] = " + ("0.f;" if gy else "y[j];"))
@@ -91,23 +108,30 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         a("    {")
         a("      floatx4 zero = {0};")
         for r in empty_rows:
-            a(f"      store({r}, zero, zero);")
+            a(f"      {store}({r}, zero, zero);")
         a("    }")
 
     def load_b(k):
+        if split:
+            a(f"    ops.load_b({tiles[k][0][1]}, b{k % 2});")
+            return
         a(f"    load_b<KS>(b{k % 2}, xs + {tiles[k][0][1]} * CIN * 2);")
 
     def chain(k):
         z = "za" if k % 2 == 0 else "zb"
-        a(f"    mfma_chain<KS>(w{run_of_tile[k] % 3}, b{k % 2}, {z}0, {z}1);")
+        if split:
+            a(f"    ops.chain(w{run_of_tile[k] % 3}, b{k % 2}, {z}0, {z}1); "
+              f"f{z[1]} = ops.scale({tiles[k][0][0]}, {tiles[k][0][1]});")
+        else:
+            a(f"    mfma_chain<KS>(w{run_of_tile[k] % 3}, b{k % 2}, {z}0, {z}1);")
         j = run_of_tile[k]
         if runs[j][1] == k and j + 2 < len(runs):
-            a(f"    load_a({runs[j + 2][0]}, w{(j + 2) % 3});")
+            a(f"    {load_a}({runs[j + 2][0]}, w{(j + 2) % 3});")
 
     if tiles:
-        a(f"    load_a({runs[0][0]}, w0);")
+        a(f"    {load_a}({runs[0][0]}, w0);")
         if len(runs) > 1:
-            a(f"    load_a({runs[1][0]}, w1);")
+            a(f"    {load_a}({runs[1][0]}, w1);")
         load_b(0)
         if len(tiles) > 1:
             load_b(1)
@@ -119,7 +143,7 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         if k in first_of_block:
             for r in first_of_block[k]:
                 if gy:
-                    a(f"    floatx4 o{r}_0, o{r}_1; load_g({r}, o{r}_0, o{r}_1);")
+                    a(f"    floatx4 o{r}_0, o{r}_1; {load_g}({r}, o{r}_0, o{r}_1);")
                 else:
                     a(f"    floatx4 o{r}_0 = {{0}}, o{r}_1 = {{0}};")
         if k + 1 < len(tiles):
@@ -127,9 +151,10 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         if k + 2 < len(tiles):
             load_b(k + 2)
         cur = "za" if k % 2 == 0 else "zb"
+        factor = f" * f{cur[1]}" if split else ""
         if gy:
             for (o, m2, c) in terms:
-                a(f"    yy[{m2}] += {_lit(c)} * dot8(o{o}_0, o{o}_1, {cur}0, {cur}1);")
+                a(f"    yy[{m2}] += {_lit(c)}{factor} * dot8(o{o}_0, o{o}_1, {cur}0, {cur}1);")
             # pin the partial sums (see the accumulators of the forward body)
             a("    asm volatile(\"\" : " + ", ".join(f'"+v"(yy[{m}])' for m in sorted({m2 for _, m2, _ in terms})) + ");")
             a("    __builtin_amdgcn_sched_barrier(0);")
@@ -143,6 +168,8 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
             by_row.setdefault(o, []).append((m2, c))
         for o, pairs in by_row.items():
             s_expr = " + ".join(f"{_lit(c)} * yy[{m2}]" for m2, c in pairs)
+            if split:
+                s_expr = f"({s_expr}){factor}"
             a(f"    {{ const float s = {s_expr}; o{o}_0 += s * {cur}0; o{o}_1 += s * {cur}1; }}")
         # pin the updated accumulators: an output row is read again only when it is stored, and without this the
         # optimiser sinks every update of a block to its end, keeping all the block's tiles alive until then
@@ -152,7 +179,7 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         a("    __builtin_amdgcn_sched_barrier(0);")
         if k in last_of_block:
             for r in last_of_block[k]:
-                a(f"    store({r}, o{r}_0, o{r}_1);")
+                a(f"    {store}({r}, o{r}_0, o{r}_1);")
     if gy:
         a("    for (int j = 0; j < D2; ++j) y[j] = yy[j];")
     a("  }")
@@ -213,6 +240,36 @@ def emit_gw(name: str, coo, seg_out, seg_in1) -> str:
     return "\n".join(L)
 
 
+def emit_split(out_dir: str) -> str:
+    """``generated/uv_split_configs.inc``: the single-precision bodies, and every table as a list of terms."""
+    chunks = ["// Generated by equitorch_amd/csrc/gen_uv.py; do not edit.", ""]
+    names = SPLIT_CONFIGS
+    for name in names:
+        io, i1, i2, kw = CONFIGS[name]
+        coo = tp_coo(tp_infos(Irreps(io), Irreps(i1), Irreps(i2), **kw)[0])
+        seg_out, seg_in1 = irrep_segments(Irreps(io)), irrep_segments(Irreps(i1))
+        for d in (0, 1):
+            chunks.append(emit_direction(name, d, coo, seg_out, seg_in1, split=True))
+        chunks.append(emit_direction(name, 0, coo, seg_out, seg_in1, gy=True, split=True))
+        terms = ", ".join(f"{{{_lit(coo.coef[t])}, {coo.M[t]}, {coo.M1[t]}, {coo.M2[t]}, {coo.p[t]}}}"
+                          for t in range(coo.coef.shape[0]))
+        chunks.append(f"static __device__ const UvsTerm UVS_{name}_terms[] = {{{terms}}};")
+        chunks.append(f"struct UVS_{name}_table {{")
+        chunks.append(f"  static constexpr int N = {coo.coef.shape[0]};")
+        chunks.append(f"  __device__ __forceinline__ static const UvsTerm* terms() {{ return UVS_{name}_terms; }}")
+        chunks.append("};")
+        chunks.append("")
+    chunks.append("#define CGTP_FOREACH_UVS_CONFIG(X) \\")
+    chunks.append(" \\\n".join(f"  X({list(CONFIGS).index(n)}, UVS_{n}_d0, UVS_{n}_d1, UVS_{n}_gy, UVS_{n}_table)"
+                              for n in names))
+    chunks.append("")
+    path, text = os.path.join(out_dir, "uv_split_configs.inc"), "\n".join(chunks)
+    if not os.path.exists(path) or open(path).read() != text:
+        with open(path, "w") as f:
+            f.write(text)
+    return path
+
+
 def main(out_dir: str = None) -> str:
     out_dir = out_dir or os.path.join(HERE, "generated")
     os.makedirs(out_dir, exist_ok=True)
@@ -240,6 +297,7 @@ def main(out_dir: str = None) -> str:
     if not os.path.exists(path) or open(path).read() != text:
         with open(path, "w") as f:
             f.write(text)
+    emit_split(out_dir)
     return path
 
 

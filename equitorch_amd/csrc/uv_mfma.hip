@@ -12,8 +12,7 @@
 // (2l+1) * 8 registers; the whole wavefront fits 256 registers, so two workgroups share a compute unit and one
 // stages its input while the other computes.  The staged rows are padded by 16 bytes per sample so that the 16
 // lanes of one LDS phase hit distinct banks.
-#include "cgtp_device.h"
-#include "cgtp_host.h"
+#include "uv_common.h"
 
 // accumulator-tile updates are written as o += s * z; let them contract to FMAs in this file
 #pragma clang fp contract(fast)
@@ -21,7 +20,6 @@
 namespace cgtp {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -44,13 +42,6 @@ __device__ __forceinline__ void mfma_chain(const bf16x8 (&a)[2][KS], const bf16x
     z0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][k], b[k], z0, 0, 0, 0);
     z1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1][k], b[k], z1, 0, 0, 0);
   }
-}
-
-__device__ __forceinline__ float dot8(const floatx4& g0, const floatx4& g1, const floatx4& z0, const floatx4& z1) {
-  float s = g0[0] * z0[0];
-  s += g0[1] * z0[1]; s += g0[2] * z0[2]; s += g0[3] * z0[3];
-  s += g1[0] * z1[0]; s += g1[1] * z1[1]; s += g1[2] * z1[2]; s += g1[3] * z1[3];
-  return s;
 }
 
 #include "generated/uv_configs.inc"

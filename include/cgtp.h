@@ -390,6 +390,20 @@ int64_t cgtp_uv_grad_w_workspace_bytes(int cfg, int64_t n_rows, int32_t cin, int
 int cgtp_uv_grad_w(int cfg, const void* x, const void* y, const void* g, void* gw, void* workspace, int64_t n_rows,
                    int32_t cin, int32_t cout, int32_t dtype, const float* path_scale, void* stream);
 
+/* The fully connected product of a compiled table (cfg as above) in single precision on the half-precision matrix cores,
+ * every fp32 operand carried as two halves (no less precise than fp32 matrix instructions).  kind 0: forward, x
+ * (n_rows, D1, cin), y (n_rows, D2), out (n_rows, DO, cout); 1: gradient of x, `x` = grad_out (n_rows, DO, cin), out
+ * (n_rows, D1, cout); 2: gradient of y, y = grad_out (n_rows, DO, cout), out (n_rows, D2), cout <= 128.  cin 32, 64 or
+ * 128, cout a multiple of 32.  w: the weight (P, contracted, produced) for kinds 0 and 2, (P, produced, contracted) for
+ * kind 1, contiguous; packed: cgtp_uvs_packed_bytes() bytes filled by cgtp_uvs_pack_weights (transposed for kind 1). */
+int64_t cgtp_uvs_packed_bytes(int32_t n_paths, int32_t cin, int32_t cout);
+int cgtp_uvs_pack_weights(const float* w, void* packed, int32_t n_paths, int32_t cin, int32_t cout, int32_t transposed,
+                          void* stream);
+int cgtp_uvs_validate(int cfg, int kind, const void* x, const void* y, const void* packed, const void* w, const void* out,
+                      int64_t n_rows, int32_t cin, int32_t cout);
+int cgtp_uvs_apply(int cfg, int kind, const void* x, const void* y, const void* packed, const void* w, void* out,
+                   int64_t n_rows, int32_t cin, int32_t cout, void* stream);
+
 /* ---- radial basis and cutoff envelopes ---------------------------------------------------------------------------
  *
  * Element-wise functions of the edge length r (n values), fp32 / fp64, one launch forward and one for the gradient.

@@ -1,0 +1,81 @@
+"""The fully connected product of the compiled tables in fp32 on the half-precision matrix cores (``cgtp_uvs_apply``): every
+operand carried as two halves, no less precise than fp32 matrix instructions."""
+import pytest
+import torch
+
+from helpers import stable_seed
+from oracle import ref_ops
+
+pytestmark = pytest.mark.gpu
+SH = {1: "0e+1o", 2: "0e+1o+2e", 3: "0e+1o+2e+3o"}
+
+
+def _operands(device, lmax, cin, cout, n, seed):
+    from equitorch_amd.nn import SO3Linear
+    mod = SO3Linear(SH[lmax], SH[lmax], SH[lmax], cin, cout, internal_weights=False, feature_mode="uv").to(device)
+    d = (lmax + 1) ** 2
+    gen = torch.Generator().manual_seed(seed)
+    return mod, [torch.randn(n, d, cin, generator=gen), torch.randn(n, d, generator=gen),
+                 torch.randn(mod.num_paths, cin, cout, generator=gen) * (cin * mod.num_paths) ** -0.5,
+                 torch.randn(n, d, cout, generator=gen)]
+
+
+def _step(mod, device, x, y, w, ct):
+    wrt = [t.to(device).requires_grad_(True) for t in (x, y, w)]
+    out = mod(*wrt)
+    return [t.detach() for t in (out, *torch.autograd.grad(out, wrt, ct.to(device)))]
+
+
+def _both_routes(monkeypatch, mod, device, operands):
+    from equitorch_amd.nn.functional import _uv_native
+    results, kinds, split = {}, [], _uv_native._split
+
+    def spy(kind, *args):
+        out = split(kind, *args)
+        kinds.append((kind, out is not None))
+        return out
+    monkeypatch.setattr(_uv_native, "_split", spy)
+    results["split"] = _step(mod, device, *operands)
+    assert sorted(kinds) == [(0, True), (1, True), (2, True)], kinds
+    monkeypatch.setattr(_uv_native, "_split", lambda *args: None)
+    results["fp32"] = _step(mod, device, *operands)
+    return results["split"], results["fp32"]
+
+
+@pytest.mark.parametrize("lmax,cin,cout,n", [(1, 32, 32, 1), (1, 128, 64, 17), (2, 64, 32, 33), (2, 128, 128, 300),
+                                             (3, 32, 128, 47), (3, 64, 64, 1000), (3, 128, 128, 555)])
+@pytest.mark.parametrize("values", ["normal", "wide"])
+def test_no_less_precise_than_fp32_matrix_instructions(device, monkeypatch, lmax, cin, cout, n, values):
+    """Both routes against the dense float64 oracle, ragged batches and every tile width; ``wide``: rows of x, paths of W
+    and single elements spread over twenty binary orders of magnitude."""
+    mod, ops = _operands(device, lmax, cin, cout, n, stable_seed("split", lmax, cin, cout, n))
+    if values == "wide":
+        gen = torch.Generator().manual_seed(3)
+        for t in ops:
+            lead = (t.shape[0],) + (1,) * (t.ndim - 1)
+            t.mul_(torch.exp2(torch.randint(-20, 21, lead, generator=gen).float()))
+        ops[0].mul_(torch.exp2(torch.randint(-10, 11, ops[0].shape, generator=gen).float()))
+    split, fp32 = _both_routes(monkeypatch, mod, device, ops)
+    T = ref_ops.dense_coupling(SH[lmax], SH[lmax], SH[lmax]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_u1v, T, ops[:3], ops[3])
+    for k, (name, want) in enumerate(zip(("out", "grad x", "grad y"), (ref_out, *ref_grads[:2]))):
+        # row by row: a row's error against its own size
+        def err(a):
+            d, w = (a.cpu().double() - want).flatten(1).norm(dim=1), want.flatten(1).norm(dim=1)
+            return float((d / w.clamp_min(1e-30)).square().mean().sqrt())
+        e_split, e_fp32 = err(split[k]), err(fp32[k])
+        print(f"{name} lmax={lmax} {cin}->{cout} n={n} {values}: split {e_split:.2e} fp32 {e_fp32:.2e}")
+        # one sample's rounding errors are a handful of draws: a factor of two between two orders of summation
+        assert e_split <= (1.1 if n >= 300 else 2.0) * e_fp32 + 3e-8, name
+
+
+@pytest.mark.parametrize("where,value", [(0, float("inf")), (0, float("nan")), (2, float("inf")), (2, float("nan")), (3, float("-inf")),
+                                         (0, 3e38), (2, 1e25), (1, float("inf"))])
+def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, where, value):
+    mod, ops = _operands(device, 2, 64, 64, 100, 5)
+    ops[where].view(-1)[567] = value
+    split, fp32 = _both_routes(monkeypatch, mod, device, ops)
+    for a, b in zip(split, fp32):
+        fin = torch.isfinite(b)
+        assert torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
+        assert float((a[fin] - b[fin]).norm()) <= 1e-6 * float(b[fin].norm())
