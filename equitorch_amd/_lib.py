@@ -72,7 +72,7 @@ class UvuMx(C.Structure):
     _fields_ = [("fwd", C.c_void_p), ("bwd", C.c_void_p),
                 ("fwd_records", C.c_int32), ("fwd_entries", C.c_int32), ("bwd_records", C.c_int32),
                 ("bwd_entries", C.c_int32), ("row_tiles", C.c_int32), ("rounds", C.c_int32), ("lanes_log2", C.c_int32),
-                ("tiles", C.c_int32)]
+                ("tiles", C.c_int32), ("bwd4", C.c_void_p), ("bwd4_items", C.c_int32), ("bwd4_chunks", C.c_int32)]
 
 
 class PswTable(C.Structure):

@@ -637,7 +637,9 @@ int cgtp_abi_layout(int which, int64_t* out, int capacity) {
                                    CGTP_OFF(cgtp_uvu_mx, fwd_records), CGTP_OFF(cgtp_uvu_mx, fwd_entries),
                                    CGTP_OFF(cgtp_uvu_mx, bwd_records), CGTP_OFF(cgtp_uvu_mx, bwd_entries),
                                    CGTP_OFF(cgtp_uvu_mx, row_tiles), CGTP_OFF(cgtp_uvu_mx, rounds),
-                                   CGTP_OFF(cgtp_uvu_mx, lanes_log2), CGTP_OFF(cgtp_uvu_mx, tiles)};
+                                   CGTP_OFF(cgtp_uvu_mx, lanes_log2), CGTP_OFF(cgtp_uvu_mx, tiles),
+                                   CGTP_OFF(cgtp_uvu_mx, bwd4), CGTP_OFF(cgtp_uvu_mx, bwd4_items),
+                                   CGTP_OFF(cgtp_uvu_mx, bwd4_chunks)};
 #undef CGTP_OFF
   const int64_t* tabs[] = {operand, tri, gen_operand, gen, uvu, uvt_item, uvt, uvt_gw, uvt_gy, uvu_tab, psw_table,
                            psw_args, uvu_mx};

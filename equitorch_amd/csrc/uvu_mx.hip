@@ -40,7 +40,7 @@ constexpr int kMxMaxPaths = 32;
 // Words of the device tables (built by the host, see cgtp_uvu_mx in cgtp.h), copied to LDS by every workgroup.
 struct MxDev {
   const uint32_t* words;
-  int n_words, n_rec, n_ent, n_rowtiles, n_rounds, lanes_log2, n_tiles;
+  int n_words, n_rec, n_ent, n_rowtiles, n_rounds, lanes_log2, n_tiles, n_chunks;
   int D1, D2, DO, P;
   int32_t* flags;      // one word per range: 1 = a result was not finite
 };
@@ -191,6 +191,49 @@ __device__ __forceinline__ void mx_flush(mx4 (&acc)[NJ], float* dst, int D, int6
   }
 }
 
+// One tile of G: sum over the channels of (w g)[row of this lane] x[.]; wr, gr: the lane's rows at channel 4 g.
+template <int NJ>
+__device__ __forceinline__ mx4 mx_channels(const float* wr, const float* gr, const float (&xt)[NJ][4]) {
+  mx4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < NJ; ++q) {
+    float wq[4], gq[4];
+    mx_get<4>(wq, wr + 16 * q);
+    mx_get<4>(gq, gr + 16 * q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z = __builtin_amdgcn_mfma_f32_16x16x4f32(wq[i] * gq[i], xt[q][i], z, 0, 0, 0);
+  }
+  return z;
+}
+// grad_y of edge e from G in LDS; 1 << lanes_log2 lanes share a component.
+__device__ __forceinline__ void mx_grad_y(const UvuDev<float>& a, const MxDev& t, const uint32_t* terms, const float* G, int64_t e,
+                                          int lane, float& bad) {
+  float sum = 0.f;
+  for (int u = 0; u < t.n_rounds; ++u) {
+    const uint32_t* term = terms + 2 * (u * kWave + lane);
+    sum = fmaf(__builtin_bit_cast(float, term[0]), G[term[1]], sum);
+  }
+  for (int off = 1; off < (1 << t.lanes_log2); off <<= 1) sum += shfl_xor(sum, off);
+  const int b = lane >> t.lanes_log2;
+  bad = fmaf(sum, 0.f, bad);
+  if ((lane & ((1 << t.lanes_log2) - 1)) == 0 && b < t.D2) a.gy[e * t.D2 + b] = sum;
+}
+// The weight gradient of edge e from its rows in LDS.
+template <int NJ, int WR>
+__device__ __forceinline__ void mx_store_grad_w(const UvuDev<float>& a, const MxDev& t, const float* rows, int pitch, int64_t e,
+                                                int g, int c0, bool c_ok, float& bad) {
+#pragma unroll
+  for (int i = 0; i < WR; ++i) {
+    if (4 * i + g < t.P) {
+      float v[NJ];
+      mx_get<NJ>(v, rows + (4 * i + g) * pitch + c0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) bad = fmaf(v[j], 0.f, bad);
+      if (c_ok) store_vec_stream<float, NJ>(a.gw + (e * t.P + 4 * i + g) * a.C + c0, v);
+    }
+  }
+}
+
 // First position past the range, and whether its first / last segment lie wholly inside it.
 struct MxRange {
   int64_t p0, p1;
@@ -337,18 +380,7 @@ __global__ void __launch_bounds__(512) uvu_mx_bwd_kernel(const UvuDev<float> a, 
       for (int s = 0; s < kMxMaxPaths / 4; ++s) {
         if (s < t.n_rowtiles) {
           const uint32_t rw = tab[parts.row + 16 * s + r];
-          const float* wr = ws + (rw & 255) * pitch + 4 * g;
-          const float* gr = gs + (rw >> 8) * pitch + 4 * g;
-          mx4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int q = 0; q < NJ; ++q) {
-            float wq[4], gq[4];
-            mx_get<4>(wq, wr + 16 * q);
-            mx_get<4>(gq, gr + 16 * q);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) z = __builtin_amdgcn_mfma_f32_16x16x4f32(wq[i] * gq[i], xt[q][i], z, 0, 0, 0);
-          }
-          G[s] = z;
+          G[s] = mx_channels<NJ>(ws + (rw & 255) * pitch + 4 * g, gs + (rw >> 8) * pitch + 4 * g, xt);
         }
       }
       mx_sync();            // the weight rows are consumed: G takes their place
@@ -360,16 +392,7 @@ __global__ void __launch_bounds__(512) uvu_mx_bwd_kernel(const UvuDev<float> a, 
         }
       }
       mx_sync();
-      // 1 << lanes_log2 lanes share a component of y
-      float sum = 0.f;
-      for (int u = 0; u < t.n_rounds; ++u) {
-        const uint32_t* term = tab + parts.term + 2 * (u * kWave + lane);
-        sum = fmaf(__builtin_bit_cast(float, term[0]), ws[term[1]], sum);
-      }
-      for (int off = 1; off < (1 << t.lanes_log2); off <<= 1) sum += shfl_xor(sum, off);
-      const int b = lane >> t.lanes_log2;
-      bad = fmaf(sum, 0.f, bad);
-      if ((lane & ((1 << t.lanes_log2) - 1)) == 0 && b < t.D2) a.gy[e * t.D2 + b] = sum;
+      mx_grad_y(a, t, tab + parts.term, ws, e, lane, bad);
       mx_sync();
     }
     if (want_gw) {          // the weight gradient is gathered in the weight rows' place
@@ -414,16 +437,7 @@ __global__ void __launch_bounds__(512) uvu_mx_bwd_kernel(const UvuDev<float> a, 
         }
       }
       mx_sync();
-#pragma unroll
-      for (int i = 0; i < WR; ++i) {
-        if (4 * i + g < t.P) {
-          float v[NJ];
-          mx_get<NJ>(v, ws + (4 * i + g) * pitch + c0);
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) bad = fmaf(v[j], 0.f, bad);
-          if (c_ok) store_vec_stream<float, NJ>(a.gw + (e * t.P + 4 * i + g) * C + c0, v);
-        }
-      }
+      mx_store_grad_w<NJ, WR>(a, t, ws, pitch, e, g, c0, c_ok, bad);
       mx_sync();
     }
   }
@@ -432,11 +446,237 @@ __global__ void __launch_bounds__(512) uvu_mx_bwd_kernel(const UvuDev<float> a, 
   if (lane == 0) t.flags[range] = any_bad;
 }
 
+// ---- backward, one channel per lane (33 to 64 channels) ----------------------------------------------------------
+// A path couples 2 l + 1 of up to 16 rows, so three quarters of a 16-row tile multiply zeros.  v_mfma_f32_4x4x1_16b_f32 takes
+// 16 blocks of four channels times four rows and one contracted row in 8 cycles, with A broadcast from one block to
+// all: no padding of the contracted rows, none of the tile beyond the multiple of four, and a lane keeps one channel
+// throughout.  The rows of x are cut into chunks of up to four rows of one irrep; an item is a path's share of a chunk, up
+// to seven rows of grad_out; a register of A holds the eight slots of two items.  D = A^T g of an item gives both
+// gradients: grad_x += w D and grad_w = sum over the rows of x D.  At 206 coefficients about 115 such instructions
+// replace 136 of 32 cycles per edge; G, whose contraction runs over the channels, stays on 16 x 16 x 4.  65 536 edges, 64
+// channels, 206 coefficients: 453 -> 371 us; 32 768 edges, forward and backward: 350 -> 307 us, 58 coefficients 169 -> 158
+// us.  The forward gains nothing this way (175 -> 180 us; 58 coefficients 47 -> 61): its single contraction waits for
+// two LDS reads per contracted row instead of three per four, so it stays on 16-row tiles.
+constexpr int kMxChunks = 8;
+struct Mx4Parts {
+  int rec, item, chunk, row, term, words;
+  __host__ __device__ Mx4Parts(int n_rec, int n_items, int n_rowtiles, int n_rounds) {
+    rec = 0;
+    item = rec + 3 * n_rec;                 // n_items (even) x (path | first row << 8 | rows << 16 | adds << 20)
+    chunk = item + n_items;                 // kMxChunks x (first row | rows << 8 | end of its pairs of items << 16)
+    row = chunk + kMxChunks;                // as MxParts
+    term = row + 16 * n_rowtiles;
+    words = (term + 128 * n_rounds + 3) & ~3;
+  }
+};
+constexpr int kMx4Pitch = 68;               // LDS row: 64 channels, and 4 for the row-wise reads of G
+struct Mx4Layout {
+  int a, w, r1, e, y, floats;
+  __host__ __device__ Mx4Layout(int D2, int DO, int P, int n_items, int n_rowtiles) {
+    int at = 0;
+    const auto take = [&](int n) { const int r = at; at += (n + 3) & ~3; return r; };
+    a = take(32 * n_items);
+    w = take(P * kMx4Pitch);
+    r1 = take((DO + 6) * kMx4Pitch);                  // an item's seven rows may reach six past the end
+    const int g_floats = 256 * n_rowtiles, gw_floats = P * kMx4Pitch;
+    e = take(g_floats > gw_floats ? g_floats : gw_floats);      // G, then the weight gradient
+    y = take(D2);
+    floats = at;
+  }
+};
+
+// Operands of a pair of items, requested one pair ahead.
+struct Mx4Pair {
+  uint32_t k[2];
+  float a, w[2], r[2][7];
+  __device__ __forceinline__ void request(uint32_t items, int pair, const float* A, const float* ws, const float* rows, int lane) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      k[h] = (uint32_t)__builtin_amdgcn_readlane((int)items, 2 * pair + h);
+      w[h] = ws[(k[h] & 255) * kMx4Pitch + lane];
+      const float* at = rows + ((k[h] >> 8) & 255) * kMx4Pitch + lane;
+#pragma unroll
+      for (int j = 0; j < 7; ++j) r[h][j] = at[j * kMx4Pitch];
+    }
+    a = A[pair * 64 + lane];
+  }
+  __device__ __forceinline__ int rows() const { return max((int)(k[0] >> 16) & 15, (int)(k[1] >> 16) & 15); }
+};
+// z[h] += the slot's four rows times b (A of block 8 h + J broadcast to all blocks)
+template <int J>
+__device__ __forceinline__ void mx4_step(mx4 (&z)[2], float a, float b0, float b1) {
+  z[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, b0, z[0], 4, J, 0);
+  z[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, b1, z[1], 4, 8 + J, 0);
+}
+// b(h, j): the operand of row j of item h
+template <class B>
+__device__ __forceinline__ void mx4_multiply(mx4 (&z)[2], float a, int rows, B&& b) {
+  mx4_step<0>(z, a, b(0, 0), b(1, 0));
+  if (rows > 1) {
+    mx4_step<1>(z, a, b(0, 1), b(1, 1));
+    mx4_step<2>(z, a, b(0, 2), b(1, 2));
+  }
+  if (rows > 3) {
+    mx4_step<3>(z, a, b(0, 3), b(1, 3));
+    mx4_step<4>(z, a, b(0, 4), b(1, 4));
+  }
+  if (rows > 5) {
+    mx4_step<5>(z, a, b(0, 5), b(1, 5));
+    mx4_step<6>(z, a, b(0, 6), b(1, 6));
+  }
+}
+
+__device__ __forceinline__ void mx4_flush(mx4 (&acc)[kMxChunks], uint32_t chunks, int n_chunks, float* dst, int64_t C, int lane,
+                                          float& bad) {
+#pragma unroll
+  for (int c = 0; c < kMxChunks; ++c) {
+    if (c < n_chunks) {
+      const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)chunks, c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bad = fmaf(acc[c][i], 0.f, bad);
+        if (i < (int)((k >> 8) & 255) && lane < C) dst[((k & 255) + i) * C + lane] = acc[c][i];
+      }
+      acc[c] = mx4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+}
+
+template <int WR>
+__global__ void __launch_bounds__(512) uvu_mx4_bwd_kernel(const UvuDev<float> a, const MxDev t) {
+  extern __shared__ __align__(16) float mx_lds[];
+  const Mx4Parts parts(t.n_rec, t.n_ent, t.n_rowtiles, t.n_rounds);
+  uint32_t* tab = reinterpret_cast<uint32_t*>(mx_lds);
+  for (int i = threadIdx.x; i < t.n_words; i += blockDim.x) tab[i] = t.words[i];
+  const Mx4Layout Y(t.D2, t.DO, t.P, t.n_ent, t.n_rowtiles);
+  const int lane = threadIdx.x & (kWave - 1), g = lane >> 4, r = lane & 15, c0 = r * 4;
+  float* mine = mx_lds + parts.words + (threadIdx.x / kWave) * Y.floats;
+  for (int i = lane; i < Y.floats; i += kWave) mine[i] = 0.f;
+  __syncthreads();
+  const int64_t range = seg_wave_index(a.n_waves);
+  if (range < 0) return;
+  const MxRange R(a, range);
+  const int64_t C = a.C;
+  const bool c_ok = c0 < a.C;
+  const bool want_gx = a.gx != nullptr, want_gy = a.gy != nullptr, want_gw = a.gw != nullptr;
+  float *A = mine + Y.a, *ws = mine + Y.w, *gs = mine + Y.r1, *E = mine + Y.e;
+  const uint32_t items = tab[parts.item + min(lane, t.n_ent - 1)], chunks = tab[parts.chunk + min(lane, kMxChunks - 1)];
+  mx4 acc[kMxChunks];
+#pragma unroll
+  for (int c = 0; c < kMxChunks; ++c) acc[c] = mx4{0.f, 0.f, 0.f, 0.f};
+  MxIndex I;
+  I.load(a, R.p0, R.p1, lane);
+  float gv[4][4], wv[WR][4], yv, bad = 0.f;
+  const auto fetch = [&](int edge, int other) __attribute__((always_inline)) {
+    yv = a.y[(int64_t)edge * t.D2 + min(lane, t.D2 - 1)];
+    mx_fetch<4, 4>(gv, a.g + (int64_t)other * t.DO * C, C, t.DO, g, c0, c_ok, false);
+    mx_fetch<4, WR>(wv, a.w + (a.w_shared ? 0 : (int64_t)edge * t.P * C), C, t.P, g, c0, c_ok, !a.w_shared);
+  };
+  fetch(MxIndex::at(I.edge, 0), MxIndex::at(I.other, 0));
+  const int n = (int)(R.p1 - R.p0);
+  int cur = -1;
+  bool first = true;
+  float xt[4][4];          // x[row r][16 q + 4 g + i]: the second operand of G for the open segment
+  mx4 xr[kMxChunks];       // the open segment's rows of x, this lane's channel
+  const auto row_of = [&](bool complete) __attribute__((always_inline)) {
+    return complete ? a.gx + (int64_t)cur * t.D1 * C : a.ws + (range * 2 + (first ? 0 : 1)) * t.D1 * C;
+  };
+  for (int k = 0; k < n; ++k) {
+    const int sid = MxIndex::at(I.sid, k & 63);
+    const int64_t e = MxIndex::at(I.edge, k & 63);
+    if (lane < t.D2) mine[Y.y + lane] = yv;
+    mx_stage<4, WR>(ws, kMx4Pitch, wv, t.P, g, c0);
+    mx_stage<4, 4>(gs, kMx4Pitch, gv, t.DO, g, c0);
+    if (sid != cur) {
+      const float* xrow = a.x + (int64_t)sid * t.D1 * C;
+      const int cl = lane < C ? lane : 0;
+#pragma unroll
+      for (int c = 0; c < kMxChunks; ++c) {
+        xr[c] = mx4{0.f, 0.f, 0.f, 0.f};
+        if (c < t.n_chunks) {
+          const uint32_t ck = (uint32_t)__builtin_amdgcn_readlane((int)chunks, c);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (i < (int)((ck >> 8) & 255)) {
+              const float v = xrow[((ck & 255) + i) * C + cl];
+              xr[c][i] = lane < C ? v : 0.f;
+            }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool in = r < t.D1 && 16 * q + 4 * g < C;        // C is a multiple of 4
+        load_vec<float, 4>(xt[q], xrow + (in ? r * C + 16 * q + 4 * g : 0));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xt[q][i] = in ? xt[q][i] : 0.f;
+      }
+      if (cur >= 0) {
+        if (want_gx) mx4_flush(acc, chunks, t.n_chunks, row_of(first ? R.first_complete : true), C, lane, bad);
+        first = false;
+      }
+      cur = sid;
+    }
+    mx_sync();
+    if (k + 1 < n) {
+      if (((k + 1) & 63) == 0) I.load(a, R.p0 + k + 1, R.p1, lane);
+      fetch(MxIndex::at(I.edge, (k + 1) & 63), MxIndex::at(I.other, (k + 1) & 63));
+    }
+    mx_couple(tab + parts.rec, t.n_rec, mine + Y.y, A, lane);
+    mx_sync();
+    if (want_gy) {
+      for (int s = 0; s < t.n_rowtiles; ++s) {
+        const uint32_t rw = tab[parts.row + 16 * s + r];
+        const mx4 G = mx_channels<4>(ws + (rw & 255) * kMx4Pitch + 4 * g, gs + (rw >> 8) * kMx4Pitch + 4 * g, xt);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) E[(16 * s + 4 * g + i) * 16 + r] = G[i];
+      }
+      mx_sync();
+      mx_grad_y(a, t, tab + parts.term, E, e, lane, bad);
+      mx_sync();
+    }
+    if (want_gx || want_gw) {
+      const int last = t.n_ent / 2 - 1;
+      int pair = 0;
+      Mx4Pair N;
+      N.request(items, 0, A, ws, gs, lane);
+#pragma unroll
+      for (int c = 0; c < kMxChunks; ++c) {
+        if (c < t.n_chunks) {
+          const int end = (int)((uint32_t)__builtin_amdgcn_readlane((int)chunks, c) >> 16);
+          for (; pair < end; ++pair) {
+            const Mx4Pair P = N;
+            N.request(items, min(pair + 1, last), A, ws, gs, lane);
+            mx4 D[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            mx4_multiply(D, P.a, P.rows(), [&](int h, int j) __attribute__((always_inline)) { return P.r[h][j]; });
+            acc[c] += P.w[0] * D[0] + P.w[1] * D[1];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              float* at = E + (P.k[h] & 255) * kMx4Pitch + lane;
+              float v = (P.k[h] >> 20) & 1 ? *at : 0.f;       // an earlier chunk of the path
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v = fmaf(xr[c][i], D[h][i], v);
+              *at = v;
+            }
+          }
+        }
+      }
+      mx_sync();
+      if (want_gw) mx_store_grad_w<4, WR>(a, t, E, kMx4Pitch, e, g, c0, c_ok, bad);
+      mx_sync();
+    }
+  }
+  if (want_gx) mx4_flush(acc, chunks, t.n_chunks, row_of((first ? R.first_complete : true) && R.last_complete), C, lane, bad);
+  const bool any_bad = __any(!(bad == 0.f));
+  if (lane == 0) t.flags[range] = any_bad;
+}
+
 // ---- host side ------------------------------------------------------------------------------------------------
 struct MxPlan {
   int nj, wr, per, waves_per_group;
+  bool wide;             // one channel per lane
   int64_t n_ranges, n_flags, ws_elems;
   size_t lds_bytes;
+  int n_words;
 };
 
 static int mx_plan(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, int backward, MxPlan* plan) {
@@ -455,11 +695,21 @@ static int mx_plan(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu
                           (backward ? (uintptr_t)a->grad_out | (uintptr_t)a->grad_x | (uintptr_t)a->grad_w : (uintptr_t)a->out);
   if (bytes & (4 * plan->nj - 1)) return CGTP_ERR_SHAPE;
   plan->wr = t->P <= 16 ? 4 : 8;
-  const MxParts parts(n_rec, n_ent, backward ? m->row_tiles : 0, backward ? m->rounds : 0, backward ? m->tiles : 0);
-  const MxLayout Y(plan->nj, t->D1, t->D2, t->DO, t->P, n_ent, m->row_tiles, backward != 0);
+  // Few coefficients and few channels leave little to contract: up to 64 coefficients and 32 channels the backward is quicker
+  // entry by entry (58 coefficients, 32 768 edges, 32 channels: 97 against 108 us; 206 coefficients: 425 against 203).
+  if (backward && plan->nj < 4 && t->nnz <= 64) return CGTP_ERR_SHAPE;
+  // one channel per lane past 32 channels, where the rows fit eight chunks (they do unless there are many scalars)
+  plan->wide = backward && plan->nj == 4 && m->bwd4 && m->bwd4_chunks > 0 && m->bwd4_chunks <= kMxChunks && m->bwd4_items > 0 &&
+               m->bwd4_items <= 64 && m->bwd4_items % 2 == 0;
+  const MxParts parts16(n_rec, n_ent, backward ? m->row_tiles : 0, backward ? m->rounds : 0, backward ? m->tiles : 0);
+  const Mx4Parts parts4(n_rec, m->bwd4_items, m->row_tiles, m->rounds);
+  const MxLayout Y16(plan->nj, t->D1, t->D2, t->DO, t->P, n_ent, m->row_tiles, backward != 0);
+  const Mx4Layout Y4(t->D2, t->DO, t->P, m->bwd4_items, m->row_tiles);
+  const int wave_floats = plan->wide ? Y4.floats : Y16.floats, words = plan->wide ? parts4.words : parts16.words;
+  plan->n_words = words;
   // as many wavefronts per compute unit as the LDS holds, at most two per SIMD in the backward (registers); workgroups
   // of up to eight wavefronts there and four in the forward, sharing one copy of the tables
-  const int64_t wave_bytes = 4 * (int64_t)Y.floats, tab_bytes = 4 * (int64_t)parts.words;
+  const int64_t wave_bytes = 4 * (int64_t)wave_floats, tab_bytes = 4 * (int64_t)words;
   int best = 0;
   for (int w = backward ? 8 : 4; w >= 1; --w) {
     const int64_t group = w * wave_bytes + tab_bytes;
@@ -508,15 +758,16 @@ static int mx_launch(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_u
     d.n_rows = a->n_rows; d.n_seg = a->n_seg; d.n_waves = plan.n_ranges;
     d.C = a->C; d.w_shared = a->w_shared; d.pos_per_wave = plan.per;
     MxDev dev = {};
-    dev.words = backward ? m->bwd : m->fwd;
+    dev.words = plan.wide ? m->bwd4 : backward ? m->bwd : m->fwd;
     dev.n_rec = backward ? m->bwd_records : m->fwd_records;
-    dev.n_ent = backward ? m->bwd_entries : m->fwd_entries;
+    dev.n_ent = plan.wide ? m->bwd4_items : backward ? m->bwd_entries : m->fwd_entries;
+    dev.n_chunks = m->bwd4_chunks;
     dev.n_rowtiles = m->row_tiles; dev.n_rounds = m->rounds; dev.lanes_log2 = m->lanes_log2; dev.n_tiles = m->tiles;
-    const MxParts parts(dev.n_rec, dev.n_ent, backward ? m->row_tiles : 0, backward ? m->rounds : 0, backward ? m->tiles : 0);
-    dev.n_words = parts.words;
+    dev.n_words = plan.n_words;
     dev.D1 = t->D1; dev.D2 = t->D2; dev.DO = t->DO; dev.P = t->P;
     dev.flags = reinterpret_cast<int32_t*>((float*)a->workspace + plan.ws_elems);
-    const void* fn = plan.nj == 1 ? mx_kernel<1>(backward, plan.wr)
+    const void* fn = plan.wide ? (plan.wr == 4 ? (const void*)uvu_mx4_bwd_kernel<4> : (const void*)uvu_mx4_bwd_kernel<8>)
+                     : plan.nj == 1 ? mx_kernel<1>(backward, plan.wr)
                                   : plan.nj == 2 ? mx_kernel<2>(backward, plan.wr) : mx_kernel<4>(backward, plan.wr);
     if (plan.lds_bytes > 48 * 1024 &&
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds_bytes) != hipSuccess)

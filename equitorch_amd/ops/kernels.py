@@ -837,9 +837,9 @@ class UvuTable:
         words = uvu_mx_words(coo)
         self.mx = None
         if words is not None:
-            self.mx = _lib.UvuMx(**{k: v for k, v in words.items() if k not in ("fwd", "bwd")})
-            self.mx_words = [torch.from_numpy(words[k].view(np.int32)).to(device) for k in ("fwd", "bwd")]
-            self.mx.fwd, self.mx.bwd = (v.data_ptr() for v in self.mx_words)
+            self.mx_words = {k: torch.from_numpy(v.view(np.int32)).to(device) for k, v in words.items()
+                             if isinstance(v, np.ndarray)}
+            self.mx = _lib.UvuMx(**{k: self.mx_words[k].data_ptr() if k in self.mx_words else v for k, v in words.items()})
 
 
 def uvu_mx_words(coo) -> Optional[dict]:
@@ -921,8 +921,39 @@ def uvu_mx_words(coo) -> Optional[dict]:
                 at[p] = u + 1
         for chunks in mine:
             tiles += [block[0] | (block[1] + 3) // 4 << 8] + chunks + [0] * (4 - len(chunks))
+    def walk4():                                    # chunks of up to four rows of x, items in pairs
+        chunks = []
+        for r0, n in sorted(set(x_rows)):
+            chunks += [(r0 + 4 * j, min(4, n - 4 * j), (r0, n)) for j in range((n + 3) // 4)]
+        covered = [r for r0, n, _ in chunks for r in range(r0, r0 + n)]
+        if len(set(covered)) != len(covered):
+            return None
+        chunks += [(r, 1, None) for r in range(D1) if r not in covered]      # rows nothing couples to
+        items, at, ends = [], {}, []
+        for r0, n, block in chunks:
+            mine = [(out_rows[p][0] + 7 * j, min(7, out_rows[p][1] - 7 * j), p) for p in range(P) if x_rows[p] == block
+                    for j in range((out_rows[p][1] + 6) // 7)]
+            for m0, rows, p in sorted(mine, key=lambda v: v[1]):
+                for k in range(rows):
+                    for r in range(n):
+                        at[p, m0 + k, r0 + r] = len(items) // 2 * 64 + (8 * (len(items) % 2) + k) * 4 + r
+                opens = r0 == block[0] and m0 == out_rows[p][0]
+                items.append(p | m0 << 8 | (rows | 1) << 16 | (not opens) << 20)
+            if len(items) % 2:
+                items.append(1 << 16 | 1 << 20)
+            ends.append(len(items) // 2)
+        if len(chunks) > 8 or not 0 < len(items) <= 64:
+            return None
+        records = []
+        for key, terms in elements.items():
+            (c0, b0), (c1, b1) = (terms + [(0.0, terms[0][1])])[:2]
+            records += [f32(c0), f32(c1), b0 | b1 << 8 | at[key] << 16]
+        words = [r0 | n << 8 | end << 16 for (r0, n, _), end in zip(chunks, ends)]
+        return records + items + words + [0] * (8 - len(words)), len(items), len(chunks)
+    x4 = walk4()
     pack = lambda *parts: np.array([w for part in parts for w in part] + [0] * 4, dtype=np.uint32)    # noqa: E731
-    return {"fwd": pack(fwd_records, fwd_entries), "bwd": pack(bwd_records, bwd_entries, row_words, term_words, tiles),
+    wide = {} if x4 is None else {"bwd4": pack(x4[0], row_words, term_words), "bwd4_items": x4[1], "bwd4_chunks": x4[2]}
+    return {**wide, "fwd": pack(fwd_records, fwd_entries), "bwd": pack(bwd_records, bwd_entries, row_words, term_words, tiles),
             "fwd_records": len(elements), "fwd_entries": len(fwd_entries), "bwd_records": len(elements),
             "bwd_entries": len(bwd_entries), "row_tiles": row_tiles, "rounds": rounds, "lanes_log2": lanes_log2,
             "tiles": len(tiles) // 5}
@@ -973,7 +1004,7 @@ def _uvu_tab_launch(a: UvuArgs, tab: UvuTable, backward: int, device) -> None:
     """Launches on the matrix cores where the table and the operands fit them (see ``uvu_mx_words`` and
     ``cgtp_uvu_mx_validate``: at most 64 channels, of which a lane takes one, two or four at a time), entry by entry
     elsewhere.  206 coefficients, 65 536 edges, 64 channels: forward 175 us against 411,
-    backward 453 against 1303; every size of the range gains (an edge costs the same wherever it lies)."""
+    backward 371 against 1303."""
     mx = tab.mx
     if mx is not None and _lib.lib.cgtp_uvu_mx_validate(C.byref(a), C.byref(tab.c), C.byref(mx), backward) == 0:
         nbytes = int(_lib.lib.cgtp_uvu_mx_workspace_bytes(C.byref(a), C.byref(tab.c), C.byref(mx), backward))

@@ -314,12 +314,19 @@ int cgtp_uvu_tab_bwd(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, void* stream
  *             64 * rounds pairs (coef, place in the matrix (path, output row) x 16 rows of x): lane l adds up component
  *             l >> lanes_log2 of grad_y;
  *             5 words per tile of the weight gradient: first row of grad_out | steps << 8, then four chunks of up to
- *             four rows of x of one path: element | path << 16 | 1 << 24 if the path has an earlier chunk | rows << 25. */
+ *             four rows of x of one path: element | path << 16 | 1 << 24 if the path has an earlier chunk | rows << 25.
+ * bwd4 (33 to 64 channels; NULL or more than eight chunks: bwd serves): the rows of x cut into chunks of up to four; records
+ * as above with the element (item / 2) * 64 + (8 * (item % 2) + row of grad_out) * 4 + row of the chunk;
+ *             items path | first row of grad_out << 8 | rows (1, 3, 5, 7) << 16 | 1 << 20 if the path has an earlier chunk;
+ *             eight chunks first row | rows << 8 | end of its items / 2 << 16; then row words and pairs as above.
+ * The backward takes more than 64 coefficients where there are at most 32 channels. */
 typedef struct cgtp_uvu_mx {
   const uint32_t* fwd;
   const uint32_t* bwd;
   int32_t fwd_records, fwd_entries, bwd_records, bwd_entries;   /* entries <= 64                                    */
   int32_t row_tiles, rounds, lanes_log2, tiles;
+  const uint32_t* bwd4;
+  int32_t bwd4_items, bwd4_chunks;                              /* items <= 64, even                                */
 } cgtp_uvu_mx;
 int64_t cgtp_uvu_mx_workspace_bytes(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, int backward);
 int cgtp_uvu_mx_validate(const cgtp_uvu_args* a, const cgtp_uvu_tab* t, const cgtp_uvu_mx* m, int backward);

@@ -185,3 +185,45 @@ def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, 
         assert torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
         # in a range without a value that is not finite the sums run in another order: norm-wise
         assert float((a[fin] - b[fin]).detach().abs().max()) <= 1e-5 * float(b[fin].abs().max())
+
+
+@pytest.mark.parametrize("irreps", TABLES)
+def test_the_wide_walk_covers_the_table(irreps):
+    """The walk of the kernels with one channel per lane: the coupling matrix of every item, put back in its place, is the
+    table's, and every path and produced row is visited once."""
+    from equitorch_amd.ops import kernels
+    coo = kernels.coo_of(_info(irreps))
+    m = kernels.uvu_mx_words(coo)
+    y = np.random.default_rng(3).standard_normal(coo.D2)
+    f32 = lambda v: float(np.uint32(v).view(np.float32))     # noqa: E731
+    for which, produced, contracted, n_prod, n_con in (("bwd", coo.M1, coo.M, coo.D1, coo.DO),):
+        words, n_items, n_chunks = m[which + "4"], m[which + "4_items"], m[which + "4_chunks"]
+        n_rec = m[which + "_records"]
+        assert n_items % 2 == 0 and n_items <= 64 and n_chunks <= 8
+        want, got = np.zeros((coo.P, n_prod, n_con)), np.zeros((coo.P, n_prod + 4, n_con + 7))
+        for c, r, k, b, p in zip(coo.coef, produced, contracted, coo.M2, coo.p):
+            want[p, r, k] += float(np.float32(c)) * y[b]
+        A = np.zeros(32 * n_items)
+        for c0, c1, k in words[:3 * n_rec].reshape(-1, 3):
+            A[k >> 16] = f32(c0) * y[k & 255] + f32(c1) * y[(k >> 8) & 255]
+        items = words[3 * n_rec:3 * n_rec + n_items]
+        chunks = words[3 * n_rec + n_items:3 * n_rec + n_items + 8][:n_chunks]
+        pair, rows_seen, paths = 0, [], set()
+        for chunk in chunks:
+            r0, n = int(chunk & 255), int((chunk >> 8) & 255)
+            rows_seen += range(r0, r0 + n)
+            while pair < (chunk >> 16):
+                for h in (0, 1):
+                    k = int(items[2 * pair + h])
+                    p, row, rows = k & 255, (k >> 8) & 255, (k >> 16) & 15
+                    assert rows in (1, 3, 5, 7) and row + rows <= n_con + 6
+                    slots = A[pair * 64 + 32 * h:pair * 64 + 32 * h + 32].reshape(8, 4)
+                    assert not slots[rows:].any() and not slots[:, n:].any()
+                    got[p, r0:r0 + 4, row:row + rows] += slots[:rows].T
+                    if slots.any():
+                        assert bool(k >> 20 & 1) == (p in paths)        # sets the path's gradient, then adds to it
+                        paths.add(p)
+                pair += 1
+        assert pair * 2 == n_items and sorted(rows_seen) == list(range(n_prod))
+        assert paths == set(range(coo.P))
+        np.testing.assert_allclose(got[:, :n_prod, :n_con], want, rtol=0, atol=1e-12)
