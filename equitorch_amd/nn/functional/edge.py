@@ -284,6 +284,11 @@ def edge_tensor_product_uu(x: Tensor, sh: Tensor, weight: Tensor, plan: EdgePlan
     cfg = kernels.uvu_config_of(tp_info_forward)
     if cfg >= 0 and x.dtype == sh.dtype == weight.dtype and x.dtype in (torch.float32, torch.float64):
         xc, yc, wc = x.contiguous(), sh.contiguous(), weight.contiguous()
+        tab = kernels.uvu_subset_table(cfg, tp_info_forward, xc, yc, wc)
+        if tab is not None:
+            kernels.log_tier("edge_tensor_product_uu", "table-driven fused gather / product / segment sum",
+                             f"{tab.nnz} coefficients, some paths of config {int(cfg)}")
+            return _EdgeUvuTable.apply(xc, yc, wc, plan, tab, tp_info_forward)
         if kernels.uvu_launchable(cfg, xc, yc, wc, segments=True):
             kernels.log_tier("edge_tensor_product_uu", "fused gather / product / segment sum", f"config {int(cfg)}")
             handle = _shim_handle(plan, cfg, xc, 0, tp_info_forward)

@@ -984,6 +984,17 @@ def _uvu_tab_args(x: Tensor, y: Tensor, w: Tensor, seg: SegIndex) -> UvuArgs:
     return a
 
 
+def _tab_probe(x: Tensor, y: Tensor, w: Tensor) -> UvuArgs:
+    """Arguments as a launch on these operands would have them, for the validation entry points."""
+    a = UvuArgs()
+    a.dtype, a.C, a.w_shared = _lib.F32, x.shape[-1], int(w.ndim == 2)
+    a.n_rows, a.n_x_rows, a.n_seg = y.shape[0], x.shape[0], x.shape[0]
+    dummy = 256
+    a.ptr = a.seg_ids = a.gather = a.out = a.grad_out = a.grad_x = a.grad_y = dummy
+    a.x, a.y, a.w = x.data_ptr() or dummy, y.data_ptr() or dummy, w.data_ptr() or dummy
+    return a
+
+
 def uvu_tab_launchable(tab: Optional[UvuTable], x: Tensor, y: Tensor, w: Tensor, need_grad_w: bool) -> bool:
     """Whether the table-driven segment kernels take these operands in both directions (fp32, up to 256 channels — 64
     unless a multiple of 4 and aligned —, per-edge weights or a shared weight that needs no gradient)."""
@@ -991,13 +1002,22 @@ def uvu_tab_launchable(tab: Optional[UvuTable], x: Tensor, y: Tensor, w: Tensor,
         return False
     if x.shape[0] == 0 or y.shape[0] == 0 or y.ndim != 2 or (w.ndim == 2 and need_grad_w):
         return False
-    a = UvuArgs()
-    a.dtype, a.C, a.w_shared = _lib.F32, x.shape[-1], int(w.ndim == 2)
-    a.n_rows, a.n_x_rows, a.n_seg = y.shape[0], x.shape[0], x.shape[0]
-    dummy = 256
-    a.ptr = a.seg_ids = a.gather = a.out = a.grad_out = a.grad_x = a.grad_y = dummy
-    a.x, a.y, a.w = x.data_ptr() or dummy, y.data_ptr() or dummy, w.data_ptr() or dummy
+    a = _tab_probe(x, y, w)
     return all(_lib.lib.cgtp_uvu_tab_validate(C.byref(a), C.byref(tab.c), d) == 0 for d in (0, 1))
+
+
+def uvu_subset_table(cfg: Cfg, tp_info, x: Tensor, y: Tensor, w: Tensor) -> Optional[UvuTable]:
+    """The table to run on the matrix cores as it is, where a compiled table only matches with paths the caller's does not
+    have: the compiled kernels then take the per-edge weights expanded by zero rows (a copy of the largest operand, there
+    and back) and work through all paths.  9 of 15 paths, 77 coefficients, 32 768 edges, forward and backward: 64 channels
+    510 -> 187 us, 16 channels 226 -> 181.  None where the matrix cores do not take it in both directions."""
+    if int(cfg) < 0 or cfg.w_rows is None or w.ndim != 3 or x.dtype != torch.float32:
+        return None
+    tab = uvu_table_of(tp_info, x.device)
+    if tab is None or tab.mx is None or not uvu_tab_launchable(tab, x, y, w, False):
+        return None
+    return tab if all(_lib.lib.cgtp_uvu_mx_validate(C.byref(_tab_probe(x, y, w)), C.byref(tab.c), C.byref(tab.mx), d) == 0
+                      for d in (0, 1)) else None
 
 
 def _uvu_tab_launch(a: UvuArgs, tab: UvuTable, backward: int, device) -> None:
