@@ -171,6 +171,10 @@ def _load():
     _uvs = [C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_int32]
     lib.cgtp_uvs_validate.argtypes = _uvs
     lib.cgtp_uvs_apply.argtypes = _uvs + [C.c_void_p]
+    lib.cgtp_uvsw_packed_bytes.restype = C.c_int64
+    lib.cgtp_uvsw_packed_bytes.argtypes = [C.c_int32] * 4
+    lib.cgtp_uvsw_validate.argtypes = _uvs + [C.c_int32]
+    lib.cgtp_uvsw_apply.argtypes = _uvs + [C.c_int32, C.c_void_p]
     lib.cgtp_uvu_mx_workspace_bytes.restype = C.c_int64
     lib.cgtp_uvu_mx_workspace_bytes.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]
     lib.cgtp_uvu_mx_validate.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]

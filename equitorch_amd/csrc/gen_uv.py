@@ -251,6 +251,10 @@ def emit_split(out_dir: str) -> str:
         for d in (0, 1):
             chunks.append(emit_direction(name, d, coo, seg_out, seg_in1, split=True))
         chunks.append(emit_direction(name, 0, coo, seg_out, seg_in1, gy=True, split=True))
+        # gradient of the second operand when it has channels as well: the gradient of x with the operands exchanged
+        swapped = coo._replace(M1=coo.M2, M2=coo.M1, D1=coo.D2, D2=coo.D1)
+        chunks.append(emit_direction(name, 1, swapped, seg_out, irrep_segments(Irreps(i2)), split=True)
+                      .replace(f"struct UVS_{name}_d1 ", f"struct UVS_{name}_d2 "))
         terms = ", ".join(f"{{{_lit(coo.coef[t])}, {coo.M[t]}, {coo.M1[t]}, {coo.M2[t]}, {coo.p[t]}}}"
                           for t in range(coo.coef.shape[0]))
         chunks.append(f"static __device__ const UvsTerm UVS_{name}_terms[] = {{{terms}}};")
@@ -260,7 +264,7 @@ def emit_split(out_dir: str) -> str:
         chunks.append("};")
         chunks.append("")
     chunks.append("#define CGTP_FOREACH_UVS_CONFIG(X) \\")
-    chunks.append(" \\\n".join(f"  X({list(CONFIGS).index(n)}, UVS_{n}_d0, UVS_{n}_d1, UVS_{n}_gy, UVS_{n}_table)"
+    chunks.append(" \\\n".join(f"  X({list(CONFIGS).index(n)}, UVS_{n}_d0, UVS_{n}_d1, UVS_{n}_gy, UVS_{n}_d2, UVS_{n}_table)"
                               for n in names))
     chunks.append("")
     path, text = os.path.join(out_dir, "uv_split_configs.inc"), "\n".join(chunks)

@@ -48,20 +48,35 @@ __device__ __forceinline__ unsigned uvs_exp(unsigned abs_bits) { return max(abs_
 __device__ __forceinline__ float uvs_scale(unsigned e) { return __builtin_bit_cast(float, (267u - e) << 23); }
 __device__ __forceinline__ float uvs_unscale(unsigned e) { return __builtin_bit_cast(float, (e - 13u) << 23); }
 
+// The weight as the caller holds it.  With channels on both operands a path has one matrix per channel l of the operand
+// that is not contracted; `matrices` is their number (else 1), and a "path" of the packed weight is a (path, l).
+struct UvsWeight {
+  const float* w;
+  int64_t stride_p, stride_k, stride_c, stride_l;
+  int matrices;
+  __device__ __forceinline__ const float* of(int i) const { return w + (i / matrices) * stride_p + (i % matrices) * stride_l; }
+};
+
 // A workgroup per path and block of 32 output channels: the path's largest magnitude (every workgroup of a path reads all of
 // it: 64 KB at 128 channels, from L2), then both halves of its block in fragment order.  Per path and block 2 (half) x 2
 // (tile) x K / 32 chunks of 1 KB, holding the 16 bytes of every lane; row r of tile t is output channel
 // 8 (r / 4) + 4 t + r % 4 of the block.  inv[p]: what undoes the scale, a NaN for a path that is not split.
-__global__ void __launch_bounds__(256) uvs_pack_kernel(const float* __restrict__ w, _Float16* __restrict__ packed,
-                                                       float* __restrict__ inv, int K, int cout, int64_t stride_p,
-                                                       int64_t stride_k, int64_t stride_c) {
+__global__ void __launch_bounds__(256) uvs_pack_kernel(UvsWeight W, _Float16* __restrict__ packed, float* __restrict__ inv, int K,
+                                                       int cout) {
   __shared__ unsigned waves_max[4];
   const int p = blockIdx.x, blk = blockIdx.y, ks = K / 32;
-  const float* wp = w + p * stride_p;
+  const float* wp = W.of(p);
+  const int64_t stride_k = W.stride_k, stride_c = W.stride_c;
   unsigned m = 0;
-  // a path is K * cout consecutive elements, either way round; a multiple of 1024
+  // lanes along the axis of consecutive elements; K and cout are multiples of 32
+  const bool k_inner = stride_k == 1;
+  const int inner = k_inner ? K : cout;
+  const int64_t si = k_inner ? stride_k : stride_c, so = k_inner ? stride_c : stride_k;
 #pragma unroll 4
-  for (int i = threadIdx.x; i < K * cout; i += 256) m = max(m, __builtin_bit_cast(unsigned, wp[i]) & 0x7fffffffu);
+  for (int i = threadIdx.x; i < K * cout; i += 256) {
+    const float v = wp[(i / inner) * so + (i % inner) * si];
+    m = max(m, __builtin_bit_cast(unsigned, v) & 0x7fffffffu);
+  }
   for (int off = 1; off < kWave; off <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, kWave));
   if ((threadIdx.x & (kWave - 1)) == 0) waves_max[threadIdx.x / kWave] = m;
   __syncthreads();
@@ -164,6 +179,7 @@ struct UvsOps {
   const unsigned char* xs;                  // this lane's base in its sample's rows
   const float* inv_x;                       // its sample's rows
   const float* inv_w;
+  int inv_stride = 1;                       // between the paths of inv_w
   __device__ __forceinline__ void load_a(int p, A& a) const {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -194,20 +210,14 @@ struct UvsOps {
       }
     }
   }
-  __device__ __forceinline__ float scale(int p, int row) const { return inv_x[row] * inv_w[p]; }
-};
-
-// The weight as the caller holds it.
-struct UvsWeight {
-  const float* w;
-  int64_t stride_p, stride_k, stride_c;
+  __device__ __forceinline__ float scale(int p, int row) const { return inv_x[row] * inv_w[p * inv_stride]; }
 };
 
 // (s x) W of one path and row for the two tiles of block `blk`, from memory, in fp32 matrix instructions.
 __device__ __forceinline__ void uvs_plain_tile(const UvsWeight& W, int p, int blk, const float* __restrict__ xrow, float s,
                                                int K, int r, int q, floatx4 (&z)[2]) {
   z[0] = z[1] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const float* wb = W.w + p * W.stride_p + (blk * 32 + 8 * (r >> 2) + (r & 3)) * W.stride_c;
+  const float* wb = W.of(p) + (blk * 32 + 8 * (r >> 2) + (r & 3)) * W.stride_c;
   for (int k = q; k < K; k += 4) {
     const float b = s * xrow[k];
 #pragma unroll
@@ -346,19 +356,134 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
   }
 }
 
+// With channels on both operands ("uvw"), contracted channels x (n, DIN, 32), the other operand z (n, D2, L):
+//   out[n, m, w] = sum_l sum_t coef_t * z[n, b_t, l] * sum_u x[n, a_t, u] * W[p_t, u, l, w]
+// is the product above summed over l, with z[., ., l] for y and a weight per (path, l).  A workgroup owns 16 samples and a
+// block of 32 produced channels; its four wavefronts take every fourth l each, keep all output rows in registers, and are
+// added through LDS in a fixed order.  Mixing z and x first, as the fp32 route does, forms 1024 products per (path, row)
+// and sample on the vector units; here they are the matrix cores', and the vector units see one multiply-add per
+// coefficient and l.  What bounds it: vector and matrix instructions of two wavefronts per SIMD in about equal parts, and
+// the weights from L2 (4 bytes an element and workgroup: 1.4 MB at 32 channels, lmax = 2).
+// 32 x 32 -> 32, lmax = 2, 32768 samples: 943 -> 268 us, both gradients alike; 500 samples: 179 -> 44 us with packing; lmax = 1,
+// 32768 samples 205 -> 73 us.  Error of the results against 64 bits 1.1e-7 to 1.4e-7, of the fp32 route 2.0e-7 to 1.4e-6.
+template <class CFG, class TAB, int KIND>
+__global__ void __launch_bounds__(256, 2) uvsw_kernel(const float* __restrict__ x, const float* __restrict__ z,
+                                                      const _Float16* __restrict__ wp, const float* __restrict__ inv_w,
+                                                      float* __restrict__ out, int64_t n_rows, int cout, UvsWeight W) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int CIN = 32, DIN = CFG::DIN, DOUT = CFG::DOUT, D2 = CFG::D2;
+  using T = UvsLds<DIN, CIN>;
+  const int64_t n0 = (int64_t)blockIdx.x * kUvsSamples;
+  const int L = W.matrices, n_mat = CFG::P * L;
+  bool ok = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
+  float* inv_x = reinterpret_cast<float*>(smem + T::kTile);
+  float* inv_p = inv_x + kUvsSamples * DIN;
+  int* words = reinterpret_cast<int*>(inv_p + n_mat);
+  float* zs = reinterpret_cast<float*>(words + 4);                // [l][row][sample]
+  for (int i = threadIdx.x; i < n_mat; i += blockDim.x) {
+    const float v = inv_w[i];
+    inv_p[i] = v;
+    ok = ok && v == v;
+  }
+  for (int i = threadIdx.x; i < kUvsSamples * D2 * L; i += blockDim.x) {
+    const int s = i / (D2 * L), rest = i - s * (D2 * L), b = rest / L, l = rest - b * L;
+    const float v = z[min(n0 + s, n_rows - 1) * (D2 * L) + rest];
+    zs[(l * D2 + b) * kUvsSamples + s] = v;
+    ok = ok && v - v == 0.f;
+  }
+  const bool plain = uvs_any(!ok, words);
+
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int n = lane & 15, q = lane >> 4;
+  const int64_t row_n = min(n0 + n, n_rows - 1);
+  const bool valid = n0 + n < n_rows;
+  const int wblk = blockIdx.y;
+  float* orow = out + (n0 + n) * DOUT * cout + wblk * 32 + 8 * q;
+  auto store = [&](int row, const floatx4& o0, const floatx4& o1) __attribute__((always_inline)) {
+    if (valid) {
+      __builtin_nontemporal_store(o0, reinterpret_cast<floatx4*>(orow + row * cout));
+      __builtin_nontemporal_store(o1, reinterpret_cast<floatx4*>(orow + row * cout + 4));
+    }
+  };
+  if (plain) {
+    for (int m = wave; m < DOUT; m += 4) {
+      floatx4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      for (int t = 0; t < TAB::N; ++t) {
+        const UvsTerm e = TAB::terms()[t];
+        const int mt = KIND == 0 ? e.o : KIND == 1 ? e.a : e.b, at = KIND == 0 ? e.a : e.o, bt = KIND == 2 ? e.a : e.b;
+        if (mt != m) continue;
+        for (int l = 0; l < L; ++l) {
+          floatx4 v[2];
+          uvs_plain_tile(W, e.p * L + l, wblk, x + (row_n * DIN + at) * CIN, e.c * z[(row_n * D2 + bt) * L + l], CIN, n, q, v);
+          o[0] += v[0];
+          o[1] += v[1];
+        }
+      }
+      store(m, o[0], o[1]);
+    }
+    return;
+  }
+  floatx4 acc[DOUT][2];
+#pragma unroll
+  for (int m = 0; m < DOUT; ++m) acc[m][0] = acc[m][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int64_t matrix = (int64_t)cout * CIN * 2;
+  for (int l = wave; l < L; l += 4) {
+    float zv[D2];
+#pragma unroll
+    for (int j = 0; j < D2; ++j) zv[j] = zs[(l * D2 + j) * kUvsSamples + n];
+    const UvsOps<DIN, CIN> ops{wp + l * matrix + (int64_t)wblk * (4 * 512) + lane * 8, L * matrix,
+                               smem + n * T::kPitch + q * 16, inv_x + n * DIN, inv_p + l, L};
+    CFG::run(ops, zv, [&](int row, const floatx4& o0, const floatx4& o1) __attribute__((always_inline)) {
+      acc[row][0] += o0;
+      acc[row][1] += o1;
+    });
+  }
+  // wavefronts 2 and 3 to 0 and 1, then 1 to 0
+  floatx4* red = reinterpret_cast<floatx4*>(smem);
+#pragma unroll
+  for (int half = 2; half >= 1; half >>= 1) {
+    __syncthreads();
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int m = 0; m < DOUT; ++m)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) red[(((wave - half) * DOUT + m) * 2 + t) * kWave + lane] = acc[m][t];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int m = 0; m < DOUT; ++m)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[m][t] += red[((wave * DOUT + m) * 2 + t) * kWave + lane];
+    }
+  }
+  if (wave == 0) {
+#pragma unroll
+    for (int m = 0; m < DOUT; ++m) store(m, acc[m][0], acc[m][1]);
+  }
+}
+
 // ---- host side ------------------------------------------------------------------------------------------------
 using UvsFn = void (*)(const float*, const float*, const _Float16*, const float*, float*, int64_t, int, UvsWeight);
 struct UvsEntry {
   int cfg;                 // index of the table among the compiled ones (cgtp_uv_find)
   int din[2], p;           // rows of the contracted operand in the forward and in the gradient of x; paths
   UvsFn fn[3][3];          // [forward, gradient of x, gradient of y][32, 64, 128 contracted channels]
+  UvsFn fn_w[3];           // channels on both operands, 32 contracted; null where the rows do not fit the registers
+  int rows_w[3][3];        // rows of the contracted, the other and the produced operand
 };
 
 // wavefronts per SIMD the registers are kept to: two, except at 128 contracted channels, where the three weight fragments in
 // flight alone take 192 registers
 constexpr int uvs_waves(int cin) { return cin < 128 ? 2 : 1; }
 
-template <class D0, class D1, class GY, class TAB>
+template <class CFG, class TAB, int KIND>
+constexpr UvsFn uvsw_fn() {
+  if constexpr (CFG::DOUT <= 9) return uvsw_kernel<CFG, TAB, KIND>;
+  else return nullptr;
+}
+
+template <class D0, class D1, class GY, class DW, class TAB>
 static UvsEntry make_uvs_entry(int cfg) {
   UvsEntry e;
   e.cfg = cfg;
@@ -371,11 +496,14 @@ static UvsEntry make_uvs_entry(int cfg) {
   CGTP_UVS_CIN(1, 64)
   CGTP_UVS_CIN(2, 128)
 #undef CGTP_UVS_CIN
+  e.fn_w[0] = uvsw_fn<D0, TAB, 0>(); e.fn_w[1] = uvsw_fn<D1, TAB, 1>(); e.fn_w[2] = uvsw_fn<DW, TAB, 2>();
+  const int rows[3][3] = {{D0::DIN, D0::D2, D0::DOUT}, {D1::DIN, D1::D2, D1::DOUT}, {DW::DIN, DW::D2, DW::DOUT}};
+  for (int k = 0; k < 9; ++k) e.rows_w[k / 3][k % 3] = rows[k / 3][k % 3];
   return e;
 }
 
 static const UvsEntry* uvs_entry(int cfg) {
-#define CGTP_X(INDEX, D0, D1, GY, TAB) make_uvs_entry<D0, D1, GY, TAB>(INDEX),
+#define CGTP_X(INDEX, D0, D1, GY, DW, TAB) make_uvs_entry<D0, D1, GY, DW, TAB>(INDEX),
   static const UvsEntry table[] = {CGTP_FOREACH_UVS_CONFIG(CGTP_X)};
 #undef CGTP_X
   for (const UvsEntry& e : table)
@@ -402,6 +530,40 @@ static int uvs_check(int cfg, int kind, const void* x, const void* y, const void
   return CGTP_OK;
 }
 
+static int uvs_pack(const UvsWeight& W, void* packed, int64_t matrices, int cin, int cout, hipStream_t stream) {
+  hipLaunchKernelGGL(uvs_pack_kernel, dim3((unsigned)matrices, (unsigned)(cout / 32)), dim3(256), 0, stream, W,
+                     (_Float16*)packed, (float*)((_Float16*)packed + matrices * cin * cout * 2), cin, cout);
+  return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+}
+
+// The weight (P, U, V, W) as kind 0 (contracts U, produces W, runs over V), 1 (W, U, V) or 2 (W, V, U) reads it.
+static UvsWeight uvsw_weight(const float* w, int kind, int u, int v, int c) {
+  const int64_t sp = (int64_t)u * v * c, su = (int64_t)v * c, sv = c;
+  if (kind == 0) return {w, sp, su, 1, sv, v};
+  if (kind == 1) return {w, sp, 1, su, sv, v};
+  return {w, sp, 1, sv, su, u};
+}
+
+static int uvsw_check(int cfg, int kind, const void* x, const void* z, const void* packed, const void* w, const void* out,
+                      int64_t n_rows, int u, int v, int c, const UvsEntry** entry, int64_t* lds) {
+  const UvsEntry* e = uvs_entry(cfg);
+  if (!e) return CGTP_ERR_CONFIG;
+  if (kind < 0 || kind > 2 || !e->fn_w[kind]) return CGTP_ERR_SHAPE;
+  if (!x || !z || !packed || !w || !out) return CGTP_ERR_NULL;
+  const int cin = kind == 0 ? u : c, cout = kind == 0 ? c : kind == 1 ? u : v, L = kind == 2 ? u : v;
+  if (n_rows < 0 || cin != 32 || cout <= 0 || cout % 32 || L <= 0) return CGTP_ERR_SHAPE;
+  if (((uintptr_t)x | (uintptr_t)packed | (uintptr_t)out) & 15u) return CGTP_ERR_ALIGN;
+  const int din = e->rows_w[kind][0], d2 = e->rows_w[kind][1], dout = e->rows_w[kind][2];
+  const int64_t staged = (int64_t)kUvsSamples * (din * cin * 4 + 16) + kUvsSamples * din * 4 + (int64_t)e->p * L * 4 + 16 +
+                         (int64_t)kUvsSamples * d2 * L * 4;
+  const int64_t sums = (int64_t)2 * dout * 2 * kWave * 16;
+  *lds = staged > sums ? staged : sums;
+  if (2 * *lds > kLdsBytes) return CGTP_ERR_LDS;                  // two workgroups per compute unit, as the registers allow
+  if ((n_rows + kUvsSamples - 1) / kUvsSamples >= (int64_t)1 << 31) return CGTP_ERR_SHAPE;
+  *entry = e;
+  return CGTP_OK;
+}
+
 }  // namespace cgtp
 
 using namespace cgtp;
@@ -418,10 +580,9 @@ int cgtp_uvs_pack_weights(const float* w, void* packed, int32_t n_paths, int32_t
   if (!w || !packed) return CGTP_ERR_NULL;
   if (n_paths <= 0 || cin <= 0 || cout <= 0 || cin % 32 || cout % 32) return CGTP_ERR_SHAPE;
   if ((uintptr_t)packed & 15u) return CGTP_ERR_ALIGN;
-  const int64_t sp = (int64_t)cin * cout, sk = transposed ? 1 : cout, sc = transposed ? cin : 1;
-  hipLaunchKernelGGL(uvs_pack_kernel, dim3((unsigned)n_paths, (unsigned)(cout / 32)), dim3(256), 0, (hipStream_t)stream, w, (_Float16*)packed,
-                     (float*)((_Float16*)packed + n_paths * sp * 2), (int)cin, (int)cout, sp, sk, sc);
-  return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+  const int64_t sp = (int64_t)cin * cout;
+  const UvsWeight W = {w, sp, transposed ? 1 : (int64_t)cout, transposed ? (int64_t)cin : 1, 0, 1};
+  return uvs_pack(W, packed, n_paths, cin, cout, (hipStream_t)stream);
 }
 
 int cgtp_uvs_validate(int cfg, int kind, const void* x, const void* y, const void* packed, const void* w, const void* out,
@@ -443,10 +604,43 @@ int cgtp_uvs_apply(int cfg, int kind, const void* x, const void* y, const void* 
   if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return CGTP_ERR_LDS;
   const int64_t sp = (int64_t)cin * cout;
-  const UvsWeight W = {(const float*)w, sp, kind == 1 ? 1 : (int64_t)cout, kind == 1 ? (int64_t)cin : 1};
+  const UvsWeight W = {(const float*)w, sp, kind == 1 ? 1 : (int64_t)cout, kind == 1 ? (int64_t)cin : 1, 0, 1};
   hipLaunchKernelGGL(fn, dim3((unsigned)((n_rows + kUvsSamples - 1) / kUvsSamples), (unsigned)(kind == 2 ? 1 : (cout + 127) / 128)),
                      dim3(256), (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)y, (const _Float16*)packed,
                      (const float*)((const _Float16*)packed + e->p * sp * 2), (float*)out, n_rows, (int)cout, W);
+  return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+}
+
+int64_t cgtp_uvsw_packed_bytes(int32_t n_paths, int32_t u, int32_t v, int32_t w) {
+  if (n_paths <= 0 || u <= 0 || v <= 0 || w <= 0) return 0;
+  // any kind: the matrices of a path run over one of the operands' channels
+  return (int64_t)n_paths * u * v * w * 4 + ((int64_t)n_paths * (u > v ? u : v) * 4 + 15) / 16 * 16;
+}
+
+int cgtp_uvsw_validate(int cfg, int kind, const void* x, const void* z, const void* packed, const void* w, const void* out,
+                       int64_t n_rows, int32_t u, int32_t v, int32_t c) {
+  const UvsEntry* e = nullptr;
+  int64_t lds = 0;
+  return uvsw_check(cfg, kind, x, z, packed, w, out, n_rows, u, v, c, &e, &lds);
+}
+
+int cgtp_uvsw_apply(int cfg, int kind, const void* x, const void* z, void* packed, const void* w, void* out, int64_t n_rows,
+                    int32_t u, int32_t v, int32_t c, void* stream) {
+  const UvsEntry* e = nullptr;
+  int64_t lds = 0;
+  int st = uvsw_check(cfg, kind, x, z, packed, w, out, n_rows, u, v, c, &e, &lds);
+  if (st != CGTP_OK || n_rows == 0) return st;
+  const int cin = kind == 0 ? u : c, cout = kind == 0 ? c : kind == 1 ? u : v;
+  const UvsWeight W = uvsw_weight((const float*)w, kind, u, v, c);
+  const int64_t matrices = (int64_t)e->p * W.matrices;
+  st = uvs_pack(W, packed, matrices, cin, cout, (hipStream_t)stream);
+  if (st != CGTP_OK) return st;
+  const UvsFn fn = e->fn_w[kind];
+  if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return CGTP_ERR_LDS;
+  hipLaunchKernelGGL(fn, dim3((unsigned)((n_rows + kUvsSamples - 1) / kUvsSamples), (unsigned)(cout / 32)), dim3(256),
+                     (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)z, (const _Float16*)packed,
+                     (const float*)((const _Float16*)packed + matrices * cin * cout * 2), (float*)out, n_rows, cout, W);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
 }
 

@@ -411,6 +411,17 @@ int cgtp_uvs_validate(int cfg, int kind, const void* x, const void* y, const voi
 int cgtp_uvs_apply(int cfg, int kind, const void* x, const void* y, const void* packed, const void* w, void* out,
                    int64_t n_rows, int32_t cin, int32_t cout, void* stream);
 
+/* The same with channels on both operands and a weight (P, u, v, c) ("uvw"), contiguous.  kind 0: forward, x (n_rows, D1, u),
+ * z (n_rows, D2, v), out (n_rows, DO, c); 1: gradient of x, x = grad_out (n_rows, DO, c), z (n_rows, D2, v), out
+ * (n_rows, D1, u); 2: gradient of z, x = grad_out, z = the first operand (n_rows, D1, u), out (n_rows, D2, v).  32
+ * contracted channels (u, c, c), a multiple of 32 produced ones, at most nine produced rows.  packed:
+ * cgtp_uvsw_packed_bytes() bytes of scratch. */
+int64_t cgtp_uvsw_packed_bytes(int32_t n_paths, int32_t u, int32_t v, int32_t w);
+int cgtp_uvsw_validate(int cfg, int kind, const void* x, const void* z, const void* packed, const void* w, const void* out,
+                       int64_t n_rows, int32_t u, int32_t v, int32_t c);
+int cgtp_uvsw_apply(int cfg, int kind, const void* x, const void* z, void* packed, const void* w, void* out, int64_t n_rows,
+                    int32_t u, int32_t v, int32_t c, void* stream);
+
 /* ---- radial basis and cutoff envelopes ---------------------------------------------------------------------------
  *
  * Element-wise functions of the edge length r (n values), fp32 / fp64, one launch forward and one for the gradient.

@@ -79,3 +79,65 @@ def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, 
         fin = torch.isfinite(b)
         assert torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
         assert float((a[fin] - b[fin]).norm()) <= 1e-6 * float(b[fin].norm())
+
+
+# ---- channels on both operands ("uvw"): cgtp_uvsw_apply -----------------------------------------------------------
+def _uvw_routes(monkeypatch, device, lmax, u, v, c, operands):
+    from equitorch_amd.nn import TensorProduct
+    from equitorch_amd.nn.functional import _uv_native
+    mod = TensorProduct(SH[lmax], SH[lmax], SH[lmax], u, v, c, feature_mode="uvw", internal_weights=False).to(device)
+    kinds, split = [], _uv_native._split_uvw
+
+    def spy(kind, *args):
+        out = split(kind, *args)
+        kinds.append((kind, out is not None))
+        return out
+    monkeypatch.setattr(_uv_native, "_split_uvw", spy)
+    new = _step(mod, device, *operands)
+    monkeypatch.setattr(_uv_native, "_split_uvw", lambda *args: None)
+    return new, _step(mod, device, *operands), sorted(kinds)
+
+
+def _uvw_operands(lmax, u, v, c, n, seed):
+    d, gen = (lmax + 1) ** 2, torch.Generator().manual_seed(seed)
+    paths = {1: 4, 2: 11}[lmax]
+    return [torch.randn(n, d, u, generator=gen), torch.randn(n, d, v, generator=gen),
+            torch.randn(paths, u, v, c, generator=gen) / u, torch.randn(n, d, c, generator=gen)]
+
+
+@pytest.mark.parametrize("lmax,u,v,c,n,taken", [(1, 32, 32, 32, 1, (1, 1, 1)), (2, 32, 32, 32, 333, (1, 1, 1)),
+                                                (2, 32, 20, 64, 50, (1, 0, 0)), (2, 64, 32, 32, 17, (0, 1, 1)),
+                                                (1, 32, 4, 32, 40, (1, 1, 0)), (2, 32, 64, 32, 31, (1, 1, 1))])
+@pytest.mark.parametrize("values", ["normal", "wide"])
+def test_uvw_no_less_precise_than_fp32_matrix_instructions(device, monkeypatch, lmax, u, v, c, n, taken, values):
+    ops = _uvw_operands(lmax, u, v, c, n, stable_seed("uvw split", lmax, u, v, c, n))
+    if values == "wide":
+        gen = torch.Generator().manual_seed(3)
+        for t in ops:
+            t.mul_(torch.exp2(torch.randint(-20, 21, (t.shape[0],) + (1,) * (t.ndim - 1), generator=gen).float()))
+        ops[0].mul_(torch.exp2(torch.randint(-10, 11, ops[0].shape, generator=gen).float()))
+    new, old, kinds = _uvw_routes(monkeypatch, device, lmax, u, v, c, ops)
+    assert kinds == [(k, bool(t)) for k, t in enumerate(taken)]
+    T = ref_ops.dense_coupling(SH[lmax], SH[lmax], SH[lmax]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_uvw, T, ops[:3], ops[3])
+    for k, (name, want) in enumerate(zip(("out", "grad x", "grad y"), (ref_out, *ref_grads[:2]))):
+        def err(a):
+            d, w = (a.cpu().double() - want).flatten(1).norm(dim=1), want.flatten(1).norm(dim=1)
+            return float((d / w.clamp_min(1e-30)).square().mean().sqrt())
+        e_new, e_old = err(new[k]), err(old[k])
+        print(f"uvw {name} lmax={lmax} {u},{v}->{c} n={n} {values}: split {e_new:.2e} fp32 {e_old:.2e}")
+        assert e_new <= (1.1 if n >= 300 else 2.0) * e_old + 3e-8, name
+
+
+@pytest.mark.parametrize("where,value", [(0, float("inf")), (1, float("nan")), (1, float("inf")), (2, float("inf")),
+                                         (3, float("-inf")), (0, 3e38), (2, 1e25)])
+def test_uvw_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, where, value):
+    ops = _uvw_operands(2, 32, 32, 32, 50, 6)
+    ops[where].view(-1)[567] = value
+    new, old, kinds = _uvw_routes(monkeypatch, device, 2, 32, 32, 32, ops)
+    for a, b in zip(new, old):
+        fin = torch.isfinite(b)
+        assert torch.equal(fin, torch.isfinite(a))
+        # the fp32 route sums chains of 1024 products times the rows of a path: rounding 6e-8 each at random, 6e-8 * sqrt(1024)
+        # = 2e-6 of the result (0.6e-6 to 1.5e-6 measured against 64 bits in the test above)
+        assert float((a[fin] - b[fin]).norm()) <= 2e-6 * float(b[fin].norm())
