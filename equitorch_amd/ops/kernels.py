@@ -6,6 +6,7 @@ enqueues on torch's current stream.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import weakref
 from typing import Optional, Tuple
 
@@ -826,20 +827,26 @@ class UvuTable:
         paths = np.concatenate([walk, [0xffff, 0xffff]]).astype(np.uint32)
         self.dims = (int(coo.D1), int(coo.D2), int(coo.DO), int(coo.P))
         self.nnz, self.n_segments = nnz, int(last_of_seg.sum())
-        self.coef = torch.from_numpy(coef).to(device)
-        self.idx = torch.from_numpy(idx.view(np.int32).copy()).to(device)
-        self.paths = torch.from_numpy(paths.view(np.int32).copy()).to(device)
+        words = _mx_words_of_content(*(int(v) for v in (coo.D1, coo.D2, coo.DO, coo.P)),
+                                     *(np.ascontiguousarray(v, dtype=d).tobytes() for v, d in
+                                       ((coo.coef, np.float64), (coo.M, np.int32), (coo.M1, np.int32), (coo.M2, np.int32),
+                                        (coo.p, np.int32))))
+        # one copy to the device for all arrays, each on a 256-byte boundary
+        arrays = {"coef": coef.view(np.uint32), "idx": idx, "paths": paths}
+        if words is not None:
+            arrays.update((k, v) for k, v in words.items() if isinstance(v, np.ndarray))
+        at, parts = {}, []
+        for k, v in arrays.items():
+            at[k] = 4 * sum(part.shape[0] for part in parts)
+            parts.append(np.concatenate([v, np.zeros(-v.shape[0] % 64, dtype=np.uint32)]))
+        self.words = torch.from_numpy(np.concatenate(parts).view(np.int32)).to(device)
+        base = self.words.data_ptr()
         t = _lib.UvuTab()
-        t.coef, t.idx, t.paths = (v.data_ptr() for v in (self.coef, self.idx, self.paths))
+        t.coef, t.idx, t.paths = (base + at[k] for k in ("coef", "idx", "paths"))
         t.nnz, t.n_segments = self.nnz, self.n_segments
         t.D1, t.D2, t.DO, t.P = self.dims
         self.c = t
-        words = uvu_mx_words(coo)
-        self.mx = None
-        if words is not None:
-            self.mx_words = {k: torch.from_numpy(v.view(np.int32)).to(device) for k, v in words.items()
-                             if isinstance(v, np.ndarray)}
-            self.mx = _lib.UvuMx(**{k: self.mx_words[k].data_ptr() if k in self.mx_words else v for k, v in words.items()})
+        self.mx = None if words is None else _lib.UvuMx(**{k: base + at[k] if k in at else v for k, v in words.items()})
 
 
 def uvu_mx_words(coo) -> Optional[dict]:
@@ -957,6 +964,14 @@ def uvu_mx_words(coo) -> Optional[dict]:
             "fwd_records": len(elements), "fwd_entries": len(fwd_entries), "bwd_records": len(elements),
             "bwd_entries": len(bwd_entries), "row_tiles": row_tiles, "rounds": rounds, "lanes_log2": lanes_log2,
             "tiles": len(tiles) // 5}
+
+
+@functools.lru_cache(maxsize=32)
+def _mx_words_of_content(D1: int, D2: int, DO: int, P: int, coef: bytes, *indices: bytes) -> Optional[dict]:
+    """:func:`uvu_mx_words` by the table's content: half a millisecond of host work that a second module over the same
+    irreps does not repeat.  Host arrays only, read by every caller and written by none."""
+    M, M1, M2, p = (np.frombuffer(v, dtype=np.int32) for v in indices)
+    return uvu_mx_words(TpCoo(np.frombuffer(coef, dtype=np.float64), M, M1, M2, p, p, D1, D2, DO, P))
 
 
 def uvu_table_of(tp_info, device) -> Optional[UvuTable]:

@@ -175,7 +175,7 @@ def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, 
     for route in ("matrix", "entries"):
         info = _info(irreps).to(device)
         if route == "entries":
-            monkeypatch.setattr(kernels, "uvu_mx_words", lambda coo: None)
+            monkeypatch.setattr(kernels, "_mx_words_of_content", lambda *content: None)
         wrt = [t.to(device).requires_grad_(True) for t in (x, y, w)]
         out = edge_tensor_product_uu(*wrt, plan, info)
         assert (kernels.uvu_table_of(info, wrt[0].device).mx is None) == (route == "entries")
@@ -227,3 +227,38 @@ def test_the_wide_walk_covers_the_table(irreps):
         assert pair * 2 == n_items and sorted(rows_seen) == list(range(n_prod))
         assert paths == set(range(coo.P))
         np.testing.assert_allclose(got[:, :n_prod, :n_con], want, rtol=0, atol=1e-12)
+
+
+@pytest.mark.gpu
+def test_recorded_in_a_graph(device):
+    """Forward and gradients recorded into a HIP graph and replayed on new inputs, eager work in between: the flags of the
+    ranges are written anew by every replay (the second one sees a value that is not finite, the third none again)."""
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    info = _info(TABLES[1]).to(device)
+    src, dst, x, y, w, ct = _edge_case(TABLES[1], 64, 40, 700, False, 9)
+    plan = EdgePlan(src.to(device), dst.to(device), 40)
+    inputs = [t.to(device).requires_grad_(True) for t in (x, y, w)]
+    ct = ct.to(device)
+
+    def step():
+        out = edge_tensor_product_uu(*inputs, plan, info)
+        return (out, *torch.autograd.grad(out, inputs, ct))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = step()
+    for replay in range(3):
+        with torch.no_grad():
+            for t in inputs:
+                t.copy_(torch.randn(t.shape, generator=torch.Generator().manual_seed(replay)))
+            if replay == 1:
+                inputs[0][3, 2, 5] = float("inf")
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(recorded, step()):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num()), replay

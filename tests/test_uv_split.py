@@ -141,3 +141,37 @@ def test_uvw_values_that_are_not_finite_stay_where_they_couple(device, monkeypat
         # the fp32 route sums chains of 1024 products times the rows of a path: rounding 6e-8 each at random, 6e-8 * sqrt(1024)
         # = 2e-6 of the result (0.6e-6 to 1.5e-6 measured against 64 bits in the test above)
         assert float((a[fin] - b[fin]).norm()) <= 2e-6 * float(b[fin].norm())
+
+
+@pytest.mark.parametrize("mode", ["uv", "uvw"])
+def test_recorded_in_a_graph(device, mode):
+    """Forward and gradients recorded into a HIP graph and replayed on new inputs and weights: the weights are packed anew by
+    every replay."""
+    if mode == "uv":
+        mod, ops = _operands(device, 2, 64, 64, 50, 4)
+    else:
+        from equitorch_amd.nn import TensorProduct
+        ops = _uvw_operands(2, 32, 32, 32, 50, 4)
+        mod = TensorProduct(SH[2], SH[2], SH[2], 32, 32, 32, feature_mode="uvw", internal_weights=False).to(device)
+    inputs, ct = [t.to(device).requires_grad_(True) for t in ops[:3]], ops[3].to(device)
+
+    def step():
+        out = mod(*inputs)
+        return (out, *torch.autograd.grad(out, inputs, ct))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = step()
+    for replay in range(3):
+        with torch.no_grad():
+            for t in inputs:
+                t.copy_(torch.randn(t.shape, generator=torch.Generator().manual_seed(replay)) * 2.0 ** (5 * replay))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(recorded, step()):
+            assert torch.equal(a, b), replay
