@@ -17,7 +17,10 @@
 //
 // What bounds it: a workgroup of four wavefronts owns 16 samples, whose rows (4 bytes an element, both halves) fill most
 // of the LDS at 128 channels and lmax = 3, and every workgroup reads all the weights from L2, 1.5 MB there.
-// @FIGURES@
+// One wavefront per SIMD at 128 channels: matrix pipeline 34 % busy, LDS reads 35 % (bank conflicts another 16 %), vector
+// instructions 30 %.  128 -> 128 channels, lmax = 3, 32768 samples: forward 1312 -> 426 us, gradient of x 1314 -> 410, of y
+// 1868 -> 422 (fp32 matrix instructions, coupling first, against this); 64 -> 64, lmax = 2: 138 / 134 / 188 -> 62 / 63 / 62;
+// 512 samples of 128 channels, lmax = 3: 161 / 161 / 228 -> 51 / 52 / 53.
 //
 // Rows of x or paths of W that hold an infinity, a NaN or a magnitude past 2^64 are not split, nor is anything multiplied
 // by a y that is not finite: the workgroup then forms its samples' results with fp32 matrix instructions, term by term
