@@ -936,7 +936,7 @@ def uvu_mx_words(coo) -> Optional[dict]:
         if len(set(covered)) != len(covered):
             return None
         chunks += [(r, 1, None) for r in range(D1) if r not in covered]      # rows nothing couples to
-        items, at, ends = [], {}, []
+        items, at, ends, opened = [], {}, [], set()
         for r0, n, block in chunks:
             mine = [(out_rows[p][0] + 7 * j, min(7, out_rows[p][1] - 7 * j), p) for p in range(P) if x_rows[p] == block
                     for j in range((out_rows[p][1] + 6) // 7)]
@@ -944,8 +944,9 @@ def uvu_mx_words(coo) -> Optional[dict]:
                 for k in range(rows):
                     for r in range(n):
                         at[p, m0 + k, r0 + r] = len(items) // 2 * 64 + (8 * (len(items) % 2) + k) * 4 + r
-                opens = r0 == block[0] and m0 == out_rows[p][0]
-                items.append(p | m0 << 8 | (rows | 1) << 16 | (not opens) << 20)
+                # the first item of a path sets its row of the weight gradient, whichever rows it holds; the others add
+                items.append(p | m0 << 8 | (rows | 1) << 16 | (p in opened) << 20)
+                opened.add(p)
             if len(items) % 2:
                 items.append(1 << 16 | 1 << 20)
             ends.append(len(items) // 2)

@@ -7,7 +7,8 @@ import torch
 from helpers import assert_close, stable_seed
 from oracle import ref_ops
 
-# (out, in1, in2): several multiplicities, one row only, 16 rows on either side, 32 rows of y, an uncoupled middle
+# (out, in1, in2): several multiplicities, one row only, 16 rows on either side, 32 rows of y, an uncoupled middle,
+# output irreps of more than seven rows (two or more items of the four-row walk per path)
 TABLES = [
     ("1o+2e+1e", "0e+1o+2e", "0e+1o"),
     ("0e+1o+2e+3o", "1o+2e+3o", "0e+1o+2e"),
@@ -15,6 +16,10 @@ TABLES = [
     ("0e", "0e", "0e+0e"),
     ("0e+1e+2e+3e", "0e+1o+2e+3o", "0e+1o"),
     ("1o+3o", "0e+3o", "0e+1o+2e+3o+4e"),
+    ("0e+4e", "0e+1o+2e", "0e+1o+2e+3o+4e"),
+    ("1o+5o", "0e+1o+2e", "0e+1o+2e+3o+4e"),
+    ("4e", "4e", "0e+2e"),
+    ("7o", "0e+4e", "3o+4e"),
 ]
 
 
@@ -190,11 +195,16 @@ def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, 
 @pytest.mark.parametrize("irreps", TABLES)
 def test_the_wide_walk_covers_the_table(irreps):
     """The walk of the kernels with one channel per lane: the coupling matrix of every item, put back in its place, is the
-    table's, and every path and produced row is visited once."""
+    table's, every path and produced row is visited once, and the gradients of one edge formed as the kernel forms them
+    (the weight gradient's rows hold another edge's values at first) are those of the table's entries."""
     from equitorch_amd.ops import kernels
     coo = kernels.coo_of(_info(irreps))
     m = kernels.uvu_mx_words(coo)
-    y = np.random.default_rng(3).standard_normal(coo.D2)
+    rng = np.random.default_rng(3)
+    y, C = rng.standard_normal(coo.D2), 3
+    x, w, g = (rng.standard_normal(s) for s in ((coo.D1, C), (coo.P, C), (coo.DO, C)))
+    gz = np.concatenate([g, np.zeros((6, C))])
+    gx, gw = np.zeros((coo.D1, C)), rng.standard_normal((coo.P, C))
     f32 = lambda v: float(np.uint32(v).view(np.float32))     # noqa: E731
     for which, produced, contracted, n_prod, n_con in (("bwd", coo.M1, coo.M, coo.D1, coo.DO),):
         words, n_items, n_chunks = m[which + "4"], m[which + "4_items"], m[which + "4_chunks"]
@@ -220,13 +230,18 @@ def test_the_wide_walk_covers_the_table(irreps):
                     slots = A[pair * 64 + 32 * h:pair * 64 + 32 * h + 32].reshape(8, 4)
                     assert not slots[rows:].any() and not slots[:, n:].any()
                     got[p, r0:r0 + 4, row:row + rows] += slots[:rows].T
-                    if slots.any():
+                    D = slots[:7].T[:n] @ gz[row:row + 7]
+                    gx[r0:r0 + n] += w[p] * D
+                    gw[p] = (gw[p] if k >> 20 & 1 else 0) + (x[r0:r0 + n] * D).sum(0)
+                    if slots.any() or not k >> 20 & 1:             # all but an item that only fills a pair
                         assert bool(k >> 20 & 1) == (p in paths)        # sets the path's gradient, then adds to it
                         paths.add(p)
                 pair += 1
         assert pair * 2 == n_items and sorted(rows_seen) == list(range(n_prod))
         assert paths == set(range(coo.P))
         np.testing.assert_allclose(got[:, :n_prod, :n_con], want, rtol=0, atol=1e-12)
+        np.testing.assert_allclose(gx, np.einsum("prk,kc,pc->rc", want, g, w), rtol=0, atol=1e-12)
+        np.testing.assert_allclose(gw, np.einsum("prk,kc,rc->pc", want, g, x), rtol=0, atol=1e-12)
 
 
 @pytest.mark.gpu
