@@ -41,7 +41,7 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
     """Body of one configuration.  ``gy``: instead of accumulating output rows, contract every tile with the rows of
     a second channelled operand ``g`` (the output gradient) into the gradient w.r.t. the harmonics,
     ``gy[b] += coef * sum_w g[m, w] * Z[w]`` (forward tables only).  ``split``: the body for single precision, in which
-    the operands' fragments and the contraction are the caller's (``Ops``) and every tile comes with a factor per lane."""
+    the operands' fragments and the contraction are the caller's (``Ops``)."""
     if direction == 0:
         out_idx, in_idx, blocks, din, dout = coo.M, coo.M1, seg_out, coo.D1, coo.DO
     else:
@@ -61,7 +61,8 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         first_of_block[len(tiles)] = list(range(b0, b1))
         tiles += list(d.items())
         last_of_block[len(tiles) - 1] = list(range(b0, b1))
-    # weight fragments live in a ring of three buffers, fetched two path-runs ahead of their first use
+    # weight fragments live in a ring of three buffers, fetched two path-runs ahead of their first use; of two in the split
+    # body, whose fragments are three times as large
     runs = []  # (path, first tile)
     for k, ((p, _), _) in enumerate(tiles):
         if not runs or runs[-1][0] != p or k in first_of_block:
@@ -80,7 +81,7 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         a("  // xs: this lane's base into the staged input tile (row a of the sample at byte a * CIN * 2);")
         a("  // load_a(p, frag): fetch the weight fragments of path p;")
     if split:
-        a("  // ops: load_a(p, A&), load_b(row, B&), chain(A, B, z0, z1), scale(p, row): the factor of the tile;")
+        a("  // ops: load_a(p, A&), load_b(row, B&), chain(A, B, Z&), sum(Z, z0, z1);")
         a("  // sink: store(row, t0, t1) emits a finished output row / load_g(row, t0, t1) this lane's channels of g")
         a("  template <class Ops, class Sink>")
         a(f"  __device__ __forceinline__ static void run(const Ops& ops, {'' if gy else 'const '}float (&y)[D2], Sink&& sink) {{")
@@ -95,9 +96,9 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         a("  __device__ __forceinline__ static void run(const unsigned char* xs, LoadA&& load_a, const float (&y)[D2],")
         a("                                             Store&& store) {")
     if split:
-        a("    typename Ops::A w0, w1, w2;")
+        a("    typename Ops::A w0, w1;")
         a("    typename Ops::B b0, b1;")
-        a("    float fa = 0.f, fb = 0.f;")
+        a("    typename Ops::Z za, zb;")
     else:
         a("    constexpr int KS = CIN / 32;")
         a("    bf16x8 w0[2][KS], w1[2][KS], w2[2][KS], b0[KS], b1[KS];")
@@ -117,16 +118,19 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
             return
         a(f"    load_b<KS>(b{k % 2}, xs + {tiles[k][0][1]} * CIN * 2);")
 
+    n_w = 2 if split else 3
+
     def chain(k):
         z = "za" if k % 2 == 0 else "zb"
         if split:
-            a(f"    ops.chain(w{run_of_tile[k] % 3}, b{k % 2}, {z}0, {z}1); "
-              f"f{z[1]} = ops.scale({tiles[k][0][0]}, {tiles[k][0][1]});")
+            a(f"    ops.chain(w{run_of_tile[k] % n_w}, b{k % 2}, {z});")
         else:
-            a(f"    mfma_chain<KS>(w{run_of_tile[k] % 3}, b{k % 2}, {z}0, {z}1);")
+            a(f"    mfma_chain<KS>(w{run_of_tile[k] % n_w}, b{k % 2}, {z}0, {z}1);")
         j = run_of_tile[k]
-        if runs[j][1] == k and j + 2 < len(runs):
-            a(f"    {load_a}({runs[j + 2][0]}, w{(j + 2) % 3});")
+        # a ring of three is refilled when a run starts, one of two when it ends
+        at = runs[j][1] if n_w == 3 else (runs[j + 1][1] if j + 1 < len(runs) else len(tiles)) - 1
+        if at == k and j + 2 < len(runs):
+            a(f"    {load_a}({runs[j + 2][0]}, w{(j + 2) % n_w});")
 
     if tiles:
         a(f"    {load_a}({runs[0][0]}, w0);")
@@ -151,10 +155,11 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
         if k + 2 < len(tiles):
             load_b(k + 2)
         cur = "za" if k % 2 == 0 else "zb"
-        factor = f" * f{cur[1]}" if split else ""
+        if split:
+            a(f"    ops.sum({cur}, {cur}0, {cur}1);")
         if gy:
             for (o, m2, c) in terms:
-                a(f"    yy[{m2}] += {_lit(c)}{factor} * dot8(o{o}_0, o{o}_1, {cur}0, {cur}1);")
+                a(f"    yy[{m2}] += {_lit(c)} * dot8(o{o}_0, o{o}_1, {cur}0, {cur}1);")
             # pin the partial sums (see the accumulators of the forward body)
             a("    asm volatile(\"\" : " + ", ".join(f'"+v"(yy[{m}])' for m in sorted({m2 for _, m2, _ in terms})) + ");")
             a("    __builtin_amdgcn_sched_barrier(0);")
@@ -168,8 +173,6 @@ def emit_direction(name: str, direction: int, coo, seg_out, seg_in1, gy: bool = 
             by_row.setdefault(o, []).append((m2, c))
         for o, pairs in by_row.items():
             s_expr = " + ".join(f"{_lit(c)} * yy[{m2}]" for m2, c in pairs)
-            if split:
-                s_expr = f"({s_expr}){factor}"
             a(f"    {{ const float s = {s_expr}; o{o}_0 += s * {cur}0; o{o}_1 += s * {cur}1; }}")
         # pin the updated accumulators: an output row is read again only when it is stored, and without this the
         # optimiser sinks every update of a block to its end, keeping all the block's tiles alive until then

@@ -6,34 +6,43 @@
 // transposed) and the gradient of y.  The order is that of uv_mfma.hip: per weight path and input row two accumulator
 // tiles Z = x W, then the coefficients as fp32 multiply-adds between accumulator tiles.
 //
-// Every fp32 operand a is carried as two halves: with a scaled by a power of two (the largest element of its row of x,
-// or of its path of W, lies in [2^13, 2^14)), h = half(a), l = half(a - h).  h + l is a to 2^-24 of it — as near as the
-// rounding of a itself — for elements down to 2^-16 of the largest, and to 2^-39 of the largest below.  Z is h h' + h l' +
-// l h' (the product l l' is below 2^-24 of the element products), each product exact in fp32 and summed in fp32, 32
-// of them to a rounding; the factor that undoes the scales joins the coefficient.  Relative error of Z against 64 bits at
-// 128 channels: 0.8e-7, of a chain of fp32 multiply-adds 2.0e-7; of the results over the range of sizes:
-// 1.2e-7 to 1.7e-7 where fp32 matrix instructions give 1.6e-7 to 5.1e-7 (lmax 1 to 3, 32 to 128 channels).
-// The same contraction in fp32 matrix instructions takes 256 cycles per 16 x 16 tile and 32 channels, this one 48.
+// Every fp32 operand a is carried as three bf16 parts, h = bf16(a), m = bf16(a - h), l = a - h - m: 8 bits each, together
+// all 24 of a, and bf16 has the exponents of fp32, so no scales (2^-110 <= |a| < 2^60; see below).  Z is h h' + h m' + m h' +
+// h l' + l h' + m m', each product exact in fp32, 32 of them summed to a rounding, the five small ones by themselves; what is
+// dropped (m l', l m', l l') is about 2^-24 of an element product at most, one rounding of it, and 2^-27 as a rule.  Errors of
+// the results against 64 bits, lmax 1 to 3, 32 to 128 channels: 0.5e-7 to 1.7e-7 where fp32 matrix instructions give 0.9e-7 to
+// 5.1e-7; with channels and elements spread over thirty binary orders never above them.  The same contraction in fp32
+// matrix instructions takes 256 cycles per 16 x 16 tile and 32 channels, this one 96.  (Two half-precision parts and three
+// products, 48 cycles, need a common scale per row and path: elements and channels far below the largest lose bits, and
+// so do products far from 1.)
 //
-// What bounds it: a workgroup of four wavefronts owns 16 samples, whose rows (4 bytes an element, both halves) fill most
-// of the LDS at 128 channels and lmax = 3, and every workgroup reads all the weights from L2, 1.5 MB there.
-// One wavefront per SIMD at 128 channels: matrix pipeline 34 % busy, LDS reads 35 % (bank conflicts another 16 %), vector
-// instructions 30 %.  128 -> 128 channels, lmax = 3, 32768 samples: forward 1312 -> 426 us, gradient of x 1314 -> 410, of y
-// 1868 -> 422 (fp32 matrix instructions, coupling first, against this); 64 -> 64, lmax = 2: 138 / 134 / 188 -> 62 / 63 / 62;
-// 512 samples of 128 channels, lmax = 3: 161 / 161 / 228 -> 51 / 52 / 53.
+// What bounds it: a workgroup of four wavefronts owns 16 samples, whose rows (4 or 6 bytes an element) fill most of the LDS at
+// 128 channels and lmax = 2 and 3, and every workgroup reads all the weights from L2, 2.3 MB there.  One wavefront per
+// SIMD at 128 channels (lmax = 3): matrix pipeline 41 % busy, vector instructions 39 %, waiting for data 18 %.  128 -> 128
+// channels, lmax = 3, 32768 samples: forward 1308 -> 677 us, gradient of x 1316 -> 679, of y 1879 -> 649 (fp32 matrix
+// instructions, coupling first, against this); 64 -> 64, lmax = 2: 140 / 135 / 188 -> 77 / 76 / 74; 500 samples of 128 channels,
+// lmax = 3: 161 / 162 / 228 -> 82 / 82 / 79.  Splitting the rows in every tile that reads them took 800 us there (vector
+// instructions 52 %): as many rows as fit are staged as parts (UvsLds), the others split between matrix instructions.
 //
-// Rows of x or paths of W that hold an infinity, a NaN or a magnitude past 2^64 are not split, nor is anything multiplied
-// by a y that is not finite: the workgroup then forms its samples' results with fp32 matrix instructions, term by term
-// of the table and the coupling first (uvs_plain_tile), so that such values reach exactly the results they couple to.
+// An x or W with an element that is not finite, from 2^60 on (Z could overflow where coupling first does not) or below 2^-110 but
+// not zero (its last part could be below the smallest subnormal), a y that is not finite, or a y of 16 and more next to an x or W below 2^-50 (Z could
+// underflow where coupling first does not) is not split: the workgroup then forms its samples' results with fp32 matrix
+// instructions, term by term of the table and the coupling first (uvs_plain_tile), so that such values reach exactly the
+// results they couple to.
 #include "uv_common.h"
+
+#include <algorithm>
 
 // accumulator-tile updates are written as o += s * z; let them contract to FMAs in this file
 #pragma clang fp contract(fast)
 
 namespace cgtp {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 struct UvsTerm {
   float c;
@@ -43,13 +52,68 @@ struct UvsTerm {
 #include "generated/uv_split_configs.inc"
 
 constexpr int kUvsSamples = 16;
-constexpr unsigned kUvsMaxExp = 127 + 64;      // biased exponent from which an operand is not split
 
-// Power of two that takes a value with biased exponent e (below kUvsMaxExp; 0 counts as the smallest normal range handled)
-// into [2^13, 2^14), and its inverse.
-__device__ __forceinline__ unsigned uvs_exp(unsigned abs_bits) { return max(abs_bits >> 23, 14u); }
-__device__ __forceinline__ float uvs_scale(unsigned e) { return __builtin_bit_cast(float, (267u - e) << 23); }
-__device__ __forceinline__ float uvs_unscale(unsigned e) { return __builtin_bit_cast(float, (e - 13u) << 23); }
+// What an operand's elements ask for, or'ed over them.
+constexpr unsigned kUvsPlain = 1;       // not to be split
+constexpr unsigned kUvsSmall = 2;       // an element of x or W below 2^-50 (and not zero): its products with another such one
+constexpr unsigned kUvsLargeY = 4;      // may be subnormal, which shows in the results only next to a y of 16 and more
+__device__ __forceinline__ unsigned uvs_asks(float a) {
+  const unsigned b = __builtin_bit_cast(unsigned, a) & 0x7fffffffu;
+  const unsigned nonzero = b - 1u;      // 0 becomes the largest
+  return (b >= (127u + 60) << 23 || nonzero < ((127u - 110) << 23) - 1 ? kUvsPlain : 0) |
+         (nonzero < ((127u - 50) << 23) - 1 ? kUvsSmall : 0);
+}
+__device__ __forceinline__ unsigned uvs_asks_y(float y) {
+  return (y - y != 0.f ? kUvsPlain : 0) | (fabsf(y) >= 16.f ? kUvsLargeY : 0);
+}
+// The three parts of pairs of elements, one conversion instruction for two (left element by element, each takes its own).
+__device__ __forceinline__ unsigned uvs_pair(float a, float b) {
+  const floatx2 v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ float uvs_low(unsigned pair) { return __builtin_bit_cast(float, pair << 16); }
+__device__ __forceinline__ float uvs_high(unsigned pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
+template <int N>
+struct UvsParts {
+  unsigned p[3][N / 2];
+  float a, b;            // what is left of the pair in work
+  // Three, three and five instructions.
+  template <int STAGE>
+  __device__ __forceinline__ void stage(int j, float x, float y) {
+    if constexpr (STAGE == 0) {
+      p[0][j] = uvs_pair(x, y);
+      a = uvs_low(p[0][j]);
+      b = uvs_high(p[0][j]);
+    } else if constexpr (STAGE == 1) {
+      a = x - a;
+      b = y - b;
+      p[1][j] = uvs_pair(a, b);
+    } else {
+      p[2][j] = uvs_pair(a - uvs_low(p[1][j]), b - uvs_high(p[1][j]));
+    }
+  }
+  __device__ __forceinline__ void pair(int j, float x, float y) {
+    stage<0>(j, x, y);
+    stage<1>(j, x, y);
+    stage<2>(j, x, y);
+  }
+};
+__device__ __forceinline__ bf16x8 uvs_frag(const unsigned (&p)[4]) {
+  return __builtin_bit_cast(bf16x8, u32x4{p[0], p[1], p[2], p[3]});
+}
+
+// Barrier; `m` or'ed over the workgroup's four wavefronts (`words`: four words of LDS).
+__device__ __forceinline__ unsigned uvs_all(unsigned m, unsigned* words) {
+  unsigned w = 0;
+#pragma unroll
+  for (unsigned bit = 1; bit <= kUvsLargeY; bit <<= 1) w |= __any((m & bit) != 0) ? bit : 0;
+  if ((threadIdx.x & (kWave - 1)) == 0) words[threadIdx.x / kWave] = w;
+  __syncthreads();
+  return words[0] | words[1] | words[2] | words[3];
+}
+__device__ __forceinline__ bool uvs_is_plain(unsigned m) {
+  return (m & kUvsPlain) || ((m & kUvsSmall) && (m & kUvsLargeY));
+}
 
 // The weight as the caller holds it.  With channels on both operands a path has one matrix per channel l of the operand
 // that is not contracted; `matrices` is their number (else 1), and a "path" of the packed weight is a (path, l).
@@ -60,197 +124,206 @@ struct UvsWeight {
   __device__ __forceinline__ const float* of(int i) const { return w + (i / matrices) * stride_p + (i % matrices) * stride_l; }
 };
 
-// A workgroup per path and block of 32 output channels: the path's largest magnitude (every workgroup of a path reads all of
-// it: 64 KB at 128 channels, from L2), then both halves of its block in fragment order.  Per path and block 2 (half) x 2
-// (tile) x K / 32 chunks of 1 KB, holding the 16 bytes of every lane; row r of tile t is output channel
-// 8 (r / 4) + 4 t + r % 4 of the block.  inv[p]: what undoes the scale, a NaN for a path that is not split.
-__global__ void __launch_bounds__(256) uvs_pack_kernel(UvsWeight W, _Float16* __restrict__ packed, float* __restrict__ inv, int K,
+// A workgroup per path and block of 32 output channels: the parts of its block in fragment order.  Per path and block 3 (part)
+// x 2 (tile) x K / 32 chunks of 1 KB, holding the 16 bytes of every lane; row r of tile t is output channel
+// 8 (r / 4) + 4 t + r % 4 of the block.  asks: a word per path and block.
+__global__ void __launch_bounds__(256) uvs_pack_kernel(UvsWeight W, __bf16* __restrict__ packed, unsigned* __restrict__ asks, int K,
                                                        int cout) {
-  __shared__ unsigned waves_max[4];
+  __shared__ unsigned words[4];
   const int p = blockIdx.x, blk = blockIdx.y, ks = K / 32;
   const float* wp = W.of(p);
-  const int64_t stride_k = W.stride_k, stride_c = W.stride_c;
   unsigned m = 0;
-  // lanes along the axis of consecutive elements; K and cout are multiples of 32
-  const bool k_inner = stride_k == 1;
-  const int inner = k_inner ? K : cout;
-  const int64_t si = k_inner ? stride_k : stride_c, so = k_inner ? stride_c : stride_k;
-#pragma unroll 4
-  for (int i = threadIdx.x; i < K * cout; i += 256) {
-    const float v = wp[(i / inner) * so + (i % inner) * si];
-    m = max(m, __builtin_bit_cast(unsigned, v) & 0x7fffffffu);
-  }
-  for (int off = 1; off < kWave; off <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, kWave));
-  if ((threadIdx.x & (kWave - 1)) == 0) waves_max[threadIdx.x / kWave] = m;
-  __syncthreads();
-  for (int i = 0; i < 4; ++i) m = max(m, waves_max[i]);
-  const bool plain = (m >> 23) >= kUvsMaxExp;
-  const unsigned e = plain ? 127u : uvs_exp(m);
-  if (threadIdx.x == 0 && blk == 0) inv[p] = plain ? __builtin_nanf("") : uvs_unscale(e);
-  const float s = uvs_scale(e);
   for (int i = threadIdx.x; i < K * 4; i += 256) {             // fragments of eight k
     const int lane = i & 63, c = i >> 6, k = c % ks, t = c / ks;
     const int r = lane & 15, q = lane >> 4;
     const int row = blk * 32 + 8 * (r >> 2) + 4 * t + (r & 3), col = k * 32 + 8 * q;
-    f16x8 h, l;
+    float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float v = wp[(col + j) * stride_k + row * stride_c] * s;
-      h[j] = (_Float16)v;
-      l[j] = (_Float16)(v - (float)h[j]);
+      v[j] = wp[(col + j) * W.stride_k + row * W.stride_c];
+      m |= uvs_asks(v[j]);
     }
-    _Float16* dst = packed + (int64_t)p * K * cout * 2 + ((int64_t)(blk * 4 + t) * ks + k) * 512 + lane * 8;
-    *reinterpret_cast<f16x8*>(dst) = h;
-    *reinterpret_cast<f16x8*>(dst + (int64_t)2 * ks * 512) = l;
+    UvsParts<8> part;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part.pair(j, v[2 * j], v[2 * j + 1]);
+    __bf16* dst = packed + (int64_t)p * K * cout * 3 + ((int64_t)(blk * 6 + t) * ks + k) * 512 + lane * 8;
+#pragma unroll
+    for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(dst + (int64_t)h * 2 * ks * 512) = uvs_frag(part.p[h]);
   }
+  m = uvs_all(m, words);
+  if (threadIdx.x == 0) asks[p * (cout / 32) + blk] = m;
 }
 
-// LDS: per sample DIN rows of (CIN high halves, CIN low halves) and 16 bytes of padding; then what undoes the scale of every
-// row, [sample][DIN]; then that of every path, and four words (uvs_any).
+// LDS: per sample DIN rows and 16 bytes of padding, then four words (uvs_all).  The rows from kRaw on hold the three parts of
+// CIN elements each, the ones before (those of the low degrees, which fewer tiles read) CIN floats that every tile splits
+// anew: as many as the LDS asks for without costing a workgroup per compute unit (two at 32 and 64 channels, one at 128).
+constexpr int uvs_raw_rows(int din, int cin) {
+  for (int raw = 0; raw < din; ++raw)
+    if (kUvsSamples * (cin * (6 * din - 2 * raw) + 16) + 16 <= (cin < 128 ? kLdsBytes / 2 : kLdsBytes)) return raw;
+  return din;
+}
 template <int DIN, int CIN>
 struct UvsLds {
-  static constexpr int kRow = CIN * 4, kPitch = DIN * kRow + 16, kTile = kUvsSamples * kPitch;
+  static constexpr int kRaw = uvs_raw_rows(DIN, CIN), kPitch = CIN * (6 * DIN - 2 * kRaw) + 16, kTile = kUvsSamples * kPitch;
+  static __device__ __forceinline__ constexpr int row(int r) { return CIN * (6 * r - 2 * (r < kRaw ? r : kRaw)); }
 };
 
-// Stages the 16 samples' rows; true if none of this thread's rows has to be left unsplit.
+// Stages the 16 samples' rows; what this thread's elements ask for.
 template <int DIN, int CIN>
-__device__ __forceinline__ bool uvs_stage(const float* __restrict__ x, int64_t n0, int64_t n_rows, unsigned char* smem) {
+__device__ __forceinline__ unsigned uvs_stage(const float* __restrict__ x, int64_t n0, int64_t n_rows, unsigned char* smem) {
   using L = UvsLds<DIN, CIN>;
-  constexpr int PIECES = CIN / 4, TOTAL = kUvsSamples * DIN * PIECES;
-  float* inv = reinterpret_cast<float*>(smem + L::kTile);
-  bool ok = true;
+  constexpr int ROW = CIN / 4, PER = DIN * ROW, TOTAL = kUvsSamples * PER;
+  unsigned m = 0;
   constexpr int UNROLL = 8;
-  static_assert(TOTAL % kWave == 0, "whole wavefronts: the lanes of a row exchange their maxima");
   for (int base = 0; base < TOTAL; base += 256 * UNROLL) {
     f32x4 v[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int i = base + u * 256 + (int)threadIdx.x;
-      if (i < TOTAL) {
-        const int s = i / (DIN * PIECES), c = i % (DIN * PIECES);
-        v[u] = *reinterpret_cast<const f32x4*>(x + min(n0 + s, n_rows - 1) * (DIN * CIN) + c * 4);
-      }
+      if (i < TOTAL) v[u] = *reinterpret_cast<const f32x4*>(x + min(n0 + i / PER, n_rows - 1) * (DIN * CIN) + i % PER * 4);
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int i = base + u * 256 + (int)threadIdx.x;
       if (i < TOTAL) {
-        const int s = i / (DIN * PIECES), c = i % (DIN * PIECES), row = c / PIECES, piece = c % PIECES;
-        unsigned m = 0;
+        float a[4];                     // a bit cast of the vector's element itself would read element 0
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float a = v[u][j];      // a bit cast of the vector's element itself would read element 0
-          m = max(m, __builtin_bit_cast(unsigned, a) & 0x7fffffffu);
+          a[j] = v[u][j];
+          m |= uvs_asks(a[j]);
         }
+        unsigned char* row = smem + i / PER * L::kPitch + L::row(i % PER / ROW);
+        if (i % PER / ROW >= L::kRaw) {
+          UvsParts<4> part;
+          part.pair(0, a[0], a[1]);
+          part.pair(1, a[2], a[3]);
 #pragma unroll
-        for (int off = 1; off < PIECES; off <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, kWave));
-        ok = ok && (m >> 23) < kUvsMaxExp;
-        const unsigned e = min(uvs_exp(m), kUvsMaxExp);
-        const float sc = uvs_scale(e);
-        f16x4 h, l;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float a = v[u][j] * sc;
-          h[j] = (_Float16)a;
-          l[j] = (_Float16)(a - (float)h[j]);
+          for (int h = 0; h < 3; ++h)
+            *reinterpret_cast<u32x2*>(row + h * CIN * 2 + i % ROW * 8) = u32x2{part.p[h][0], part.p[h][1]};
+        } else {
+          *reinterpret_cast<f32x4*>(row + i % ROW * 16) = v[u];
         }
-        unsigned char* dst = smem + s * L::kPitch + row * L::kRow + piece * 8;
-        *reinterpret_cast<f16x4*>(dst) = h;
-        *reinterpret_cast<f16x4*>(dst + CIN * 2) = l;
-        if (piece == 0) inv[s * DIN + row] = uvs_unscale(e);
       }
     }
   }
-  return ok;
-}
-
-// Barrier; whether `v` holds in any thread of the workgroup's four wavefronts (`words`: four words of LDS).
-__device__ __forceinline__ bool uvs_any(bool v, int* words) {
-  const bool any = __any(v);
-  if ((threadIdx.x & (kWave - 1)) == 0) words[threadIdx.x / kWave] = any;
-  __syncthreads();
-  return words[0] | words[1] | words[2] | words[3];
+  return m;
 }
 
 template <int DIN, int CIN>
 struct UvsOps {
+  using L = UvsLds<DIN, CIN>;
   static constexpr int KS = CIN / 32;
-  struct A { f16x8 f[2][2][KS]; };          // [half][tile][step]
-  struct B { f16x8 f[2][KS]; };
-  const _Float16* wp;                       // this lane's fragments of path 0
+  struct A { bf16x8 f[3][2][KS]; };         // [part][tile][step]
+  struct B { u32x4 v[KS][L::kRaw == DIN ? 2 : 3]; bool raw; };
+  struct Z { floatx4 z[2], s[2]; };         // sums of the large products and of the small ones
+  const __bf16* wp;                         // this lane's fragments of path 0
   int64_t path_stride;
-  const unsigned char* xs;                  // this lane's base in its sample's rows
-  const float* inv_x;                       // its sample's rows
-  const float* inv_w;
-  int inv_stride = 1;                       // between the paths of inv_w
+  const unsigned char* xs;                  // its sample's rows
+  int q;                                    // its eight elements of a step
   __device__ __forceinline__ void load_a(int p, A& a) const {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 3; ++h)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int k = 0; k < KS; ++k)
-          a.f[h][t][k] = *reinterpret_cast<const f16x8*>(wp + p * path_stride + ((h * 2 + t) * KS + k) * 512);
+          a.f[h][t][k] = *reinterpret_cast<const bf16x8*>(wp + p * path_stride + ((h * 2 + t) * KS + k) * 512);
   }
   __device__ __forceinline__ void load_b(int row, B& b) const {
+    b.raw = row < L::kRaw;
+    const unsigned char* at = xs + L::row(row) + q * (b.raw ? 32 : 16);
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int k = 0; k < KS; ++k)
 #pragma unroll
-      for (int k = 0; k < KS; ++k)
-        b.f[h][k] = *reinterpret_cast<const f16x8*>(xs + row * (CIN * 4) + h * (CIN * 2) + k * 64);
+      for (int h = 0; h < (L::kRaw == DIN ? 2 : 3); ++h)
+        if (h < 2 || !b.raw)
+          b.v[k][h] = *reinterpret_cast<const u32x4*>(at + k * (b.raw ? 128 : 64) + h * (b.raw ? 16 : CIN * 2));
   }
-  // the small products first
-  __device__ __forceinline__ void chain(const A& a, const B& b, floatx4& z0, floatx4& z1) const {
-    z0 = floatx4{0.f, 0.f, 0.f, 0.f};
-    z1 = floatx4{0.f, 0.f, 0.f, 0.f};
+  // A tile.  A row staged as floats is split here, a step ahead of the matrix instructions that take it: one matrix
+  // instruction (16 cycles) and a few vector ones beside it in turn.
+  __device__ __forceinline__ void chain(const A& a, const B& b, Z& out) const {
 #pragma unroll
-    for (int part = 0; part < 3; ++part) {
-      const int ha = part == 0 ? 1 : 0, hb = part == 1 ? 1 : 0;
+    for (int t = 0; t < 2; ++t) out.z[t] = out.s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const auto element = [&](int k, int j) __attribute__((always_inline)) {
+      const unsigned w = b.v[k][j / 4][j % 4];
+      return __builtin_bit_cast(float, w);
+    };
+    UvsParts<8> part[2];
+    if (b.raw) {
 #pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        z0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.f[ha][0][k], b.f[hb][k], z0, 0, 0, 0);
-        z1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.f[ha][1][k], b.f[hb][k], z1, 0, 0, 0);
+      for (int j = 0; j < 4; ++j) part[0].pair(j, element(0, 2 * j), element(0, 2 * j + 1));
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      bf16x8 x[3];
+#pragma unroll
+      for (int h = 0; h < 3; ++h)
+        x[h] = b.raw || L::kRaw == DIN ? uvs_frag(part[k & 1].p[h]) : __builtin_bit_cast(bf16x8, b.v[k][L::kRaw == DIN ? 0 : h]);
+#pragma unroll
+      for (int i = 0; i < 12; ++i) {
+        const int t = i & 1, c = i >> 1;          // h h' of the two tiles, then the small products
+        const int ha = c == 1 ? 2 : c == 2 || c == 4 ? 1 : 0, hb = c == 3 ? 2 : c == 2 || c == 5 ? 1 : 0;
+        floatx4& sum = c == 0 ? out.z[t] : out.s[t];
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.f[ha][t][k], x[hb], sum, 0, 0, 0);
+        if (b.raw && k + 1 < KS) {
+          const int j = i / 3;
+          const float v = element(k + 1, 2 * j), w = element(k + 1, 2 * j + 1);
+          if (i % 3 == 0) part[(k + 1) & 1].template stage<0>(j, v, w);
+          else if (i % 3 == 1) part[(k + 1) & 1].template stage<1>(j, v, w);
+          else part[(k + 1) & 1].template stage<2>(j, v, w);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
   }
-  __device__ __forceinline__ float scale(int p, int row) const { return inv_x[row] * inv_w[p * inv_stride]; }
+  static __device__ __forceinline__ void sum(const Z& in, floatx4& z0, floatx4& z1) {
+    z0 = in.z[0] + in.s[0];
+    z1 = in.z[1] + in.s[1];
+  }
 };
 
 // (s x) W of one path and row for the two tiles of block `blk`, from memory, in fp32 matrix instructions.
+template <int K>
 __device__ __forceinline__ void uvs_plain_tile(const UvsWeight& W, int p, int blk, const float* __restrict__ xrow, float s,
-                                               int K, int r, int q, floatx4 (&z)[2]) {
+                                               int r, int q, floatx4 (&z)[2]) {
   z[0] = z[1] = floatx4{0.f, 0.f, 0.f, 0.f};
   const float* wb = W.of(p) + (blk * 32 + 8 * (r >> 2) + (r & 3)) * W.stride_c;
-  for (int k = q; k < K; k += 4) {
-    const float b = s * xrow[k];
+  constexpr int STEPS = 8;      // of which the loads are in flight together
+  static_assert(K % (4 * STEPS) == 0, "whole groups of steps");
+#pragma unroll 1
+  for (int k0 = q; k0 < K; k0 += 4 * STEPS) {
+    float b[STEPS], w[STEPS][2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-      z[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wb[k * W.stride_k + 4 * t * W.stride_c], b, z[t], 0, 0, 0);
+    for (int i = 0; i < STEPS; ++i) {
+      b[i] = s * xrow[k0 + 4 * i];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) w[i][t] = wb[(k0 + 4 * i) * W.stride_k + 4 * t * W.stride_c];
+    }
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) z[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][t], b[i], z[t], 0, 0, 0);
   }
 }
 
 // DIR 0: forward, 1: gradient of x (terms with the rows of out and x exchanged).
 template <class CFG, class TAB, int DIR, int CIN, int WAVES>
 __global__ void __launch_bounds__(256, WAVES) uvs_kernel(const float* __restrict__ x, const float* __restrict__ y,
-                                                         const _Float16* __restrict__ wp, const float* __restrict__ inv_w,
+                                                         const __bf16* __restrict__ wp, const unsigned* __restrict__ asks_w,
                                                          float* __restrict__ out, int64_t n_rows, int cout, UvsWeight W) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int DIN = CFG::DIN, DOUT = CFG::DOUT, D2 = CFG::D2;
   using L = UvsLds<DIN, CIN>;
   const int64_t n0 = (int64_t)blockIdx.x * kUvsSamples;
-  bool ok = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
-  float* inv_x = reinterpret_cast<float*>(smem + L::kTile);
-  float* inv_p = inv_x + kUvsSamples * DIN;
-  for (int i = threadIdx.x; i < CFG::P; i += blockDim.x) {
-    const float v = inv_w[i];
-    inv_p[i] = v;
-    ok = ok && v == v;
+  unsigned m = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
+  const int n_blocks = cout / 32;
+  for (int i = threadIdx.x; i < CFG::P * 4; i += blockDim.x) {
+    const int blk = blockIdx.y * 4 + (i & 3);
+    if (blk < n_blocks) m |= asks_w[(i >> 2) * n_blocks + blk];
   }
-  for (int i = threadIdx.x; i < kUvsSamples * D2; i += blockDim.x) {
-    const float v = y[min(n0 + i / D2, n_rows - 1) * D2 + i % D2];
-    ok = ok && v - v == 0.f;
-  }
-  const bool plain = uvs_any(!ok, reinterpret_cast<int*>(inv_p + CFG::P));
+  for (int i = threadIdx.x; i < kUvsSamples * D2; i += blockDim.x)
+    m |= uvs_asks_y(y[min(n0 + i / D2, n_rows - 1) * D2 + i % D2]);
+  const bool plain = uvs_is_plain(uvs_all(m, reinterpret_cast<unsigned*>(smem + L::kTile)));
 
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int n = lane & 15, q = lane >> 4;
@@ -266,25 +339,25 @@ __global__ void __launch_bounds__(256, WAVES) uvs_kernel(const float* __restrict
     }
   };
   if (plain) {
-    for (int m = 0; m < DOUT; ++m) {
+    for (int row = 0; row < DOUT; ++row) {
       floatx4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
       for (int t = 0; t < TAB::N; ++t) {
         const UvsTerm e = TAB::terms()[t];
-        if ((DIR == 0 ? e.o : e.a) != m) continue;
+        if ((DIR == 0 ? e.o : e.a) != row) continue;
         floatx4 z[2];
-        uvs_plain_tile(W, e.p, wblk, x + (row_n * DIN + (DIR == 0 ? e.a : e.o)) * CIN, e.c * y[row_n * D2 + e.b], CIN, n, q, z);
+        uvs_plain_tile<CIN>(W, e.p, wblk, x + (row_n * DIN + (DIR == 0 ? e.a : e.o)) * CIN, e.c * y[row_n * D2 + e.b], n, q, z);
         o[0] += z[0];
         o[1] += z[1];
       }
-      store(m, o[0], o[1]);
+      store(row, o[0], o[1]);
     }
     return;
   }
   float yv[D2];
 #pragma unroll
   for (int j = 0; j < D2; ++j) yv[j] = y[row_n * D2 + j];
-  const UvsOps<DIN, CIN> ops{wp + (int64_t)wblk * (4 * (CIN / 32) * 512) + lane * 8, (int64_t)cout * CIN * 2,
-                             smem + n * L::kPitch + q * 16, inv_x + n * DIN, inv_p};
+  const UvsOps<DIN, CIN> ops{wp + (int64_t)wblk * (6 * (CIN / 32) * 512) + lane * 8, (int64_t)cout * CIN * 3,
+                        smem + n * L::kPitch, q};
   CFG::run(ops, yv, store);
 }
 
@@ -292,26 +365,24 @@ __global__ void __launch_bounds__(256, WAVES) uvs_kernel(const float* __restrict
 // four lanes of a sample and the wavefronts (channel blocks, cout <= 128) are then added in a fixed order.
 template <class CFG, class TAB, int CIN, int WAVES>
 __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restrict__ x, const float* __restrict__ g,
-                                                            const _Float16* __restrict__ wp, const float* __restrict__ inv_w,
+                                                            const __bf16* __restrict__ wp, const unsigned* __restrict__ asks_w,
                                                             float* __restrict__ gy, int64_t n_rows, int cout, UvsWeight W) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int DIN = CFG::DIN, DOUT = CFG::DOUT, D2 = CFG::D2;
   using L = UvsLds<DIN, CIN>;
   const int64_t n0 = (int64_t)blockIdx.x * kUvsSamples;
-  bool ok = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
-  float* inv_x = reinterpret_cast<float*>(smem + L::kTile);
-  float* inv_p = inv_x + kUvsSamples * DIN;
-  for (int i = threadIdx.x; i < CFG::P; i += blockDim.x) {
-    const float v = inv_w[i];
-    inv_p[i] = v;
-    ok = ok && v == v;
+  unsigned m = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
+  const int n_blocks = cout / 32;
+  for (int i = threadIdx.x; i < CFG::P * 4; i += blockDim.x) {
+    const int blk = blockIdx.y * 4 + (i & 3);
+    if (blk < n_blocks) m |= asks_w[(i >> 2) * n_blocks + blk];
   }
-  const bool plain = uvs_any(!ok, reinterpret_cast<int*>(inv_p + CFG::P));
+  const bool plain = uvs_is_plain(uvs_all(m, reinterpret_cast<unsigned*>(smem + L::kTile)));
 
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int n = lane & 15, q = lane >> 4, n_blk = cout / 32;
+  const int n = lane & 15, q = lane >> 4;
   const int64_t row_n = min(n0 + n, n_rows - 1);
-  const float* grow = g + row_n * DOUT * cout + min(wave, n_blk - 1) * 32 + 8 * q;
+  const float* grow = g + row_n * DOUT * cout + min(wave, n_blocks - 1) * 32 + 8 * q;
   float part[D2];
 #pragma unroll
   for (int j = 0; j < D2; ++j) part[j] = 0.f;
@@ -319,12 +390,12 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
     g0 = *reinterpret_cast<const floatx4*>(grow + row * cout);
     g1 = *reinterpret_cast<const floatx4*>(grow + row * cout + 4);
   };
-  if (wave < n_blk) {
+  if (wave < n_blocks) {
     if (plain) {
       for (int t = 0; t < TAB::N; ++t) {
         const UvsTerm e = TAB::terms()[t];
         floatx4 z[2], g0, g1;
-        uvs_plain_tile(W, e.p, wave, x + (row_n * DIN + e.a) * CIN, 1.f, CIN, n, q, z);
+        uvs_plain_tile<CIN>(W, e.p, wave, x + (row_n * DIN + e.a) * CIN, 1.f, n, q, z);
         load_g(e.o, g0, g1);
         const float v = e.c * dot8(g0, g1, z[0], z[1]);
 #pragma unroll
@@ -332,8 +403,8 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
           if (j == e.b) part[j] += v;
       }
     } else {
-      const UvsOps<DIN, CIN> ops{wp + (int64_t)wave * (4 * (CIN / 32) * 512) + lane * 8, (int64_t)cout * CIN * 2,
-                                 smem + n * L::kPitch + q * 16, inv_x + n * DIN, inv_p};
+      const UvsOps<DIN, CIN> ops{wp + (int64_t)wave * (6 * (CIN / 32) * 512) + lane * 8, (int64_t)cout * CIN * 3,
+                            smem + n * L::kPitch, q};
       CFG::run(ops, part, load_g);
     }
 #pragma unroll
@@ -347,14 +418,14 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
   }
   __syncthreads();  // every wavefront is done with the staged rows; reuse the front of LDS for the partial sums
   float* red = reinterpret_cast<float*>(smem);
-  if (wave < n_blk && q == 0) {
+  if (wave < n_blocks && q == 0) {
 #pragma unroll
     for (int j = 0; j < D2; ++j) red[(wave * kUvsSamples + n) * D2 + j] = part[j];
   }
   __syncthreads();
   for (int i = threadIdx.x; i < kUvsSamples * D2; i += blockDim.x) {
     float s = 0.f;
-    for (int w = 0; w < n_blk; ++w) s += red[w * kUvsSamples * D2 + i];
+    for (int w = 0; w < n_blocks; ++w) s += red[w * kUvsSamples * D2 + i];
     if (n0 + i / D2 < n_rows) gy[n0 * D2 + i] = s;
   }
 }
@@ -366,35 +437,30 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
 // added through LDS in a fixed order.  Mixing z and x first, as the fp32 route does, forms 1024 products per (path, row)
 // and sample on the vector units; here they are the matrix cores', and the vector units see one multiply-add per
 // coefficient and l.  What bounds it: vector and matrix instructions of two wavefronts per SIMD in about equal parts, and
-// the weights from L2 (4 bytes an element and workgroup: 1.4 MB at 32 channels, lmax = 2).
-// 32 x 32 -> 32, lmax = 2, 32768 samples: 943 -> 268 us, both gradients alike; 500 samples: 179 -> 44 us with packing; lmax = 1,
-// 32768 samples 205 -> 73 us.  Error of the results against 64 bits 1.1e-7 to 1.4e-7, of the fp32 route 2.0e-7 to 1.4e-6.
+// the weights from L2 (6 bytes an element and workgroup: 2.2 MB at 32 channels, lmax = 2).
+// 32 x 32 -> 32, lmax = 2, 32768 samples: 925 -> 386 us, both gradients alike; 500 samples: 178 -> 58 us with packing; lmax = 1,
+// 32768 samples 197 -> 103 us.  Error of the results against 64 bits 0.7e-7 to 1.2e-7, of the
+// fp32 route 2.0e-7 to 15.8e-7.
 template <class CFG, class TAB, int KIND>
 __global__ void __launch_bounds__(256, 2) uvsw_kernel(const float* __restrict__ x, const float* __restrict__ z,
-                                                      const _Float16* __restrict__ wp, const float* __restrict__ inv_w,
+                                                      const __bf16* __restrict__ wp, const unsigned* __restrict__ asks_w,
                                                       float* __restrict__ out, int64_t n_rows, int cout, UvsWeight W) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int CIN = 32, DIN = CFG::DIN, DOUT = CFG::DOUT, D2 = CFG::D2;
   using T = UvsLds<DIN, CIN>;
   const int64_t n0 = (int64_t)blockIdx.x * kUvsSamples;
   const int L = W.matrices, n_mat = CFG::P * L;
-  bool ok = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
-  float* inv_x = reinterpret_cast<float*>(smem + T::kTile);
-  float* inv_p = inv_x + kUvsSamples * DIN;
-  int* words = reinterpret_cast<int*>(inv_p + n_mat);
+  unsigned m = uvs_stage<DIN, CIN>(x, n0, n_rows, smem);
+  unsigned* words = reinterpret_cast<unsigned*>(smem + T::kTile);
   float* zs = reinterpret_cast<float*>(words + 4);                // [l][row][sample]
-  for (int i = threadIdx.x; i < n_mat; i += blockDim.x) {
-    const float v = inv_w[i];
-    inv_p[i] = v;
-    ok = ok && v == v;
-  }
+  for (int i = threadIdx.x; i < n_mat; i += blockDim.x) m |= asks_w[i * (cout / 32) + blockIdx.y];
   for (int i = threadIdx.x; i < kUvsSamples * D2 * L; i += blockDim.x) {
     const int s = i / (D2 * L), rest = i - s * (D2 * L), b = rest / L, l = rest - b * L;
     const float v = z[min(n0 + s, n_rows - 1) * (D2 * L) + rest];
     zs[(l * D2 + b) * kUvsSamples + s] = v;
-    ok = ok && v - v == 0.f;
+    m |= uvs_asks_y(v);
   }
-  const bool plain = uvs_any(!ok, words);
+  const bool plain = uvs_is_plain(uvs_all(m, words));
 
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int n = lane & 15, q = lane >> 4;
@@ -409,33 +475,33 @@ __global__ void __launch_bounds__(256, 2) uvsw_kernel(const float* __restrict__ 
     }
   };
   if (plain) {
-    for (int m = wave; m < DOUT; m += 4) {
+    for (int row = wave; row < DOUT; row += 4) {
       floatx4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
       for (int t = 0; t < TAB::N; ++t) {
         const UvsTerm e = TAB::terms()[t];
         const int mt = KIND == 0 ? e.o : KIND == 1 ? e.a : e.b, at = KIND == 0 ? e.a : e.o, bt = KIND == 2 ? e.a : e.b;
-        if (mt != m) continue;
+        if (mt != row) continue;
         for (int l = 0; l < L; ++l) {
           floatx4 v[2];
-          uvs_plain_tile(W, e.p * L + l, wblk, x + (row_n * DIN + at) * CIN, e.c * z[(row_n * D2 + bt) * L + l], CIN, n, q, v);
+          uvs_plain_tile<CIN>(W, e.p * L + l, wblk, x + (row_n * DIN + at) * CIN, e.c * z[(row_n * D2 + bt) * L + l], n, q, v);
           o[0] += v[0];
           o[1] += v[1];
         }
       }
-      store(m, o[0], o[1]);
+      store(row, o[0], o[1]);
     }
     return;
   }
   floatx4 acc[DOUT][2];
 #pragma unroll
   for (int m = 0; m < DOUT; ++m) acc[m][0] = acc[m][1] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int64_t matrix = (int64_t)cout * CIN * 2;
+  const int64_t matrix = (int64_t)cout * CIN * 3;
   for (int l = wave; l < L; l += 4) {
     float zv[D2];
 #pragma unroll
     for (int j = 0; j < D2; ++j) zv[j] = zs[(l * D2 + j) * kUvsSamples + n];
-    const UvsOps<DIN, CIN> ops{wp + l * matrix + (int64_t)wblk * (4 * 512) + lane * 8, L * matrix,
-                               smem + n * T::kPitch + q * 16, inv_x + n * DIN, inv_p + l, L};
+    const UvsOps<DIN, CIN> ops{wp + l * matrix + (int64_t)wblk * (6 * 512) + lane * 8, L * matrix,
+                          smem + n * T::kPitch, q};
     CFG::run(ops, zv, [&](int row, const floatx4& o0, const floatx4& o1) __attribute__((always_inline)) {
       acc[row][0] += o0;
       acc[row][1] += o1;
@@ -467,16 +533,18 @@ __global__ void __launch_bounds__(256, 2) uvsw_kernel(const float* __restrict__ 
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------
-using UvsFn = void (*)(const float*, const float*, const _Float16*, const float*, float*, int64_t, int, UvsWeight);
+using UvsFn = void (*)(const float*, const float*, const __bf16*, const unsigned*, float*, int64_t, int, UvsWeight);
 struct UvsEntry {
   int cfg;                 // index of the table among the compiled ones (cgtp_uv_find)
-  int din[2], p;           // rows of the contracted operand in the forward and in the gradient of x; paths
+  int p;                   // paths
+  int64_t lds[3][3];       // bytes, as fn
+  int64_t lds_w[3];        // of the staged rows, as fn_w
   UvsFn fn[3][3];          // [forward, gradient of x, gradient of y][32, 64, 128 contracted channels]
   UvsFn fn_w[3];           // channels on both operands, 32 contracted; null where the rows do not fit the registers
-  int rows_w[3][3];        // rows of the contracted, the other and the produced operand
+  int rows_w[3][2];        // rows of the operand that is not contracted, and of the produced one
 };
 
-// wavefronts per SIMD the registers are kept to: two, except at 128 contracted channels, where the three weight fragments in
+// wavefronts per SIMD the registers are kept to: two, except at 128 contracted channels, where the two weight fragments in
 // flight alone take 192 registers
 constexpr int uvs_waves(int cin) { return cin < 128 ? 2 : 1; }
 
@@ -490,18 +558,22 @@ template <class D0, class D1, class GY, class DW, class TAB>
 static UvsEntry make_uvs_entry(int cfg) {
   UvsEntry e;
   e.cfg = cfg;
-  e.din[0] = D0::DIN; e.din[1] = D1::DIN; e.p = D0::P;
+  e.p = D0::P;
 #define CGTP_UVS_CIN(i, CIN)                               \
   e.fn[0][i] = uvs_kernel<D0, TAB, 0, CIN, uvs_waves(CIN)>;   \
   e.fn[1][i] = uvs_kernel<D1, TAB, 1, CIN, uvs_waves(CIN)>;   \
-  e.fn[2][i] = uvs_gy_kernel<GY, TAB, CIN, uvs_waves(CIN)>;
+  e.fn[2][i] = uvs_gy_kernel<GY, TAB, CIN, uvs_waves(CIN)>;   \
+  e.lds[0][i] = UvsLds<D0::DIN, CIN>::kTile + 16;             \
+  e.lds[1][i] = UvsLds<D1::DIN, CIN>::kTile + 16;             \
+  e.lds[2][i] = UvsLds<GY::DIN, CIN>::kTile + 16;
   CGTP_UVS_CIN(0, 32)
   CGTP_UVS_CIN(1, 64)
   CGTP_UVS_CIN(2, 128)
 #undef CGTP_UVS_CIN
+  e.lds_w[0] = UvsLds<D0::DIN, 32>::kTile; e.lds_w[1] = UvsLds<D1::DIN, 32>::kTile; e.lds_w[2] = UvsLds<DW::DIN, 32>::kTile;
   e.fn_w[0] = uvsw_fn<D0, TAB, 0>(); e.fn_w[1] = uvsw_fn<D1, TAB, 1>(); e.fn_w[2] = uvsw_fn<DW, TAB, 2>();
-  const int rows[3][3] = {{D0::DIN, D0::D2, D0::DOUT}, {D1::DIN, D1::D2, D1::DOUT}, {DW::DIN, DW::D2, DW::DOUT}};
-  for (int k = 0; k < 9; ++k) e.rows_w[k / 3][k % 3] = rows[k / 3][k % 3];
+  const int rows[3][2] = {{D0::D2, D0::DOUT}, {D1::D2, D1::DOUT}, {DW::D2, DW::DOUT}};
+  for (int k = 0; k < 6; ++k) e.rows_w[k / 2][k % 2] = rows[k / 2][k % 2];
   return e;
 }
 
@@ -525,8 +597,7 @@ static int uvs_check(int cfg, int kind, const void* x, const void* y, const void
   *ci = cin == 32 ? 0 : cin == 64 ? 1 : cin == 128 ? 2 : -1;
   if (*ci < 0) return CGTP_ERR_SHAPE;
   if (((uintptr_t)x | (uintptr_t)packed | (uintptr_t)(kind == 2 ? y : out)) & 15u) return CGTP_ERR_ALIGN;
-  const int din = e->din[kind == 1];
-  *lds = (int64_t)kUvsSamples * (din * cin * 4 + 16) + kUvsSamples * din * 4 + e->p * 4 + 16;
+  *lds = e->lds[kind][*ci];
   if (*lds > kLdsBytes) return CGTP_ERR_LDS;
   if ((n_rows + kUvsSamples - 1) / kUvsSamples >= (int64_t)1 << 31) return CGTP_ERR_SHAPE;
   *entry = e;
@@ -535,7 +606,7 @@ static int uvs_check(int cfg, int kind, const void* x, const void* y, const void
 
 static int uvs_pack(const UvsWeight& W, void* packed, int64_t matrices, int cin, int cout, hipStream_t stream) {
   hipLaunchKernelGGL(uvs_pack_kernel, dim3((unsigned)matrices, (unsigned)(cout / 32)), dim3(256), 0, stream, W,
-                     (_Float16*)packed, (float*)((_Float16*)packed + matrices * cin * cout * 2), cin, cout);
+                     (__bf16*)packed, (unsigned*)((__bf16*)packed + matrices * cin * cout * 3), cin, cout);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
 }
 
@@ -556,9 +627,8 @@ static int uvsw_check(int cfg, int kind, const void* x, const void* z, const voi
   const int cin = kind == 0 ? u : c, cout = kind == 0 ? c : kind == 1 ? u : v, L = kind == 2 ? u : v;
   if (n_rows < 0 || cin != 32 || cout <= 0 || cout % 32 || L <= 0) return CGTP_ERR_SHAPE;
   if (((uintptr_t)x | (uintptr_t)packed | (uintptr_t)out) & 15u) return CGTP_ERR_ALIGN;
-  const int din = e->rows_w[kind][0], d2 = e->rows_w[kind][1], dout = e->rows_w[kind][2];
-  const int64_t staged = (int64_t)kUvsSamples * (din * cin * 4 + 16) + kUvsSamples * din * 4 + (int64_t)e->p * L * 4 + 16 +
-                         (int64_t)kUvsSamples * d2 * L * 4;
+  const int d2 = e->rows_w[kind][0], dout = e->rows_w[kind][1];
+  const int64_t staged = e->lds_w[kind] + 16 + (int64_t)kUvsSamples * d2 * L * 4;
   const int64_t sums = (int64_t)2 * dout * 2 * kWave * 16;
   *lds = staged > sums ? staged : sums;
   if (2 * *lds > kLdsBytes) return CGTP_ERR_LDS;                  // two workgroups per compute unit, as the registers allow
@@ -575,7 +645,7 @@ extern "C" {
 
 int64_t cgtp_uvs_packed_bytes(int32_t n_paths, int32_t cin, int32_t cout) {
   if (n_paths <= 0 || cin <= 0 || cout <= 0 || cin % 32 || cout % 32) return 0;
-  return (int64_t)n_paths * cin * cout * 4 + ((int64_t)n_paths * 4 + 15) / 16 * 16;
+  return (int64_t)n_paths * cin * cout * 6 + ((int64_t)n_paths * (cout / 32) * 4 + 15) / 16 * 16;
 }
 
 int cgtp_uvs_pack_weights(const float* w, void* packed, int32_t n_paths, int32_t cin, int32_t cout, int32_t transposed,
@@ -609,15 +679,16 @@ int cgtp_uvs_apply(int cfg, int kind, const void* x, const void* y, const void* 
   const int64_t sp = (int64_t)cin * cout;
   const UvsWeight W = {(const float*)w, sp, kind == 1 ? 1 : (int64_t)cout, kind == 1 ? (int64_t)cin : 1, 0, 1};
   hipLaunchKernelGGL(fn, dim3((unsigned)((n_rows + kUvsSamples - 1) / kUvsSamples), (unsigned)(kind == 2 ? 1 : (cout + 127) / 128)),
-                     dim3(256), (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)y, (const _Float16*)packed,
-                     (const float*)((const _Float16*)packed + e->p * sp * 2), (float*)out, n_rows, (int)cout, W);
+                     dim3(256), (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)y, (const __bf16*)packed,
+                     (const unsigned*)((const __bf16*)packed + e->p * sp * 3), (float*)out, n_rows, (int)cout, W);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
 }
 
 int64_t cgtp_uvsw_packed_bytes(int32_t n_paths, int32_t u, int32_t v, int32_t w) {
   if (n_paths <= 0 || u <= 0 || v <= 0 || w <= 0) return 0;
-  // any kind: the matrices of a path run over one of the operands' channels
-  return (int64_t)n_paths * u * v * w * 4 + ((int64_t)n_paths * (u > v ? u : v) * 4 + 15) / 16 * 16;
+  // any kind: the matrices of a path run over one of the operands' channels, the blocks of 32 over another's
+  const int64_t most = std::max({(int64_t)v * w, (int64_t)v * u, (int64_t)u * v}) / 32;
+  return (int64_t)n_paths * u * v * w * 6 + (n_paths * most * 4 + 15) / 16 * 16;
 }
 
 int cgtp_uvsw_validate(int cfg, int kind, const void* x, const void* z, const void* packed, const void* w, const void* out,
@@ -642,8 +713,8 @@ int cgtp_uvsw_apply(int cfg, int kind, const void* x, const void* z, void* packe
   if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return CGTP_ERR_LDS;
   hipLaunchKernelGGL(fn, dim3((unsigned)((n_rows + kUvsSamples - 1) / kUvsSamples), (unsigned)(cout / 32)), dim3(256),
-                     (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)z, (const _Float16*)packed,
-                     (const float*)((const _Float16*)packed + matrices * cin * cout * 2), (float*)out, n_rows, cout, W);
+                     (size_t)lds, (hipStream_t)stream, (const float*)x, (const float*)z, (const __bf16*)packed,
+                     (const unsigned*)((const __bf16*)packed + matrices * cin * cout * 3), (float*)out, n_rows, cout, W);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
 }
 

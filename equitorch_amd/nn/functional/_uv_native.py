@@ -249,9 +249,9 @@ def apply(x: Tensor, y: Tensor, wp: Tensor, tp_info, role: str, dout: int, cout:
 def _split(kind: int, x: Tensor, y: Tensor, w: Tensor, tp_info, rows_out: int) -> Optional[Tensor]:
     """The product of a compiled table in fp32 on the half-precision matrix cores (``cgtp_uvs_apply``; ``kind`` 0: forward, 1:
     gradient of the first operand, 2: gradient of the second), or None where the fp32 matrix instructions serve: tables
-    that are not compiled in as they are, channels other than 32, 64, 128.  No size is left out: from 512 to 32768
-    samples, lmax 1 to 3 and 32 to 128 channels it takes 0.3 to 1.0 of their time (512 samples, lmax = 1, 32 channels: 13 to
-    17 us on both, launches alone)."""
+    that are not compiled in as they are, contracted channels other than 32, 64, 128.  From 100 to 32768 samples, lmax 1
+    to 3, equal channels it takes 0.3 to 0.9 of their time (100 samples, lmax = 1, 32 channels: 14 to 18 us on both,
+    launches alone)."""
     if isinstance(tp_info, CooTable) or x.dtype != torch.float32:
         return None
     cfg = kernels.uv_config_of(tp_info)
@@ -277,7 +277,7 @@ def _split_uvw(kind: int, x: Tensor, z: Tensor, w: Tensor, tp_info, rows_out: in
     """The same for channels on both operands (``cgtp_uvsw_apply``), ``w (P, U, V, W)``; ``kind`` 0: forward, 1: gradient of the
     first operand (``x`` = grad_out, ``z`` = the second operand), 2: gradient of the second (``x`` = grad_out, ``z`` = the
     first).  32 contracted channels, which one matrix instruction takes whole, a multiple of 32 produced ones, up to nine
-    produced rows (lmax = 2: the registers hold them all).  Takes 0.25 to 0.7 of the time of the fp32 matrix instructions from 500 to 32768
+    produced rows (lmax = 2: the registers hold them all).  Takes 0.3 to 0.7 of the time of the fp32 matrix instructions from 100 to 32768
     samples."""
     if isinstance(tp_info, CooTable) or x.dtype != torch.float32:
         return None

@@ -398,7 +398,7 @@ int cgtp_uv_grad_w(int cfg, const void* x, const void* y, const void* g, void* g
                    int32_t cin, int32_t cout, int32_t dtype, const float* path_scale, void* stream);
 
 /* The fully connected product of a compiled table (cfg as above) in single precision on the half-precision matrix cores,
- * every fp32 operand carried as two halves (no less precise than fp32 matrix instructions).  kind 0: forward, x
+ * every fp32 operand carried as three bf16 parts (no less precise than fp32 matrix instructions, and of their range).  kind 0: forward, x
  * (n_rows, D1, cin), y (n_rows, D2), out (n_rows, DO, cout); 1: gradient of x, `x` = grad_out (n_rows, DO, cin), out
  * (n_rows, D1, cout); 2: gradient of y, y = grad_out (n_rows, DO, cout), out (n_rows, D2), cout <= 128.  cin 32, 64 or
  * 128, cout a multiple of 32.  w: the weight (P, contracted, produced) for kinds 0 and 2, (P, produced, contracted) for

@@ -1,5 +1,5 @@
 """The fully connected product of the compiled tables in fp32 on the half-precision matrix cores (``cgtp_uvs_apply``): every
-operand carried as two halves, no less precise than fp32 matrix instructions."""
+operand carried as three bf16 parts, no less precise than fp32 matrix instructions and of their range."""
 import pytest
 import torch
 
@@ -81,6 +81,65 @@ def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, 
         assert float((a[fin] - b[fin]).norm()) <= 1e-6 * float(b[fin].norm())
 
 
+def _per_channel(got, want):
+    """Error of every (row, channel) over the samples against its own size (rows alone for a result without channels)."""
+    d = (got.cpu().double() - want).norm(dim=0) / want.norm(dim=0)
+    return float(d.square().mean().sqrt()), float(d.max())
+
+
+def _no_worse(name, split, fp32, want, slack):
+    for which, new, old in zip(("mean", "largest"), _per_channel(split, want), _per_channel(fp32, want)):
+        print(f"{name}: {which} error over the channels: split {new:.2e} fp32 {old:.2e}")
+        # each channel's error is that of a few hundred draws: the largest of them scatters more than the mean
+        assert new <= slack[which == "largest"] * old + 3e-8, (name, which)
+
+
+@pytest.mark.parametrize("lmax,cin,cout", [(1, 128, 64), (2, 64, 64), (3, 64, 32), (3, 128, 128)])
+def test_every_channel_keeps_its_precision(device, monkeypatch, lmax, cin, cout):
+    """Channels of x, of grad_out and of the weight (on either axis) that are up to 2^-30 of the largest, with the products
+    of x, W and grad_out balanced, so that every channel counts; errors per row and channel against its own size."""
+    mod, ops = _operands(device, lmax, cin, cout, 200, stable_seed("channels", lmax, cin, cout))
+    gen = torch.Generator().manual_seed(11)
+    a, b = (torch.exp2(torch.randint(0, 31, (c,), generator=gen).float()) for c in (cin, cout))
+    ops[0] /= a
+    ops[2] *= a[:, None] / b
+    ops[3] *= b
+    split, fp32 = _both_routes(monkeypatch, mod, device, ops)
+    T = ref_ops.dense_coupling(SH[lmax], SH[lmax], SH[lmax]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_u1v, T, ops[:3], ops[3])
+    for name, new, old, want in zip(("out", "grad x", "grad y"), split, fp32, (ref_out, *ref_grads[:2])):
+        _no_worse(f"{name} lmax={lmax} {cin}->{cout}", new, old, want, (1.1, 1.5))
+
+
+# exponents of x, y, W and grad_out: results that are ordinary fp32 numbers, of operands or products that are far from 1
+RANGES = [(0, 0, 0, 100), (0, 0, -5, 115), (-70, 0, -40, 0), (-40, 0, -40, -30), (-60, 60, -60, 30), (-90, 80, -60, 100),
+          (-105, 0, 0, 0), (0, 0, -105, 0), (-107, 0, 1, 0), (2, 2, -106, 0), (-115, 0, 2, -100), (59, -40, 59, 0), (70, -30, 55, -50), (63, 20, 40, 0), (10, 90, 10, 10)]
+
+
+def _scaled(ops, exponents):
+    return [t * 2.0 ** e for t, e in zip(ops, exponents)]
+
+
+def _check_range(names, split, fp32, refs, exponents):
+    for name, new, old, want in zip(names, split, fp32, refs):
+        if not torch.isfinite(old).all():
+            continue
+        assert torch.isfinite(new).all(), (name, exponents)
+        if want.abs().max() > 2.0 ** -110:         # below, the terms of the sums are subnormal numbers on either route
+            _no_worse(f"{name} of {exponents}", new, old, want, (1.5, 2.5))
+
+
+@pytest.mark.parametrize("exponents", RANGES)
+def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponents):
+    mod, ops = _operands(device, 2, 64, 32, 70, 21)
+    ops = _scaled(ops, exponents)
+    ops[0][3, 2, 5] = 0.0              # an exact zero has no exponent
+    split, fp32 = _both_routes(monkeypatch, mod, device, ops)
+    T = ref_ops.dense_coupling(SH[2], SH[2], SH[2]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_u1v, T, ops[:3], ops[3])
+    _check_range(("out", "grad x", "grad y"), split, fp32, (ref_out, *ref_grads[:2]), exponents)
+
+
 # ---- channels on both operands ("uvw"): cgtp_uvsw_apply -----------------------------------------------------------
 def _uvw_routes(monkeypatch, device, lmax, u, v, c, operands):
     from equitorch_amd.nn import TensorProduct
@@ -141,6 +200,31 @@ def test_uvw_values_that_are_not_finite_stay_where_they_couple(device, monkeypat
         # the fp32 route sums chains of 1024 products times the rows of a path: rounding 6e-8 each at random, 6e-8 * sqrt(1024)
         # = 2e-6 of the result (0.6e-6 to 1.5e-6 measured against 64 bits in the test above)
         assert float((a[fin] - b[fin]).norm()) <= 2e-6 * float(b[fin].norm())
+
+
+def test_uvw_every_channel_keeps_its_precision(device, monkeypatch):
+    u, v, c = 32, 32, 32
+    ops = _uvw_operands(2, u, v, c, 150, stable_seed("uvw channels"))
+    gen = torch.Generator().manual_seed(12)
+    a, z, b = (torch.exp2(torch.randint(0, 21, (k,), generator=gen).float()) for k in (u, v, c))
+    ops[0] /= a
+    ops[1] /= z
+    ops[2] *= a[:, None, None] * z[:, None] / b
+    ops[3] *= b
+    new, old, _ = _uvw_routes(monkeypatch, device, 2, u, v, c, ops)
+    T = ref_ops.dense_coupling(SH[2], SH[2], SH[2]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_uvw, T, ops[:3], ops[3])
+    for name, a, b, want in zip(("out", "grad x", "grad y"), new, old, (ref_out, *ref_grads[:2])):
+        _no_worse(f"uvw {name}", a, b, want, (1.1, 1.5))
+
+
+@pytest.mark.parametrize("exponents", RANGES)
+def test_uvw_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponents):
+    ops = _scaled(_uvw_operands(2, 32, 32, 32, 40, 22), exponents)
+    new, old, _ = _uvw_routes(monkeypatch, device, 2, 32, 32, 32, ops)
+    T = ref_ops.dense_coupling(SH[2], SH[2], SH[2]).float().double()
+    ref_out, ref_grads = ref_ops.dense_grads(ref_ops.dense_uvw, T, ops[:3], ops[3])
+    _check_range(("out", "grad x", "grad y"), new, old, (ref_out, *ref_grads[:2]), exponents)
 
 
 @pytest.mark.parametrize("mode", ["uv", "uvw"])
