@@ -596,6 +596,10 @@ static int uvs_check(int cfg, int kind, const void* x, const void* y, const void
   if (n_rows < 0 || cout <= 0 || cout % 32 || (kind == 2 && cout > 128)) return CGTP_ERR_SHAPE;
   *ci = cin == 32 ? 0 : cin == 64 ? 1 : cin == 128 ? 2 : -1;
   if (*ci < 0) return CGTP_ERR_SHAPE;
+  // One block of produced channels keeps one wavefront in four busy, at 128 contracted channels the only one of its compute
+  // unit: 128 -> 32, 32768 samples, lmax 1, 2, 3: 62, 213, 612 us where fp32 matrix instructions take 45, 158, 515 (128 -> 64:
+  // 67, 219, 645 for 70, 293, 716; 64 -> 32, two workgroups per compute unit: 22, 58, 170 for 29, 93, 208).
+  if (cin == 128 && cout == 32) return CGTP_ERR_SHAPE;
   if (((uintptr_t)x | (uintptr_t)packed | (uintptr_t)(kind == 2 ? y : out)) & 15u) return CGTP_ERR_ALIGN;
   *lds = e->lds[kind][*ci];
   if (*lds > kLdsBytes) return CGTP_ERR_LDS;

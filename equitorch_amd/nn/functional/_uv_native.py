@@ -249,7 +249,7 @@ def apply(x: Tensor, y: Tensor, wp: Tensor, tp_info, role: str, dout: int, cout:
 def _split(kind: int, x: Tensor, y: Tensor, w: Tensor, tp_info, rows_out: int) -> Optional[Tensor]:
     """The product of a compiled table in fp32 on the half-precision matrix cores (``cgtp_uvs_apply``; ``kind`` 0: forward, 1:
     gradient of the first operand, 2: gradient of the second), or None where the fp32 matrix instructions serve: tables
-    that are not compiled in as they are, contracted channels other than 32, 64, 128.  From 100 to 32768 samples, lmax 1
+    that are not compiled in as they are, contracted channels other than 32, 64, 128, and 128 -> 32.  From 100 to 32768 samples, lmax 1
     to 3, equal channels it takes 0.3 to 0.9 of their time (100 samples, lmax = 1, 32 channels: 14 to 18 us on both,
     launches alone)."""
     if isinstance(tp_info, CooTable) or x.dtype != torch.float32:

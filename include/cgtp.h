@@ -398,11 +398,12 @@ int cgtp_uv_grad_w(int cfg, const void* x, const void* y, const void* g, void* g
                    int32_t cin, int32_t cout, int32_t dtype, const float* path_scale, void* stream);
 
 /* The fully connected product of a compiled table (cfg as above) in single precision on the half-precision matrix cores,
- * every fp32 operand carried as three bf16 parts (no less precise than fp32 matrix instructions, and of their range).  kind 0: forward, x
- * (n_rows, D1, cin), y (n_rows, D2), out (n_rows, DO, cout); 1: gradient of x, `x` = grad_out (n_rows, DO, cin), out
- * (n_rows, D1, cout); 2: gradient of y, y = grad_out (n_rows, DO, cout), out (n_rows, D2), cout <= 128.  cin 32, 64 or
- * 128, cout a multiple of 32.  w: the weight (P, contracted, produced) for kinds 0 and 2, (P, produced, contracted) for
- * kind 1, contiguous; packed: cgtp_uvs_packed_bytes() bytes filled by cgtp_uvs_pack_weights (transposed for kind 1). */
+ * every fp32 operand carried as three bf16 parts (no less precise than fp32 matrix instructions, and of their range).
+ * kind 0: forward, x (n_rows, D1, cin), y (n_rows, D2), out (n_rows, DO, cout); 1: gradient of x, `x` = grad_out (n_rows,
+ * DO, cin), out (n_rows, D1, cout); 2: gradient of y, y = grad_out (n_rows, DO, cout), out (n_rows, D2), cout <= 128.  cin 32,
+ * 64 or 128, cout a multiple of 32, at 128 from 64 on.  w: the weight (P, contracted, produced) for kinds 0 and 2, (P,
+ * produced, contracted) for kind 1, contiguous; packed: cgtp_uvs_packed_bytes() bytes filled by cgtp_uvs_pack_weights
+ * (transposed for kind 1). */
 int64_t cgtp_uvs_packed_bytes(int32_t n_paths, int32_t cin, int32_t cout);
 int cgtp_uvs_pack_weights(const float* w, void* packed, int32_t n_paths, int32_t cin, int32_t cout, int32_t transposed,
                           void* stream);

@@ -207,6 +207,20 @@ def test_uv_matrix_core_entry_points_validate_on_the_host():
     assert L.cgtp_uv_grad_w(cfg, p16, p16, p16, p16, p16, 100, 128, 160, _lib.BF16, None, None) == 2
 
 
+def test_single_precision_split_entry_points_validate_on_the_host():
+    from equitorch_amd import _lib
+    lib, cfg, at = _lib.lib, 1, 4096                                # lmax 2
+    ok = lambda kind, cin, cout, x=at, y=at, out=at, n=100: lib.cgtp_uvs_validate(cfg, kind, x, y, at, at, out, n, cin, cout)  # noqa: E731
+    for kind in (0, 1, 2):
+        assert [ok(kind, c, c) for c in (32, 64, 128)] == [0, 0, 0]
+        assert [ok(kind, *c) for c in ((32, 128), (64, 32), (128, 64), (32, 96))] == [0] * 4
+        assert ok(kind, 128, 32) != 0                               # slower than fp32 matrix instructions
+        assert all(ok(kind, *c) != 0 for c in ((16, 32), (96, 96), (256, 64), (64, 48)))
+        assert ok(kind, 64, 64, x=at + 4) != 0
+    assert ok(0, 128, 160) == 0 and ok(2, 128, 160) != 0            # the sums of grad_y are one workgroup's
+    assert ok(0, 64, 64, out=at + 4) != 0 and ok(2, 64, 64, y=at + 4) != 0
+
+
 def test_spherical_harmonics_entry_points_validate_on_the_host():
     from equitorch_amd import _lib
     L = _lib.lib

@@ -27,6 +27,7 @@ def _step(mod, device, x, y, w, ct):
 
 
 def _both_routes(monkeypatch, mod, device, operands):
+    """Results on both routes; the split one takes all three products but those with 128 contracted and 32 produced channels."""
     from equitorch_amd.nn.functional import _uv_native
     results, kinds, split = {}, [], _uv_native._split
 
@@ -36,7 +37,8 @@ def _both_routes(monkeypatch, mod, device, operands):
         return out
     monkeypatch.setattr(_uv_native, "_split", spy)
     results["split"] = _step(mod, device, *operands)
-    assert sorted(kinds) == [(0, True), (1, True), (2, True)], kinds
+    cin, cout = operands[2].shape[1:]
+    assert sorted(kinds) == [(0, (cin, cout) != (128, 32)), (1, (cout, cin) != (128, 32)), (2, (cin, cout) != (128, 32))], kinds
     monkeypatch.setattr(_uv_native, "_split", lambda *args: None)
     results["fp32"] = _step(mod, device, *operands)
     return results["split"], results["fp32"]
