@@ -1022,18 +1022,48 @@ def uvu_tab_launchable(tab: Optional[UvuTable], x: Tensor, y: Tensor, w: Tensor,
     return all(_lib.lib.cgtp_uvu_tab_validate(C.byref(a), C.byref(tab.c), d) == 0 for d in (0, 1))
 
 
+def _subset_pays(channels: int, n_edges: int, paths: int, all_paths: int) -> bool:
+    """Whether a table with ``paths`` of a compiled table's ``all_paths`` is quicker as it is.  Forward and backward in us, as
+    it is | on the compiled kernels with expanded weights (paths of all paths):
+
+        200 000 edges   16 channels     32          36          48          64
+           6 of 15       843 |  910    970 | 1565      -      1064 | 2708     -
+           9 of 15       993 |  931   1212 | 1602      -      1286 | 2758     -
+          14 of 15          -             -        1670 | 2643  1697 | 2825  1272 | 3186
+           8 of 11       918 |  559   1080 |  873      -      1147 | 1344     -
+          10 of 11          -             -        1302 | 1242  1326 | 1369   982 | 1656
+          15 of 18      1483 |  948   1867 | 1663      -      1934 | 2644     -
+          22 of 23          -             -        3586 | 3124  3615 | 3811  2805 | 4742
+          23 of 23          -             -        3814 | 2911  3843 | 3605  3050 | 4551   (in another order)
+          17 of 34      1766 | 1931   2170 | 3575      -      2634 | 5943     -
+        8000 edges
+           9 of 15       140 |  225    139 |  223
+
+    The matrix cores take 16 channels for every number up to 16, 32 up to 32 and 64 up to 64, the compiled kernels what
+    there are, and all paths (200 000 edges, 4 channels, 9 of 15 paths: 940 | 477).  Up to some 250 000 pairs of an edge
+    and a path (120 000 where 64 channels are taken for fewer: 10 000 edges, 36 channels, 23 of 23 paths: 229 | 190) both are
+    short, and the copies and launches of the expansion decide."""
+    if n_edges * paths <= (250_000 if channels <= 32 else 120_000) or channels == 64:
+        return True
+    share = 0.6 if channels <= 32 else 0.74 if channels < 48 else 0.95
+    return channels > 16 and paths <= share * all_paths
+
+
 def uvu_subset_table(cfg: Cfg, tp_info, x: Tensor, y: Tensor, w: Tensor) -> Optional[UvuTable]:
     """The table to run on the matrix cores as it is, where a compiled table only matches with paths the caller's does not
     have: the compiled kernels then take the per-edge weights expanded by zero rows (a copy of the largest operand, there
-    and back) and work through all paths.  9 of 15 paths, 77 coefficients, 32 768 edges, forward and backward: 64 channels
-    510 -> 187 us, 16 channels 226 -> 181.  None where the matrix cores do not take it in both directions."""
-    if int(cfg) < 0 or cfg.w_rows is None or w.ndim != 3 or x.dtype != torch.float32:
+    and back) and work through all paths.  None where that is quicker all the same (``_subset_pays``) or the matrix cores
+    do not take the table and the operands in both directions (``cgtp_uvu_mx_validate``)."""
+    if int(cfg) < 0 or cfg.w_rows is None or w.ndim != 3 or x.dtype != torch.float32 or y.ndim != 2:
+        return None
+    channels, n_edges, paths = x.shape[-1], y.shape[0], w.shape[1]
+    if channels > 64 or not x.shape[0] or not n_edges or not _subset_pays(channels, n_edges, paths, len(cfg.w_rows)):
         return None
     tab = uvu_table_of(tp_info, x.device)
-    if tab is None or tab.mx is None or not uvu_tab_launchable(tab, x, y, w, False):
+    if tab is None or tab.mx is None or (channels <= 32 and tab.nnz <= 64):      # the last: refused by the backward
         return None
-    return tab if all(_lib.lib.cgtp_uvu_mx_validate(C.byref(_tab_probe(x, y, w)), C.byref(tab.c), C.byref(tab.mx), d) == 0
-                      for d in (0, 1)) else None
+    a = _tab_probe(x, y, w)
+    return tab if all(_lib.lib.cgtp_uvu_mx_validate(C.byref(a), C.byref(tab.c), C.byref(tab.mx), d) == 0 for d in (1, 0)) else None
 
 
 def _uvu_tab_launch(a: UvuArgs, tab: UvuTable, backward: int, device) -> None:

@@ -244,6 +244,71 @@ def test_the_wide_walk_covers_the_table(irreps):
         np.testing.assert_allclose(gw, np.einsum("prk,kc,rc->pc", want, g, x), rtol=0, atol=1e-12)
 
 
+# tables with some of a compiled table's paths (own paths of all): lmax 1 (2 of 4), 2 (8 of 11, 9 of 15), 3 (17, 28 of 34)
+SUBSETS = [("0o+1e", "0e+1o", "0e+1e"), ("0o+1e+2o", "0e+1e+2o", "0e+1o+2e"), ("0e+1e+2e", "0e+1o+2e", "0e+1o+2e"),
+           ("0e+1e+2e+3e", "0e+1e+2e+3o", "0e+1e+2o+3o"), ("0e+1e+2e+3e", "0e+1o+2o+3o", "0e+1o+2o+3o")]
+
+
+def _subset_taken(irreps, channels, n_edges):
+    from equitorch_amd.irreps import Irreps
+    from equitorch_amd.ops import kernels
+    info = _info(irreps)
+    cfg = kernels.uvu_config_of(info)
+    assert int(cfg) >= 0 and cfg.w_rows is not None
+    x, y, w = torch.empty(16, Irreps(irreps[1]).dim, channels), torch.empty(n_edges, Irreps(irreps[2]).dim), None
+    w = torch.empty(n_edges, kernels.coo_of(info).P, channels)
+    return kernels.uvu_subset_table(cfg, info, x, y, w) is not None
+
+
+def test_where_a_table_with_some_paths_runs_as_it_is():
+    """At 64 channels and for short lists always; otherwise by the share of the compiled table's paths, by the width the
+    channels are padded to.  Never where the kernels do not take the table or the channels."""
+    from equitorch_amd.ops.kernels import _subset_pays
+    small, p8, p9, p17, p28 = SUBSETS
+    for irreps in (p8, p9, p17, p28):
+        assert _subset_taken(irreps, 64, 50000) and all(_subset_taken(irreps, c, 3000) for c in (8, 16, 32, 48))
+        assert not _subset_taken(irreps, 68, 1000) and not _subset_taken(irreps, 63, 1000)
+    assert not _subset_taken(small, 32, 1000) and _subset_taken(small, 64, 1000)
+    tables = (p8, p9, p17, p28)                                      # 0.73, 0.6, 0.5, 0.82 of the paths
+    for channels, taken in ((8, (0, 0, 0, 0)), (16, (0, 0, 0, 0)), (32, (0, 1, 1, 0)), (36, (1, 1, 1, 0)), (48, (1, 1, 1, 1))):
+        assert [_subset_taken(t, channels, 50000) for t in tables] == [bool(v) for v in taken], channels
+    assert [_subset_taken(p9, 16, n) for n in (27777, 27778)] == [True, False]
+    # a compiled table's paths in another order, or but one
+    assert [_subset_pays(c, 65536, 23, 23) for c in (32, 36, 60, 64)] == [False, False, False, True]
+    assert [_subset_pays(c, 65536, 10, 11) for c in (36, 48, 64)] == [False, True, True]
+    assert [_subset_pays(c, 8000, 23, 23) for c in (16, 32, 36, 60)] == [True, True, False, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("irreps", SUBSETS)
+@pytest.mark.parametrize("channels,n_nodes,n_edges", [(64, 40, 700), (36, 3, 2000), (24, 300, 900), (8, 30, 400)])
+def test_a_table_with_some_paths_on_both_routes(device, monkeypatch, irreps, channels, n_nodes, n_edges):
+    """As it is and on the compiled table with expanded weights, both against the oracle."""
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    from equitorch_amd.ops import kernels
+    info = _info(irreps).to(device)
+    src, dst, x, y, w, ct = _edge_case(irreps, channels, n_nodes, n_edges, False, stable_seed("subset", irreps, channels))
+    plan = EdgePlan(src.to(device), dst.to(device), n_nodes)
+    T = ref_ops.dense_coupling(*irreps).float().double()
+
+    def ref_fn(T, x, sh, w):
+        return ref_ops.scatter_sum(ref_ops.dense_u1u(T, x.index_select(0, src), sh, w), dst, n_nodes)
+    ref_out, ref_grads = ref_ops.dense_grads(ref_fn, T, (x, y, w), ct)
+    launches = []
+    launch = kernels._uvu_tab_launch
+    monkeypatch.setattr(kernels, "_uvu_tab_launch", lambda *args: (launches.append(1), launch(*args)))
+    for route in ("as it is", "expanded"):
+        if route == "expanded":
+            monkeypatch.setattr(kernels, "uvu_subset_table", lambda *args: None)
+        wrt = [t.to(device).requires_grad_(True) for t in (x, y, w)]
+        out = edge_tensor_product_uu(*wrt, plan, info)
+        grads = torch.autograd.grad(out, wrt, ct.to(device))
+        for name, got, want in zip(("out", "grad x", "grad y", "grad w"), (out, *grads), (ref_out, *ref_grads)):
+            assert_close(got, want, 1e-5, f"{irreps} C={channels} {route}: {name}", norm="max")
+        assert len(launches) == (2 if route == "as it is" and (channels > 32 or irreps != SUBSETS[0]) else 0)
+        launches.clear()
+
+
 @pytest.mark.gpu
 def test_recorded_in_a_graph(device):
     """Forward and gradients recorded into a HIP graph and replayed on new inputs, eager work in between: the flags of the
