@@ -218,23 +218,25 @@ class _EdgeUvuRadial(Function):
 
 class _EdgeUvuTable(Function):
     """Gather, product and segment sum in one launch for a table that is not compiled in: the table-driven segment
-    kernels (``cgtp_uvu_tab_fwd`` / ``cgtp_uvu_tab_bwd``), tables read through the scalar cache, the per-edge
-    operands and the segment sums in LDS."""
+    kernels, on the matrix cores (``cgtp_uvu_mx_fwd`` / ``_bwd``; ``as_it_is``: wherever these take it) or entry by entry
+    (``cgtp_uvu_tab_fwd`` / ``_bwd``), tables read through the scalar cache, the per-edge operands and the segment sums
+    in LDS."""
 
     @staticmethod
-    def forward(ctx, x: Tensor, sh: Tensor, w: Tensor, plan: EdgePlan, tab, tp_info: TensorProductInfo):
-        out = kernels.uvu_tab_forward(tab, x, sh, w, plan.fwd_index)
+    def forward(ctx, x: Tensor, sh: Tensor, w: Tensor, plan: EdgePlan, tab, tp_info: TensorProductInfo, as_it_is: bool):
+        out = kernels.uvu_tab_forward(tab, x, sh, w, plan.fwd_index, as_it_is)
         ctx.save_for_backward(x, sh, w)
-        ctx.plan, ctx.tab, ctx.tp_info = plan, tab, tp_info
+        ctx.plan, ctx.tab, ctx.tp_info, ctx.as_it_is = plan, tab, tp_info, as_it_is
         return out
 
     @staticmethod
     def backward(ctx, g):
         x, sh, w = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return (*_higher_order(_unfused(ctx.plan, ctx.tp_info), (x, sh, w), ctx.needs_input_grad[:3], g), None, None, None)
-        res = kernels.uvu_tab_backward(ctx.tab, x, sh, w, g.contiguous(), ctx.needs_input_grad[:3], ctx.plan.bwd_index)
-        return (*res, None, None, None)
+            return (*_higher_order(_unfused(ctx.plan, ctx.tp_info), (x, sh, w), ctx.needs_input_grad[:3], g), None, None, None, None)
+        res = kernels.uvu_tab_backward(ctx.tab, x, sh, w, g.contiguous(), ctx.needs_input_grad[:3], ctx.plan.bwd_index,
+                                       ctx.as_it_is)
+        return (*res, None, None, None, None)
 
 
 class _EdgeUvuRows(Function):
@@ -288,7 +290,7 @@ def edge_tensor_product_uu(x: Tensor, sh: Tensor, weight: Tensor, plan: EdgePlan
         if tab is not None:
             kernels.log_tier("edge_tensor_product_uu", "table-driven fused gather / product / segment sum",
                              f"{tab.nnz} coefficients, some paths of config {int(cfg)}")
-            return _EdgeUvuTable.apply(xc, yc, wc, plan, tab, tp_info_forward)
+            return _EdgeUvuTable.apply(xc, yc, wc, plan, tab, tp_info_forward, True)
         if kernels.uvu_launchable(cfg, xc, yc, wc, segments=True):
             kernels.log_tier("edge_tensor_product_uu", "fused gather / product / segment sum", f"config {int(cfg)}")
             handle = _shim_handle(plan, cfg, xc, 0, tp_info_forward)
@@ -305,7 +307,7 @@ def edge_tensor_product_uu(x: Tensor, sh: Tensor, weight: Tensor, plan: EdgePlan
         if kernels.uvu_tab_launchable(tab, xc, yc, wc, weight.requires_grad and torch.is_grad_enabled()):
             kernels.log_tier("edge_tensor_product_uu", "table-driven fused gather / product / segment sum",
                              f"{tab.nnz} coefficients")
-            return _EdgeUvuTable.apply(xc, yc, wc, plan, tab, tp_info_forward)
+            return _EdgeUvuTable.apply(xc, yc, wc, plan, tab, tp_info_forward, False)
     kernels.log_tier("edge_tensor_product_uu", "index_select + tensor_product_u1u + sparse_scale")
     msg = tensor_product_u1u(x.index_select(0, plan.src), sh, weight, tp_info_forward)
     e, d, c = msg.shape

@@ -1066,19 +1066,58 @@ def uvu_subset_table(cfg: Cfg, tp_info, x: Tensor, y: Tensor, w: Tensor) -> Opti
     return tab if all(_lib.lib.cgtp_uvu_mx_validate(C.byref(a), C.byref(tab.c), C.byref(tab.mx), d) == 0 for d in (1, 0)) else None
 
 
-def _uvu_tab_launch(a: UvuArgs, tab: UvuTable, backward: int, device) -> None:
+def _mx_pays(backward: int, channels: int, n_rows: int, n_seg: int, nnz: int, shared: bool) -> bool:
+    """Whether the matrix-core kernels are quicker than the walk entry by entry.  Kernel times in us, per-edge weights, matrix
+    cores | entry by entry (coefficients):
+
+        forward           10 000 edges                 200 000 edges
+        channels       4         16         64         4          16         32          48         64
+             2      14 | 32    14 | 20    15 | 17   119 | 41   125 | 40   142 | 57    152 | 92   113 | 93
+            39      19 | 46    20 | 36    25 | 42   227 | 66   252 | 136  286 | 244   354 | 472  232 | 480
+            70      18 | 60    19 | 42    23 | 42   201 | 79   218 | 146  247 | 236   277 | 238  199 | 242
+           105      17 | 71    18 | 48    25 | 53   178 | 158  199 | 178  219 | 289   235 | 498  154 | 503
+           147      21 | 103   21 | 69    27 | 72   259 | 250  279 | 276  318 | 462   402 | 841  284 | 851
+           206      30 | 128   31 | 91    45 | 102  449 | 539  488 | 525  623 | 711   732 | 1266 516 | 1274
+        backward
+            30      28 | 64    27 | 52    34 | 56   329 | 89   341 | 190  391 | 322   408 | 591  346 | 599
+            70      33 | 105   34 | 85    46 | 89   451 | 225  470 | 318  551 | 549   627 | 1014 554 | 1031
+           147      42 | 194   42 | 154   61 | 161  606 | 828  632 | 853  761 | 1558  935 | 2017 800 | 2036
+
+    The coupling matrix of an edge and the contraction over 16, 32 or 64 channels cost the same for fewer, while the walk
+    takes as many edges per wavefront as their channels fit; a short list leaves the walk few wavefronts.  (Up to three
+    channels the walk takes one per lane and half the time.  50 coefficients, 64 channels, a shared weight: 336 | 255.)
+    Segments of one position (a plain batch) cost the matrix cores a row of results each, 65 536 rows: 147 coefficients, 4
+    and 16 channels, forward 100 | 113 and 113 | 94, backward 244 | 208 and 260 | 334; 39, 48 channels, backward 406 | 329."""
+    if nnz < 16:
+        return False
+    if n_rows <= 16384:
+        return True
+    if channels > 51:
+        return nnz >= 56 or not shared or bool(backward)
+    short = 2 * n_seg > n_rows                # segments of one position or so
+    if channels > 32:
+        return nnz >= (28 if backward and not short else 73)
+    if channels > 16:
+        return nnz >= (65 if backward else 100)
+    if nnz < 140:
+        return False
+    return bool(backward) and channels > 8 if short else channels > 3 and (bool(backward) or nnz >= 300 or n_rows <= 131072)
+
+
+def _uvu_tab_launch(a: UvuArgs, tab: UvuTable, backward: int, device, as_it_is: bool) -> None:
     """Launches on the matrix cores where the table and the operands fit them (see ``uvu_mx_words`` and
-    ``cgtp_uvu_mx_validate``: at most 64 channels, of which a lane takes one, two or four at a time), entry by entry
-    elsewhere.  206 coefficients, 65 536 edges, 64 channels: forward 175 us against 411,
-    backward 371 against 1303."""
+    ``cgtp_uvu_mx_validate``: at most 64 channels, of which a lane takes one, two or four at a time) and they are the
+    quicker ones (``_mx_pays``; ``as_it_is``: the caller has decided, see ``uvu_subset_table``), entry by entry elsewhere."""
     mx = tab.mx
-    if mx is not None and _lib.lib.cgtp_uvu_mx_validate(C.byref(a), C.byref(tab.c), C.byref(mx), backward) == 0:
+    if mx is not None and (as_it_is or _mx_pays(backward, a.C, a.n_rows, a.n_seg, tab.nnz, bool(a.w_shared))):
+        # negative where the kernels do not take the launch; the launch itself checks again, with the workspace
         nbytes = int(_lib.lib.cgtp_uvu_mx_workspace_bytes(C.byref(a), C.byref(tab.c), C.byref(mx), backward))
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        a.workspace = ws.data_ptr()
-        launch = _lib.lib.cgtp_uvu_mx_bwd if backward else _lib.lib.cgtp_uvu_mx_fwd
-        _lib.check(launch(C.byref(a), C.byref(tab.c), C.byref(mx), _lib.stream_ptr(device)), "cgtp_uvu_mx")
-        return
+        if nbytes >= 0:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            a.workspace = ws.data_ptr()
+            launch = _lib.lib.cgtp_uvu_mx_bwd if backward else _lib.lib.cgtp_uvu_mx_fwd
+            _lib.check(launch(C.byref(a), C.byref(tab.c), C.byref(mx), _lib.stream_ptr(device)), "cgtp_uvu_mx")
+            return
     ws = _uvu_tab_workspace(a, tab, backward, device)
     launch = _lib.lib.cgtp_uvu_tab_bwd if backward else _lib.lib.cgtp_uvu_tab_fwd
     _lib.check(launch(C.byref(a), C.byref(tab.c), _lib.stream_ptr(device)), "cgtp_uvu_tab")
@@ -1095,16 +1134,16 @@ def _uvu_tab_workspace(a: UvuArgs, tab: UvuTable, backward: int, device):
     return ws
 
 
-def uvu_tab_forward(tab: UvuTable, x: Tensor, y: Tensor, w: Tensor, seg: SegIndex) -> Tensor:
+def uvu_tab_forward(tab: UvuTable, x: Tensor, y: Tensor, w: Tensor, seg: SegIndex, as_it_is: bool = False) -> Tensor:
     """``out[s] = sum_{q in segment s} TP(x[seg.gather[q]], y[e_q], w[e_q])`` for any table, one launch."""
     a = _uvu_tab_args(x, y, w, seg)
     out = torch.empty((a.n_seg, tab.dims[2], x.shape[-1]), dtype=x.dtype, device=x.device)
     a.out = out.data_ptr()
-    _uvu_tab_launch(a, tab, 0, x.device)
+    _uvu_tab_launch(a, tab, 0, x.device, as_it_is)
     return out
 
 
-def uvu_tab_backward(tab: UvuTable, x: Tensor, y: Tensor, w: Tensor, g: Tensor, need, seg: SegIndex):
+def uvu_tab_backward(tab: UvuTable, x: Tensor, y: Tensor, w: Tensor, g: Tensor, need, seg: SegIndex, as_it_is: bool = False):
     """-> (grad_x, grad_y, grad_w) over the list sorted by the other end (``seg``: segments = rows of x)."""
     a = _uvu_tab_args(x, y, w, seg)
     a.grad_out = g.data_ptr()
@@ -1112,7 +1151,7 @@ def uvu_tab_backward(tab: UvuTable, x: Tensor, y: Tensor, w: Tensor, g: Tensor, 
     gy = torch.empty_like(y) if need[1] else None
     gw = torch.empty_like(w) if need[2] else None
     a.grad_x, a.grad_y, a.grad_w = _lib.ptr(gx), _lib.ptr(gy), _lib.ptr(gw)
-    _uvu_tab_launch(a, tab, 1, x.device)
+    _uvu_tab_launch(a, tab, 1, x.device, as_it_is)
     return gx, gy, gw
 
 

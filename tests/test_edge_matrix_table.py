@@ -141,10 +141,12 @@ def _paths(irreps):
 @pytest.mark.parametrize("channels,n_nodes,n_edges,hub", [(64, 5, 1, False), (60, 40, 700, True), (48, 3, 9000, False),
                                                           (32, 300, 2049, True), (18, 50, 600, False), (16, 70, 900, False),
                                                           (5, 30, 400, True), (36, 3000, 2500, False)])
-def test_product_and_gradients(device, irreps, channels, n_nodes, n_edges, hub):
+def test_product_and_gradients(device, monkeypatch, irreps, channels, n_nodes, n_edges, hub):
     """One, two and four channels per lane with and without idle lanes; one edge, ranges of more than 64 positions,
     nodes without edges, a node whose edges span many ranges; every subset of gradients the kernels tell apart."""
     from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    from equitorch_amd.ops import kernels
+    monkeypatch.setattr(kernels, "_mx_pays", lambda *args: True)          # the kernels, also where the walk is quicker
     info = _info(irreps).to(device)
     src, dst, x, y, w, ct = _edge_case(irreps, channels, n_nodes, n_edges, hub, stable_seed("mx", irreps, channels))
     plan = EdgePlan(src.to(device), dst.to(device), n_nodes)
@@ -277,6 +279,51 @@ def test_where_a_table_with_some_paths_runs_as_it_is():
     assert [_subset_pays(c, 65536, 23, 23) for c in (32, 36, 60, 64)] == [False, False, False, True]
     assert [_subset_pays(c, 65536, 10, 11) for c in (36, 48, 64)] == [False, True, True]
     assert [_subset_pays(c, 8000, 23, 23) for c in (16, 32, 36, 60)] == [True, True, False, False]
+
+
+def test_where_the_walk_entry_by_entry_is_quicker():
+    from equitorch_amd.ops.kernels import _mx_pays
+    takes = lambda backward, nnz, n, shared=False, degree=16: [_mx_pays(backward, c, n, n // degree, nnz, shared)  # noqa: E731
+                                                               for c in (1, 4, 16, 32, 48, 64)]
+    for backward in (0, 1):
+        assert takes(backward, 2, 1000) == takes(backward, 2, 200000) == [False] * 6
+        assert takes(backward, 39, 1000) == takes(backward, 206, 16384) == [True] * 6
+    assert takes(0, 39, 200000) == [False] * 5 + [True] and takes(0, 105, 200000) == [False] * 3 + [True] * 3
+    assert takes(0, 206, 100000) == [False] + [True] * 5 and takes(0, 206, 200000) == [False] * 3 + [True] * 3
+    assert takes(0, 351, 200000) == [False] + [True] * 5
+    assert takes(1, 39, 200000) == [False] * 4 + [True] * 2 and takes(1, 70, 200000) == [False] * 3 + [True] * 3
+    assert takes(1, 147, 500000) == [False] + [True] * 5
+    assert takes(0, 147, 65536, degree=1) == [False] * 3 + [True] * 3 and takes(1, 147, 65536, degree=1) == [False] * 2 + [True] * 4
+    assert takes(1, 39, 65536, degree=1) == [False] * 5 + [True]
+    assert takes(0, 50, 200000, True) == [False] * 6 and takes(1, 50, 200000, True) == [False] * 4 + [True] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels,n_edges,want", [(16, 20000, [False, False]), (64, 20000, [True, True]), (48, 20000, [False, True]),
+                                                   (16, 2000, [True, False])])
+def test_long_lists_take_the_quicker_kernels(device, monkeypatch, channels, n_edges, want):
+    """Which kernels run for 39 coefficients (forward, backward), and that the results are the oracle's."""
+    from equitorch_amd import _lib
+    from equitorch_amd.nn.functional import EdgePlan, edge_tensor_product_uu
+    irreps = TABLES[0]
+    info = _info(irreps).to(device)
+    src, dst, x, y, w, ct = _edge_case(irreps, channels, 500, n_edges, False, stable_seed("quicker", channels, n_edges))
+    plan = EdgePlan(src.to(device), dst.to(device), 500)
+    ran = []
+    for name, mx in (("cgtp_uvu_mx_fwd", True), ("cgtp_uvu_mx_bwd", True), ("cgtp_uvu_tab_fwd", False), ("cgtp_uvu_tab_bwd", False)):
+        entry = getattr(_lib.lib, name)
+        monkeypatch.setattr(_lib.lib, name, lambda *args, entry=entry, mx=mx: (ran.append(mx), entry(*args))[1])
+    wrt = [t.to(device).requires_grad_(True) for t in (x, y, w)]
+    out = edge_tensor_product_uu(*wrt, plan, info)
+    grads = torch.autograd.grad(out, wrt, ct.to(device))
+    assert ran == want
+    T = ref_ops.dense_coupling(*irreps).float().double()
+
+    def ref_fn(T, x, sh, w):
+        return ref_ops.scatter_sum(ref_ops.dense_u1u(T, x.index_select(0, src), sh, w), dst, 500)
+    ref_out, ref_grads = ref_ops.dense_grads(ref_fn, T, (x, y, w), ct)
+    for name, got, ref in zip(("out", "grad x", "grad y", "grad w"), (out, *grads), (ref_out, *ref_grads)):
+        assert_close(got, ref, 1e-5, f"C={channels} {name}", norm="max")
 
 
 @pytest.mark.gpu
