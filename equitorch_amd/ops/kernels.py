@@ -511,15 +511,21 @@ class SegIndex:
             pos = ptr[:-1][seg] + (targets - first[seg]) * slots
             self._wave_pos[slots] = torch.from_numpy(np.concatenate([pos, [n_pos]]).astype(np.int64)).to(self.ptr.device)
 
-    def prefers_aligned(self, slots: int, backward: bool) -> bool:
-        """Whether a launch with ``slots`` edges per step runs on the segment-aligned ranges.  The backward, with its
-        long steps, never does (lmax 2, C = 64, 65 536 edges: 94.4 us balanced, 102 aligned); neither does a forward
-        with one or two edges per step (lmax 3: 114.6 against 123.4 us), one whose steps do not fill the chip, where a
-        node's edges in one wavefront would take longer than the launch (8192 edges: 15.6 against 17.4 us at lmax 2,
-        27.7 against 48.9 at lmax 3), or one with a node of far more edges than the average wavefront takes.  Otherwise
-        aligned ranges save the partial rows and the fix-up (54.4 against 55.1 us; lmax 1, 200 000 edges: 61.9 against 70)."""
-        return (not backward and slots > 2 and self.wave_seg is not None and self.n_positions > _RESIDENT_WAVES * slots
-                and self.longest <= max(48, self.n_positions >> 10))
+    def prefers_aligned(self, slots: int, backward: bool, nnz: int) -> bool:
+        """Whether a launch with ``slots`` edges per step over a table of ``nnz`` coefficients runs on the segment-aligned
+        ranges.  The backward, with its long steps, never does (lmax 2, C = 64, 65 536 edges: 94.4 us balanced, 102 aligned).
+        A forward on aligned ranges has no partial rows and no fix-up pass, about 5 us, and fewer ranges to end, each with a
+        sum over its slots, but lasts at least as long as the steps of the longest segment: it pays while these are not too
+        many more than a wavefront's share, at 0.15 us a step and 0.01 per coefficient.  Aligned against balanced: 60 000
+        edges of degree 64, lmax 2, 16 channels (6 steps of 16 edges for 2) 20.1 against 25.4 us, lmax 3, 4 channels (3 of 32 for
+        1) 27.6 against 38.6; 8192 edges, C = 64, lmax 2 (8 steps of 4 for 1) 17.4 against 15.6, lmax 3 48.9 against 27.7;
+        65 536 edges, lmax 2 54.4 against 55.1.  With one or two edges per step the ranges' different lengths cost more
+        (lmax 3: 123.4 against 114.6), but for the smallest tables (lmax 1, C = 128, 60 000 edges of degree 4: 44.9 against
+        50.1)."""
+        if backward or self.wave_seg is None or (slots <= 2 and nnz > 32):
+            return False
+        excess = -(-self.longest // slots) - max(1.0, self.n_positions / (slots * _RESIDENT_WAVES))
+        return excess * (0.15 + 0.01 * nnz) <= 5.0 + 0.25 * slots
 
     @staticmethod
     def aligned_ranges(ptr: Tensor, positions_per_wave: int) -> Optional[Tensor]:
@@ -557,7 +563,8 @@ def seg_ranges(cfg: int, seg: SegIndex, dtype_code: int, channels: int, backward
     if _lib.lib.cgtp_uvu_blockwise_only(int(cfg)):
         return None, None
     slots = int(_lib.lib.cgtp_uvu_slots(int(cfg), dtype_code, channels, int(backward)))
-    if _RANGE_MODE == "balanced" or (_RANGE_MODE == "auto" and not seg.prefers_aligned(slots, backward or long_steps)):
+    if _RANGE_MODE == "balanced" or (_RANGE_MODE == "auto" and not seg.prefers_aligned(
+            slots, backward or long_steps, _compiled_tables("uvu")[int(cfg)][0][4])):
         wave_pos = seg.balanced_positions(slots)
         if wave_pos is not None:
             return None, wave_pos
