@@ -464,8 +464,8 @@ class SegIndex:
     rounds of resident wavefronts (``balanced_positions``).  Kernel times at C = 64, average degree 14-20, forward |
     backward in us, with 32 positions per range as for every list before and with this rule:
 
-        lmax 2:   420 edges 19.9 | 36.7 -> 10.1 | 14.6    8192: 28.3 | 44.1 -> 15.6 | 25.3    32768: 31.6 | 53.3 -> 28.9 | 53.2
-        lmax 3:   420 edges 73.5 | 196  -> 19.0 | 43.8    8192: 78.1 | 202  -> 27.7 | 58.2    32768: 88.8 | 210  -> 64.6 | 144
+        lmax 2:   420 edges 19.9 | 37.4 ->  9.5 | 12.5    8192: 27.6 | 45.7 -> 14.9 | 28.2    32768: 33.0 | 56.1 -> 28.8 | 55.1
+        lmax 3:   420 edges 67.4 | 190  -> 15.9 | 26.5    8192: 82.0 | 202  -> 28.6 | 61.5    32768: 91.5 | 207  -> 65.6 | 156
 
     ``positions_per_wave``: a fixed number of positions per range instead of the rule (both kinds of range)."""
 
@@ -514,18 +514,19 @@ class SegIndex:
     def prefers_aligned(self, slots: int, backward: bool, nnz: int) -> bool:
         """Whether a launch with ``slots`` edges per step over a table of ``nnz`` coefficients runs on the segment-aligned
         ranges.  The backward, with its long steps, never does (lmax 2, C = 64, 65 536 edges: 94.4 us balanced, 102 aligned).
-        A forward on aligned ranges has no partial rows and no fix-up pass, about 5 us, and fewer ranges to end, each with a
+        A forward on aligned ranges has no partial rows and no fix-up pass, about 4 us, and fewer ranges to end, each with a
         sum over its slots, but lasts at least as long as the steps of the longest segment: it pays while these are not too
-        many more than a wavefront's share, at 0.15 us a step and 0.01 per coefficient.  Aligned against balanced: 60 000
+        many more than a wavefront's share, at 0.1 us a step and 0.01 per coefficient.  Aligned against balanced: 60 000
         edges of degree 64, lmax 2, 16 channels (6 steps of 16 edges for 2) 20.1 against 25.4 us, lmax 3, 4 channels (3 of 32 for
-        1) 27.6 against 38.6; 8192 edges, C = 64, lmax 2 (8 steps of 4 for 1) 17.4 against 15.6, lmax 3 48.9 against 27.7;
+        1) 27.6 against 38.6; C = 64, lmax 2, 420 edges (6 steps of 4 for 1) whole calls 12.4 against 14.4, one launch less,
+        but 7 steps 12.5 against 9.5 in the kernels, 8192 edges (7 for 1) 16.3 against 14.9, lmax 3 48.9 against 28.6;
         65 536 edges, lmax 2 54.4 against 55.1.  With one or two edges per step the ranges' different lengths cost more
         (lmax 3: 123.4 against 114.6), but for the smallest tables (lmax 1, C = 128, 60 000 edges of degree 4: 44.9 against
         50.1)."""
         if backward or self.wave_seg is None or (slots <= 2 and nnz > 32):
             return False
         excess = -(-self.longest // slots) - max(1.0, self.n_positions / (slots * _RESIDENT_WAVES))
-        return excess * (0.15 + 0.01 * nnz) <= 5.0 + 0.25 * slots
+        return excess * (0.1 + 0.01 * nnz) <= 4.5 + 0.25 * slots
 
     @staticmethod
     def aligned_ranges(ptr: Tensor, positions_per_wave: int) -> Optional[Tensor]:
