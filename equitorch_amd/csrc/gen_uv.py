@@ -258,12 +258,15 @@ def emit_split(out_dir: str) -> str:
         swapped = coo._replace(M1=coo.M2, M2=coo.M1, D1=coo.D2, D2=coo.D1)
         chunks.append(emit_direction(name, 1, swapped, seg_out, irrep_segments(Irreps(i2)), split=True)
                       .replace(f"struct UVS_{name}_d1 ", f"struct UVS_{name}_d2 "))
-        terms = ", ".join(f"{{{_lit(coo.coef[t])}, {coo.M[t]}, {coo.M1[t]}, {coo.M2[t]}, {coo.p[t]}}}"
-                          for t in range(coo.coef.shape[0]))
-        chunks.append(f"static __device__ const UvsTerm UVS_{name}_terms[] = {{{terms}}};")
+        # the terms in the order of (row of the result, path) of every kind of launch
+        T = range(coo.coef.shape[0])
+        orders = [sorted(T, key=lambda t: (int(rows[t]), int(coo.p[t]))) for rows in (coo.M, coo.M1, coo.M2)]
+        terms = ", ".join("{" + ", ".join(f"{{{_lit(coo.coef[t])}, {coo.M[t]}, {coo.M1[t]}, {coo.M2[t]}, {coo.p[t]}}}"
+                                          for t in order) + "}" for order in orders)
+        chunks.append(f"static __device__ const UvsTerm UVS_{name}_terms[3][{len(T)}] = {{{terms}}};")
         chunks.append(f"struct UVS_{name}_table {{")
-        chunks.append(f"  static constexpr int N = {coo.coef.shape[0]};")
-        chunks.append(f"  __device__ __forceinline__ static const UvsTerm* terms() {{ return UVS_{name}_terms; }}")
+        chunks.append(f"  static constexpr int N = {len(T)};")
+        chunks.append(f"  __device__ __forceinline__ static const UvsTerm* terms(int kind) {{ return UVS_{name}_terms[kind]; }}")
         chunks.append("};")
         chunks.append("")
     chunks.append("#define CGTP_FOREACH_UVS_CONFIG(X) \\")

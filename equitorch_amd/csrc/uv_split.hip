@@ -27,7 +27,7 @@
 // An x or W with an element that is not finite, from 2^60 on (Z could overflow where coupling first does not) or below 2^-110 but
 // not zero (its last part could be below the smallest subnormal), a y that is not finite, or a y of 16 and more next to an x or W below 2^-50 (Z could
 // underflow where coupling first does not) is not split: the workgroup then forms its samples' results with fp32 matrix
-// instructions, term by term of the table and the coupling first (uvs_plain_tile), so that such values reach exactly the
+// instructions, the coupling first (UvsPlain), so that such values reach exactly the
 // results they couple to.
 #include "uv_common.h"
 
@@ -282,27 +282,62 @@ struct UvsOps {
   }
 };
 
-// (s x) W of one path and row for the two tiles of block `blk`, from memory, in fp32 matrix instructions.
+// ---- workgroups whose operands are not split: fp32 matrix instructions, operands from memory ---------------------
+// The coupling comes first, path by path and row by row of the result, so the table is walked in the order of (row, path).
+// A lane of the contraction's quarter q holds K / 4 consecutive elements of its sample; any order of k will do where both
+// operands agree.  One wavefront per SIMD or two, waiting for memory most of the time.  128 -> 128 channels, lmax 3: a launch
+// with one such workgroup 613 us (term by term 2433), 4096 samples that all are 647 (fp32 instructions throughout: 181).
 template <int K>
-__device__ __forceinline__ void uvs_plain_tile(const UvsWeight& W, int p, int blk, const float* __restrict__ xrow, float s,
-                                               int r, int q, floatx4 (&z)[2]) {
-  z[0] = z[1] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const float* wb = W.of(p) + (blk * 32 + 8 * (r >> 2) + (r & 3)) * W.stride_c;
-  constexpr int STEPS = 8;      // of which the loads are in flight together
-  static_assert(K % (4 * STEPS) == 0, "whole groups of steps");
-#pragma unroll 1
-  for (int k0 = q; k0 < K; k0 += 4 * STEPS) {
-    float b[STEPS], w[STEPS][2];
+struct UvsPlain {
+  static constexpr int N = K / 4;
+  float u[N];
+  __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-      b[i] = s * xrow[k0 + 4 * i];
+    for (int i = 0; i < N; ++i) u[i] = 0.f;
+  }
+  __device__ __forceinline__ void mix(const float* __restrict__ xrow, float s, int q) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) w[i][t] = wb[(k0 + 4 * i) * W.stride_k + 4 * t * W.stride_c];
+    for (int i = 0; i < N; i += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(xrow + q * N + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[i + j] += s * v[j];
     }
+  }
+  // o += u W for the two tiles of block `blk`.
+  __device__ __forceinline__ void multiply(const UvsWeight& W, int matrix, int blk, int r, int q, floatx4 (&o)[2]) const {
+    const float* wb = W.of(matrix) + (blk * 32 + 8 * (r >> 2) + (r & 3)) * W.stride_c + q * N * W.stride_k;
+    floatx4 z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr int STEPS = 8;      // of which the loads are in flight together
 #pragma unroll
-    for (int i = 0; i < STEPS; ++i)
+    for (int i0 = 0; i0 < N; i0 += STEPS) {
+      float w[STEPS][2];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) z[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][t], b[i], z[t], 0, 0, 0);
+      for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) w[i][t] = wb[(i0 + i) * W.stride_k + 4 * t * W.stride_c];
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) z[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][t], u[i0 + i], z[t], 0, 0, 0);
+    }
+    o[0] += z[0];
+    o[1] += z[1];
+  }
+};
+// Rows of the result, of the contracted operand and of the other one; KIND as for the launches with channels on both operands.
+template <int KIND>
+__device__ __forceinline__ int uvs_row_of(const UvsTerm& e) { return KIND == 0 ? e.o : KIND == 1 ? e.a : e.b; }
+template <int KIND>
+__device__ __forceinline__ int uvs_in_of(const UvsTerm& e) { return KIND == 0 ? e.a : e.o; }
+template <int KIND>
+__device__ __forceinline__ int uvs_other_of(const UvsTerm& e) { return KIND == 2 ? e.a : e.b; }
+// The terms of (row, path) from t on; `t` moves behind them.
+template <class TAB, int KIND, class F>
+__device__ __forceinline__ void uvs_segment(int& t, int row, int path, F&& f) {
+  for (; t < TAB::N; ++t) {
+    const UvsTerm e = TAB::terms(KIND)[t];
+    if (uvs_row_of<KIND>(e) != row || e.p != path) break;
+    f(e);
   }
 }
 
@@ -339,15 +374,17 @@ __global__ void __launch_bounds__(256, WAVES) uvs_kernel(const float* __restrict
     }
   };
   if (plain) {
+    UvsPlain<CIN> P;
+    int t = 0;
     for (int row = 0; row < DOUT; ++row) {
       floatx4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-      for (int t = 0; t < TAB::N; ++t) {
-        const UvsTerm e = TAB::terms()[t];
-        if ((DIR == 0 ? e.o : e.a) != row) continue;
-        floatx4 z[2];
-        uvs_plain_tile<CIN>(W, e.p, wblk, x + (row_n * DIN + (DIR == 0 ? e.a : e.o)) * CIN, e.c * y[row_n * D2 + e.b], n, q, z);
-        o[0] += z[0];
-        o[1] += z[1];
+      while (t < TAB::N && uvs_row_of<DIR>(TAB::terms(DIR)[t]) == row) {
+        const int path = TAB::terms(DIR)[t].p;
+        P.clear();
+        uvs_segment<TAB, DIR>(t, row, path, [&](const UvsTerm& e) __attribute__((always_inline)) {
+          P.mix(x + (row_n * DIN + uvs_in_of<DIR>(e)) * CIN, e.c * y[row_n * D2 + e.b], q);
+        });
+        P.multiply(W, path, wblk, n, q, o);
       }
       store(row, o[0], o[1]);
     }
@@ -392,15 +429,21 @@ __global__ void __launch_bounds__(256, WAVES) uvs_gy_kernel(const float* __restr
   };
   if (wave < n_blocks) {
     if (plain) {
-      for (int t = 0; t < TAB::N; ++t) {
-        const UvsTerm e = TAB::terms()[t];
-        floatx4 z[2], g0, g1;
-        uvs_plain_tile<CIN>(W, e.p, wave, x + (row_n * DIN + e.a) * CIN, 1.f, n, q, z);
-        load_g(e.o, g0, g1);
-        const float v = e.c * dot8(g0, g1, z[0], z[1]);
+      UvsPlain<CIN> P;
+      for (int t = 0; t < TAB::N;) {      // in the order of (row of x, path), whose terms share Z
+        const int row = TAB::terms(1)[t].a, path = TAB::terms(1)[t].p;
+        floatx4 z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        P.clear();
+        P.mix(x + (row_n * DIN + row) * CIN, 1.f, q);
+        P.multiply(W, path, wave, n, q, z);
+        uvs_segment<TAB, 1>(t, row, path, [&](const UvsTerm& e) __attribute__((always_inline)) {
+          floatx4 g0, g1;
+          load_g(e.o, g0, g1);
+          const float v = e.c * dot8(g0, g1, z[0], z[1]);
 #pragma unroll
-        for (int j = 0; j < D2; ++j)
-          if (j == e.b) part[j] += v;
+          for (int j = 0; j < D2; ++j)
+            if (j == e.b) part[j] += v;
+        });
       }
     } else {
       const UvsOps<DIN, CIN> ops{wp + (int64_t)wave * (6 * (CIN / 32) * 512) + lane * 8, (int64_t)cout * CIN * 3,
@@ -475,20 +518,25 @@ __global__ void __launch_bounds__(256, 2) uvsw_kernel(const float* __restrict__ 
     }
   };
   if (plain) {
-    for (int row = wave; row < DOUT; row += 4) {
+    UvsPlain<CIN> P;
+    int t = 0;
+    for (int row = 0; row < DOUT; ++row) {
       floatx4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-      for (int t = 0; t < TAB::N; ++t) {
-        const UvsTerm e = TAB::terms()[t];
-        const int mt = KIND == 0 ? e.o : KIND == 1 ? e.a : e.b, at = KIND == 0 ? e.a : e.o, bt = KIND == 2 ? e.a : e.b;
-        if (mt != row) continue;
-        for (int l = 0; l < L; ++l) {
-          floatx4 v[2];
-          uvs_plain_tile<CIN>(W, e.p * L + l, wblk, x + (row_n * DIN + at) * CIN, e.c * z[(row_n * D2 + bt) * L + l], n, q, v);
-          o[0] += v[0];
-          o[1] += v[1];
+      while (t < TAB::N && uvs_row_of<KIND>(TAB::terms(KIND)[t]) == row) {
+        const int path = TAB::terms(KIND)[t].p;
+        int end = t;
+        uvs_segment<TAB, KIND>(end, row, path, [](const UvsTerm&) {});
+        for (int l = 0; l < L && (row & 3) == wave; ++l) {
+          P.clear();
+          int i = t;
+          uvs_segment<TAB, KIND>(i, row, path, [&](const UvsTerm& e) __attribute__((always_inline)) {
+            P.mix(x + (row_n * DIN + uvs_in_of<KIND>(e)) * CIN, e.c * z[(row_n * D2 + uvs_other_of<KIND>(e)) * L + l], q);
+          });
+          P.multiply(W, path * L + l, wblk, n, q, o);
         }
+        t = end;
       }
-      store(row, o[0], o[1]);
+      if ((row & 3) == wave) store(row, o[0], o[1]);
     }
     return;
   }
