@@ -121,6 +121,14 @@ class UvtGyArgs(C.Structure):
                 ("cx", C.c_int32), ("cout", C.c_int32), ("dtype", C.c_int32)]
 
 
+class UvlArgs(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("packed", C.c_void_p), ("w", C.c_void_p), ("out", C.c_void_p),
+                ("steps", C.c_void_p), ("tasks", C.c_void_p), ("groups", C.c_void_p),
+                ("blocks", C.c_void_p), ("n_rows", C.c_int64), ("stride_p", C.c_int64), ("stride_k", C.c_int64), ("stride_c", C.c_int64),
+                ("n_blocks", C.c_int32), ("n_groups", C.c_int32), ("rows_per_task", C.c_int32), ("max_steps", C.c_int32),
+                ("dx", C.c_int32), ("dout", C.c_int32), ("cx", C.c_int32), ("cout", C.c_int32)]
+
+
 def _load():
     if not os.path.exists(_LIB_PATH):
         raise ImportError(
@@ -175,6 +183,10 @@ def _load():
     lib.cgtp_uvsw_packed_bytes.argtypes = [C.c_int32] * 4
     lib.cgtp_uvsw_validate.argtypes = _uvs + [C.c_int32]
     lib.cgtp_uvsw_apply.argtypes = _uvs + [C.c_int32, C.c_void_p]
+    lib.cgtp_uvl_packed_bytes.restype = C.c_int64
+    lib.cgtp_uvl_packed_bytes.argtypes = [C.c_int32] * 3
+    lib.cgtp_uvl_validate.argtypes = [C.POINTER(UvlArgs)]
+    lib.cgtp_uvl_apply.argtypes = [C.POINTER(UvlArgs), C.c_void_p]
     lib.cgtp_uvu_mx_workspace_bytes.restype = C.c_int64
     lib.cgtp_uvu_mx_workspace_bytes.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]
     lib.cgtp_uvu_mx_validate.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]

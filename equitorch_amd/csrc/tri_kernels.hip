@@ -640,14 +640,26 @@ int cgtp_abi_layout(int which, int64_t* out, int capacity) {
                                    CGTP_OFF(cgtp_uvu_mx, lanes_log2), CGTP_OFF(cgtp_uvu_mx, tiles),
                                    CGTP_OFF(cgtp_uvu_mx, bwd4), CGTP_OFF(cgtp_uvu_mx, bwd4_items),
                                    CGTP_OFF(cgtp_uvu_mx, bwd4_chunks)};
+  static const int64_t uvl_args[] = {sizeof(cgtp_uvl_args), CGTP_OFF(cgtp_uvl_args, x), CGTP_OFF(cgtp_uvl_args, packed),
+                                     CGTP_OFF(cgtp_uvl_args, w), CGTP_OFF(cgtp_uvl_args, out),
+                                     CGTP_OFF(cgtp_uvl_args, steps), CGTP_OFF(cgtp_uvl_args, tasks),
+                                     CGTP_OFF(cgtp_uvl_args, groups), CGTP_OFF(cgtp_uvl_args, blocks),
+                                     CGTP_OFF(cgtp_uvl_args, n_rows),
+                                     CGTP_OFF(cgtp_uvl_args, stride_p), CGTP_OFF(cgtp_uvl_args, stride_k),
+                                     CGTP_OFF(cgtp_uvl_args, stride_c), CGTP_OFF(cgtp_uvl_args, n_blocks),
+                                     CGTP_OFF(cgtp_uvl_args, n_groups), CGTP_OFF(cgtp_uvl_args, rows_per_task),
+                                     CGTP_OFF(cgtp_uvl_args, max_steps),
+                                     CGTP_OFF(cgtp_uvl_args, dx), CGTP_OFF(cgtp_uvl_args, dout),
+                                     CGTP_OFF(cgtp_uvl_args, cx), CGTP_OFF(cgtp_uvl_args, cout)};
 #undef CGTP_OFF
   const int64_t* tabs[] = {operand, tri, gen_operand, gen, uvu, uvt_item, uvt, uvt_gw, uvt_gy, uvu_tab, psw_table,
-                           psw_args, uvu_mx};
+                           psw_args, uvu_mx, uvl_args};
   const int counts[] = {(int)(sizeof(operand) / 8), (int)(sizeof(tri) / 8), (int)(sizeof(gen_operand) / 8),
                         (int)(sizeof(gen) / 8), (int)(sizeof(uvu) / 8), (int)(sizeof(uvt_item) / 8),
                         (int)(sizeof(uvt) / 8), (int)(sizeof(uvt_gw) / 8), (int)(sizeof(uvt_gy) / 8),
-                        (int)(sizeof(uvu_tab) / 8), (int)(sizeof(psw_table) / 8), (int)(sizeof(psw_args) / 8), (int)(sizeof(uvu_mx) / 8)};
-  if (which < 0 || which >= 13) return -1;
+                        (int)(sizeof(uvu_tab) / 8), (int)(sizeof(psw_table) / 8), (int)(sizeof(psw_args) / 8), (int)(sizeof(uvu_mx) / 8),
+                        (int)(sizeof(uvl_args) / 8)};
+  if (which < 0 || which >= 14) return -1;
   for (int i = 0; out && i < counts[which] && i < capacity; ++i) out[i] = tabs[which][i];
   return counts[which];
 }

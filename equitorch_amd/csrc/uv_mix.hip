@@ -1,0 +1,375 @@
+// Channel mixing in single precision on the half-precision matrix cores (IrrepsLinear, SO2Linear('uv'), any table):
+//
+//   out[n, m, w] = sum_{entries e of row m} coef_e * sum_u x[n, a_e, u] * W[p_e, u, w]
+//
+// forward, and the gradient of x with the rows' roles exchanged and the weight read transposed.  Operands are three bf16
+// parts each and a product is six matrix instructions (uv_parts.h); the coefficient goes into the packed weight.
+//
+// A workgroup owns 64 NT samples and a group of rows of the result, one or two at a time (two where the same rows of x reach both, the
+// +m and -m rows of an SO(2) layer: read and split once); a wavefront 16 NT of the samples, 16 TW channels.  A unit of work is
+// 32 contracted channels of one row of x: the wavefront's part comes through LDS of its own in whole lines, is split, and is multiplied
+// with the unit's weight fragments, which the four wavefronts share through LDS (the vector L1 delivers 64 bytes a cycle, and
+// fragments loaded by each wavefront would take all of it).  Both are requested two units ahead.  The workgroups of one block of
+// samples are neighbours on one XCD: rows of x are read again for every group of rows they reach, from its L2.
+//
+// What bounds it: matrix instructions, at the clock of 1.6 to 1.8 GHz that the card keeps under them (SO2Linear, lmax = 4, 64
+// channels, 32768 samples: 134 us of the 270 at 1.7 GHz; without them the launch takes 155, L2 and stores).
+// Measured there: 571 us on fp32 matrix instructions (uvt_apply_kernel) -> 273; lmax 2: 32 channels, 4096 samples 12.9 -> 11.0; IrrepsLinear
+// 64 -> 64, lmax 2, 65536 samples 126 -> 75, 128 -> 128, lmax 3, 32768 samples 308 -> 170.  One workgroup per pair of rows, 325 us: a
+// third of its time went into starting; half lines of x from memory straight into the operands, 300; three wavefronts per
+// SIMD (spills), eight in a workgroup, matrix and vector instructions in turn by hand: no change.  Errors of the results
+// against 64 bits: 0.3e-7 to 3.0e-7, of fp32 matrix instructions 0.5e-7 to 3.7e-7.
+//
+// Values: elements that are not finite or overflow as parts show in the results, and elements below 2^-110 (but not zero; their
+// last part could be below the smallest subnormal) are looked for; a wavefront that sees either forms its results
+// again with fp32 matrix instructions from memory.
+#include "uv_parts.h"
+
+#pragma clang fp contract(fast)
+
+namespace cgtp {
+
+struct UvlDev {
+  const float* x;
+  const u32x4* packed;
+  const unsigned* asks;               // a word per (block, block of produced channels)
+  const float* w;
+  float* out;
+  const cgtp_uvl_step* steps;
+  const cgtp_uvl_task* tasks;
+  const cgtp_uvl_group* groups;
+  const cgtp_uvl_block* blocks;
+  int64_t n_rows, stride_p, stride_k, stride_c;
+  int dx, dout, cx, cout, n_groups;
+  int kc;                             // units of 32 contracted channels
+  int cblocks, sblocks;               // blocks of 16 TW produced channels, of samples
+};
+
+// A workgroup per (block, block of produced channels): parts of coef * W in fragment order, [unit][part][tile][lane] of 16 bytes.
+template <int TW>
+__global__ void __launch_bounds__(256) uvl_pack_kernel(const cgtp_uvl_block* __restrict__ blocks, const float* __restrict__ w,
+                                                       u32x4* __restrict__ packed, unsigned* __restrict__ asks, int kc, int cx,
+                                                       int cout, int64_t stride_p, int64_t stride_k, int64_t stride_c) {
+  __shared__ unsigned plain;
+  if (threadIdx.x == 0) plain = 0;
+  __syncthreads();
+  const cgtp_uvl_block b = blocks[blockIdx.x];
+  const float* wp = w + b.path * stride_p;
+  u32x4* dst = packed + (int64_t)(blockIdx.x * gridDim.y + blockIdx.y) * kc * (TW * 192);
+  unsigned m = 0;
+  for (int i = threadIdx.x; i < kc * TW * 64; i += 256) {
+    const int lane = i & 63, t = (i >> 6) % TW, k = (i >> 6) / TW;
+    // the columns a lane of uvl_kernel holds for unit k; those of the unit before get zeros
+    const int ch = blockIdx.y * 16 * TW + 16 * t + (lane & 15), first = max(min(k * 32, cx - 32), 0) + 8 * (lane >> 4);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int col = first + j;
+      const bool in = col >= k * 32 && col < cx && ch < cout;
+      const float u = wp[(in ? col : 0) * stride_k + (in ? ch : 0) * stride_c];
+      v[j] = in ? b.coef * u : 0.f;
+      m |= uvs_asks(v[j]) & kUvsPlain;
+    }
+    UvsParts<8> part;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part.pair(j, v[2 * j], v[2 * j + 1]);
+#pragma unroll
+    for (int h = 0; h < 3; ++h) dst[((k * 3 + h) * TW + t) * 64 + lane] = u32x4{part.p[h][0], part.p[h][1], part.p[h][2], part.p[h][3]};
+  }
+  if (m) plain = 1;          // whoever writes, writes the same
+  __syncthreads();
+  if (threadIdx.x == 0) asks[blockIdx.x * gridDim.y + blockIdx.y] = plain;
+}
+
+// RW rows of the result at a time.  Per unit of 32 channels a wavefront issues 24 NT RW matrix instructions (TW = 4).
+template <int TW, int NT, int RW>
+__global__ void __launch_bounds__(256, NT * RW == 4 ? 2 : 3) uvl_kernel(const UvlDev a) {
+  constexpr int CHUNK = TW * 192;                   // 16-byte words of a block's fragments of a unit
+  __shared__ u32x4 lds[2][RW][CHUNK];
+  __shared__ f32x4 xlds[4][NT * 128];
+  // workgroups b, b + 8, ... run on one XCD: the groups of one block of samples there one after the other
+  const int parts = a.n_groups * a.cblocks, j = blockIdx.x >> 3, at_part = j % parts;
+  const int sb = j / parts * 8 + (blockIdx.x & 7);
+  if (sb >= a.sblocks) return;
+  const cgtp_uvl_group group = a.groups[at_part / a.cblocks];
+  const int cb = at_part % a.cblocks;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t first = (int64_t)sb * (64 * NT) + wave * (16 * NT);
+  const int64_t n0 = min(first, a.n_rows - 1);      // past the end: the last row again
+  const int row_elems = a.dx * a.cx, left = (int)min(a.n_rows - n0, (int64_t)(16 * NT));
+  const float* xw = a.x + n0 * row_elems;
+  // A wavefront's rows go through LDS of its own: a load takes whole lines of eight samples (16 bytes a lane), where the lanes'
+  // matrix operands are 32 bytes of each of 16 samples, half lines whichever way they are loaded.  Piece p of a sample lies at
+  // place p ^ (sample % 8), so that neither side has bank conflicts.  A unit's channels start 32 before the last one at most (the weight
+  // has zeros where they overlap the unit before); with fewer than 32, the pieces past them are others (and the weight has zeros).
+  unsigned at[2 * NT];
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i)
+    at[i] = 4u * (min(8 * i + (lane >> 3), left - 1) * row_elems + min(4 * ((lane & 7) ^ (lane >> 3)), a.cx - 4));
+  f32x4* mine_x = xlds[wave];
+
+  // lane l holds step l of the group (64 at most)
+  const int steps = group.step_end - group.step_begin, units = steps * a.kc;
+  const cgtp_uvl_step mine = a.steps[group.step_begin + min(lane, steps - 1)];
+  unsigned plain_w = 0;
+#pragma unroll
+  for (int w = 0; w < RW; ++w) plain_w |= mine.block[w] >= 0 ? a.asks[mine.block[w] * a.cblocks + cb] : 0;
+  floatx4 acc[RW][TW][NT];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < RW; ++w)
+#pragma unroll
+      for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[w][t][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  // Steps begin .. end again in fp32 matrix instructions, operands from memory.
+  auto form_plain = [&](int begin, int end) __attribute__((always_inline)) {
+    clear();
+    for (int s = begin; s <= end; ++s) {
+      const float* xr = xw + __builtin_amdgcn_readlane(mine.row, s) * a.cx;
+#pragma unroll
+      for (int w = 0; w < RW; ++w) {
+        const int b = __builtin_amdgcn_readlane(mine.block[w], s);
+        if (b < 0) continue;
+        const cgtp_uvl_block of = a.blocks[b];
+        const float* wp = a.w + of.path * a.stride_p;
+        for (int k = q; k < a.cx; k += 4) {          // cx is a multiple of 4: the same count in every lane
+          float xv[NT];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) xv[i] = of.coef * xr[min(16 * i + r, left - 1) * row_elems + k];
+#pragma unroll
+          for (int t = 0; t < TW; ++t) {
+            const int ch = min(cb * 16 * TW + 16 * t + r, a.cout - 1);
+            const float wv = wp[k * a.stride_k + ch * a.stride_c];
+#pragma unroll
+            for (int i = 0; i < NT; ++i) acc[w][t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv[i], acc[w][t][i], 0, 0, 0);
+          }
+        }
+      }
+    }
+  };
+  struct Cursor { int s, k; };
+  auto advance = [&](Cursor& c) __attribute__((always_inline)) {
+    if (++c.k == a.kc) {
+      c.k = 0;
+      c.s = min(c.s + 1, steps - 1);                 // past the last unit: anything that is there
+    }
+  };
+  f32x4 raw[2 * NT];
+  auto load_x = [&](const Cursor& c) __attribute__((always_inline)) {
+    const char* xr = reinterpret_cast<const char*>(xw + __builtin_amdgcn_readlane(mine.row, c.s) * a.cx + max(min(c.k * 32, a.cx - 32), 0));
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) raw[i] = *reinterpret_cast<const f32x4*>(xr + at[i]);
+  };
+  auto put_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) mine_x[i * 64 + lane] = raw[i];
+  };
+  constexpr int PER = (CHUNK + 255) / 256;
+  u32x4 wreg[RW][PER];
+#pragma unroll
+  for (int w = 0; w < RW; ++w)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) wreg[w][i] = u32x4{0, 0, 0, 0};
+  auto load_w = [&](const Cursor& c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < RW; ++w) {
+      const int b = __builtin_amdgcn_readlane(mine.block[w], c.s);
+      if (b >= 0) {
+        const u32x4* src = a.packed + ((int64_t)(b * a.cblocks + cb) * a.kc + c.k) * CHUNK;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (PER * 256 == CHUNK || tid + i * 256 < CHUNK) wreg[w][i] = src[(unsigned)(tid + i * 256)];
+      }
+    }
+  };
+  auto put_w = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < RW; ++w)
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (PER * 256 == CHUNK || tid + i * 256 < CHUNK) lds[buf][w][tid + i * 256] = wreg[w][i];
+  };
+
+  clear();
+  unsigned plain = plain_w;
+  int s_first = 0;                                   // of the rows in work
+  Cursor cx{0, 0}, cw{0, 0}, now{0, 0};
+  load_w(cw);
+  advance(cw);
+  load_x(cx);
+  advance(cx);
+  put_w(0);
+  put_x();
+  load_x(cx);
+  advance(cx);
+  load_w(cw);
+  advance(cw);
+  __syncthreads();
+  for (int u = 0; u < units; ++u) {
+    UvsParts<8> part[NT];
+    float low = 1.f;
+    f32x4 v[NT][2];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) v[i][h] = mine_x[(16 * i + r) * 8 + ((2 * q + h) ^ (r & 7))];
+    put_x();
+    load_x(cx);
+    advance(cx);
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+          const float v0 = v[i][h][k], v1 = v[i][h][k + 1];
+          part[i].pair(2 * h + k / 2, v0, v1);
+          low = uvs_least(v0, v1, low);
+        }
+    if (__any(low < 0x1p-110f)) {                    // a zero, as a rule
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float e = v[i][h][k];
+            plain |= uvs_asks(e) & kUvsPlain;
+          }
+    }
+    put_w((u + 1) & 1);
+    load_w(cw);
+    advance(cw);
+#pragma unroll
+    for (int w = 0; w < RW; ++w) {
+      if (__builtin_amdgcn_readlane(mine.block[w], now.s) >= 0) {
+        const u32x4* frag = lds[u & 1][w] + lane;
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+          bf16x8 f[3];
+#pragma unroll
+          for (int h = 0; h < 3; ++h) f[h] = __builtin_bit_cast(bf16x8, frag[(h * TW + t) * 64]);
+#pragma unroll
+          for (int c = 0; c < 6; ++c) {              // the small products first
+            constexpr int ha[6] = {2, 1, 0, 1, 0, 0}, hb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+              acc[w][t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ha[c]], uvs_frag(part[i].p[hb[c]]), acc[w][t][i], 0, 0, 0);
+          }
+        }
+      }
+    }
+    const int end = __builtin_amdgcn_readlane(mine.task, now.s);
+    if (end >= 0 && now.k == a.kc - 1) {             // the last unit of these rows
+      const cgtp_uvl_task task = a.tasks[end];
+#pragma unroll
+      for (int w = 0; w < RW; ++w)
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const float v = acc[w][t][i][k];
+              plain |= v - v != 0.f;
+            }
+      if (__any(plain)) form_plain(s_first, now.s);
+#pragma unroll
+      for (int w = 0; w < RW; ++w) {
+        if (task.row[w] < 0 || first >= a.n_rows) continue;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          if (16 * i + r < left) {
+            float* o = a.out + ((n0 + 16 * i + r) * a.dout + task.row[w]) * a.cout;
+#pragma unroll
+            for (int t = 0; t < TW; ++t) {
+              const int ch = cb * 16 * TW + 16 * t + 4 * q;
+              if (ch < a.cout) *reinterpret_cast<floatx4*>(o + ch) = acc[w][t][i];
+            }
+          }
+        }
+      }
+      clear();
+      plain = plain_w;
+      s_first = now.s + 1;
+    }
+    advance(now);
+    __syncthreads();
+  }
+}
+
+struct UvlPlan {
+  UvlDev dev;
+  int tw, nt;
+  int64_t grid;
+};
+
+static int uvl_tiles(int cout) { return cout % 64 == 0 || cout % 64 > 32 ? 4 : 2; }
+
+static int uvl_plan(const cgtp_uvl_args* a, UvlPlan* p) {
+  if (!a || !a->x || !a->packed || !a->w || !a->out || !a->steps || !a->tasks || !a->groups || !a->blocks) return CGTP_ERR_NULL;
+  if (a->n_rows < 0 || a->n_blocks <= 0 || a->n_groups <= 0 || a->dx <= 0 || a->dout <= 0 || a->cx <= 0 || a->cout <= 0 || a->cx % 4 ||
+      a->cout % 4 || (int64_t)a->dx * a->cx > 1 << 22 || a->rows_per_task < 1 || a->rows_per_task > 2 || a->max_steps > kWave)
+    return CGTP_ERR_SHAPE;
+  if (((uintptr_t)a->x | (uintptr_t)a->packed | (uintptr_t)a->out) & 15u) return CGTP_ERR_ALIGN;
+  p->tw = uvl_tiles(a->cout);
+  UvlDev& d = p->dev;
+  d.kc = (a->cx + 31) / 32;
+  d.cblocks = (a->cout + 16 * p->tw - 1) / (16 * p->tw);
+  const int64_t parts = (int64_t)a->n_groups * d.cblocks;
+  // samples per workgroup: 256 over the rows, fewer while the launch would have less than two workgroups per compute unit
+  p->nt = 4 / a->rows_per_task;
+  while (p->nt > 1 && (a->n_rows + 64 * p->nt - 1) / (64 * p->nt) * parts < 512) p->nt /= 2;
+  const int64_t samples = 64 * p->nt, sblocks = (a->n_rows + samples - 1) / samples;
+  p->grid = (sblocks + 7) / 8 * 8 * parts;
+  if (p->grid >= (int64_t)1 << 31 || a->n_blocks > 65535 || d.cblocks > 65535) return CGTP_ERR_SHAPE;
+  d.sblocks = (int)sblocks;
+  d.x = (const float*)a->x; d.packed = (const u32x4*)a->packed; d.w = (const float*)a->w; d.out = (float*)a->out;
+  d.asks = (const unsigned*)(d.packed + (int64_t)a->n_blocks * d.cblocks * d.kc * (p->tw * 192));
+  d.steps = a->steps; d.tasks = a->tasks; d.groups = a->groups; d.blocks = a->blocks; d.n_groups = a->n_groups;
+  d.n_rows = a->n_rows; d.stride_p = a->stride_p; d.stride_k = a->stride_k; d.stride_c = a->stride_c;
+  d.dx = a->dx; d.dout = a->dout; d.cx = a->cx; d.cout = a->cout;
+  return CGTP_OK;
+}
+
+template <int TW>
+static auto uvl_fn(int nt, int rw) {
+  return rw == 2 ? (nt == 2 ? uvl_kernel<TW, 2, 2> : uvl_kernel<TW, 1, 2>)
+                 : nt == 4 ? uvl_kernel<TW, 4, 1> : nt == 2 ? uvl_kernel<TW, 2, 1> : uvl_kernel<TW, 1, 1>;
+}
+
+}  // namespace cgtp
+
+using namespace cgtp;
+
+extern "C" {
+
+int64_t cgtp_uvl_packed_bytes(int32_t n_blocks, int32_t cx, int32_t cout) {
+  if (n_blocks <= 0 || cx <= 0 || cout <= 0) return 0;
+  const int64_t tw = uvl_tiles(cout), cblocks = (cout + 16 * tw - 1) / (16 * tw);
+  return n_blocks * cblocks * ((cx + 31) / 32 * (tw * 192 * 16) + 4);
+}
+
+int cgtp_uvl_validate(const cgtp_uvl_args* a) {
+  UvlPlan p;
+  return uvl_plan(a, &p);
+}
+
+int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream) {
+  UvlPlan p;
+  const int st = uvl_plan(a, &p);
+  if (st != CGTP_OK || a->n_rows == 0) return st;
+  const UvlDev& d = p.dev;
+  hipLaunchKernelGGL(p.tw == 4 ? uvl_pack_kernel<4> : uvl_pack_kernel<2>, dim3((unsigned)a->n_blocks, (unsigned)d.cblocks), dim3(256), 0,
+                     (hipStream_t)stream, a->blocks, d.w, (u32x4*)a->packed, (unsigned*)d.asks, d.kc, d.cx, d.cout, d.stride_p,
+                     d.stride_k, d.stride_c);
+  if (hipGetLastError() != hipSuccess) return CGTP_ERR_LAUNCH;
+  void (*fn)(const UvlDev) = p.tw == 4 ? uvl_fn<4>(p.nt, a->rows_per_task) : uvl_fn<2>(p.nt, a->rows_per_task);
+  hipLaunchKernelGGL(fn, dim3((unsigned)p.grid), dim3(256), 0, (hipStream_t)stream, d);
+  return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+}
+
+}  // extern "C"

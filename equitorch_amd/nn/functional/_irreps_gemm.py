@@ -408,13 +408,13 @@ def _table_driven_path(x: Tensor, weight: Tensor, plan: LinearPlan, in_size: int
         zeros = np.zeros(len(rows), dtype=np.int32)
         coo = TpCoo(sc.astype(np.float64), m.astype(np.int32), m1.astype(np.int32), zeros, pw.astype(np.int32), zeros,
                     int(in_size), 1, int(plan.out_size), int(plan.n_paths))
-        return _uv_native.CooTable(coo, anchor, lambda xx, yy, ww: _Mix.apply(xx, ww, plan, False, in_size) * yy[:, :, None])
+        return _uv_native.CooTable(coo, anchor, lambda xx, yy, ww: _Mix.apply(xx, ww, plan, False, in_size) * yy[:, :, None], mixing=True)
 
     table = cached(anchor, ("linear_as_coo_table", in_size, plan.n_paths, plan.out_size), build)
     if table is False:
         return None
     ones = _ones_column(x.shape[0], x.dtype, x.device)
-    if not _uv_native.u1v_supported(x, ones, weight, table):
+    if not (_uv_native.u1v_supported(x, ones, weight, table) or _uv_native.mix_fits(x, weight, table)):
         return None
     kernels.log_tier("irreps_linear", "table-driven matrix-core kernels")
     return _uv_native.u1v(x, ones, weight, table)

@@ -81,7 +81,9 @@ def _blocks(info, in_size: int, n_weights: int, device, dtype):
         # where every output component sits in the concatenation of the blocks' results (all covered), or None
         inverse = torch.argsort(order) if order.shape[0] == n_out else None
         return blocks, n_out, order, inverse
-    return cached(anchor, ("so2_blocks", in_size, n_weights, str(device), dtype), build)
+    # the first call may be inside a transform (jvp, vmap), whose tensors are no data to keep
+    with torch._C._DisableFuncTorch():
+        return cached(anchor, ("so2_blocks", in_size, n_weights, str(device), dtype), build)
 
 
 def so2_linear_uv_shared(input: Tensor, weight: Tensor, info, in_size: int, n_weights: int) -> Tensor:

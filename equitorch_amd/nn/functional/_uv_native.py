@@ -11,7 +11,7 @@ ordered by output row; this module cuts that list from the table for each of the
     ('uvw' only) g2[M2]   <- rows M of grad_out,   first operand rows M1,  weight permuted
 """
 import ctypes as C
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import numpy as np
 import torch
@@ -28,10 +28,11 @@ class CooTable:
     """A product table given directly by its coordinates (``coo``: ``TpCoo`` fields M, M1, M2, p, coef and the extents)
     instead of a ``TensorProductInfo`` — the tables of the channel-mixing layers, whose second operand is the scalar 1.
     ``anchor``: a tensor that lives as long as the table (cache key); ``fallback(x, y, w)``: a differentiable
-    evaluation of the same product for gradients of higher order."""
+    evaluation of the same product for gradients of higher order.  ``mixing``: the second operand is the scalar 1 in every
+    sample (channel mixing)."""
 
-    def __init__(self, coo, anchor: Tensor, fallback):
-        self.coo, self.anchor, self.fallback = coo, anchor, fallback
+    def __init__(self, coo, anchor: Tensor, fallback, mixing: bool = False):
+        self.coo, self.anchor, self.fallback, self.mixing = coo, anchor, fallback, mixing
 
 
 def _anchor(table) -> Tensor:
@@ -218,8 +219,21 @@ def pack(w: Tensor, n_paths: int, k: int, cout: int, stride_p: int, stride_k: in
     return packed
 
 
-def apply(x: Tensor, y: Tensor, wp: Tensor, tp_info, role: str, dout: int, cout: int) -> Tensor:
-    """One launch of ``cgtp_uvt_apply``: ``x (N, dx, cx)``, ``y (N, dy)`` or ``(N, dy, cy)`` -> ``(N, dout, cout)``."""
+class StoredWeight(NamedTuple):
+    """A weight ``(P, U, W)`` as the caller holds it, packed by :func:`apply` for the kernel that serves."""
+    w: Tensor
+    transposed: bool
+
+
+def apply(x: Tensor, y: Tensor, wp, tp_info, role: str, dout: int, cout: int) -> Tensor:
+    """``x (N, dx, cx)``, ``y (N, dy)`` or ``(N, dy, cy)`` -> ``(N, dout, cout)``: one launch of ``cgtp_uvt_apply``, with
+    ``wp`` a weight packed for it, or (a :class:`StoredWeight`) of ``cgtp_uvl_apply`` for channel mixing in fp32."""
+    if isinstance(wp, StoredWeight):
+        out = _mix_split(x, wp.w, tp_info, wp.transposed)
+        if out is not None:
+            return out
+        p, u, wc = wp.w.shape
+        wp = pack(wp.w, p, wc, u, u * wc, 1, wc) if wp.transposed else pack(wp.w, p, u, wc, u * wc, wc, 1)
     n, dx, cx = x.shape
     dy = y.shape[1]
     cy = y.shape[2] if y.ndim == 3 else 0
@@ -295,6 +309,129 @@ def _split_uvw(kind: int, x: Tensor, z: Tensor, w: Tensor, tp_info, rows_out: in
     return out
 
 
+class _MixTable:
+    """A channel-mixing table for ``cgtp_uvl_apply`` (``transposed``: the gradient of its input): the rows of the result by two
+    where most of the rows of the input that reach one reach both (the ``+m`` and ``-m`` rows of an SO(2) layer, which then
+    load and split them once), else one by one, and their steps."""
+
+    def __init__(self, coo, transposed: bool):
+        rows_out, rows_in, n_out = (coo.M1, coo.M, coo.D1) if transposed else (coo.M, coo.M1, coo.DO)
+        blocks = {}                                    # (path, coefficient) -> its place in the packed weight
+        terms = [{} for _ in range(n_out)]             # row of the result: row of the input -> blocks
+        for o, i, p, c in zip(rows_out, rows_in, coo.p, coo.coef):
+            b = blocks.setdefault((int(p), np.float32(c)), len(blocks))
+            terms[int(o)].setdefault(int(i), []).append(b)
+        pairs, alone = [], set(range(n_out))
+        for m in range(n_out):
+            if m in alone:
+                most = max(sorted(alone - {m}), key=lambda k: len(terms[m].keys() & terms[k].keys()), default=None)
+                if most is not None and 2 * len(terms[m].keys() & terms[most].keys()) > max(len(terms[m]), len(terms[most])):
+                    pairs.append((m, most))
+                    alone -= {m, most}
+        if 4 * sum(len(terms[m].keys() & terms[k].keys()) for m, k in pairs) < sum(len(t) for t in terms):
+            pairs, alone = [], set(range(n_out))
+        self.rows_per_task = 2 if pairs else 1
+        self.tasks, self.steps = sorted(pairs + [(m, -1) for m in alone]), []
+        for m, k in self.tasks:
+            steps = []
+            for i in sorted(terms[m].keys() | (terms[k].keys() if k >= 0 else set())):
+                b0, b1 = terms[m].get(i, []), terms[k].get(i, []) if k >= 0 else []
+                steps += [(i, b0[t] if t < len(b0) else -1, b1[t] if t < len(b1) else -1)
+                          for t in range(max(len(b0), len(b1)))]
+            self.steps.append(steps or [(0, -1, -1)])
+        self.n_out, self.n_blocks = n_out, max(len(blocks), 1)
+        self.blocks = np.array([(p, c.view(np.int32)) for p, c in blocks] or [(0, 0)], dtype=np.int32)
+        self.longest = max(map(len, self.steps))
+        # the numbers of groups to choose from, with the most steps of a group
+        self.choices = {g: self.dealt(g)[1] for g in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, len(self.tasks)) if g <= len(self.tasks)}
+
+    def dealt(self, n_groups: int):
+        """The tasks in ``n_groups`` groups: the longest first, each to the group with the fewest steps so far."""
+        groups, count = [[] for _ in range(n_groups)], [0] * n_groups
+        for t in sorted(range(len(self.tasks)), key=lambda t: -len(self.steps[t])):
+            g = count.index(min(count))
+            groups[g].append(t)
+            count[g] += len(self.steps[t])
+        return groups, max(count)
+
+    def groups_for(self, n: int, column_blocks: int) -> int:
+        """Groups (workgroups a block of samples is cut into): what lets whole rounds of two workgroups per compute unit end
+        soonest, a workgroup costing its steps and about two more to start."""
+        blocks = -(-n * self.rows_per_task // 256) * column_blocks
+        fits = [(-(-blocks * g // 512) * (most + 2), g) for g, most in self.choices.items() if most <= _MIX_STEPS]
+        return min(fits)[1]
+
+
+_MIX_STEPS = 64
+
+
+class _MixWalk:
+    """The table dealt to every number of groups there is to choose from, on the device in one piece: a batch of another size
+    copies nothing.  ``at[n_groups]``: where its steps, its groups and the tasks and blocks they share begin, in bytes."""
+
+    def __init__(self, table: _MixTable, device):
+        parts = [np.array(v, dtype=np.int32).ravel() for v in (table.tasks, table.blocks)]
+        parts[0] = np.resize(parts[0], -(-parts[0].size // 4) * 4)          # steps are read 16 bytes at a time
+        parts[1] = np.resize(parts[1], -(-parts[1].size // 4) * 4)
+        end, self.at, self.max_steps = sum(p.size for p in parts), {}, {}
+        for n_groups, most in table.choices.items():
+            steps, ptr = [], []
+            for group in table.dealt(n_groups)[0]:
+                ptr.append((len(steps), len(steps) + sum(len(table.steps[t]) for t in group)))
+                for t in group:
+                    steps += [(*s, -1) for s in table.steps[t][:-1]] + [(*table.steps[t][-1], t)]
+            ptr += [(0, 0)] * (len(ptr) % 2)
+            parts += [np.array(v, dtype=np.int32).ravel() for v in (steps, ptr)]
+            self.at[n_groups] = tuple(4 * v for v in (end, end + parts[-2].size, 0, parts[0].size))
+            self.max_steps[n_groups] = most
+            end += parts[-2].size + parts[-1].size
+        self.words = torch.from_numpy(np.concatenate(parts)).to(device)
+
+
+def _mix_table(table, transposed: bool) -> _MixTable:
+    return kernels.cached(_anchor(table), ("uvl_table", transposed), lambda: _MixTable(table.coo, transposed))
+
+
+def mix_fits(x: Tensor, w: Tensor, table) -> bool:
+    """Whether channel mixing with this table runs on the half-precision matrix cores in both directions.  The calls it
+    takes from the library route, which is plain tensor algebra, leave the transforms of that to it: vmap, forward mode and
+    tracing see no autograd function there."""
+    c = table.coo
+    if (torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or torch.jit.is_tracing()):
+        return False
+    return (x.dtype == w.dtype == torch.float32 and x.shape[0] > 0 and x.data_ptr() % 16 == 0 and w.shape[1] % 4 == 0
+            and w.shape[2] % 4 == 0 and w.shape[0] == c.P and tuple(x.shape[1:]) == (c.D1, w.shape[1])
+            and max(c.D1 * w.shape[1], c.DO * w.shape[2]) <= 1 << 22
+            and all(_mix_table(table, t).longest <= _MIX_STEPS for t in (False, True)))
+
+
+def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor]:
+    """Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``), or None where the fp32 matrix
+    instructions serve.  Over 400 launches (IrrepsLinear of lmax 1 to 4, SO2Linear of lmax 2 to 6, 8 to 256 channels on either side,
+    100 to 30000 samples) it takes 0.4 to 1.0 of their time; past 128 contracted channels and below 2048 samples its
+    workgroups are few and long (256 -> 256, lmax 4, 700 samples: 43 us against 38)."""
+    if not (isinstance(table, CooTable) and table.mixing) or x.dtype != torch.float32:
+        return None
+    n, dx, cx = x.shape
+    cout = w.shape[1] if transposed else w.shape[2]
+    mix = _mix_table(table, transposed)
+    if mix.longest > _MIX_STEPS or (cx > 128 and n < 2048 and chunk_of(n, dx, 1, mix.n_out, cx, 0, cout) > 0):
+        return None
+    n_groups = mix.groups_for(n, -(-cout // 64))
+    walk = kernels.cached(_anchor(table), ("uvl_walk", transposed, str(x.device)), lambda: _MixWalk(mix, x.device))
+    packed = torch.empty(int(_lib.lib.cgtp_uvl_packed_bytes(mix.n_blocks, cx, cout)), dtype=torch.uint8, device=x.device)
+    out = torch.empty((n, mix.n_out, cout), dtype=x.dtype, device=x.device)
+    steps, groups, tasks, blocks = (walk.words.data_ptr() + v for v in walk.at[n_groups])
+    a = _lib.UvlArgs(x.data_ptr(), packed.data_ptr(), w.data_ptr(), out.data_ptr(), steps, tasks, groups, blocks,
+                     n, w.stride(0), w.stride(2 if transposed else 1), w.stride(1 if transposed else 2),
+                     mix.n_blocks, n_groups, mix.rows_per_task, walk.max_steps[n_groups], dx, mix.n_out, cx, cout)
+    if _lib.lib.cgtp_uvl_validate(C.byref(a)) != 0:
+        return None
+    _lib.check(_lib.lib.cgtp_uvl_apply(C.byref(a), _lib.stream_ptr(x.device)), "cgtp_uvl_apply")
+    return out
+
+
 def _coo(tp_info):
     return tp_info.coo if isinstance(tp_info, CooTable) else kernels.coo_of(tp_info)
 
@@ -318,7 +455,7 @@ class _U1vNative(Function):
         p, u, wc = w.shape
         out = _split(0, x, y, w, tp_info, c.DO)
         if out is None:
-            out = apply(x, y, pack(w, p, u, wc, u * wc, wc, 1), tp_info, "out", c.DO, wc)
+            out = apply(x, y, StoredWeight(w, False), tp_info, "out", c.DO, wc)
         ctx.save_for_backward(x, y, w)
         ctx.tp_info = tp_info
         return out
@@ -342,7 +479,7 @@ class _U1vNative(Function):
         if need[0]:
             gx = _split(1, g, y, w, tp_info, c.D1)
             if gx is None:
-                gx = apply(g, y, pack(w, p, wc, u, u * wc, 1, wc), tp_info, "in1", c.D1, u)
+                gx = apply(g, y, StoredWeight(w, True), tp_info, "in1", c.D1, u)
         if need[2]:
             gw = grad_w(x, y, g, tp_info)
         if need[1]:

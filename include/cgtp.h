@@ -423,6 +423,35 @@ int cgtp_uvsw_validate(int cfg, int kind, const void* x, const void* z, const vo
 int cgtp_uvsw_apply(int cfg, int kind, const void* x, const void* z, void* packed, const void* w, void* out, int64_t n_rows,
                     int32_t u, int32_t v, int32_t c, void* stream);
 
+/* Channel mixing in single precision on the half-precision matrix cores (operands as above), any table:
+ *   out[n, m, w] = sum_{entries e of row m} coef_e * sum_u x[n, row_e, u] * W[path_e, u, w]
+ * x (n_rows, dx, cx), out (n_rows, dout, cout), contiguous, cx and cout multiples of 4; W read through element strides (path,
+ * contracted, produced).  A task makes one or two rows of out (rows_per_task; row[1] = -1: none): it is a run of steps,
+ * each a row of x times a block for either row of out (-1: none), the last with the task's index (`task`, else -1); a row
+ * of out without terms has a task of one step without blocks.  Blocks are the distinct (path, coefficient) pairs.  A group is
+ * the work of one workgroup for its samples: the steps of whole tasks, 1 to 64 (max_steps: the most of any).  steps, tasks, groups
+ * and blocks in device memory, packed: cgtp_uvl_packed_bytes() bytes of scratch.  The layers are IrrepsLinear and
+ * SO2Linear('uv') with a shared weight (reference equitorch/nn/linears.py:268-571). */
+typedef struct { int32_t row, block[2], task; } cgtp_uvl_step;
+typedef struct { int32_t row[2]; } cgtp_uvl_task;
+typedef struct { int32_t step_begin, step_end; } cgtp_uvl_group;
+typedef struct { int32_t path; float coef; } cgtp_uvl_block;
+typedef struct {
+  const void* x;
+  void* packed;
+  const void* w;
+  void* out;
+  const cgtp_uvl_step* steps;
+  const cgtp_uvl_task* tasks;
+  const cgtp_uvl_group* groups;
+  const cgtp_uvl_block* blocks;
+  int64_t n_rows, stride_p, stride_k, stride_c;
+  int32_t n_blocks, n_groups, rows_per_task, max_steps, dx, dout, cx, cout;
+} cgtp_uvl_args;
+int64_t cgtp_uvl_packed_bytes(int32_t n_blocks, int32_t cx, int32_t cout);
+int cgtp_uvl_validate(const cgtp_uvl_args* a);
+int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream);
+
 /* ---- radial basis and cutoff envelopes ---------------------------------------------------------------------------
  *
  * Element-wise functions of the edge length r (n values), fp32 / fp64, one launch forward and one for the gradient.

@@ -1,0 +1,217 @@
+"""Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``; IrrepsLinear and SO2Linear('uv') with a shared
+weight): every operand carried as three bf16 parts, no less precise than fp32 matrix instructions and of their range."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import stable_seed
+
+SH = {l: "+".join(f"{k}{'eo'[k % 2]}" for k in range(l + 1)) for l in range(7)}
+
+
+def _coo(kind, l):
+    """Table of a layer as entries (row of the result, row of the input, weight, coefficient)."""
+    from equitorch_amd import nn as enn
+    from equitorch_amd.nn.functional import _irreps_gemm as G
+    if kind == "so2":
+        mod = enn.SO2Linear(SH[l], SH[l], 4, 4, feature_mode="uv")
+        plan = G.plan_of_product_info(mod.info_forward, mod.irreps_in.dim, mod.num_weights)
+    else:
+        mod = enn.IrrepsLinear(SH[l], "2e+0e+1o+0e", 4, 4)
+        plan = G.plan_of_linear_info(mod.forward_info)
+    return [(p.o0 + j, p.i0 + j, p.w, p.scale) for p in plan.paths for j in range(p.k)], plan, (l + 1) ** 2
+
+
+def _table(entries, n_in, n_out, n_w):
+    from equitorch_amd._tables import TpCoo
+    from equitorch_amd.nn.functional import _uv_native as N
+    m, m1, p, c = (np.asarray(v) for v in zip(*entries))
+    z = np.zeros(len(m), dtype=np.int32)
+    coo = TpCoo(c.astype(np.float64), m.astype(np.int32), m1.astype(np.int32), z, p.astype(np.int32), z, n_in, 1, n_out, n_w)
+    return N.CooTable(coo, torch.zeros(1), None, mixing=True)
+
+
+@pytest.mark.parametrize("kind,l", [("so2", 2), ("so2", 6), ("lin", 2), ("own", 0)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_the_steps_are_the_table(kind, l, transposed):
+    """Tasks, steps and groups for every number of groups against the table's entries; ``own``: several weights and coefficients
+    for one pair of rows, and rows of either side that no entry reaches."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    if kind == "own":
+        entries, n_in, n_out, n_w = [(0, 2, 1, 0.5), (0, 2, 0, -2.0), (3, 2, 1, 0.5), (3, 0, 1, 1.5), (0, 0, 2, 3.0), (1, 4, 2, 1.0)], 6, 5, 3
+    else:
+        entries, plan, n_in = _coo(kind, l)
+        n_out, n_w = plan.out_size, plan.n_paths
+    table = N._MixTable(_table(entries, n_in, n_out, n_w).coo, transposed)
+    want = sorted(((i, m) if transposed else (m, i)) + (p, np.float32(c)) for m, i, p, c in entries)
+    walk = N._MixWalk(table, "cpu")
+    words = walk.words.numpy()
+    n_steps = sum(map(len, table.steps))
+    for g, (at_steps, at_groups, at_tasks, at_blocks) in walk.at.items():
+        assert at_steps % 16 == 0 and at_groups % 8 == 0 and at_tasks % 8 == 0 and at_blocks % 8 == 0
+        steps = words[at_steps // 4:].reshape(-1)[:4 * n_steps].reshape(-1, 4)
+        groups = words[at_groups // 4:][:2 * g].reshape(-1, 2)
+        tasks = words[at_tasks // 4:][:2 * len(table.tasks)].reshape(-1, 2)
+        blocks = words[at_blocks // 4:][:2 * table.n_blocks].reshape(-1, 2)
+        assert groups[0, 0] == 0 and groups[-1, 1] == len(steps) and (groups[1:, 0] == groups[:-1, 1]).all()
+        assert (groups[:, 1] > groups[:, 0]).all() and (groups[:, 1] - groups[:, 0]).max() == walk.max_steps[g]
+        assert all(steps[e - 1, 3] >= 0 for _, e in groups)                 # whole tasks
+        got, rows, begin = [], [], 0
+        for s, (row, b0, b1, task) in enumerate(steps):
+            if task < 0:
+                continue
+            for i, x0, x1, _ in steps[begin:s + 1]:
+                for row_out, b in zip(tasks[task], (x0, x1)):
+                    if b >= 0:
+                        assert row_out >= 0
+                        got.append((int(row_out), int(i), int(blocks[b, 0]), blocks[b, 1:].view(np.float32)[0]))
+            rows += [int(r) for r in tasks[task] if r >= 0]
+            begin = s + 1
+        assert sorted(got) == want and sorted(rows) == list(range(table.n_out))
+    if kind == "so2":
+        assert table.rows_per_task == 2
+    assert table.groups_for(10 ** 6, 1) >= 1 and max(len(s) for s in table.steps) == table.longest
+
+
+# ---- on the GPU ------------------------------------------------------------------------------------------------------
+def _module(kind, l, cin, cout, device):
+    from equitorch_amd import nn as enn
+    torch.manual_seed(stable_seed("mix", kind, l, cin, cout))
+    if kind == "so2":
+        return enn.SO2Linear(SH[l], SH[l], cin, cout, feature_mode="uv").to(device)
+    return enn.IrrepsLinear(SH[l], SH[l] if kind == "lin" else "2e+0e+1o+0e", cin, cout).to(device)
+
+
+def _run(mod, x, g):
+    x = x.detach().requires_grad_(True)
+    out = mod(x)
+    return [t.detach() for t in (out, torch.autograd.grad(out, [x], g)[0])]
+
+
+def _routes(monkeypatch, kind, l, cin, cout, x, g, device, scale=1.0):
+    """Results of the split kernels, of the route without them and of float64."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    mod = _module(kind, l, cin, cout, device)
+    with torch.no_grad():
+        mod.weight.mul_(scale)
+    taken, split = [], N._mix_split
+
+    def spy(*args):
+        out = split(*args)
+        taken.append(out is not None)
+        return out
+    monkeypatch.setattr(N, "_mix_split", spy)
+    new = _run(mod, x.to(device), g.to(device))
+    assert taken == [True, True]
+    monkeypatch.setattr(N, "_mix_split", lambda *args: None)
+    monkeypatch.setattr(N, "mix_fits", lambda *args: False)
+    old = _run(mod, x.to(device), g.to(device))
+    ref = _run(mod.double(), x.double().to(device), g.double().to(device))
+    return new, old, ref
+
+
+def _operands(kind, l, cin, cout, n, seed):
+    gen = torch.Generator().manual_seed(seed)
+    rows_out = (l + 1) ** 2 if kind != "own" else 10
+    return torch.randn(n, (l + 1) ** 2, cin, generator=gen), torch.randn(n, rows_out, cout, generator=gen)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n", [
+    ("lin", 1, 4, 4, 1), ("lin", 2, 12, 20, 65), ("own", 3, 36, 100, 129), ("lin", 2, 64, 64, 3000), ("lin", 3, 128, 96, 700),
+    ("lin", 1, 160, 32, 2500), ("so2", 2, 32, 32, 63), ("so2", 4, 64, 64, 1000), ("so2", 6, 48, 48, 257), ("so2", 3, 40, 132, 31)])
+@pytest.mark.parametrize("values", ["normal", "wide"])
+def test_no_less_precise_than_fp32_matrix_instructions(device, monkeypatch, kind, l, cin, cout, n, values):
+    """Ragged batches, channels that fill no tile, rows no entry reaches; ``wide``: samples and elements spread over twenty
+    binary orders of magnitude."""
+    x, g = _operands(kind, l, cin, cout, n, stable_seed("mix operands", kind, l, cin, cout, n))
+    if values == "wide":
+        gen = torch.Generator().manual_seed(3)
+        for t in (x, g):
+            t.mul_(torch.exp2(torch.randint(-20, 21, (n, 1, 1), generator=gen).float()))
+            t.mul_(torch.exp2(torch.randint(-10, 11, t.shape, generator=gen).float()))
+    new, old, ref = _routes(monkeypatch, kind, l, cin, cout, x, g, device)
+    for name, a, b, want in zip(("out", "grad x"), new, old, ref):
+        def err(t):
+            d, w = (t.double() - want).flatten(1).norm(dim=1), want.flatten(1).norm(dim=1)
+            return float((d / w.clamp_min(1e-30)).square().mean().sqrt())
+        print(f"{name} {kind} lmax={l} {cin}->{cout} n={n} {values}: split {err(a):.2e} fp32 {err(b):.2e}")
+        # one sample's rounding errors are a handful of draws: a factor of two between two orders of summation
+        assert err(a) <= (1.1 if n >= 300 else 2.0) * err(b) + 3e-8, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where,value", [("x", float("inf")), ("x", float("nan")), ("g", float("-inf")), ("x", 3.4e38), ("w", float("inf"))])
+@pytest.mark.parametrize("kind", ["lin", "so2"])
+def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, kind, where, value):
+    from equitorch_amd.nn.functional import _uv_native as N
+    x, g = _operands(kind, 2, 32, 64, 150, 7)
+    mod = _module(kind, 2, 32, 64, device)
+    {"x": x, "g": g, "w": mod.weight.data}[where].view(-1)[567] = value
+    new = _run(mod, x.to(device), g.to(device))
+    monkeypatch.setattr(N, "_mix_split", lambda *args: None)
+    for a, b in zip(new, _run(mod, x.to(device), g.to(device))):
+        fin = torch.isfinite(b)
+        assert torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
+        assert float((a[fin] - b[fin]).norm()) <= 1e-6 * float(b[fin].norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exponent,scale", [(0, 0), (-70, -40), (-105, 0), (-115, 0), (-118, 30), (0, -112), (-60, -50), (60, 60), (100, -20), (-113, 100)])
+def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponent, scale):
+    x, g = _operands("so2", 2, 64, 32, 70, 8)
+    x[3, 2, 5] = 0.0                   # an exact zero has no exponent
+    x, g = x * 2.0 ** exponent, g * 2.0 ** exponent
+    new, old, ref = _routes(monkeypatch, "so2", 2, 64, 32, x, g, device, 2.0 ** scale)
+    for name, a, b, want in zip(("out", "grad x"), new, old, ref):
+        assert torch.isfinite(a).all() == torch.isfinite(b).all()
+        if want.abs().max() > 2.0 ** -110 and torch.isfinite(b).all():    # below, the products are subnormal numbers on either route
+            def err(t):
+                d = (t.double() - want).norm(dim=0) / want.norm(dim=0)
+                return float(d.square().mean().sqrt())
+            print(f"{name} of 2^{exponent}, 2^{scale}: split {err(a):.2e} fp32 {err(b):.2e}")
+            assert err(a) <= 1.5 * err(b) + 3e-8, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["lin", "so2"])
+def test_recorded_in_a_graph(device, kind):
+    """Forward and gradients recorded and replayed on new inputs and weights: the weight is packed anew by every replay."""
+    mod = _module(kind, 2, 32, 64, device)
+    x, g = (t.to(device) for t in _operands(kind, 2, 32, 64, 100, 9))
+    x.requires_grad_(True)
+
+    def step():
+        out = mod(x)
+        return (out, *torch.autograd.grad(out, [x, mod.weight], g))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = step()
+    for replay in range(3):
+        with torch.no_grad():
+            gen = torch.Generator().manual_seed(replay)
+            for t in (x, mod.weight):
+                t.copy_(torch.randn(t.shape, generator=gen) * 2.0 ** (5 * replay))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(recorded, step()):
+            assert torch.equal(a, b), replay
+
+
+@pytest.mark.gpu
+def test_transforms_of_the_library_route_stay(device):
+    """An SO(2) layer too large for the fp32 kernels was tensor algebra: forward mode and vmap still take it."""
+    mod = _module("so2", 6, 64, 64, device)
+    x, t = (v.to(device) for v in _operands("so2", 6, 64, 64, 20, 10))
+    want = mod(t).detach()             # the layer's plan is made by a plain call
+    out, tangent = torch.func.jvp(mod, (x,), (t,))
+    assert float((out - mod(x)).detach().norm()) <= 2e-6 * float(out.detach().norm())
+    assert float((tangent - want).detach().norm()) <= 2e-6 * float(want.norm())
+    batched = torch.func.vmap(lambda v: mod(v))(x.view(2, 10, *x.shape[1:]))
+    assert float((batched.flatten(0, 1) - out).detach().norm()) <= 2e-6 * float(out.detach().norm())
