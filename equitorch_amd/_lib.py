@@ -129,6 +129,13 @@ class UvlArgs(C.Structure):
                 ("dx", C.c_int32), ("dout", C.c_int32), ("cx", C.c_int32), ("cout", C.c_int32)]
 
 
+class UvgArgs(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("y", C.c_void_p), ("g", C.c_void_p), ("gw", C.c_void_p), ("workspace", C.c_void_p),
+                ("jobs", C.c_void_p), ("job_ptr", C.c_void_p), ("slot_ptr", C.c_void_p), ("n_rows", C.c_int64),
+                ("cfg", C.c_int32), ("n_ranges", C.c_int32), ("n_wgs", C.c_int32), ("n_slots", C.c_int32),
+                ("c", C.c_int32), ("cy", C.c_int32)]
+
+
 def _load():
     if not os.path.exists(_LIB_PATH):
         raise ImportError(
@@ -187,6 +194,8 @@ def _load():
     lib.cgtp_uvl_packed_bytes.argtypes = [C.c_int32] * 3
     lib.cgtp_uvl_validate.argtypes = [C.POINTER(UvlArgs)]
     lib.cgtp_uvl_apply.argtypes = [C.POINTER(UvlArgs), C.c_void_p]
+    lib.cgtp_uvg_validate.argtypes = [C.POINTER(UvgArgs)]
+    lib.cgtp_uvg_apply.argtypes = [C.POINTER(UvgArgs), C.c_void_p]
     lib.cgtp_uvu_mx_workspace_bytes.restype = C.c_int64
     lib.cgtp_uvu_mx_workspace_bytes.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]
     lib.cgtp_uvu_mx_validate.argtypes = [C.POINTER(UvuArgs), C.POINTER(UvuTab), C.POINTER(UvuMx), C.c_int]

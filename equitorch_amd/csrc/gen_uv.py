@@ -243,6 +243,44 @@ def emit_gw(name: str, coo, seg_out, seg_in1) -> str:
     return "\n".join(L)
 
 
+def emit_split_gw(name: str, coo) -> str:
+    """The paths of a table for the weight gradient in single precision: of a path's rows of x and of g the ones that are
+    more are mixed with y into as many rows as the others are (fewer products that way), row by row.  ``m.y(b)`` is row b of
+    y, ``m.add(o, s)`` adds s times mixed-side row ``o`` of the path, ``m.fence()`` ends a group of two."""
+    L, turned = [], 0
+    for p in range(coo.P):
+        mine = [t for t in range(coo.coef.shape[0]) if coo.p[t] == p]
+        x_rows, g_rows = (sorted({int(col[t]) for t in mine}) for col in (coo.M1, coo.M))
+        for rows in (x_rows, g_rows):
+            assert rows == list(range(rows[0], rows[0] + len(rows)))
+        swapped = len(g_rows) > len(x_rows)
+        turned |= swapped << p
+        mixed, plain = (g_rows, x_rows) if swapped else (x_rows, g_rows)
+        L += [f"struct UVG_{name}_p{p} {{",
+              f"  static constexpr bool SWAPPED = {str(swapped).lower()};      // g is mixed, not x",
+              f"  static constexpr int O0 = {mixed[0]}, NO = {len(mixed)}, R0 = {plain[0]}, NR = {len(plain)};",
+              "  template <int R, class Mix>",
+              "  __device__ __forceinline__ static void mix(Mix&& m) {"]
+        for r, row in enumerate(plain):
+            L.append(f"    if constexpr (R == {r}) {{")
+            adds = 0
+            for o, mrow in enumerate(mixed):
+                terms = [t for t in mine if (int(coo.M1[t]), int(coo.M[t])) == ((row, mrow) if swapped else (mrow, row))]
+                if terms:
+                    L.append(f"      m.add({o}, " + " + ".join(f"{_lit(coo.coef[t])} * m.y({coo.M2[t]})" for t in terms) + ");")
+                    adds += 1
+                    if adds % 2 == 0:
+                        L.append("      m.fence();")
+            L.append("    }")
+        L += ["  }", "};"]
+    L += [f"struct UVG_{name} {{", f"  static constexpr int D1 = {coo.D1}, D2 = {coo.D2}, DO = {coo.DO}, P = {coo.P};",
+          f"  static constexpr unsigned SWAPPED = {turned}u;      // a bit per path",
+          "  template <class F>", "  __device__ __forceinline__ static void path(int p, F&& f) {", "    switch (p) {"]
+    L += [f"      case {p}: f(UVG_{name}_p{p}{{}}); break;" for p in range(coo.P)]
+    L += ["      default: break;", "    }", "  }", "};", ""]
+    return "\n".join(L)
+
+
 def emit_split(out_dir: str) -> str:
     """``generated/uv_split_configs.inc``: the single-precision bodies, and every table as a list of terms."""
     chunks = ["// Generated by equitorch_amd/csrc/gen_uv.py; do not edit.", ""]
@@ -273,10 +311,14 @@ def emit_split(out_dir: str) -> str:
     chunks.append(" \\\n".join(f"  X({list(CONFIGS).index(n)}, UVS_{n}_d0, UVS_{n}_d1, UVS_{n}_gy, UVS_{n}_d2, UVS_{n}_table)"
                               for n in names))
     chunks.append("")
-    path, text = os.path.join(out_dir, "uv_split_configs.inc"), "\n".join(chunks)
-    if not os.path.exists(path) or open(path).read() != text:
-        with open(path, "w") as f:
-            f.write(text)
+    gw = ["// Generated by equitorch_amd/csrc/gen_uv.py; do not edit.", ""]
+    gw += [emit_split_gw(n, tp_coo(tp_infos(*map(Irreps, CONFIGS[n][:3]), **CONFIGS[n][3])[0])) for n in names]
+    gw += ["#define CGTP_FOREACH_UVG_CONFIG(X) " + " ".join(f"X({list(CONFIGS).index(n)}, UVG_{n})" for n in names), ""]
+    path = os.path.join(out_dir, "uv_split_configs.inc")
+    for path, text in ((path, "\n".join(chunks)), (os.path.join(out_dir, "uv_split_gw_configs.inc"), "\n".join(gw))):
+        if not os.path.exists(path) or open(path).read() != text:
+            with open(path, "w") as f:
+                f.write(text)
     return path
 
 

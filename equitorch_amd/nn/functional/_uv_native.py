@@ -129,9 +129,96 @@ class _PathWalk(_Coefficients):
         self._coef, self._device, self._term_c = coef, device, {}
 
 
+class _GradWWalk:
+    """The work of ``cgtp_uvg_apply`` for a table, dealt to ``n_wgs`` workgroups."""
+    SHARES = 64
+
+    def __init__(self, coo, n_wgs: int, device):
+        cost = []
+        for p in range(coo.P):
+            mine = np.asarray(coo.p) == p
+            rows = len(set(np.asarray(coo.M1)[mine].tolist())), len(set(np.asarray(coo.M)[mine].tolist()))
+            # of a step: its products (as many as the side with fewer rows has), and the rows that are read
+            cost.append(min(rows) + 0.15 * sum(rows))
+        jobs = self.deal(cost, n_wgs)
+        slots, slot_ptr = {}, [0]
+        for p in range(coo.P):
+            for w, mine in enumerate(jobs):
+                for path, _ in mine:
+                    if path == p:
+                        slots[w, p] = len(slots)
+            slot_ptr.append(len(slots))
+        flat = [(p, slots[w, p], mask & 0xffffffff, mask >> 32) for w, mine in enumerate(jobs) for p, mask in mine]
+        job_ptr = np.cumsum([0] + [len(mine) for mine in jobs])
+        parts = [np.array(flat, dtype=np.uint32).view(np.int32), job_ptr.astype(np.int32), np.array(slot_ptr, dtype=np.int32)]
+        self.words = torch.from_numpy(np.concatenate([p.ravel() for p in parts])).to(device)
+        self.at = [4 * sum(p.size for p in parts[:k]) for k in range(len(parts))]
+        self.n_slots = len(slots)
+
+    @classmethod
+    def deal(cls, cost, n_wgs: int):
+        """Per workgroup its ``(path, mask)``: the 64 shares of every path, dealt in the order of the paths so that all
+        workgroups carry the same cost, the shares of a path spread over its steps."""
+        room = sum(cost) * cls.SHARES / n_wgs
+        jobs, w, left = [[] for _ in range(n_wgs)], 0, room
+        for p, c in enumerate(cost):
+            todo, portions = cls.SHARES, []
+            while todo:
+                take = min(todo, max(0, int(left / c + 0.5))) if w < n_wgs - 1 else todo
+                if take:
+                    portions.append((w, take))
+                    todo -= take
+                    left -= take * c
+                if todo:
+                    w, left = w + 1, left + room           # what was taken too much or too little carries over
+            given, masks = [0] * len(portions), [0] * len(portions)
+            for bit in range(cls.SHARES):
+                k = max(range(len(portions)), key=lambda i: portions[i][1] * (bit + 1) / cls.SHARES - given[i])
+                given[k] += 1
+                masks[k] |= 1 << bit
+            for (g, _), mask in zip(portions, masks):
+                if mask:
+                    jobs[g].append((p, mask))
+        return jobs
+
+
+def _split_grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Optional[Tensor]:
+    """:func:`grad_w` in fp32 on the half-precision matrix cores (``cgtp_uvg_apply``), or None where the fp32 matrix
+    instructions serve: tables that are not compiled in as they are, different numbers of channels, and where they are
+    quicker or more precise.  Without channels on ``y`` that is up to 64 channels (lmax 3, 64 channels, 32768 samples 405 against
+    545 us, but errors of 5.3e-7 against 4.9e-7), lmax 1 (4000 samples, 128 channels: 38 us against 28) and small batches (lmax 3, 1000 samples,
+    128 channels 77 us against 67; below 4096 samples errors of 2.7e-7 against 2.5e-7); with channels, below 24 of them (16: 128 us against
+    110; 20: 417 and 405) and small batches (lmax 2, 1000 samples 107 us against 77; lmax 1, 2100 samples 50 and 44)."""
+    if isinstance(tp_info, CooTable) or x.dtype != torch.float32 or x.shape[0] == 0 or x.shape[2] != g.shape[2]:
+        return None
+    cfg = kernels.uv_config_of(tp_info)
+    if int(cfg) < 0 or cfg.path_scale is not None or cfg.w_rows is not None:
+        return None
+    (n, _, c), cy = x.shape, y.shape[2] if y.ndim == 3 else 0
+    coo = _coo(tp_info)
+    if (min(c, cy) < 24 or n < (2048 if coo.P > 4 else 8192)) if cy else (c <= 64 or n < (2048 if coo.P <= 11 else 4096)):
+        return None
+    steps, n_wgs = -(-n // 16), 64                       # of a range: 32 compute units, two wavefronts per SIMD
+    n_ranges = 8 * max(1, steps // 1024)
+    walk = kernels.cached(_anchor(tp_info), ("uvg_walk", n_wgs, str(x.device)), lambda: _GradWWalk(coo, n_wgs, x.device))
+    gw = torch.empty((coo.P, c * max(cy, 1), c), dtype=x.dtype, device=x.device)
+    jobs, job_ptr, slot_ptr = (walk.words.data_ptr() + v for v in walk.at)
+    a = _lib.UvgArgs(x.data_ptr(), y.data_ptr(), g.data_ptr(), gw.data_ptr(), 256, jobs, job_ptr, slot_ptr, n, int(cfg), n_ranges, n_wgs,
+                     walk.n_slots, c, cy)
+    if _lib.lib.cgtp_uvg_validate(C.byref(a)) != 0:
+        return None
+    ws = torch.empty(n_ranges * walk.n_slots * gw[0].numel(), dtype=x.dtype, device=x.device)
+    a.workspace = ws.data_ptr()
+    _lib.check(_lib.lib.cgtp_uvg_apply(C.byref(a), _lib.stream_ptr(x.device)), "cgtp_uvg_apply")
+    return gw
+
+
 def grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Tensor:
-    """``gw[p, k, w] = sum_n sum_{(p, M)} inter[n, (p, M), k] g[n, M, w]`` (``cgtp_uvt_grad_w``): ``(P, K, C_out)`` with
-    ``K = C_x`` or ``C_x * C_y``; the caller reshapes."""
+    """``gw[p, k, w] = sum_n sum_{(p, M)} inter[n, (p, M), k] g[n, M, w]`` (``cgtp_uvt_grad_w``, in fp32 ``cgtp_uvg_apply``):
+    ``(P, K, C_out)`` with ``K = C_x`` or ``C_x * C_y``; the caller reshapes."""
+    gw = _split_grad_w(x, y, g, tp_info)
+    if gw is not None:
+        return gw
     walk = kernels.cached(_anchor(tp_info), ("uvt_path_walk", str(x.device)),
                           lambda: _PathWalk(_coo(tp_info), x.device))
     n, dx, cx = x.shape

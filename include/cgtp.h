@@ -452,6 +452,30 @@ int64_t cgtp_uvl_packed_bytes(int32_t n_blocks, int32_t cx, int32_t cout);
 int cgtp_uvl_validate(const cgtp_uvl_args* a);
 int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream);
 
+/* The weight gradient of the fully connected product of a compiled table (cfg as above) in single precision on the
+ * half-precision matrix cores (operands as above), as many channels of g as of x:
+ *   gw[p, k, (l,) w] = sum_n sum_{terms t of p} coef_t * x[n, a_t, k] * y[n, b_t(, l)] * g[n, m_t, w]
+ * x (n_rows, D1, c), y (n_rows, D2) with cy = 0, c <= 128, or (n_rows, D2, cy) with cy a multiple of 4, c <= 32; g (n_rows, DO, c),
+ * gw (P, c, (cy,) c), contiguous, c a multiple of 4.  The samples are cut into n_ranges ranges, and in each the work is dealt
+ * to n_wgs workgroups: job_ptr[w] .. job_ptr[w + 1] are those of workgroup w, a job the steps of 16 samples of a path whose number
+ * in the range, mod 64, is in its mask (not empty).  Every job has a slot of the workspace, n_ranges * n_slots slots of c *
+ * max(cy, 1) * c floats; the slots of path p are slot_ptr[p] .. slot_ptr[p + 1].  Tables in device memory. */
+typedef struct { int32_t path, slot, mask_low, mask_high; } cgtp_uvg_job;
+typedef struct {
+  const void* x;
+  const void* y;
+  const void* g;
+  void* gw;
+  void* workspace;
+  const cgtp_uvg_job* jobs;
+  const int32_t* job_ptr;
+  const int32_t* slot_ptr;
+  int64_t n_rows;
+  int32_t cfg, n_ranges, n_wgs, n_slots, c, cy;
+} cgtp_uvg_args;
+int cgtp_uvg_validate(const cgtp_uvg_args* a);
+int cgtp_uvg_apply(const cgtp_uvg_args* a, void* stream);
+
 /* ---- radial basis and cutoff envelopes ---------------------------------------------------------------------------
  *
  * Element-wise functions of the edge length r (n values), fp32 / fp64, one launch forward and one for the gradient.
