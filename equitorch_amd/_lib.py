@@ -129,6 +129,13 @@ class UvlArgs(C.Structure):
                 ("dx", C.c_int32), ("dout", C.c_int32), ("cx", C.c_int32), ("cout", C.c_int32)]
 
 
+class UvlGwArgs(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("g", C.c_void_p), ("gw", C.c_void_p), ("workspace", C.c_void_p),
+                ("pairs", C.c_void_p), ("path_ptr", C.c_void_p), ("n_rows", C.c_int64),
+                ("n_paths", C.c_int32), ("max_pairs", C.c_int32), ("dx", C.c_int32), ("dg", C.c_int32),
+                ("cx", C.c_int32), ("cout", C.c_int32)]
+
+
 class UvgArgs(C.Structure):
     _fields_ = [("x", C.c_void_p), ("y", C.c_void_p), ("g", C.c_void_p), ("gw", C.c_void_p), ("workspace", C.c_void_p),
                 ("jobs", C.c_void_p), ("job_ptr", C.c_void_p), ("slot_ptr", C.c_void_p), ("n_rows", C.c_int64),
@@ -194,6 +201,9 @@ def _load():
     lib.cgtp_uvl_packed_bytes.argtypes = [C.c_int32] * 3
     lib.cgtp_uvl_validate.argtypes = [C.POINTER(UvlArgs)]
     lib.cgtp_uvl_apply.argtypes = [C.POINTER(UvlArgs), C.c_void_p]
+    lib.cgtp_uvl_grad_w_workspace_bytes.restype = C.c_int64
+    lib.cgtp_uvl_grad_w_workspace_bytes.argtypes = [C.POINTER(UvlGwArgs)]
+    lib.cgtp_uvl_grad_w.argtypes = [C.POINTER(UvlGwArgs), C.c_void_p]
     lib.cgtp_uvg_validate.argtypes = [C.POINTER(UvgArgs)]
     lib.cgtp_uvg_apply.argtypes = [C.POINTER(UvgArgs), C.c_void_p]
     lib.cgtp_uvu_mx_workspace_bytes.restype = C.c_int64

@@ -659,15 +659,23 @@ int cgtp_abi_layout(int which, int64_t* out, int capacity) {
                                      CGTP_OFF(cgtp_uvg_args, n_ranges), CGTP_OFF(cgtp_uvg_args, n_wgs),
                                      CGTP_OFF(cgtp_uvg_args, n_slots), CGTP_OFF(cgtp_uvg_args, c),
                                      CGTP_OFF(cgtp_uvg_args, cy)};
+  static const int64_t uvl_gw_args[] = {sizeof(cgtp_uvl_gw_args), CGTP_OFF(cgtp_uvl_gw_args, x),
+                                        CGTP_OFF(cgtp_uvl_gw_args, g), CGTP_OFF(cgtp_uvl_gw_args, gw),
+                                        CGTP_OFF(cgtp_uvl_gw_args, workspace), CGTP_OFF(cgtp_uvl_gw_args, pairs),
+                                        CGTP_OFF(cgtp_uvl_gw_args, path_ptr), CGTP_OFF(cgtp_uvl_gw_args, n_rows),
+                                        CGTP_OFF(cgtp_uvl_gw_args, n_paths), CGTP_OFF(cgtp_uvl_gw_args, max_pairs),
+                                        CGTP_OFF(cgtp_uvl_gw_args, dx), CGTP_OFF(cgtp_uvl_gw_args, dg),
+                                        CGTP_OFF(cgtp_uvl_gw_args, cx), CGTP_OFF(cgtp_uvl_gw_args, cout)};
 #undef CGTP_OFF
   const int64_t* tabs[] = {operand, tri, gen_operand, gen, uvu, uvt_item, uvt, uvt_gw, uvt_gy, uvu_tab, psw_table,
-                           psw_args, uvu_mx, uvl_args, uvg_args};
+                           psw_args, uvu_mx, uvl_args, uvg_args, uvl_gw_args};
   const int counts[] = {(int)(sizeof(operand) / 8), (int)(sizeof(tri) / 8), (int)(sizeof(gen_operand) / 8),
                         (int)(sizeof(gen) / 8), (int)(sizeof(uvu) / 8), (int)(sizeof(uvt_item) / 8),
                         (int)(sizeof(uvt) / 8), (int)(sizeof(uvt_gw) / 8), (int)(sizeof(uvt_gy) / 8),
                         (int)(sizeof(uvu_tab) / 8), (int)(sizeof(psw_table) / 8), (int)(sizeof(psw_args) / 8), (int)(sizeof(uvu_mx) / 8),
-                        (int)(sizeof(uvl_args) / 8), (int)(sizeof(uvg_args) / 8)};
-  if (which < 0 || which >= 15) return -1;
+                        (int)(sizeof(uvl_args) / 8), (int)(sizeof(uvg_args) / 8),
+                        (int)(sizeof(uvl_gw_args) / 8)};
+  if (which < 0 || which >= 16) return -1;
   for (int i = 0; out && i < counts[which] && i < capacity; ++i) out[i] = tabs[which][i];
   return counts[which];
 }

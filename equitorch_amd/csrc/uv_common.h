@@ -16,4 +16,7 @@ __device__ __forceinline__ float dot8(const floatx4& g0, const floatx4& g1, cons
   return s;
 }
 
+// gw[i] = sum over the chunks c of part[c * n + i] in a fixed order (uvt_kernels.hip); n a multiple of 4.
+int uvt_reduce_chunks(const float* part, float* gw, int64_t n_chunks, int64_t n, hipStream_t stream);
+
 }  // namespace cgtp

@@ -301,6 +301,221 @@ __global__ void __launch_bounds__(256, NT * RW == 4 ? 2 : 3) uvl_kernel(const Uv
   }
 }
 
+// ---- gradient of the weight: gW[p, k, w] = sum_n sum_{entries e of p} coef_e * x[n, a_e, k] * g[n, m_e, w] ---------------------
+struct UvlGwDev {
+  const float* x;
+  const float* g;
+  float* part;                        // (n_chunks, n_paths, cx, cout)
+  const cgtp_uvl_pair* pairs;
+  const int32_t* path_ptr;
+  int64_t n_rows;
+  int n_paths, dx, dg, cx, cout, chunk, n_chunks, kblocks, wblocks;
+};
+
+// A wavefront owns a block of 16 TI x 16 TJ of a path's gradient and a chunk of samples by itself, as uvt_grad_w_small_kernel does: what
+// it loads of 32 samples (TI or TJ consecutive channels of eight samples a lane) is the layout of the matrix operands, so nothing is
+// exchanged and there is no barrier.  The four wavefronts of a workgroup have four paths in a row: the (w_+, w_-) pairs of an
+// SO(2) layer read the same rows, the second time from the L1; the paths of a chunk run on one XCD.
+// What bounds it: splitting both operands (64 elements a lane and 32 samples: 390 vector instructions next to 96 matrix ones of 16
+// cycles) and the rows from L2.  SO2Linear, lmax 4, 64 channels, 32768 samples 548 -> 346 us, 1000 samples 36 -> 30; IrrepsLinear 64 -> 64,
+// lmax 2, 65536 samples 118 -> 84, 128 -> 128, lmax 3, 32768 samples 241 -> 219.
+template <int TI, int TJ>
+__global__ void __launch_bounds__(256, 2) uvl_gw_kernel(const UvlGwDev a) {
+  typedef typename VecOf<float, TI>::type VI;
+  typedef typename VecOf<float, TJ>::type VJ;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), r = lane & 15, q = lane >> 4;
+  const int groups = (a.n_paths + 3) / 4, parts = groups * a.kblocks * a.wblocks, j = blockIdx.x >> 3;
+  const int at = j % parts, chunk = j / parts * 8 + (blockIdx.x & 7), p = at % groups * 4 + wave;
+  if (chunk >= a.n_chunks || p >= a.n_paths) return;
+  const int k0 = at / groups % a.kblocks * (16 * TI), w0 = at / groups / a.kblocks * (16 * TJ);
+  const int64_t n_begin = (int64_t)chunk * a.chunk, n_end = min(n_begin + a.chunk, a.n_rows);
+  const int kc = min(k0 + TI * r, a.cx - TI), wc = min(w0 + TJ * r, a.cout - TJ);      // channels past the last are not stored
+  const int xs = a.dx * a.cx, gs = a.dg * a.cout, e0 = a.path_ptr[p], entries = a.path_ptr[p + 1] - e0;
+  const int steps = (int)((n_end - n_begin + 31) / 32), units = steps * entries;
+  floatx4 acc[TI][TJ];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int t = 0; t < TJ; ++t) acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  unsigned plain = 0;
+  if (units > 0) {
+    // lane l holds entry l of the path (64 at most)
+    const cgtp_uvl_pair mine = a.pairs[e0 + min(lane, entries - 1)];
+    auto coef_of = [&](int e) __attribute__((always_inline)) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.coef), e));
+    };
+    const unsigned xat = 4u * (unsigned)(8 * q * xs + kc), gat = 4u * (unsigned)(8 * q * gs + wc);
+    VI xr[8];
+    VJ gr[8];
+    auto load = [&](int step, int e) __attribute__((always_inline)) {
+      const int64_t n0 = n_begin + (int64_t)step * 32;
+      const char* xrow = reinterpret_cast<const char*>(a.x + n0 * xs + __builtin_amdgcn_readlane(mine.row_x, e) * a.cx);
+      const char* grow = reinterpret_cast<const char*>(a.g + n0 * gs + __builtin_amdgcn_readlane(mine.row_g, e) * a.cout);
+      if (n0 + 32 <= n_end) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xr[i] = *reinterpret_cast<const VI*>(xrow + (int64_t)i * xs * 4 + xat);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) gr[i] = *reinterpret_cast<const VJ*>(grow + (int64_t)i * gs * 4 + gat);
+      } else {
+        int left = (int)(n_end - n0);
+        asm volatile("" : "+v"(left));                 // its addresses are not kept around the loop
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int n = 8 * q + i, nc = min(n, left - 1);
+          const VI u = *reinterpret_cast<const VI*>(xrow + 4u * (unsigned)(nc * xs + kc));
+          const VJ v = *reinterpret_cast<const VJ*>(grow + 4u * (unsigned)(nc * gs + wc));
+#pragma unroll
+          for (int k = 0; k < TI; ++k) xr[i][k] = n < left ? u[k] : 0.f;
+#pragma unroll
+          for (int k = 0; k < TJ; ++k) gr[i][k] = n < left ? v[k] : 0.f;
+        }
+      }
+    };
+    int step = 0, e = 0;
+    load(0, 0);
+    for (int u = 0; u < units; ++u) {
+      const float sign = u & 1 ? -1.f : 1.f, c = sign * coef_of(e);
+      UvsParts<8> xp[TI];
+      VJ gv[8];
+      float low = 1.f;
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float v0 = c * xr[2 * k][i], v1 = c * xr[2 * k + 1][i];
+          xp[i].pair(k, v0, v1);
+          low = uvs_least(v0, v1, low);
+        }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) gv[k] = gr[k];
+#pragma unroll
+      for (int k = 0; k < 8; k += 2)
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) {
+          const float v0 = gv[k][t], v1 = gv[k + 1][t];
+          low = uvs_least(v0, v1, low);
+        }
+      if (__any(low < 0x1p-110f)) {                    // a zero, as a rule
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+#pragma unroll
+          for (int i = 0; i < TI; ++i) {
+            const float v = c * xr[k][i];
+            plain |= uvs_asks(v) & kUvsPlain;
+          }
+#pragma unroll
+          for (int t = 0; t < TJ; ++t) {
+            const float v = gv[k][t];
+            plain |= uvs_asks(v) & kUvsPlain;
+          }
+        }
+      }
+      if (++e == entries) {
+        e = 0;
+        ++step;
+      }
+      if (u + 1 < units) load(step, e);
+#pragma unroll
+      for (int t = 0; t < TJ; ++t) {
+        UvsParts<8> gp;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float v0 = gv[2 * k][t], v1 = gv[2 * k + 1][t];
+          gp.pair(k, v0, v1);
+        }
+        // The products of 32 samples are summed by themselves, every other time with the sign turned: the matrix instruction rounds
+        // downwards, which in a sum over many samples is no small part of the error (IrrepsLinear 64 -> 64, 65536 samples: all
+        // parts added to the chunk's sums 7.2e-7, by themselves 6.0e-7, with alternating signs 2.3e-7; fp32 instructions 4.5e-7).
+        floatx4 sum[TI];
+#pragma unroll
+        for (int i = 0; i < TI; ++i) sum[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int h = 0; h < 6; ++h) {                  // the small products first
+          constexpr int ha[6] = {2, 1, 0, 1, 0, 0}, hb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+          for (int i = 0; i < TI; ++i)
+            sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uvs_frag(xp[i].p[ha[h]]), uvs_frag(gp.p[hb[h]]), sum[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < TI; ++i) acc[i][t] += sign * sum[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int t = 0; t < TJ; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float v = acc[i][t][k];
+          plain |= v - v != 0.f;
+        }
+    if (__any(plain)) {                                // fp32 matrix instructions, operands from memory
+      clear();
+      for (int s = 0; s < entries; ++s) {
+        const float c = coef_of(s);
+        const float* xrow = a.x + __builtin_amdgcn_readlane(mine.row_x, s) * a.cx + kc;
+        const float* grow = a.g + __builtin_amdgcn_readlane(mine.row_g, s) * a.cout + wc;
+        for (int64_t n0 = n_begin; n0 < n_end; n0 += 4) {
+          const int64_t n = min(n0 + q, n_end - 1);
+          const float f = n0 + q < n_end ? 1.f : 0.f;
+          const VI u = *reinterpret_cast<const VI*>(xrow + n * xs);
+          const VJ v = *reinterpret_cast<const VJ*>(grow + n * gs);
+#pragma unroll
+          for (int i = 0; i < TI; ++i) {
+            const float ui = f != 0.f ? c * u[i] : 0.f;
+#pragma unroll
+            for (int t = 0; t < TJ; ++t) {
+              const float vt = f != 0.f ? v[t] : 0.f;
+              acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ui, vt, acc[i][t], 0, 0, 0);
+            }
+          }
+        }
+      }
+    }
+  }
+  // element e of tile (i, t): channel TI (4 q + e) + i of the contracted axis's block, TJ r + t of the other's
+  float* out = a.part + ((int64_t)chunk * a.n_paths + p) * a.cx * a.cout;
+  if (w0 + TJ * r < a.cout) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = k0 + TI * (4 * q + e) + i;
+        if (k < a.cx) {
+          VJ v;
+#pragma unroll
+          for (int t = 0; t < TJ; ++t) v[t] = acc[i][t][e];
+          *reinterpret_cast<VJ*>(out + (int64_t)k * a.cout + w0 + TJ * r) = v;
+        }
+      }
+  }
+}
+
+// Samples per wavefront: 32 or more, at most 8192 wavefronts and 512 partial results (the rule of uvt_grad_w_small_kernel).
+static int64_t uvl_gw_chunk(const cgtp_uvl_gw_args* a) {
+  const int64_t blocks = (int64_t)((a->cx + 63) / 64) * ((a->cout + 63) / 64) * a->n_paths;
+  int64_t chunk = 32;
+  while ((a->n_rows + chunk - 1) / chunk > 512 || (a->n_rows + chunk - 1) / chunk * blocks > 8192) {
+    chunk *= 2;
+    if (chunk >= a->n_rows) break;
+  }
+  return chunk;
+}
+
+static int uvl_gw_check(const cgtp_uvl_gw_args* a) {
+  if (!a || !a->x || !a->g || !a->gw || !a->pairs || !a->path_ptr) return CGTP_ERR_NULL;
+  if (a->n_rows <= 0 || a->n_paths <= 0 || a->dx <= 0 || a->dg <= 0 || a->cx <= 0 || a->cout <= 0 || a->cx % 4 || a->cout % 4 ||
+      (int64_t)a->dx * a->cx > 1 << 22 || (int64_t)a->dg * a->cout > 1 << 22 || a->max_pairs > kWave)
+    return CGTP_ERR_SHAPE;
+  if (((uintptr_t)a->x | (uintptr_t)a->g | (uintptr_t)a->gw | (uintptr_t)a->workspace) & 15u) return CGTP_ERR_ALIGN;
+  const int64_t blocks = (int64_t)((a->cx + 63) / 64) * ((a->cout + 63) / 64) * ((a->n_paths + 3) / 4);
+  const int64_t chunks = (a->n_rows + uvl_gw_chunk(a) - 1) / uvl_gw_chunk(a);
+  return (chunks + 7) / 8 * 8 * blocks < (int64_t)1 << 31 ? CGTP_OK : CGTP_ERR_SHAPE;
+}
+
 struct UvlPlan {
   UvlDev dev;
   int tw, nt;
@@ -370,6 +585,33 @@ int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream) {
   void (*fn)(const UvlDev) = p.tw == 4 ? uvl_fn<4>(p.nt, a->rows_per_task) : uvl_fn<2>(p.nt, a->rows_per_task);
   hipLaunchKernelGGL(fn, dim3((unsigned)p.grid), dim3(256), 0, (hipStream_t)stream, d);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+}
+
+int64_t cgtp_uvl_grad_w_workspace_bytes(const cgtp_uvl_gw_args* a) {
+  if (uvl_gw_check(a) != CGTP_OK) return 0;
+  const int64_t chunk = uvl_gw_chunk(a);
+  return (a->n_rows + chunk - 1) / chunk * a->n_paths * a->cx * a->cout * 4;
+}
+
+int cgtp_uvl_grad_w(const cgtp_uvl_gw_args* a, void* stream) {
+  const int st = uvl_gw_check(a);
+  if (st != CGTP_OK) return st;
+  if (!a->workspace) return CGTP_ERR_WORKSPACE;
+  UvlGwDev d;
+  d.x = (const float*)a->x; d.g = (const float*)a->g; d.part = (float*)a->workspace;
+  d.pairs = a->pairs; d.path_ptr = a->path_ptr;
+  d.n_rows = a->n_rows; d.n_paths = a->n_paths; d.dx = a->dx; d.dg = a->dg; d.cx = a->cx; d.cout = a->cout;
+  const int64_t chunk = uvl_gw_chunk(a), n_chunks = (a->n_rows + chunk - 1) / chunk;
+  d.chunk = (int)chunk;
+  d.n_chunks = (int)n_chunks;
+  const bool ki = a->cx <= 32, wj = a->cout <= 32;     // two channels a lane where 32 cover the axis
+  d.kblocks = ki ? 1 : (a->cx + 63) / 64;
+  d.wblocks = wj ? 1 : (a->cout + 63) / 64;
+  const int64_t grid = (n_chunks + 7) / 8 * 8 * ((a->n_paths + 3) / 4) * d.kblocks * d.wblocks;
+  void (*fn)(const UvlGwDev) = ki ? (wj ? uvl_gw_kernel<2, 2> : uvl_gw_kernel<2, 4>) : wj ? uvl_gw_kernel<4, 2> : uvl_gw_kernel<4, 4>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, d);
+  if (hipGetLastError() != hipSuccess) return CGTP_ERR_LAUNCH;
+  return uvt_reduce_chunks((const float*)a->workspace, (float*)a->gw, n_chunks, (int64_t)a->n_paths * a->cx * a->cout, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -18,8 +18,7 @@
 //
 // The file compiles twice: as it is for fp32 (v_mfma_f32_16x16x4_f32), and from uvt_kernels_f64.hip with CGTP_UVT_F64
 // defined for fp64 (v_mfma_f64_16x16x4_f64, same lane layouts); each set lives in its own namespace.
-#include "cgtp_device.h"
-#include "cgtp_host.h"
+#include "uv_common.h"
 
 #ifdef CGTP_UVT_F64
 #define UVT_NS uvt_f64
@@ -1318,6 +1317,11 @@ int grad_y(const cgtp_uvt_gy_args* a, void* stream) {
 // The double-precision set of the same kernels and entry points: uvt_kernels_f64.hip compiles this file with
 // CGTP_UVT_F64 defined.
 namespace cgtp {
+int uvt_reduce_chunks(const float* part, float* gw, int64_t n_chunks, int64_t n, hipStream_t stream) {
+  hipLaunchKernelGGL(uvt_f32::uvt_gw_reduce_kernel, dim3((unsigned)((n / 4 + uvt_f32::kGwReduceCols - 1) / uvt_f32::kGwReduceCols)),
+                     dim3(uvt_f32::kGwReduceCols * uvt_f32::kGwReduceSlices), 0, stream, part, gw, n_chunks, n / 4);
+  return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
+}
 namespace uvt_f64 {
 int pack_weights(const void* w, void* packed, int32_t n_paths, int64_t K, int32_t cout, int64_t stride_p, int64_t stride_k,
                  int64_t stride_c, int32_t dtype, void* stream);

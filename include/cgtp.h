@@ -452,6 +452,23 @@ int64_t cgtp_uvl_packed_bytes(int32_t n_blocks, int32_t cx, int32_t cout);
 int cgtp_uvl_validate(const cgtp_uvl_args* a);
 int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream);
 
+/* Its weight gradient: gw[p, k, w] = sum_n sum_{pairs e of path p} coef_e * x[n, row_x, k] * g[n, row_g, w]; x (n_rows, dx, cx), g (n_rows,
+ * dg, cout), gw (n_paths, cx, cout), contiguous, cx and cout multiples of 4.  path_ptr[p] .. path_ptr[p + 1] are the pairs of path
+ * p, at most 64 (max_pairs: the most of any; none: zeros).  workspace: cgtp_uvl_grad_w_workspace_bytes() bytes. */
+typedef struct { int32_t row_x, row_g; float coef; int32_t reserved_; } cgtp_uvl_pair;
+typedef struct {
+  const void* x;
+  const void* g;
+  void* gw;
+  void* workspace;
+  const cgtp_uvl_pair* pairs;
+  const int32_t* path_ptr;
+  int64_t n_rows;
+  int32_t n_paths, max_pairs, dx, dg, cx, cout;
+} cgtp_uvl_gw_args;
+int64_t cgtp_uvl_grad_w_workspace_bytes(const cgtp_uvl_gw_args* a);
+int cgtp_uvl_grad_w(const cgtp_uvl_gw_args* a, void* stream);
+
 /* The weight gradient of the fully connected product of a compiled table (cfg as above) in single precision on the
  * half-precision matrix cores (operands as above), as many channels of g as of x:
  *   gw[p, k, (l,) w] = sum_n sum_{terms t of p} coef_t * x[n, a_t, k] * y[n, b_t(, l)] * g[n, m_t, w]

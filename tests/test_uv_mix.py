@@ -1,4 +1,4 @@
-"""Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``; IrrepsLinear and SO2Linear('uv') with a shared
+"""Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``, ``cgtp_uvl_grad_w``; IrrepsLinear and SO2Linear('uv') with a shared
 weight): every operand carried as three bf16 parts, no less precise than fp32 matrix instructions and of their range."""
 import numpy as np
 import pytest
@@ -171,6 +171,64 @@ def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponent, sc
                 return float(d.square().mean().sqrt())
             print(f"{name} of 2^{exponent}, 2^{scale}: split {err(a):.2e} fp32 {err(b):.2e}")
             assert err(a) <= 1.5 * err(b) + 3e-8, name
+
+
+# ---- gradient of the weight --------------------------------------------------------------------------------------------
+def _weight_gradients(monkeypatch, kind, l, cin, cout, x, g, device):
+    from equitorch_amd.nn.functional import _uv_native as N
+    mod = _module(kind, l, cin, cout, device)
+    taken, split = [], N._mix_grad_w
+
+    def spy(*args):
+        taken.append(args)
+        return split(*args)
+    monkeypatch.setattr(N, "_mix_grad_w", spy)
+    new, = torch.autograd.grad(mod(x.to(device)), [mod.weight], g.to(device))
+    (xs, gs, table), = taken
+    ones = torch.ones(xs.shape[0], 1, device=device)
+    monkeypatch.setattr(N, "_mix_grad_w", lambda *args: None)
+    return new, N.grad_w(xs, ones, gs, table), N.grad_w(xs.double(), ones.double(), gs.double(), table)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n", [("lin", 1, 4, 4, 1), ("lin", 2, 12, 20, 65), ("own", 3, 36, 100, 129), ("lin", 2, 64, 64, 70001),
+                                               ("lin", 3, 128, 96, 700), ("so2", 2, 32, 64, 31), ("so2", 4, 64, 32, 2077), ("so2", 6, 48, 48, 257)])
+@pytest.mark.parametrize("values", ["normal", "wide"])
+def test_the_weight_gradient_is_no_less_precise(device, monkeypatch, kind, l, cin, cout, n, values):
+    x, g = _operands(kind, l, cin, cout, n, stable_seed("mix gw", kind, l, cin, cout, n))
+    if values == "wide":
+        gen = torch.Generator().manual_seed(3)
+        for t in (x, g):
+            t.mul_(torch.exp2(torch.randint(-10, 11, (n, 1, 1), generator=gen).float()))
+        x[n // 2 + 1:n // 2 + 9] = 0.0
+    new, old, ref = _weight_gradients(monkeypatch, kind, l, cin, cout, x, g, device)
+    e_new, e_old = (float((t.double() - ref).norm() / ref.norm()) for t in (new, old))
+    print(f"grad W {kind} lmax={l} {cin}->{cout} n={n} {values}: split {e_new:.2e} fp32 {e_old:.2e}")
+    assert e_new <= e_old + 3e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where,value", [(0, float("inf")), (1, float("nan")), (1, float("-inf")), (0, 3.39e38)])
+def test_the_weight_gradient_of_values_that_are_not_finite(device, monkeypatch, where, value):
+    ops = list(_operands("so2", 2, 32, 64, 150, 7))
+    ops[1 - where] *= 2.0 ** -8
+    ops[where].view(-1)[567] = value
+    new, old, _ = _weight_gradients(monkeypatch, "so2", 2, 32, 64, *ops, device)
+    fin = torch.isfinite(old)
+    assert torch.equal(fin, torch.isfinite(new)) and torch.equal(new[~fin & ~old.isnan()], old[~fin & ~old.isnan()])
+    assert float((new[fin].double() - old[fin].double()).norm()) <= 1e-6 * float(old[fin].double().norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exponents", [(0, 0), (-105, 0), (-118, 100), (0, -113), (-60, -48), (60, 60)])
+def test_the_weight_gradient_has_the_range_of_fp32(device, monkeypatch, exponents):
+    ops = [t * 2.0 ** e for t, e in zip(_operands("lin", 2, 64, 32, 300, 8), exponents)]
+    new, old, ref = _weight_gradients(monkeypatch, "lin", 2, 64, 32, *ops, device)
+    assert torch.equal(torch.isfinite(new), torch.isfinite(old))
+    if ref.abs().max() > 2.0 ** -100:
+        e_new, e_old = (float((t.double() - ref).norm() / ref.norm()) for t in (new, old))
+        print(f"{exponents}: split {e_new:.2e} fp32 {e_old:.2e}")
+        assert e_new <= 1.5 * e_old + 3e-8
 
 
 @pytest.mark.gpu
