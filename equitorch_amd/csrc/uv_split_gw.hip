@@ -16,13 +16,14 @@
 //
 // The steps are cut into ranges, one per XCD at a time, and the workgroups of a range (two wavefronts per SIMD) share the work of its
 // paths evenly: path p has 64 shares of its steps (step mod 64), dealt to workgroups by cost.  They walk the range side by
-// side, so that its rows come from memory once and then from the XCD's L2.  The sums of a few products at a time (12 or 32) are added
+// side, so that its rows come from memory once and then from the XCD's L2.  The sums of some products at a time (24 or 64) are added
 // to a slot of the workspace (chains as short as those of the fp32 kernel); the slots are added in their order.
 //
 // What bounds it: waiting (43 % of the wavefronts' time at two per SIMD: rows from the last-level cache, three quarters of the requests
 // that miss the L1 at lmax = 3; barriers), then vector and matrix instructions in about equal parts (250 vector ones to 24 matrix
-// ones of 32 cycles per product and wavefront).  128 channels, 32768 samples: lmax 3 1253 -> 935 us, lmax 2 444 -> 327; 4096 samples
-// 196 -> 131 and 80 -> 69; "uvw" 32 x 32 -> 32, lmax 2, 32768 samples 1280 -> 900 us, 4096 235 -> 155.  Tables walked at run time
+// ones of 32 cycles per product and wavefront).  128 channels, 32768 samples: lmax 3 1253 -> 855 us, lmax 2 444 -> 318; 4096 samples
+// 196 -> 130 and 80 -> 60; "uvw" 32 x 32 -> 32, lmax 2, 32768 samples 1280 -> 855 us, 4096 235 -> 162.  With all sums of one sign, 32 products
+// each: lmax 3 5.4e-7 in 935 us, 64: 7.2e-7.  Tables walked at run time
 // instead of generated: 1390; one wavefront per l with "uvw": 1300.
 //
 // Values: as in uv_mix.hip; where a workgroup sees an element that is not to be split, or a sum that is not finite, it forms
@@ -255,6 +256,8 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
 
       float* out = a.slots + ((int64_t)range * a.n_slots + J.slot) * a.slot_elems;
       bool first = true;
+      // The matrix instruction rounds downwards: sums turn their sign from one to the next, of a job and over the workgroups and ranges.
+      float sign = (range + wg) & 1 ? -1.f : 1.f;
       int s = next_step(s_begin - 1);
       do {
         // a window: a few steps of the job
@@ -291,7 +294,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
                 Mix m{yl + (LV ? (wave * LN + i) * kStep : ybuf * YN) + 8 * q, raw, floatx8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
                 PATH::template mix<R>(m);
                 UvsParts<8> part;
-                split(m.v, part);
+                split(sign * m.v, part);
                 __builtin_amdgcn_sched_barrier(0);
                 if (i == SETS - 1) {
                   if (!LV && R == 0 && more) load_y(sn);
@@ -341,7 +344,8 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
         if (__any(redo) && lane == 0) atomicOr(&redo_all, 1u);
         redo = 0;
         __syncthreads();
-        if (redo_all) {                                  // fp32 matrix instructions, operands from memory
+        const bool again = redo_all;
+        if (again) {                                     // fp32 matrix instructions, operands from memory
           clear();
           int sp = s_window;
           for (int k = 0; k < STEPS && sp < s_end; ++k, sp = next_step(sp)) {
@@ -376,6 +380,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
         // element e of a tile: mixed channel 8 (e / 4) + 4 q + e % 4 of the wavefront's 32, plain channel r of the tile's
         // A slot is [mixed channel][l][plain channel] whichever side is mixed: whole lines here, turned by the reduction.
         const int r_now = opaque(r), q_now = opaque(q);
+        const float turn = again ? 1.f : sign;
 #pragma unroll
         for (int i = 0; i < SETS; ++i) {
           const int l = LV ? wave * LN + i : 0;
@@ -389,13 +394,14 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
                 const int mc = m0 + 8 * (e >> 2) + 4 * q_now + (e & 3);
                 if (mc < C) {
                   float* at = out + (mc * a.L + l) * C + c;
-                  *at = first ? acc[i][tb][e] : *at + acc[i][tb][e];
+                  *at = first ? turn * acc[i][tb][e] : *at + turn * acc[i][tb][e];
                 }
               }
             }
           }
         }
         first = false;
+        sign = -sign;
       } while (s < s_end);
     });
   }
@@ -485,10 +491,10 @@ int uvg_plan(const cgtp_uvg_args* a, UvgPlan* p) {
   d.C = a->c;
   const int64_t steps = (a->n_rows + kStep - 1) / kStep;
   // Sums as short as keep the errors at those of the fp32 kernel, whose chunks shrink with the batch and with the table (128
-  // channels, relative to 64 bits: lmax 2, 8192 samples 3.6e-7 with 32 products, 2.6e-7 with 12, fp32 3.1e-7; lmax 3, 32768 samples
-  // 5.4e-7 and 6.7e-7, 4096 3.4e-7 and 3.5e-7; with channels on y 3.6e-7 and 5.7e-7).  Adding a sum to its slot takes as long as several
-  // products: lmax 3, 32768 samples 935 us with 32, 1040 with 24, 870 with 64 (7.2e-7).
-  d.window = lv || e->p > 11 || a->n_rows >= 16384 ? 32 : 12;
+  // channels, relative to 64 bits: lmax 3, 32768 samples 4.6e-7 with 64 products, 7.0e-7 with 256, fp32 6.7e-7; lmax 2, 32768
+  // samples 4.5e-7 and 5.8e-7, 8192 samples 3.1e-7 with 32 and fp32; with channels on y 4.5e-7 and 5.8e-7).  Adding a sum to its
+  // slot takes as long as several products: lmax 3, 32768 samples 940 us with 32, 855 with 64, 797 with 256.
+  d.window = lv || e->p > 11 || a->n_rows >= 16384 ? 64 : 24;
   d.n_ranges = a->n_ranges;
   d.n_wgs = a->n_wgs;
   d.n_slots = a->n_slots;

@@ -220,10 +220,10 @@ class _GradWWalk:
 def _split_grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Optional[Tensor]:
     """:func:`grad_w` in fp32 on the half-precision matrix cores (``cgtp_uvg_apply``), or None where the fp32 matrix
     instructions serve: tables that are not compiled in as they are, different numbers of channels, and where they are
-    quicker or more precise.  Without channels on ``y`` that is up to 64 channels (lmax 3, 64 channels, 32768 samples 405 against
-    545 us, but errors of 5.3e-7 against 4.9e-7), lmax 1 (4000 samples, 128 channels: 38 us against 28) and small batches (lmax 3, 1000 samples,
-    128 channels 77 us against 67; below 4096 samples errors of 2.7e-7 against 2.5e-7); with channels, below 24 of them (16: 128 us against
-    110; 20: 417 and 405) and small batches (lmax 2, 1000 samples 107 us against 77; lmax 1, 2100 samples 50 and 44)."""
+    quicker or more precise.  Without channels on ``y`` that is up to 64 channels (8192 samples, lmax 3: 91 us against 148, but
+    errors of 3.7e-7 against 2.8e-7), lmax 1 (4000 samples, 128 channels: 38 us against 28) and small batches (lmax 3, 1000
+    samples, 128 channels 77 us against 67; up to 4096 samples equal errors); with channels, below 24 of them (16: 128 us against 110; 20: 417 and 405) and
+    small batches (lmax 2, 1000 samples 107 us against 77; lmax 1, 2100 samples 50 and 44)."""
     if isinstance(tp_info, CooTable) or x.dtype != torch.float32 or x.shape[0] == 0 or x.shape[2] != g.shape[2]:
         return None
     cfg = kernels.uv_config_of(tp_info)
@@ -231,7 +231,7 @@ def _split_grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Optional[Tensor]:
         return None
     (n, _, c), cy = x.shape, y.shape[2] if y.ndim == 3 else 0
     coo = _coo(tp_info)
-    if (min(c, cy) < 24 or n < (2048 if coo.P > 4 else 8192)) if cy else (c <= 64 or n < (2048 if coo.P <= 11 else 4096)):
+    if (min(c, cy) < 24 or n < (2048 if coo.P > 4 else 8192)) if cy else (c <= 64 or n < (2048 if coo.P <= 11 else 5000)):
         return None
     steps, n_wgs = -(-n // 16), 64                       # of a range: 32 compute units, two wavefronts per SIMD
     n_ranges = 8 * max(1, steps // 1024)
