@@ -468,6 +468,7 @@ class _MixTable:
         self.longest = max(map(len, self.steps))
         # the numbers of groups to choose from, with the most steps of a group
         self.choices = {g: self.dealt(g)[1] for g in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, len(self.tasks)) if g <= len(self.tasks)}
+        self.costs = [(g, most + 2) for g, most in self.choices.items() if most <= _MIX_STEPS]
 
     def dealt(self, n_groups: int):
         """The tasks in ``n_groups`` groups: the longest first, each to the group with the fewest steps so far."""
@@ -482,8 +483,12 @@ class _MixTable:
         """Groups (workgroups a block of samples is cut into): what lets whole rounds of two workgroups per compute unit end
         soonest, a workgroup costing its steps and about two more to start."""
         blocks = -(-n * self.rows_per_task // 256) * column_blocks
-        fits = [(-(-blocks * g // 512) * (most + 2), g) for g, most in self.choices.items() if most <= _MIX_STEPS]
-        return min(fits)[1]
+        least, best = None, 0
+        for g, cost in self.costs:
+            time = -(-blocks * g // 512) * cost
+            if least is None or time < least:
+                least, best = time, g
+        return best
 
 
 _MIX_STEPS = 64
@@ -510,6 +515,7 @@ class _MixWalk:
             self.max_steps[n_groups] = most
             end += parts[-2].size + parts[-1].size
         self.words = torch.from_numpy(np.concatenate(parts)).to(device)
+        self.address = {g: tuple(self.words.data_ptr() + v for v in at) for g, at in self.at.items()}
 
 
 def _mix_table(table, transposed: bool) -> _MixTable:
@@ -546,13 +552,14 @@ def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor
     walk = kernels.cached(_anchor(table), ("uvl_walk", transposed, str(x.device)), lambda: _MixWalk(mix, x.device))
     packed = torch.empty(int(_lib.lib.cgtp_uvl_packed_bytes(mix.n_blocks, cx, cout)), dtype=torch.uint8, device=x.device)
     out = torch.empty((n, mix.n_out, cout), dtype=x.dtype, device=x.device)
-    steps, groups, tasks, blocks = (walk.words.data_ptr() + v for v in walk.at[n_groups])
+    steps, groups, tasks, blocks = walk.address[n_groups]
     a = _lib.UvlArgs(x.data_ptr(), packed.data_ptr(), w.data_ptr(), out.data_ptr(), steps, tasks, groups, blocks,
                      n, w.stride(0), w.stride(2 if transposed else 1), w.stride(1 if transposed else 2),
                      mix.n_blocks, n_groups, mix.rows_per_task, walk.max_steps[n_groups], dx, mix.n_out, cx, cout)
-    if _lib.lib.cgtp_uvl_validate(C.byref(a)) != 0:
+    status = _lib.lib.cgtp_uvl_apply(C.byref(a), _lib.stream_ptr(x.device))
+    if status in (2, 3):               # extents or an alignment it does not take: nothing was launched
         return None
-    _lib.check(_lib.lib.cgtp_uvl_apply(C.byref(a), _lib.stream_ptr(x.device)), "cgtp_uvl_apply")
+    _lib.check(status, "cgtp_uvl_apply")
     return out
 
 
