@@ -185,6 +185,12 @@ def _covered(plan: LinearPlan) -> bool:
     return end >= plan.out_size
 
 
+def _right_operand(w: Tensor) -> Tensor:
+    """A transposed right operand of a batched product.  In 16 bits it is laid out anew: the library's product of such a view
+    ends in a memory fault (gradient of the input of a bf16 layer, 256 channels)."""
+    return w.contiguous() if w.dtype in (torch.bfloat16, torch.float16) else w
+
+
 def _mix_raw(x: Tensor, w: Tensor, plan: LinearPlan, w_t: bool) -> Tensor:
     """``out[n, o0+j, :] += scale * x[n, i0+j, :] @ W[(n,) p]`` for every path; ``w_t``: use ``W^T``."""
     n, _, cin = x.shape
@@ -203,7 +209,7 @@ def _mix_raw(x: Tensor, w: Tensor, plan: LinearPlan, w_t: bool) -> Tensor:
             if alpha is None:                                          # rows with different scales: fold them in
                 wb, alpha = wb * _row_scales(grp, wb), 1.0
             if w_t:
-                wb = wb.transpose(1, 2)
+                wb = _right_operand(wb.transpose(1, 2))
             ot = os_.transpose(0, 1)                                   # (rows, N, cout), rows strided by D_out * cout
             torch.baddbmm(ot, xs.transpose(0, 1), wb, beta=beta, alpha=alpha, out=ot)
         else:
@@ -212,7 +218,7 @@ def _mix_raw(x: Tensor, w: Tensor, plan: LinearPlan, w_t: bool) -> Tensor:
             while at < grp.rows:
                 pw = grp.w_of_row[at]
                 k = next((j for j in range(at, grp.rows) if grp.w_of_row[j] != pw), grp.rows) - at
-                wp = w[:, pw].transpose(1, 2) if w_t else w[:, pw]
+                wp = _right_operand(w[:, pw].transpose(1, 2)) if w_t else w[:, pw]
                 k = next((j for j in range(at, at + k) if grp.scale_of_row[j] != grp.scale_of_row[at]), at + k) - at
                 dst = os_[:, at:at + k, :]
                 torch.baddbmm(dst, xs[:, at:at + k, :], wp, beta=beta, alpha=grp.scale_of_row[at], out=dst)
