@@ -26,8 +26,9 @@
 // each: lmax 3 5.4e-7 in 935 us, 64: 7.2e-7.  Tables walked at run time
 // instead of generated: 1390; one wavefront per l with "uvw": 1300.
 //
-// Values: as in uv_mix.hip; where a workgroup sees an element that is not to be split, or a sum that is not finite, it forms
-// those sums again with fp32 matrix instructions.
+// Values: as in uv_mix.hip; where a workgroup sees an element that is not to be split, a zero that may be what y left of g (paths
+// whose g is mixed), or a sum that is not finite, it forms those sums again with fp32 matrix instructions.  Looking at zeros costs
+// nothing where there are none and 2 to 8 % with every other element or sample zero.
 #include "uv_parts.h"
 
 #pragma clang fp contract(fast)
@@ -38,6 +39,7 @@ namespace {
 #include "generated/uv_split_gw_configs.inc"
 
 constexpr int kStep = 16;              // samples of a matrix instruction
+constexpr unsigned kLeastY = (127u - 30) << 24;        // 2^-30 as by_magnitude() has it
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx8 __attribute__((ext_vector_type(8)));
@@ -47,6 +49,9 @@ __device__ __forceinline__ int opaque(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+
+// Orders by magnitude, a zero as the largest.
+__device__ __forceinline__ unsigned by_magnitude(float v) { return (__builtin_bit_cast(unsigned, v) << 1) - 1u; }
 
 struct UvgDev {
   const float* x;
@@ -103,6 +108,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
   __shared__ u32x4 bl[2 * CHUNK];
   __shared__ __align__(16) float yl[LV ? YN * LW : 2 * YN];        // [2: step][row of y][sample], with LV [row][l][sample]
   __shared__ unsigned redo_all;
+  __shared__ unsigned least_y;                           // of the y so far, zeros aside; 2^-30 where none is below
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r = lane & 31, q = lane >> 5, C = a.C;
 
@@ -115,6 +121,8 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
   const bool makes = TB == NW || tid < TB * 64;
   const int pc = tid % (32 * TB), oct = tid / (32 * TB), pcol = min(pc, C - 1);
   u32x4* const plain_to = bl + (pc >> 5) * 64 + oct * 32 + (pc & 31);
+
+  if (tid == 0) least_y = kLeastY;                       // the first window's barrier is behind it
 
   for (int job = a.job_ptr[wg]; job < a.job_ptr[wg + 1]; ++job) {
     const cgtp_uvg_job J = a.jobs[job];
@@ -176,7 +184,8 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
           }
         }
       };
-      auto split = [&](const floatx8& v, UvsParts<8>& part) __attribute__((always_inline)) {
+      // `zeros` looks at a v with elements of next to nothing, zeros as a rule.
+      auto split = [&](const floatx8& v, UvsParts<8>& part, auto&& zeros) __attribute__((always_inline)) {
         float low = 1.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -184,18 +193,34 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
           part.pair(j, v0, v1);
           low = uvs_least(v0, v1, low);
         }
-        if (__any(low < 0x1p-110f)) {                    // a zero, as a rule
+        if (__any(low < 0x1p-110f)) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             const float e = v[j];
             redo |= uvs_asks(e) & kUvsPlain;
           }
+          zeros(v);
         }
+      };
+      // Coupled to g first, y may take a product below the smallest number where x would have kept it above.  A zero is that only
+      // next to a g and a y of a product below 2^-110 (a sum of terms in y cancels to no less than 2^-35 of them).
+      auto look_at_zero = [&](unsigned zero) __attribute__((always_inline)) {
+        if (!PATH::SWAPPED || !__any(zero)) return;
+        unsigned least = ~0u;
+#pragma unroll
+        for (int o = 0; o < NO; ++o)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float e = raw[o][j];
+            least = min(least, by_magnitude(__builtin_bit_cast(float, opaque(__builtin_bit_cast(int, e)))));
+          }
+        const float g = __builtin_bit_cast(float, least >> 1), y = __builtin_bit_cast(float, least_y >> 1);
+        redo |= zero && g * y < 0x1p-110f;               // no g but zeros: not a number, and not below
       };
       auto put_plain = [&](int buf) __attribute__((always_inline)) {
         if (!makes) return;
         UvsParts<8> part;
-        split(praw, part);
+        split(praw, part, [](const floatx8&) {});
 #pragma unroll
         for (int h = 0; h < 3; ++h)
           plain_to[buf * CHUNK + h * TB * 64] = u32x4{part.p[h][0], part.p[h][1], part.p[h][2], part.p[h][3]};
@@ -203,16 +228,22 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
       // The rows of y of a step.  Without channels i = (sample, row) and a step ahead; with them sample by sample, when the step
       // begins (it lasts several thousand cycles).
       float yreg[YWORDS];
+      auto note_y = [&](unsigned least) __attribute__((always_inline)) {       // read past the barrier behind it
+        if (PATH::SWAPPED && least < kLeastY) atomicMin(&least_y, least);
+      };
       auto load_y = [&](int s) __attribute__((always_inline)) {
         const int64_t n0 = (int64_t)s * kStep, last = min(a.n_rows - n0, (int64_t)kStep) * CFG::D2;
         if constexpr (LV) {
           const int per = a.L / 4, total = YN * per;
+          unsigned least = ~0u;
           for (int i = tid; i < total; i += THREADS) {
             const int e = i / per, l4 = i - e * per;
             const f32x4 v = *reinterpret_cast<const f32x4*>(a.y + (n0 * CFG::D2 + (e < last ? e : 0)) * a.L + l4 * 4);
 #pragma unroll
             for (int k = 0; k < 4; ++k) yl[(e % CFG::D2 * LW + l4 * 4 + k) * kStep + e / CFG::D2] = v[k];
+            least = min(min(least, by_magnitude(v[0])), min(by_magnitude(v[1]), min(by_magnitude(v[2]), by_magnitude(v[3]))));
           }
+          note_y(least);
         } else {
 #pragma unroll
           for (int k = 0; k < YWORDS; ++k) {
@@ -222,11 +253,14 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
         }
       };
       auto put_y = [&](int buf) __attribute__((always_inline)) {
+        unsigned least = ~0u;
 #pragma unroll
         for (int k = 0; k < YWORDS; ++k) {
           const int i = opaque(k * THREADS + tid);
           if (i < YN) yl[buf * YN + i % CFG::D2 * kStep + i / CFG::D2] = yreg[k];
+          if (i < YN) least = min(least, by_magnitude(yreg[k]));
         }
+        note_y(least);
       };
       struct Mix {
         const float* ys;
@@ -288,13 +322,18 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
                 for (int h = 0; h < 3; ++h) f[h] = __builtin_bit_cast(bf16x8, frag[(h * TB + tb) * 64]);
               };
               if (LV) fragments(0);
+              unsigned zero = 0;                         // a mixed element is zero
 #pragma unroll
               for (int i = 0; i < SETS; ++i) {
                 if (LV && wave * LN + i >= a.L) continue;
                 Mix m{yl + (LV ? (wave * LN + i) * kStep : ybuf * YN) + 8 * q, raw, floatx8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
                 PATH::template mix<R>(m);
                 UvsParts<8> part;
-                split(sign * m.v, part);
+                split(sign * m.v, part, [&](const floatx8& v) __attribute__((always_inline)) {
+#pragma unroll
+                  for (int j = 0; j < 8; ++j) zero |= v[j] == 0.f;
+                });
+                if (!LV) look_at_zero(zero);
                 __builtin_amdgcn_sched_barrier(0);
                 if (i == SETS - 1) {
                   if (!LV && R == 0 && more) load_y(sn);
@@ -310,6 +349,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
                   }
                 }
               }
+              if (LV) look_at_zero(zero);
               if (LV && R == NR - 1 && more) load_mixed(sn);
               __builtin_amdgcn_sched_barrier(0);
               // the plain row of the next product, and the request for the one after

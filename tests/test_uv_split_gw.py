@@ -120,6 +120,30 @@ def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponents, c
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cy", [0, 24])
+@pytest.mark.parametrize("scaled", ["all", "some samples", "some channels"])
+def test_products_that_only_vanish_in_one_order(device, monkeypatch, cy, scaled):
+    """y and grad_out whose product is below the smallest number, next to an x that makes up for it: zero where grad_out is
+    mixed with y first, and no small matter where y meets x first, as in the fp32 kernel."""
+    ops = _operands(2, 24 if cy else 80, cy, 2100, 9)
+    at = {"all": slice(None), "some samples": slice(700, 703), "some channels": (slice(None), slice(None), slice(3, 5))}[scaled]
+    for t, e in zip(ops, (100, -80, -80)):
+        if t.ndim == 3 or scaled != "some channels":
+            t[at] *= 2.0 ** e
+        else:
+            t *= 2.0 ** e
+    if scaled == "some samples":       # the others are zero: what the result is made of is theirs alone
+        for t in ops:
+            t[:700], t[703:] = 0.0, 0.0
+    new, old, ref = _routes(device, monkeypatch, 2, ops)
+    assert float(ref.abs().max()) > 2.0 ** -70
+    for p in range(ref.shape[0]):
+        e_new, e_old = (float((t[p].double() - ref[p]).norm() / ref[p].norm()) for t in (new, old))
+        print(f"cy={cy} {scaled} path {p}: split {e_new:.2e} fp32 {e_old:.2e}")
+        assert e_new <= 2.0 * e_old + 3e-8
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cy", [0, 32])
 def test_recorded_in_a_graph(device, cy):
     from equitorch_amd.nn import SO3Linear
