@@ -29,10 +29,10 @@ class CooTable:
     instead of a ``TensorProductInfo`` — the tables of the channel-mixing layers, whose second operand is the scalar 1.
     ``anchor``: a tensor that lives as long as the table (cache key); ``fallback(x, y, w)``: a differentiable
     evaluation of the same product for gradients of higher order.  ``mixing``: the second operand is the scalar 1 in every
-    sample (channel mixing)."""
+    sample (channel mixing).  ``algebra``: the fallback is tensor algebra, which takes gradients that are batched or traced."""
 
-    def __init__(self, coo, anchor: Tensor, fallback, mixing: bool = False):
-        self.coo, self.anchor, self.fallback, self.mixing = coo, anchor, fallback, mixing
+    def __init__(self, coo, anchor: Tensor, fallback, mixing: bool = False, algebra: bool = False):
+        self.coo, self.anchor, self.fallback, self.mixing, self.algebra = coo, anchor, fallback, mixing, algebra
 
 
 def _anchor(table) -> Tensor:
@@ -522,13 +522,20 @@ def _mix_table(table, transposed: bool) -> _MixTable:
     return kernels.cached(_anchor(table), ("uvl_table", transposed), lambda: _MixTable(table.coo, transposed))
 
 
+def _observed(*tensors: Tensor) -> bool:
+    """Whether something looks at the operations on these tensors one by one (a transform, forward mode, tracing, a dispatch
+    mode, a tensor subclass, autocast): tensor algebra serves it, an autograd function over raw pointers does not."""
+    functorch = torch._C._functorch
+    return (functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled("cuda")
+            or any(type(t) not in (Tensor, torch.nn.Parameter) or functorch.is_legacy_batchedtensor(t) for t in tensors))
+
+
 def mix_fits(x: Tensor, w: Tensor, table) -> bool:
-    """Whether channel mixing with this table runs on the half-precision matrix cores in both directions.  The calls it
-    takes from the library route, which is plain tensor algebra, leave the transforms of that to it: vmap, forward mode and
-    tracing see no autograd function there."""
+    """Whether channel mixing with this table, too large for the fp32 kernels, runs on the half-precision matrix cores in
+    both directions."""
     c = table.coo
-    if (torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
-            or torch.jit.is_tracing()):
+    if _observed(x, w):
         return False
     return (x.dtype == w.dtype == torch.float32 and x.shape[0] > 0 and x.data_ptr() % 16 == 0 and w.shape[1] % 4 == 0
             and w.shape[2] % 4 == 0 and w.shape[0] == c.P and tuple(x.shape[1:]) == (c.D1, w.shape[1])
@@ -597,11 +604,12 @@ class _U1vNative(Function):
         x, y, w = ctx.saved_tensors
         need = ctx.needs_input_grad[:3]
         tp_info = ctx.tp_info
-        if torch.is_grad_enabled():       # higher-order derivative: the differentiable route throughout
+        higher = torch.is_grad_enabled()  # higher-order derivative: the differentiable route throughout
+        if higher or (isinstance(tp_info, CooTable) and tp_info.algebra and _observed(g)):
             with torch.enable_grad():
                 out = tp_info.fallback(x, y, w) if isinstance(tp_info, CooTable) else _uv_gemm.u1v(x, y, w, tp_info)
                 wanted = [t for t, n in zip((x, y, w), need) if n]
-                got = iter(torch.autograd.grad(out, wanted, g, create_graph=True, allow_unused=True))
+                got = iter(torch.autograd.grad(out, wanted, g, create_graph=higher, allow_unused=True))
             return tuple(next(got) if n else None for n in need) + (None,)
         c = _coo(tp_info)
         p, u, wc = w.shape

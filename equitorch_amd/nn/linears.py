@@ -290,14 +290,17 @@ class SO2Linear(nn.Module):
                 x3 = input.reshape(-1, *input.shape[-2:]).contiguous()
                 if not plan.paths:
                     return G.no_paths(x3, weight, plan).reshape(*input.shape[:-2], plan.out_size, weight.shape[-1])
-                out = G._table_driven_path(x3, weight.contiguous(), plan, self.irreps_in.dim, anchor)
-                if out is None and x3.shape[0] > 0:
-                    out = G._adapted_path(x3, weight.contiguous(), plan, self.irreps_in.dim, anchor)
-                if out is not None:
-                    return out.reshape(*input.shape[:-2], plan.out_size, out.shape[-1])
                 # one GEMM per order |m| over the components of that order side by side
                 from .functional._so2_gemm import so2_linear_uv_shared
-                return so2_linear_uv_shared(input, weight, self.info_forward, self.irreps_in.dim, self.num_weights)
+
+                def algebra(x, w, info=self.info_forward, in_size=self.irreps_in.dim, n_weights=self.num_weights):
+                    return so2_linear_uv_shared(x, w, info, in_size, n_weights)
+                out = G._table_driven_path(x3, weight.contiguous(), plan, self.irreps_in.dim, anchor, algebra)
+                if out is None and x3.shape[0] > 0:
+                    out = G._adapted_path(x3, weight.contiguous(), plan, self.irreps_in.dim, anchor, algebra)
+                if out is not None:
+                    return out.reshape(*input.shape[:-2], plan.out_size, out.shape[-1])
+                return algebra(input, weight)
             # per-sample weights: every table entry is a (C_in, C_out) GEMM on one component, batched over samples
             from .functional import _irreps_gemm as G
             plan = G.plan_of_product_info(self.info_forward, self.irreps_in.dim, self.num_weights)

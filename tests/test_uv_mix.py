@@ -273,3 +273,38 @@ def test_transforms_of_the_library_route_stay(device):
     assert float((tangent - want).detach().norm()) <= 2e-6 * float(want.norm())
     batched = torch.func.vmap(lambda v: mod(v))(x.view(2, 10, *x.shape[1:]))
     assert float((batched.flatten(0, 1) - out).detach().norm()) <= 2e-6 * float(out.detach().norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["batched gradients", "vmap of the gradient", "second order", "operators seen", "autocast"])
+def test_what_tensor_algebra_takes_is_taken(device, monkeypatch, what):
+    """A layer that was tensor algebra, in all that sees its operations one by one: as on the library route."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from equitorch_amd.nn.functional import _uv_native as N
+    x, t = (v.to(device) for v in _operands("so2", 6, 64, 64, 6, 11))
+    gs = torch.randn(3, *t.shape, generator=torch.Generator().manual_seed(12)).to(device)
+
+    def results():
+        mod = _module("so2", 6, 64, 64, device)
+        leaf = x.clone().requires_grad_(True)
+        if what == "batched gradients":
+            return torch.autograd.grad(mod(leaf), [leaf, mod.weight], gs, is_grads_batched=True)
+        if what == "vmap of the gradient":
+            out = mod(leaf)
+            return torch.func.vmap(lambda g: torch.autograd.grad(out, [leaf, mod.weight], g, retain_graph=True))(gs)
+        if what == "second order":
+            first = torch.autograd.grad(mod(leaf), [leaf, mod.weight], t, create_graph=True)
+            return torch.autograd.grad(sum((f * f).sum() for f in first), [leaf, mod.weight])
+        if what == "operators seen":
+            with FlopCounterMode(display=False) as count:
+                out = mod(x)
+            assert count.get_total_flops() > 0
+            return [out]
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return [mod(x)]
+    got = results()
+    monkeypatch.setattr(N, "mix_fits", lambda *args: False)
+    for a, b in zip(got, results()):
+        assert a.dtype == b.dtype
+        assert float((a.double() - b.double()).detach().norm()) <= 4e-6 * float(b.detach().double().norm())
