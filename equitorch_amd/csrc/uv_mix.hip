@@ -18,7 +18,7 @@
 // 64 -> 64, lmax 2, 65536 samples 126 -> 75, 128 -> 128, lmax 3, 32768 samples 308 -> 170.  One workgroup per pair of rows, 325 us: a
 // third of its time went into starting; half lines of x from memory straight into the operands, 300; three wavefronts per
 // SIMD (spills), eight in a workgroup, matrix and vector instructions in turn by hand: no change.  Errors of the results
-// against 64 bits: 0.3e-7 to 3.0e-7, of fp32 matrix instructions 0.5e-7 to 3.7e-7.
+// against 64 bits, rows of 1 to 96 units: 0.4e-7 to 2.3e-7, of fp32 matrix instructions 0.9e-7 to 8.0e-7.
 //
 // Values: elements that are not finite or overflow as parts show in the results, and elements below 2^-110 (but not zero; their
 // last part could be below the smallest subnormal) are looked for; a wavefront that sees either forms its results
@@ -252,13 +252,21 @@ __global__ void __launch_bounds__(256, NT * RW == 4 ? 2 : 3) uvl_kernel(const Uv
           bf16x8 f[3];
 #pragma unroll
           for (int h = 0; h < 3; ++h) f[h] = __builtin_bit_cast(bf16x8, frag[(h * TW + t) * 64]);
+          // A unit's six products are summed by themselves: the matrix instruction rounds downwards, six times a unit at the size
+          // of the row's sum where they are added to it (12 units of 32 channels 3.6e-7, by themselves 1.0e-7; 512 of them
+          // 2.1e-6 and 4.3e-7; fp32 instructions 4.3e-7 for 12; SO2Linear, lmax 4, 64 channels 1152 -> 1161 us a step).
+          floatx4 sum[NT];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) sum[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int c = 0; c < 6; ++c) {              // the small products first
             constexpr int ha[6] = {2, 1, 0, 1, 0, 0}, hb[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
             for (int i = 0; i < NT; ++i)
-              acc[w][t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ha[c]], uvs_frag(part[i].p[hb[c]]), acc[w][t][i], 0, 0, 0);
+              sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ha[c]], uvs_frag(part[i].p[hb[c]]), sum[i], 0, 0, 0);
           }
+#pragma unroll
+          for (int i = 0; i < NT; ++i) acc[w][t][i] += sum[i];
         }
       }
     }

@@ -79,6 +79,8 @@ def _module(kind, l, cin, cout, device):
     torch.manual_seed(stable_seed("mix", kind, l, cin, cout))
     if kind == "so2":
         return enn.SO2Linear(SH[l], SH[l], cin, cout, feature_mode="uv").to(device)
+    if kind == "copies":               # a result's row of l inputs, and an input's of l results; the others are many
+        return enn.IrrepsLinear(f"{l}x0e+8o+9o", f"8o+{l}x0e+9o", cin, cout).to(device)
     return enn.IrrepsLinear(SH[l], SH[l] if kind == "lin" else "2e+0e+1o+0e", cin, cout).to(device)
 
 
@@ -88,12 +90,14 @@ def _run(mod, x, g):
     return [t.detach() for t in (out, torch.autograd.grad(out, [x], g)[0])]
 
 
-def _routes(monkeypatch, kind, l, cin, cout, x, g, device, scale=1.0):
+def _routes(monkeypatch, kind, l, cin, cout, x, g, device, scale=1.0, sign=False):
     """Results of the split kernels, of the route without them and of float64."""
     from equitorch_amd.nn.functional import _uv_native as N
     mod = _module(kind, l, cin, cout, device)
     with torch.no_grad():
         mod.weight.mul_(scale)
+        if sign:
+            mod.weight.abs_()
     taken, split = [], N._mix_split
 
     def spy(*args):
@@ -138,6 +142,25 @@ def test_no_less_precise_than_fp32_matrix_instructions(device, monkeypatch, kind
         print(f"{name} {kind} lmax={l} {cin}->{cout} n={n} {values}: split {err(a):.2e} fp32 {err(b):.2e}")
         # one sample's rounding errors are a handful of draws: a factor of two between two orders of summation
         assert err(a) <= (1.1 if n >= 300 else 2.0) * err(b) + 3e-8, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n", [("so2", 6, 48, 48, 700), ("so2", 5, 64, 96, 500), ("lin", 4, 256, 64, 900), ("so2", 6, 256, 32, 300),
+                                               ("copies", 4, 64, 36, 400), ("copies", 2, 128, 128, 600)])
+@pytest.mark.parametrize("sign", [False, True])
+def test_long_rows_are_no_less_precise_than_the_library(device, monkeypatch, kind, l, cin, cout, n, sign):
+    """Rows past the fp32 kernels' sizes were products of the library, which sums in blocks; ``sign``: inputs and weights of one
+    sign, where a rounding to one side does not average out.  Both are random errors of a few hundred sums each: a tenth."""
+    mod = _module(kind, l, cin, cout, "cpu")
+    gen = torch.Generator().manual_seed(stable_seed("long", kind, l, cin, cout))
+    x, g = torch.randn(n, mod.irreps_in.dim, cin, generator=gen), torch.randn(n, mod.irreps_out.dim, cout, generator=gen)
+    if sign:
+        x, g = x.abs(), g.abs()
+    new, old, ref = _routes(monkeypatch, kind, l, cin, cout, x, g, device, sign=sign)
+    for name, a, b, want in zip(("out", "grad x"), new, old, ref):
+        e_new, e_old = (float((t.double() - want).norm() / want.norm()) for t in (a, b))
+        print(f"{name} {kind} {l} {cin}->{cout} sign={sign}: split {e_new:.2e} library {e_old:.2e}")
+        assert e_new <= 1.1 * e_old, name
 
 
 @pytest.mark.gpu
