@@ -393,12 +393,13 @@ def _ones_column(n: int, dtype, device) -> Tensor:
     return buf[:n]
 
 
-def _table_driven_path(x: Tensor, weight: Tensor, plan: LinearPlan, in_size: int, anchor: Tensor, algebra=None):
+def _table_driven_path(x: Tensor, weight: Tensor, plan: LinearPlan, in_size: int, anchor: Tensor, algebra=None,
+                       widened: bool = False):
     """fp32 with a shared weight: the layer as a fully connected product with the scalar 1 on the table-driven
     matrix-core kernels (``cgtp_uvt_*``: forward, grad input and grad weight in one launch each, rows read and written
     in place): every path of the plan becomes ``k`` table entries (output row, input row, 0, weight, scale).  None
     when the extents do not fit those kernels.  ``algebra(x, weight)``: the layer as tensor algebra, where it has one; tables
-    too large for the fp32 kernels take it for gradients of higher order and under transforms."""
+    too large for the fp32 kernels go to it for gradients of higher order and under transforms.  ``widened``: from 16 bits."""
     import numpy as np
 
     from ..._tables import TpCoo
@@ -422,7 +423,7 @@ def _table_driven_path(x: Tensor, weight: Tensor, plan: LinearPlan, in_size: int
         return None
     ones = _ones_column(x.shape[0], x.dtype, x.device)
     if not _uv_native.u1v_supported(x, ones, weight, table):
-        if not _uv_native.mix_fits(x, weight, table):
+        if not _uv_native.mix_fits(x, weight, table, algebra is not None, widened):
             return None
         if algebra is not None:
             table = _uv_native.CooTable(table.coo, anchor, lambda xx, yy, ww: algebra(xx, ww) * yy[:, :, None], mixing=True,
@@ -471,7 +472,7 @@ def _adapted_path(x: Tensor, weight: Tensor, plan: LinearPlan, in_size: int, anc
         xa, wa = pad(xa, (0, -cin % 4)), pad(wa, (0, -cout % 4, 0, -cin % 4))
     if xa is x:
         return None
-    out = _table_driven_path(xa, wa, plan, in_size, anchor, algebra) if wa.ndim == 3 else _streaming_path(xa, wa, plan, in_size, anchor)
+    out = _table_driven_path(xa, wa, plan, in_size, anchor, algebra, widened=xa.dtype != dtype) if wa.ndim == 3 else _streaming_path(xa, wa, plan, in_size, anchor)
     if out is None:
         return None
     if out.shape[-1] != cout:

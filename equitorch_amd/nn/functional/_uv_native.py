@@ -491,7 +491,7 @@ class _MixTable:
         return best
 
 
-_MIX_STEPS = 64
+_MIX_STEPS = 64          # of a group, one lane each
 
 
 class _MixWalk:
@@ -531,16 +531,31 @@ def _observed(*tensors: Tensor) -> bool:
             or any(type(t) not in (Tensor, torch.nn.Parameter) or functorch.is_legacy_batchedtensor(t) for t in tensors))
 
 
-def mix_fits(x: Tensor, w: Tensor, table) -> bool:
+def mix_fits(x: Tensor, w: Tensor, table, one_product: bool, widened: bool) -> bool:
     """Whether channel mixing with this table, too large for the fp32 kernels, runs on the half-precision matrix cores in
-    both directions."""
+    both directions.  ``one_product``: the library has all entries of a row in one product (SO(2) layers, forward and gradients of
+    50 to 16000 samples, 48 to 256 channels 0.1 to 0.8 of its time), else one for each entry, which wins where the launches do
+    not count: past 1.5e9 multiplications (lmax 6, 96 channels, 16000 samples 692 us against 677, lmax 3, 64 -> 256 453 against 353,
+    below 0.4 to 0.9) and past 256 channels (lmax 6, 384, 300 samples 314 against 250).  ``widened`` from 16 bits, in which the library
+    is quicker: SO(2) layers up to 1.7e10 multiplications (lmax 6, 64 channels, 4000 samples 399 us against 1387, lmax 5, 256, 1000 897
+    against 1384; past it lmax 4, 192, 4000 1545 against 1225, lmax 6, 256, 4000 4598 against 2543).
+    Long rows stay on the library, which sums in blocks and entries of their own.  Relative to 64 bits, operands of one sign,
+    kernel and library: one product of 12 entries of 256 channels (96 units of 32) 1.4e-7 and 2.0e-7; entries of their own, one of 384
+    channels 0.6e-7 and 3.1e-7, 3 of 640 1.0e-7 and 0.8e-7, 24 of 128 1.5e-7 and 0.9e-7."""
     c = table.coo
     if _observed(x, w):
         return False
+    if x.shape[0] * len(c.p) * w.shape[1] * w.shape[2] > {(False, False): 1.5e9, (False, True): 0, (True, True): 1.7e10}.get(
+            (one_product, widened), float("inf")):
+        return False
+
+    def short(transposed: bool) -> bool:
+        steps = _mix_table(table, transposed).longest
+        return steps <= _MIX_STEPS and steps * -(-w.shape[1 + transposed] // 32) <= (96 if one_product else 8)
     return (x.dtype == w.dtype == torch.float32 and x.shape[0] > 0 and x.data_ptr() % 16 == 0 and w.shape[1] % 4 == 0
             and w.shape[2] % 4 == 0 and w.shape[0] == c.P and tuple(x.shape[1:]) == (c.D1, w.shape[1])
             and max(c.D1 * w.shape[1], c.DO * w.shape[2]) <= 1 << 22
-            and all(_mix_table(table, t).longest <= _MIX_STEPS for t in (False, True)))
+            and short(False) and short(True))
 
 
 def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor]:

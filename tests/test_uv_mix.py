@@ -164,6 +164,18 @@ def test_long_rows_are_no_less_precise_than_the_library(device, monkeypatch, kin
 
 
 @pytest.mark.gpu
+def test_what_stays_on_the_library(device, monkeypatch):
+    """Rows whose sums the library forms more precisely, and products it forms as quickly."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    monkeypatch.setattr(N, "_mix_split", lambda *args: pytest.fail("a kernel was called"))
+    for kind, l, c, n in (("copies", 24, 128, 70), ("copies", 60, 256, 70), ("so2", 6, 288, 70), ("lin", 4, 320, 70), ("lin", 4, 128, 4000)):
+        mod = _module(kind, l, c, c, device)
+        x = torch.randn(n, mod.irreps_in.dim, c, generator=torch.Generator().manual_seed(1)).to(device)
+        want = _module(kind, l, c, c, device).double()(x.double())
+        assert float((mod(x).double() - want).detach().norm()) <= 1e-6 * float(want.detach().norm())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("where,value", [("x", float("inf")), ("x", float("nan")), ("g", float("-inf")), ("x", 3.4e38), ("w", float("inf"))])
 @pytest.mark.parametrize("kind", ["lin", "so2"])
 def test_values_that_are_not_finite_stay_where_they_couple(device, monkeypatch, kind, where, value):
