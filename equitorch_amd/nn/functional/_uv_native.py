@@ -188,7 +188,14 @@ class _GradWWalk:
         parts = [np.array(flat, dtype=np.uint32).view(np.int32), job_ptr.astype(np.int32), np.array(slot_ptr, dtype=np.int32)]
         self.words = torch.from_numpy(np.concatenate([p.ravel() for p in parts])).to(device)
         self.at = [4 * sum(p.size for p in parts[:k]) for k in range(len(parts))]
-        self.n_slots = len(slots)
+        self.n_slots, self.n_paths = len(slots), coo.P
+
+    def ranges(self, steps: int) -> int:
+        """Ranges the steps are cut into, each with slots of its own: 128 steps or more in each, and no more than the fp32 kernel has
+        partial results (128 of every path) where the eight of the XCDs leave room for it: 155 MB for "uvw", lmax 2, 32 channels,
+        past 32768 samples.  (With ranges of 128 steps throughout 1.24 GB at 262144 samples, 5946 us against 6823; lmax 1 1478
+        against 1424, without channels on y the same; fp32 instructions 1310 at 32768 samples, here 820.)"""
+        return 8 * max(1, min(steps // 1024, 16 * self.n_paths // self.n_slots))
 
     @classmethod
     def deal(cls, cost, n_wgs: int):
@@ -234,8 +241,8 @@ def _split_grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Optional[Tensor]:
     if (min(c, cy) < 24 or n < (2048 if coo.P > 4 else 8192)) if cy else (c <= 64 or n < (2048 if coo.P <= 11 else 5000)):
         return None
     steps, n_wgs = -(-n // 16), 64                       # of a range: 32 compute units, two wavefronts per SIMD
-    n_ranges = 8 * max(1, steps // 1024)
     walk = kernels.cached(_anchor(tp_info), ("uvg_walk", n_wgs, str(x.device)), lambda: _GradWWalk(coo, n_wgs, x.device))
+    n_ranges = walk.ranges(steps)
     gw = torch.empty((coo.P, c * max(cy, 1), c), dtype=x.dtype, device=x.device)
     jobs, job_ptr, slot_ptr = (walk.words.data_ptr() + v for v in walk.at)
     a = _lib.UvgArgs(x.data_ptr(), y.data_ptr(), g.data_ptr(), gw.data_ptr(), 256, jobs, job_ptr, slot_ptr, n, int(cfg), n_ranges, n_wgs,

@@ -47,6 +47,18 @@ def test_the_tables_name_every_job_once():
         assert (np.diff(slot_ptr) > 0).all()
 
 
+@pytest.mark.parametrize("l", [1, 2, 3])
+def test_the_workspace_does_not_grow_with_the_batch(l):
+    """As many slots as the fp32 kernel has partial results, or eight ranges' where that is more."""
+    from equitorch_amd.nn import SO3Linear
+    from equitorch_amd.nn.functional import _uv_native as N
+    coo = N._coo(SO3Linear(SH[l], SH[l], SH[l], 4, 4, internal_weights=False, feature_mode="uv").tp_info_forward)
+    walk = N._GradWWalk(coo, 64, "cpu")
+    for n in (2048, 8192, 32768, 1 << 17, 1 << 20, 1 << 26):
+        ranges = walk.ranges(-(-n // 16))
+        assert ranges % 8 == 0 and 8 <= ranges and ranges * walk.n_slots <= max(128 * coo.P, 8 * walk.n_slots)
+
+
 # ---- on the GPU ------------------------------------------------------------------------------------------------------
 def _operands(l, c, cy, n, seed):
     d, gen = (l + 1) ** 2, torch.Generator().manual_seed(seed)
@@ -117,6 +129,27 @@ def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponents, c
         e_new, e_old = (float((t.double() - ref).norm() / ref.norm()) for t in (new, old))
         print(f"{exponents} cy={cy}: split {e_new:.2e} fp32 {e_old:.2e}")
         assert e_new <= 1.5 * e_old + 3e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("l,c,cy", [(2, 32, 32), (3, 96, 0)])
+def test_a_large_batch_in_little_memory(device, monkeypatch, l, c, cy):
+    from equitorch_amd.nn import SO3Linear
+    from equitorch_amd.nn.functional import _uv_native as N
+    info = SO3Linear(SH[l], SH[l], SH[l], 4, 4, internal_weights=False, feature_mode="uv").to(device).tp_info_forward
+    x, y, g = (t.to(device) for t in _operands(l, c, cy, 150001, 11))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    new = N._split_grad_w(x, y, g, info)
+    used = torch.cuda.max_memory_allocated() - before
+    assert used <= 130 * new.numel() * 4 + (1 << 22)        # 128 partial results, the gradient, the tables
+    monkeypatch.setattr(N, "_split_grad_w", lambda *args: None)
+    old = N.grad_w(x, y, g, info)
+    ref = N.grad_w(x.double(), y.double(), g.double(), info)
+    e_new, e_old = (float((t.double() - ref).norm() / ref.norm()) for t in (new, old))
+    print(f"lmax={l} c={c} cy={cy}: {used / 1e6:.0f} MB, split {e_new:.2e} fp32 {e_old:.2e}")
+    assert e_new <= 1.1 * e_old
 
 
 @pytest.mark.gpu
