@@ -57,6 +57,7 @@ __global__ void __launch_bounds__(256) uvl_pack_kernel(const cgtp_uvl_block* __r
   const float* wp = w + b.path * stride_p;
   u32x4* dst = packed + (int64_t)(blockIdx.x * gridDim.y + blockIdx.y) * kc * (TW * 192);
   unsigned m = 0;
+  const float lift = b.coef != 0.f ? 0x1p+60f : 0.f;
   for (int i = threadIdx.x; i < kc * TW * 64; i += 256) {
     const int lane = i & 63, t = (i >> 6) % TW, k = (i >> 6) / TW;
     // the columns a lane of uvl_kernel holds for unit k; those of the unit before get zeros
@@ -66,9 +67,11 @@ __global__ void __launch_bounds__(256) uvl_pack_kernel(const cgtp_uvl_block* __r
     for (int j = 0; j < 8; ++j) {
       const int col = first + j;
       const bool in = col >= k * 32 && col < cx && ch < cout;
-      const float u = wp[(in ? col : 0) * stride_k + (in ? ch : 0) * stride_c];
-      v[j] = in ? b.coef * u : 0.f;
-      m |= uvs_asks(v[j]) & kUvsPlain;
+      const float e = wp[(in ? col : 0) * stride_k + (in ? ch : 0) * stride_c], u = in ? e : 0.f;
+      v[j] = b.coef * u;
+      // what the coefficient left of a subnormal weight, but not of a large x (no branch: that would sink the loads, 11 -> 15 us
+      // a launch of 128 -> 128 channels)
+      m |= (uvs_asks(v[j]) & kUvsPlain) | ((unsigned)(v[j] == 0.f) & (unsigned)(u * lift != 0.f));
     }
     UvsParts<8> part;
 #pragma unroll

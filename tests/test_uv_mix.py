@@ -208,6 +208,24 @@ def test_the_range_of_operands_is_that_of_fp32(device, monkeypatch, exponent, sc
             assert err(a) <= 1.5 * err(b) + 3e-8, name
 
 
+@pytest.mark.gpu
+def test_weights_that_a_coefficient_takes_to_zero(device, monkeypatch):
+    """The smallest subnormal weights next to large inputs: a coefficient below one half (rows of order 0) may meet x, not them."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    x, g = (t * 2.0 ** 100 for t in _operands("so2", 4, 32, 32, 70, 13))
+    mod = _module("so2", 4, 32, 32, device)
+    with torch.no_grad():
+        mod.weight.copy_(mod.weight.sign() * 2.0 ** -149)
+    new = _run(mod, x.to(device), g.to(device))
+    monkeypatch.setattr(N, "_mix_split", lambda *args: None)
+    old = _run(mod, x.to(device), g.to(device))
+    ref = _run(mod.double(), x.double().to(device), g.double().to(device))
+    for name, a, b, want in zip(("out", "grad x"), new, old, ref):
+        e_new, e_old = ((t.double() - want).norm(dim=(0, 2)) / want.norm(dim=(0, 2)) for t in (a, b))
+        print(f"{name}: split {float(e_new.max()):.2e} fp32 {float(e_old.max()):.2e}")
+        assert bool((e_new <= 2.0 * e_old + 3e-8).all()), name
+
+
 # ---- gradient of the weight --------------------------------------------------------------------------------------------
 def _weight_gradients(monkeypatch, kind, l, cin, cout, x, g, device):
     from equitorch_amd.nn.functional import _uv_native as N
