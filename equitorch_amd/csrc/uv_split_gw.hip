@@ -108,7 +108,9 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
   __shared__ u32x4 bl[2 * CHUNK];
   __shared__ __align__(16) float yl[LV ? YN * LW : 2 * YN];        // [2: step][row of y][sample], with LV [row][l][sample]
   __shared__ unsigned redo_all;
-  __shared__ unsigned least_y;                           // of the y so far, zeros aside; 2^-30 where none is below
+  // of the y so far, zeros aside; 2^-30 where none is below.  Without channels on y by turns of the steps: the next step's y is noted
+  // while some wavefronts still read this one's.
+  __shared__ unsigned least_y[LV ? 1 : 2];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r = lane & 31, q = lane >> 5, C = a.C;
 
@@ -122,7 +124,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
   const int pc = tid % (32 * TB), oct = tid / (32 * TB), pcol = min(pc, C - 1);
   u32x4* const plain_to = bl + (pc >> 5) * 64 + oct * 32 + (pc & 31);
 
-  if (tid == 0) least_y = kLeastY;                       // the first window's barrier is behind it
+  if (tid < (LV ? 1 : 2)) least_y[tid] = kLeastY;        // the first window's barrier is behind it
 
   for (int job = a.job_ptr[wg]; job < a.job_ptr[wg + 1]; ++job) {
     const cgtp_uvg_job J = a.jobs[job];
@@ -204,7 +206,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
       };
       // Coupled to g first, y may take a product below the smallest number where x would have kept it above.  A zero is that only
       // next to a g and a y of a product below 2^-110 (a sum of terms in y cancels to no less than 2^-35 of them).
-      auto look_at_zero = [&](unsigned zero) __attribute__((always_inline)) {
+      auto look_at_zero = [&](unsigned zero, int ybuf) __attribute__((always_inline)) {
         if (!PATH::SWAPPED || !__any(zero)) return;
         unsigned least = ~0u;
 #pragma unroll
@@ -214,7 +216,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
             const float e = raw[o][j];
             least = min(least, by_magnitude(__builtin_bit_cast(float, opaque(__builtin_bit_cast(int, e)))));
           }
-        const float g = __builtin_bit_cast(float, least >> 1), y = __builtin_bit_cast(float, least_y >> 1);
+        const float g = __builtin_bit_cast(float, least >> 1), y = __builtin_bit_cast(float, least_y[LV ? 0 : ybuf] >> 1);
         redo |= zero && g * y < 0x1p-110f;               // no g but zeros: not a number, and not below
       };
       auto put_plain = [&](int buf) __attribute__((always_inline)) {
@@ -228,8 +230,8 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
       // The rows of y of a step.  Without channels i = (sample, row) and a step ahead; with them sample by sample, when the step
       // begins (it lasts several thousand cycles).
       float yreg[YWORDS];
-      auto note_y = [&](unsigned least) __attribute__((always_inline)) {       // read past the barrier behind it
-        if (PATH::SWAPPED && least < kLeastY) atomicMin(&least_y, least);
+      auto note_y = [&](unsigned least, int buf) __attribute__((always_inline)) {       // read past the barrier behind it
+        if (PATH::SWAPPED && least < kLeastY) atomicMin(&least_y[buf], least);
       };
       auto load_y = [&](int s) __attribute__((always_inline)) {
         const int64_t n0 = (int64_t)s * kStep, last = min(a.n_rows - n0, (int64_t)kStep) * CFG::D2;
@@ -243,7 +245,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
             for (int k = 0; k < 4; ++k) yl[(e % CFG::D2 * LW + l4 * 4 + k) * kStep + e / CFG::D2] = v[k];
             least = min(min(least, by_magnitude(v[0])), min(by_magnitude(v[1]), min(by_magnitude(v[2]), by_magnitude(v[3]))));
           }
-          note_y(least);
+          note_y(least, 0);
         } else {
 #pragma unroll
           for (int k = 0; k < YWORDS; ++k) {
@@ -260,7 +262,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
           if (i < YN) yl[buf * YN + i % CFG::D2 * kStep + i / CFG::D2] = yreg[k];
           if (i < YN) least = min(least, by_magnitude(yreg[k]));
         }
-        note_y(least);
+        note_y(least, buf);
       };
       struct Mix {
         const float* ys;
@@ -333,7 +335,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
 #pragma unroll
                   for (int j = 0; j < 8; ++j) zero |= v[j] == 0.f;
                 });
-                if (!LV) look_at_zero(zero);
+                if (!LV) look_at_zero(zero, ybuf);
                 __builtin_amdgcn_sched_barrier(0);
                 if (i == SETS - 1) {
                   if (!LV && R == 0 && more) load_y(sn);
@@ -349,7 +351,7 @@ __global__ void __launch_bounds__(64 * NW, 2) uvg_kernel(const UvgDev a) {
                   }
                 }
               }
-              if (LV) look_at_zero(zero);
+              if (LV) look_at_zero(zero, 0);
               if (LV && R == NR - 1 && more) load_mixed(sn);
               __builtin_amdgcn_sched_barrier(0);
               // the plain row of the next product, and the request for the one after
