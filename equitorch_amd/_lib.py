@@ -126,7 +126,8 @@ class UvlArgs(C.Structure):
                 ("steps", C.c_void_p), ("tasks", C.c_void_p), ("groups", C.c_void_p),
                 ("blocks", C.c_void_p), ("n_rows", C.c_int64), ("stride_p", C.c_int64), ("stride_k", C.c_int64), ("stride_c", C.c_int64),
                 ("n_blocks", C.c_int32), ("n_groups", C.c_int32), ("rows_per_task", C.c_int32), ("max_steps", C.c_int32),
-                ("dx", C.c_int32), ("dout", C.c_int32), ("cx", C.c_int32), ("cout", C.c_int32)]
+                ("dx", C.c_int32), ("dout", C.c_int32), ("cx", C.c_int32), ("cout", C.c_int32),
+                ("by_unit", C.c_int32)]
 
 
 class UvlGwArgs(C.Structure):

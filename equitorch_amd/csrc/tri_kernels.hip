@@ -650,7 +650,8 @@ int cgtp_abi_layout(int which, int64_t* out, int capacity) {
                                      CGTP_OFF(cgtp_uvl_args, n_groups), CGTP_OFF(cgtp_uvl_args, rows_per_task),
                                      CGTP_OFF(cgtp_uvl_args, max_steps),
                                      CGTP_OFF(cgtp_uvl_args, dx), CGTP_OFF(cgtp_uvl_args, dout),
-                                     CGTP_OFF(cgtp_uvl_args, cx), CGTP_OFF(cgtp_uvl_args, cout)};
+                                     CGTP_OFF(cgtp_uvl_args, cx), CGTP_OFF(cgtp_uvl_args, cout),
+                                     CGTP_OFF(cgtp_uvl_args, by_unit)};
   static const int64_t uvg_args[] = {sizeof(cgtp_uvg_args), CGTP_OFF(cgtp_uvg_args, x), CGTP_OFF(cgtp_uvg_args, y),
                                      CGTP_OFF(cgtp_uvg_args, g), CGTP_OFF(cgtp_uvg_args, gw),
                                      CGTP_OFF(cgtp_uvg_args, workspace), CGTP_OFF(cgtp_uvg_args, jobs),

@@ -18,7 +18,7 @@
 // 64 -> 64, lmax 2, 65536 samples 126 -> 75, 128 -> 128, lmax 3, 32768 samples 308 -> 170.  One workgroup per pair of rows, 325 us: a
 // third of its time went into starting; half lines of x from memory straight into the operands, 300; three wavefronts per
 // SIMD (spills), eight in a workgroup, matrix and vector instructions in turn by hand: no change.  Errors of the results
-// against 64 bits, rows of 1 to 96 units: 0.4e-7 to 2.3e-7, of fp32 matrix instructions 0.9e-7 to 8.0e-7.
+// against 64 bits: 0.4e-7 to 3.8e-7, of fp32 matrix instructions 0.9e-7 to 4.5e-7 (BY_UNIT below).
 //
 // Values: elements that are not finite or overflow as parts show in the results, and elements below 2^-110 (but not zero; their
 // last part could be below the smallest subnormal) are looked for; a wavefront that sees either forms its results
@@ -85,7 +85,14 @@ __global__ void __launch_bounds__(256) uvl_pack_kernel(const cgtp_uvl_block* __r
 }
 
 // RW rows of the result at a time.  Per unit of 32 channels a wavefront issues 24 NT RW matrix instructions (TW = 4).
-template <int TW, int NT, int RW>
+//
+// BY_UNIT: the matrix instruction rounds downwards, six times a unit at the size of the row's sum where all six products are added to
+// it: 0.75 to 0.85 of the error of fp32 matrix instructions, and so for the tables those take (1 to 24 units of 32 channels, random
+// operands or of one sign: 0.4e-7 to 3.8e-7, 0.9e-7 to 4.5e-7).  The larger tables were products of the library, which sums in
+// blocks: for them a unit's six are summed by themselves (24 units 3.2e-7 -> 1.0e-7, 96 units 7.7e-7 -> 1.8e-7, of one sign 4.9e-7 ->
+// 1.4e-7; a sum of the five small products beside the one of the large ones: 2.7e-7).  It takes 1 to 6 % more time: SO2Linear, lmax 4,
+// 64 channels, 32768 samples 259 -> 269 us.
+template <int TW, int NT, int RW, bool BY_UNIT>
 __global__ void __launch_bounds__(256, NT * RW == 4 ? 2 : 3) uvl_kernel(const UvlDev a) {
   constexpr int CHUNK = TW * 192;                   // 16-byte words of a block's fragments of a unit
   __shared__ u32x4 lds[2][RW][CHUNK];
@@ -255,21 +262,24 @@ __global__ void __launch_bounds__(256, NT * RW == 4 ? 2 : 3) uvl_kernel(const Uv
           bf16x8 f[3];
 #pragma unroll
           for (int h = 0; h < 3; ++h) f[h] = __builtin_bit_cast(bf16x8, frag[(h * TW + t) * 64]);
-          // A unit's six products are summed by themselves: the matrix instruction rounds downwards, six times a unit at the size
-          // of the row's sum where they are added to it (12 units of 32 channels 3.6e-7, by themselves 1.0e-7; 512 of them
-          // 2.1e-6 and 4.3e-7; fp32 instructions 4.3e-7 for 12; SO2Linear, lmax 4, 64 channels 1152 -> 1161 us a step).
           floatx4 sum[NT];
+          if constexpr (BY_UNIT) {
 #pragma unroll
-          for (int i = 0; i < NT; ++i) sum[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < NT; ++i) sum[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
 #pragma unroll
           for (int c = 0; c < 6; ++c) {              // the small products first
             constexpr int ha[6] = {2, 1, 0, 1, 0, 0}, hb[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
-            for (int i = 0; i < NT; ++i)
-              sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ha[c]], uvs_frag(part[i].p[hb[c]]), sum[i], 0, 0, 0);
+            for (int i = 0; i < NT; ++i) {
+              floatx4& to = BY_UNIT ? sum[i] : acc[w][t][i];
+              to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ha[c]], uvs_frag(part[i].p[hb[c]]), to, 0, 0, 0);
+            }
           }
+          if constexpr (BY_UNIT) {
 #pragma unroll
-          for (int i = 0; i < NT; ++i) acc[w][t][i] += sum[i];
+            for (int i = 0; i < NT; ++i) acc[w][t][i] += sum[i];
+          }
         }
       }
     }
@@ -538,7 +548,8 @@ static int uvl_tiles(int cout) { return cout % 64 == 0 || cout % 64 > 32 ? 4 : 2
 static int uvl_plan(const cgtp_uvl_args* a, UvlPlan* p) {
   if (!a || !a->x || !a->packed || !a->w || !a->out || !a->steps || !a->tasks || !a->groups || !a->blocks) return CGTP_ERR_NULL;
   if (a->n_rows < 0 || a->n_blocks <= 0 || a->n_groups <= 0 || a->dx <= 0 || a->dout <= 0 || a->cx <= 0 || a->cout <= 0 || a->cx % 4 ||
-      a->cout % 4 || (int64_t)a->dx * a->cx > 1 << 22 || a->rows_per_task < 1 || a->rows_per_task > 2 || a->max_steps > kWave)
+      a->cout % 4 || (int64_t)a->dx * a->cx > 1 << 22 || a->rows_per_task < 1 || a->rows_per_task > 2 || a->max_steps > kWave || a->by_unit < 0 ||
+      a->by_unit > 1)
     return CGTP_ERR_SHAPE;
   if (((uintptr_t)a->x | (uintptr_t)a->packed | (uintptr_t)a->out) & 15u) return CGTP_ERR_ALIGN;
   p->tw = uvl_tiles(a->cout);
@@ -561,10 +572,10 @@ static int uvl_plan(const cgtp_uvl_args* a, UvlPlan* p) {
   return CGTP_OK;
 }
 
-template <int TW>
+template <int TW, bool BY_UNIT>
 static auto uvl_fn(int nt, int rw) {
-  return rw == 2 ? (nt == 2 ? uvl_kernel<TW, 2, 2> : uvl_kernel<TW, 1, 2>)
-                 : nt == 4 ? uvl_kernel<TW, 4, 1> : nt == 2 ? uvl_kernel<TW, 2, 1> : uvl_kernel<TW, 1, 1>;
+  return rw == 2 ? (nt == 2 ? uvl_kernel<TW, 2, 2, BY_UNIT> : uvl_kernel<TW, 1, 2, BY_UNIT>)
+                 : nt == 4 ? uvl_kernel<TW, 4, 1, BY_UNIT> : nt == 2 ? uvl_kernel<TW, 2, 1, BY_UNIT> : uvl_kernel<TW, 1, 1, BY_UNIT>;
 }
 
 }  // namespace cgtp
@@ -593,7 +604,8 @@ int cgtp_uvl_apply(const cgtp_uvl_args* a, void* stream) {
                      (hipStream_t)stream, a->blocks, d.w, (u32x4*)a->packed, (unsigned*)d.asks, d.kc, d.cx, d.cout, d.stride_p,
                      d.stride_k, d.stride_c);
   if (hipGetLastError() != hipSuccess) return CGTP_ERR_LAUNCH;
-  void (*fn)(const UvlDev) = p.tw == 4 ? uvl_fn<4>(p.nt, a->rows_per_task) : uvl_fn<2>(p.nt, a->rows_per_task);
+  void (*fn)(const UvlDev) = p.tw == 4 ? (a->by_unit ? uvl_fn<4, true>(p.nt, a->rows_per_task) : uvl_fn<4, false>(p.nt, a->rows_per_task))
+                                       : a->by_unit ? uvl_fn<2, true>(p.nt, a->rows_per_task) : uvl_fn<2, false>(p.nt, a->rows_per_task);
   hipLaunchKernelGGL(fn, dim3((unsigned)p.grid), dim3(256), 0, (hipStream_t)stream, d);
   return hipGetLastError() == hipSuccess ? CGTP_OK : CGTP_ERR_LAUNCH;
 }

@@ -579,12 +579,15 @@ def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor
         return None
     n_groups = mix.groups_for(n, -(-cout // 64))
     walk = kernels.cached(_anchor(table), ("uvl_walk", transposed, str(x.device)), lambda: _MixWalk(mix, x.device))
+    # tables the fp32 kernels do not take were products of the library, whose sums are more precise than theirs
+    by_unit = kernels.cached(_anchor(table), ("uvl_by_unit", w.shape[1], w.shape[2]),
+                             lambda: int(not u1v_fits(n, w.shape[1], w.shape[2], table, x.dtype)))
     packed = torch.empty(int(_lib.lib.cgtp_uvl_packed_bytes(mix.n_blocks, cx, cout)), dtype=torch.uint8, device=x.device)
     out = torch.empty((n, mix.n_out, cout), dtype=x.dtype, device=x.device)
     steps, groups, tasks, blocks = walk.address[n_groups]
     a = _lib.UvlArgs(x.data_ptr(), packed.data_ptr(), w.data_ptr(), out.data_ptr(), steps, tasks, groups, blocks,
                      n, w.stride(0), w.stride(2 if transposed else 1), w.stride(1 if transposed else 2),
-                     mix.n_blocks, n_groups, mix.rows_per_task, walk.max_steps[n_groups], dx, mix.n_out, cx, cout)
+                     mix.n_blocks, n_groups, mix.rows_per_task, walk.max_steps[n_groups], dx, mix.n_out, cx, cout, by_unit)
     status = _lib.lib.cgtp_uvl_apply(C.byref(a), _lib.stream_ptr(x.device))
     if status in (2, 3):               # extents or an alignment it does not take: nothing was launched
         return None

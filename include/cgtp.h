@@ -430,7 +430,8 @@ int cgtp_uvsw_apply(int cfg, int kind, const void* x, const void* z, void* packe
  * each a row of x times a block for either row of out (-1: none), the last with the task's index (`task`, else -1); a row
  * of out without terms has a task of one step without blocks.  Blocks are the distinct (path, coefficient) pairs.  A group is
  * the work of one workgroup for its samples: the steps of whole tasks, 1 to 64 (max_steps: the most of any).  steps, tasks, groups
- * and blocks in device memory, packed: cgtp_uvl_packed_bytes() bytes of scratch.  The layers are IrrepsLinear and
+ * and blocks in device memory, packed: cgtp_uvl_packed_bytes() bytes of scratch.  by_unit (0 or 1): the products of 32
+ * channels are summed by themselves, for a third of the errors of fp32 matrix instructions (0: four fifths).  The layers are IrrepsLinear and
  * SO2Linear('uv') with a shared weight (reference equitorch/nn/linears.py:268-571). */
 typedef struct { int32_t row, block[2], task; } cgtp_uvl_step;
 typedef struct { int32_t row[2]; } cgtp_uvl_task;
@@ -446,7 +447,7 @@ typedef struct {
   const cgtp_uvl_group* groups;
   const cgtp_uvl_block* blocks;
   int64_t n_rows, stride_p, stride_k, stride_c;
-  int32_t n_blocks, n_groups, rows_per_task, max_steps, dx, dout, cx, cout;
+  int32_t n_blocks, n_groups, rows_per_task, max_steps, dx, dout, cx, cout, by_unit;
 } cgtp_uvl_args;
 int64_t cgtp_uvl_packed_bytes(int32_t n_blocks, int32_t cx, int32_t cout);
 int cgtp_uvl_validate(const cgtp_uvl_args* a);
