@@ -11,6 +11,8 @@ ordered by output row; this module cuts that list from the table for each of the
     ('uvw' only) g2[M2]   <- rows M of grad_out,   first operand rows M1,  weight permuted
 """
 import ctypes as C
+import functools
+import heapq
 from typing import NamedTuple, Optional
 
 import numpy as np
@@ -19,6 +21,7 @@ from torch import Tensor
 from torch.autograd import Function
 
 from ... import _lib
+from ..._tables import TpCoo
 from ...ops import kernels
 
 FIRST, LAST = 1, 2
@@ -169,26 +172,9 @@ class _GradWWalk:
     SHARES = 64
 
     def __init__(self, coo, n_wgs: int, device):
-        cost = []
-        for p in range(coo.P):
-            mine = np.asarray(coo.p) == p
-            rows = len(set(np.asarray(coo.M1)[mine].tolist())), len(set(np.asarray(coo.M)[mine].tolist()))
-            # of a step: its products (as many as the side with fewer rows has), and the rows that are read
-            cost.append(min(rows) + 0.15 * sum(rows))
-        jobs = self.deal(cost, n_wgs)
-        slots, slot_ptr = {}, [0]
-        for p in range(coo.P):
-            for w, mine in enumerate(jobs):
-                for path, _ in mine:
-                    if path == p:
-                        slots[w, p] = len(slots)
-            slot_ptr.append(len(slots))
-        flat = [(p, slots[w, p], mask & 0xffffffff, mask >> 32) for w, mine in enumerate(jobs) for p, mask in mine]
-        job_ptr = np.cumsum([0] + [len(mine) for mine in jobs])
-        parts = [np.array(flat, dtype=np.uint32).view(np.int32), job_ptr.astype(np.int32), np.array(slot_ptr, dtype=np.int32)]
-        self.words = torch.from_numpy(np.concatenate([p.ravel() for p in parts])).to(device)
-        self.at = [4 * sum(p.size for p in parts[:k]) for k in range(len(parts))]
-        self.n_slots, self.n_paths = len(slots), coo.P
+        words, self.at, self.n_slots = _grad_w_words(n_wgs, int(coo.P), *(np.ascontiguousarray(v, dtype=np.int32).tobytes()
+                                                                          for v in (coo.M, coo.M1, coo.p)))
+        self.words, self.n_paths = torch.tensor(words, device=device), coo.P
 
     def ranges(self, steps: int) -> int:
         """Ranges the steps are cut into, each with slots of its own: 128 steps or more in each, and no more than the fp32 kernel has
@@ -202,8 +188,8 @@ class _GradWWalk:
         """Per workgroup its ``(path, mask)``: the 64 shares of every path, dealt in the order of the paths so that all
         workgroups carry the same cost, the shares of a path spread over its steps."""
         room = sum(cost) * cls.SHARES / n_wgs
-        jobs, w, left = [[] for _ in range(n_wgs)], 0, room
-        for p, c in enumerate(cost):
+        portions_of, w, left = [], 0, room
+        for c in cost:
             todo, portions = cls.SHARES, []
             while todo:
                 take = min(todo, max(0, int(left / c + 0.5))) if w < n_wgs - 1 else todo
@@ -213,15 +199,46 @@ class _GradWWalk:
                     left -= take * c
                 if todo:
                     w, left = w + 1, left + room           # what was taken too much or too little carries over
-            given, masks = [0] * len(portions), [0] * len(portions)
-            for bit in range(cls.SHARES):
-                k = max(range(len(portions)), key=lambda i: portions[i][1] * (bit + 1) / cls.SHARES - given[i])
-                given[k] += 1
-                masks[k] |= 1 << bit
-            for (g, _), mask in zip(portions, masks):
-                if mask:
-                    jobs[g].append((p, mask))
+            portions_of.append(portions)
+        most = max(map(len, portions_of))
+        takes = np.array([[take for _, take in portions] + [0] * (most - len(portions)) for portions in portions_of])
+        jobs = [[] for _ in range(n_wgs)]
+        for p, masks in enumerate(cls.masks(takes)):
+            for (g, _), mask in zip(portions_of[p], masks):
+                jobs[g].append((p, mask))
         return jobs
+
+    @classmethod
+    def masks(cls, takes):
+        """``takes``: a row of portions for each path, filled up with zeros.  A bit for each of a path's shares to the portion
+        that is most behind its part of them."""
+        behind, at, owner = np.zeros_like(takes), np.arange(len(takes)), np.zeros((len(takes), cls.SHARES), dtype=np.int64)
+        for bit in range(cls.SHARES):
+            behind += takes
+            owner[:, bit] = k = behind.argmax(axis=1)
+            behind[at, k] -= cls.SHARES
+        bits = owner[:, None, :] == np.arange(takes.shape[1])[:, None]
+        return np.packbits(bits, axis=-1, bitorder="little").view("<u8")[..., 0].tolist()
+
+
+@functools.lru_cache(maxsize=32)
+def _grad_w_words(n_wgs: int, n_paths: int, *indices: bytes):
+    """The arrays of a :class:`_GradWWalk` by the table's content (host work that a second module of the table does not
+    repeat): jobs, their places by workgroup and the slots by path in one array, where each begins in bytes, slots."""
+    M, M1, path = (np.frombuffer(v, dtype=np.int32).astype(np.int64) for v in indices)
+
+    def rows(idx):
+        return np.bincount(np.unique(path << 32 | idx) >> 32, minlength=n_paths)
+    # of a step: its products (as many as the side with fewer rows has), and the rows that are read
+    cost = (np.minimum(rows(M1), rows(M)) + 0.15 * (rows(M1) + rows(M))).tolist()
+    jobs = _GradWWalk.deal(cost, n_wgs)
+    by_path = sorted((p, w) for w, mine in enumerate(jobs) for p, _ in mine)
+    slots = {job: k for k, job in enumerate(by_path)}
+    flat = [(p, slots[p, w], mask & 0xffffffff, mask >> 32) for w, mine in enumerate(jobs) for p, mask in mine]
+    parts = [np.array(flat, dtype=np.uint32).view(np.int32), np.cumsum([0] + [len(mine) for mine in jobs]).astype(np.int32),
+             np.searchsorted([p for p, _ in by_path], np.arange(n_paths + 1)).astype(np.int32)]
+    return np.concatenate([v.ravel() for v in parts]), [4 * sum(v.size for v in parts[:k]) for k in range(len(parts))], len(slots)
+
 
 
 def _split_grad_w(x: Tensor, y: Tensor, g: Tensor, tp_info) -> Optional[Tensor]:
@@ -440,6 +457,9 @@ def _split_uvw(kind: int, x: Tensor, z: Tensor, w: Tensor, tp_info, rows_out: in
     return out
 
 
+_MIX_STEPS = 64          # of a group, one lane each
+
+
 class _MixTable:
     """A channel-mixing table for ``cgtp_uvl_apply`` (``transposed``: the gradient of its input): the rows of the result by two
     where most of the rows of the input that reach one reach both (the ``+m`` and ``-m`` rows of an SO(2) layer, which then
@@ -447,44 +467,112 @@ class _MixTable:
 
     def __init__(self, coo, transposed: bool):
         rows_out, rows_in, n_out = (coo.M1, coo.M, coo.D1) if transposed else (coo.M, coo.M1, coo.DO)
-        blocks = {}                                    # (path, coefficient) -> its place in the packed weight
-        terms = [{} for _ in range(n_out)]             # row of the result: row of the input -> blocks
-        for o, i, p, c in zip(rows_out, rows_in, coo.p, coo.coef):
-            b = blocks.setdefault((int(p), np.float32(c)), len(blocks))
-            terms[int(o)].setdefault(int(i), []).append(b)
-        pairs, alone = [], set(range(n_out))
-        for m in range(n_out):
-            if m in alone:
-                most = max(sorted(alone - {m}), key=lambda k: len(terms[m].keys() & terms[k].keys()), default=None)
-                if most is not None and 2 * len(terms[m].keys() & terms[most].keys()) > max(len(terms[m]), len(terms[most])):
-                    pairs.append((m, most))
-                    alone -= {m, most}
-        if 4 * sum(len(terms[m].keys() & terms[k].keys()) for m, k in pairs) < sum(len(t) for t in terms):
-            pairs, alone = [], set(range(n_out))
+        o, i, p = (np.asarray(v, dtype=np.int64) for v in (rows_out, rows_in, coo.p))
+        coef = np.asarray(coo.coef, dtype=np.float64).astype(np.float32)
+        # (path, coefficient) has a place in the packed weight
+        keys, block = np.unique(p << 32 | coef.view(np.uint32), return_inverse=True)
+        self.blocks = np.stack([(keys >> 32), (keys & 0xffffffff)], axis=1).astype(np.uint32).view(np.int32)
+        if not len(keys):
+            self.blocks = np.zeros((1, 2), dtype=np.int32)
+        self.n_out, self.n_blocks = n_out, len(self.blocks)
+        pairs, alone, shared = self._pairs(o, i, n_out)
+        if 4 * shared < len(np.unique(o * (1 << 32) + i)):
+            pairs, alone = [], list(range(n_out))
         self.rows_per_task = 2 if pairs else 1
-        self.tasks, self.steps = sorted(pairs + [(m, -1) for m in alone]), []
-        for m, k in self.tasks:
-            steps = []
-            for i in sorted(terms[m].keys() | (terms[k].keys() if k >= 0 else set())):
-                b0, b1 = terms[m].get(i, []), terms[k].get(i, []) if k >= 0 else []
-                steps += [(i, b0[t] if t < len(b0) else -1, b1[t] if t < len(b1) else -1)
-                          for t in range(max(len(b0), len(b1)))]
-            self.steps.append(steps or [(0, -1, -1)])
-        self.n_out, self.n_blocks = n_out, max(len(blocks), 1)
-        self.blocks = np.array([(p, c.view(np.int32)) for p, c in blocks] or [(0, 0)], dtype=np.int32)
-        self.longest = max(map(len, self.steps))
-        # the numbers of groups to choose from, with the most steps of a group
-        self.choices = {g: self.dealt(g)[1] for g in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, len(self.tasks)) if g <= len(self.tasks)}
+        self.tasks = sorted(pairs + [(m, -1) for m in alone])
+        # a step: a row of the input and a block for each row of the task; entries of one row and input row one after the other
+        tasks = np.array(self.tasks, dtype=np.int64).reshape(-1, 2)
+        task_of, side_of = np.zeros(n_out, dtype=np.int64), np.zeros(n_out, dtype=np.int64)
+        for side in (0, 1):
+            real = tasks[:, side] >= 0
+            task_of[tasks[real, side]], side_of[tasks[real, side]] = np.nonzero(real)[0], side
+        order = np.lexsort([i, o])
+        o, i, block = o[order], i[order], block.ravel()[order]
+        at = np.arange(len(o))
+        new = np.ones(len(o), dtype=bool)
+        new[1:] = (o[1:] != o[:-1]) | (i[1:] != i[:-1])
+        turn = at - np.maximum.accumulate(np.where(new, at, 0))
+        empty = np.nonzero(np.bincount(task_of[o], minlength=len(tasks)) == 0)[0]       # written as zeros: a step without blocks
+        n_in, most = int(i.max(initial=0)) + 1, int(turn.max(initial=0)) + 1
+        keys, step = np.unique(np.concatenate([(task_of[o] * n_in + i) * most + turn, empty * n_in * most]), return_inverse=True)
+        steps = np.full((len(keys), 4), -1, dtype=np.int32)
+        steps[:, 0] = keys // most % n_in
+        steps[step.ravel()[:len(o)], 1 + side_of[o]] = block
+        task = keys // most // n_in
+        last = np.ones(len(task), dtype=bool)
+        last[:-1] = task[1:] != task[:-1]
+        steps[last, 3] = task[last]
+        ends = (np.nonzero(last)[0] + 1).tolist()
+        self.steps = [steps[b:e] for b, e in zip([0] + ends, ends)]
+        self._sizes = list(map(len, self.steps))
+        self._longest_first = sorted(range(len(ends)), key=lambda t: -self._sizes[t])
+        self.longest = max(self._sizes)
+        # the numbers of groups to choose from, with the most steps of a group and their cost: a group's steps are a lane each
+        dealt = {g: self.dealt(g) for g in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, len(self.tasks)) if g <= len(self.tasks)}
+        self.choices = {g: most for g, (_, most) in dealt.items()}
         self.costs = [(g, most + 2) for g, most in self.choices.items() if most <= _MIX_STEPS]
+        self._dealt = {g: dealt[g][0] for g, _ in self.costs}
+
+    @staticmethod
+    def _pairs(o, i, n_out: int):
+        """Pairs of rows of the result, the rows left, and the rows of the input that both rows of a pair share, added up: of
+        rows that the same rows of the input reach two by two, and of the rest as many as share most of them."""
+        reach = np.unique(o * (1 << 32) + i)
+        row, at = reach >> 32, reach & 0xffffffff
+        ends = np.searchsorted(row, np.arange(n_out + 1))
+        rows_in = [at[ends[m]:ends[m + 1]] for m in range(n_out)]
+        pairs, shared, waiting = [], 0, {}
+        for m, mine in enumerate(rows_in):
+            if len(mine):
+                first = waiting.pop(key := mine.tobytes(), None)
+                if first is None:
+                    waiting[key] = m
+                else:
+                    pairs.append((first, m))
+                    shared += len(mine)
+        alone = np.ones(n_out, dtype=bool)
+        alone[[m for pair in pairs for m in pair]] = False
+        if len(waiting) > 1:
+            by_in = np.argsort(at, kind="stable")
+            in_ends = np.searchsorted(at[by_in], np.arange(int(at.max()) + 2))
+            reached = row[by_in]
+            for m in sorted(waiting.values()):
+                if alone[m]:
+                    both = np.bincount(np.concatenate([reached[in_ends[k]:in_ends[k + 1]] for k in rows_in[m]]), minlength=n_out)
+                    both = np.where(alone, both, 0)
+                    both[m] = 0
+                    most = int(both.argmax())
+                    if 2 * both[most] > max(len(rows_in[m]), len(rows_in[most])):
+                        pairs.append((m, most))
+                        alone[[m, most]] = False
+                        shared += int(both[most])
+        return pairs, np.nonzero(alone)[0].tolist(), shared
 
     def dealt(self, n_groups: int):
         """The tasks in ``n_groups`` groups: the longest first, each to the group with the fewest steps so far."""
-        groups, count = [[] for _ in range(n_groups)], [0] * n_groups
-        for t in sorted(range(len(self.tasks)), key=lambda t: -len(self.steps[t])):
-            g = count.index(min(count))
+        groups, count = [[] for _ in range(n_groups)], [(0, g) for g in range(n_groups)]
+        for t in self._longest_first:
+            steps, g = count[0]
             groups[g].append(t)
-            count[g] += len(self.steps[t])
-        return groups, max(count)
+            heapq.heapreplace(count, (steps + self._sizes[t], g))
+        return groups, max(count)[0]
+
+    @functools.cached_property
+    def words(self):
+        """What the kernel reads, dealt to every number of groups there is to choose from, in one array, and where the steps, the
+        groups and the tasks and blocks they share begin, in bytes, for each."""
+        parts = [np.array(v, dtype=np.int32).ravel() for v in (self.tasks, self.blocks)]
+        parts = [np.resize(v, -(-v.size // 4) * 4) for v in parts]          # steps are read 16 bytes at a time
+        end, at = sum(v.size for v in parts), {}
+        for n_groups, groups in self._dealt.items():
+            ptr, begin = [], 0
+            for group in groups:
+                ptr += [begin, begin := begin + sum(self._sizes[t] for t in group)]
+            ptr += [0] * (len(ptr) % 4)
+            parts += [np.concatenate([self.steps[t] for group in groups for t in group]).ravel(), np.array(ptr, dtype=np.int32)]
+            at[n_groups] = tuple(4 * v for v in (end, end + parts[-2].size, 0, parts[0].size))
+            end += parts[-2].size + parts[-1].size
+        return np.concatenate(parts), at
 
     def groups_for(self, n: int, column_blocks: int) -> int:
         """Groups (workgroups a block of samples is cut into): what lets whole rounds of two workgroups per compute unit end
@@ -498,35 +586,29 @@ class _MixTable:
         return best
 
 
-_MIX_STEPS = 64          # of a group, one lane each
-
-
 class _MixWalk:
-    """The table dealt to every number of groups there is to choose from, on the device in one piece: a batch of another size
-    copies nothing.  ``at[n_groups]``: where its steps, its groups and the tasks and blocks they share begin, in bytes."""
+    """The words of a :class:`_MixTable` on the device, copied in one piece: a batch of another size copies nothing."""
 
     def __init__(self, table: _MixTable, device):
-        parts = [np.array(v, dtype=np.int32).ravel() for v in (table.tasks, table.blocks)]
-        parts[0] = np.resize(parts[0], -(-parts[0].size // 4) * 4)          # steps are read 16 bytes at a time
-        parts[1] = np.resize(parts[1], -(-parts[1].size // 4) * 4)
-        end, self.at, self.max_steps = sum(p.size for p in parts), {}, {}
-        for n_groups, most in table.choices.items():
-            steps, ptr = [], []
-            for group in table.dealt(n_groups)[0]:
-                ptr.append((len(steps), len(steps) + sum(len(table.steps[t]) for t in group)))
-                for t in group:
-                    steps += [(*s, -1) for s in table.steps[t][:-1]] + [(*table.steps[t][-1], t)]
-            ptr += [(0, 0)] * (len(ptr) % 2)
-            parts += [np.array(v, dtype=np.int32).ravel() for v in (steps, ptr)]
-            self.at[n_groups] = tuple(4 * v for v in (end, end + parts[-2].size, 0, parts[0].size))
-            self.max_steps[n_groups] = most
-            end += parts[-2].size + parts[-1].size
-        self.words = torch.from_numpy(np.concatenate(parts)).to(device)
+        words, self.at = table.words
+        self.max_steps = table.choices
+        self.words = torch.tensor(words, device=device)
         self.address = {g: tuple(self.words.data_ptr() + v for v in at) for g, at in self.at.items()}
 
 
+@functools.lru_cache(maxsize=64)
+def _mix_table_of_content(transposed: bool, D1: int, DO: int, coef: bytes, *indices: bytes) -> _MixTable:
+    """:class:`_MixTable` by the table's content: host work that a second layer over the same irreps does not repeat.  Host arrays
+    only, read by every caller and written by none."""
+    M, M1, p = (np.frombuffer(v, dtype=np.int32) for v in indices)
+    return _MixTable(TpCoo(np.frombuffer(coef, dtype=np.float64), M, M1, None, p, None, D1, 1, DO, 0), transposed)
+
+
 def _mix_table(table, transposed: bool) -> _MixTable:
-    return kernels.cached(_anchor(table), ("uvl_table", transposed), lambda: _MixTable(table.coo, transposed))
+    c = table.coo
+    return kernels.cached(_anchor(table), ("uvl_table", transposed), lambda: _mix_table_of_content(
+        transposed, int(c.D1), int(c.DO), np.ascontiguousarray(c.coef, dtype=np.float64).tobytes(),
+        *(np.ascontiguousarray(v, dtype=np.int32).tobytes() for v in (c.M, c.M1, c.p))))
 
 
 def _observed(*tensors: Tensor) -> bool:

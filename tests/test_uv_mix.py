@@ -31,14 +31,19 @@ def _table(entries, n_in, n_out, n_w):
     return N.CooTable(coo, torch.zeros(1), None, mixing=True)
 
 
-@pytest.mark.parametrize("kind,l", [("so2", 2), ("so2", 6), ("lin", 2), ("own", 0)])
+@pytest.mark.parametrize("kind,l", [("so2", 2), ("so2", 6), ("lin", 2), ("own", 0), ("any", 1), ("any", 2), ("any", 3)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_the_steps_are_the_table(kind, l, transposed):
     """Tasks, steps and groups for every number of groups against the table's entries; ``own``: several weights and coefficients
-    for one pair of rows, and rows of either side that no entry reaches."""
+    for one pair of rows, and rows of either side that no entry reaches; ``any``: entries at random."""
     from equitorch_amd.nn.functional import _uv_native as N
     if kind == "own":
         entries, n_in, n_out, n_w = [(0, 2, 1, 0.5), (0, 2, 0, -2.0), (3, 2, 1, 0.5), (3, 0, 1, 1.5), (0, 0, 2, 3.0), (1, 4, 2, 1.0)], 6, 5, 3
+    elif kind == "any":
+        rng = np.random.default_rng(l)
+        n_in, n_out, n_w = 11 * l, 7 * l, 3
+        entries = [(int(a), int(b), int(c), float(s)) for a, b, c, s in zip(*(rng.integers(0, k, 40 * l) for k in (n_out, n_in, n_w)),
+                                                                            rng.choice([1.0, 0.5], 40 * l))]
     else:
         entries, plan, n_in = _coo(kind, l)
         n_out, n_w = plan.out_size, plan.n_paths
@@ -71,6 +76,26 @@ def test_the_steps_are_the_table(kind, l, transposed):
     if kind == "so2":
         assert table.rows_per_task == 2
     assert table.groups_for(10 ** 6, 1) >= 1 and max(len(s) for s in table.steps) == table.longest
+
+
+def test_rows_that_the_same_rows_reach_are_paired():
+    """Copies of irreps mixed with copies: two rows at a time, also where an odd row is left over or reached by nearly the same."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    full = [(m, i, 0, 1.0) for m in range(5) for i in range(6)]
+    assert N._MixTable(_table(full, 6, 5, 1).coo, False).tasks == [(0, 1), (2, 3), (4, -1)]
+    most = [e for e in full if e[:2] != (4, 0)] + [(5, i, 0, 1.0) for i in range(6)]       # 4 has five of the six of 5
+    assert N._MixTable(_table(most, 6, 6, 1).coo, False).tasks == [(0, 1), (2, 3), (4, 5)]
+    apart = [(m, i, 0, 1.0) for m in range(4) for i in range(6) if i % 4 == m]
+    assert N._MixTable(_table(apart, 6, 4, 1).coo, False).tasks == [(m, -1) for m in range(4)]
+
+
+def test_layers_of_one_table_share_its_steps():
+    """A second layer over the same irreps repeats no host work; another table or direction has steps of its own."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    tables = [_table(entries, n_in, plan.out_size, plan.n_paths) for entries, plan, n_in in (_coo("so2", 2), _coo("so2", 2), _coo("lin", 2))]
+    first, second, other = (N._mix_table(t, False) for t in tables)
+    assert first is second and first is not other and N._mix_table(tables[0], True) is not first
+    assert first.words[0] is second.words[0]
 
 
 # ---- on the GPU ------------------------------------------------------------------------------------------------------
