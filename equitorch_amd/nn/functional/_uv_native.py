@@ -148,11 +148,14 @@ class _MixPairs:
 def _mix_grad_w(x: Tensor, g: Tensor, table) -> Optional[Tensor]:
     """:func:`grad_w` of channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_grad_w``), or None where the fp32
     matrix instructions serve: past 128 channels, where their blocks of 128 x 128 read the rows less often (256 -> 256, 4096
-    samples: 69 us against 78).  IrrepsLinear and SO2Linear, 8 to 128 channels, 500 to 65536 samples: 0.60 to 0.98 of their time."""
+    samples: 69 us against 78), and for the same reason past 64 with the few single pairs of SO2Linear of lmax 1 (six paths, eight
+    pairs; 128 channels, 4096 samples 32.5 us against 29.4, 65536 203 against 180; lmax 2, 19 and 29: 54.9 against 64.6 and 539 against
+    620).  IrrepsLinear and SO2Linear, 8 to 128 channels, 500 to 65536 samples: 0.5 to 1.0 of their time (SO2Linear of lmax 2, 64 channels, 2000
+    samples 1.05)."""
     if not (isinstance(table, CooTable) and table.mixing) or x.dtype != torch.float32 or x.shape[0] == 0:
         return None
     (n, dx, cx), (_, dg, cout), n_paths = x.shape, g.shape, table.coo.P
-    if max(cx, cout) > 128:
+    if max(cx, cout) > 128 or (min(cx, cout) > 64 and n_paths <= 8 and len(table.coo.p) < 2 * n_paths and n > 2000):
         return None
     pairs = kernels.cached(_anchor(table), ("uvl_pairs", str(x.device)), lambda: _MixPairs(table.coo, x.device))
     gw = torch.empty((n_paths, cx, cout), dtype=x.dtype, device=x.device)
@@ -507,6 +510,12 @@ class _MixTable:
         self._sizes = list(map(len, self.steps))
         self._longest_first = sorted(range(len(ends)), key=lambda t: -self._sizes[t])
         self.longest = max(self._sizes)
+        # whether the fp32 kernel, which deals the rows to a power of two of wavefronts, has no longer chains
+        row_entries = sorted(np.bincount(o, minlength=n_out).tolist(), reverse=True)
+        chains = [0] * (1 << min(n_out.bit_length() - 1, 4))
+        for k in row_entries:
+            heapq.heapreplace(chains, chains[0] + k)
+        self.even = max(chains) <= self.longest
         # the numbers of groups to choose from, with the most steps of a group and their cost: a group's steps are a lane each
         dealt = {g: self.dealt(g) for g in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, len(self.tasks)) if g <= len(self.tasks)}
         self.choices = {g: most for g, (_, most) in dealt.items()}
@@ -647,17 +656,29 @@ def mix_fits(x: Tensor, w: Tensor, table, one_product: bool, widened: bool) -> b
             and short(False) and short(True))
 
 
+def _few_and_long(mix: _MixTable, n: int, cx: int, cout: int) -> bool:
+    """Whether the workgroups of ``cgtp_uvl_apply`` are so few and long that the fp32 kernel, of 16 samples each, ends sooner: past 128
+    contracted channels and below 2048 samples (256 -> 256, lmax 4, 700 samples: 43 us against 38), and small results made two
+    rows at a time where that kernel has no longer chains either, the pack included: SO2Linear of lmax 1, 128 -> 48 channels, 1500
+    samples 18.1 us against 14.3, 8000 20.5 against 22.1; 64 -> 64, 1500 12.6 against 11.9; of lmax 2, 128 -> 16, 4096 24.0 against 18.6, 64 ->
+    16 15.2 against 14.2, 128 -> 20 24.4 and 24.1; two scalars, 128 -> 128, 4096 19.0 against 15.5."""
+    if cx > 128 and n < 2048:
+        return True
+    return (mix.rows_per_task == 2 and mix.even and cx > (64 if 16 < cout <= 32 else 32)
+            and n < (10000 if cx > 64 and cout <= 16 else 5000) and mix.n_out * cout <= (256 if mix.n_out <= 4 else 144))
+
+
 def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor]:
     """Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``), or None where the fp32 matrix
-    instructions serve.  Over 400 launches (IrrepsLinear of lmax 1 to 4, SO2Linear of lmax 2 to 6, 8 to 256 channels on either side,
-    100 to 30000 samples) it takes 0.4 to 1.0 of their time; past 128 contracted channels and below 2048 samples its
-    workgroups are few and long (256 -> 256, lmax 4, 700 samples: 43 us against 38)."""
+    instructions serve.  Over 1000 launches (IrrepsLinear of lmax 1 to 4 and of copies of an irrep, SO2Linear of lmax 1 to 6, 8 to
+    256 channels on either side, 100 to 65000 samples) it takes 0.4 to 1.0 of their time, apart from those of
+    :func:`_few_and_long` and, up to 1.05, SO2Linear of lmax 1 and 2 with 96 and more to 16 channels about 12000 samples."""
     if not (isinstance(table, CooTable) and table.mixing) or x.dtype != torch.float32:
         return None
     n, dx, cx = x.shape
     cout = w.shape[1] if transposed else w.shape[2]
     mix = _mix_table(table, transposed)
-    if mix.longest > _MIX_STEPS or (cx > 128 and n < 2048 and chunk_of(n, dx, 1, mix.n_out, cx, 0, cout) > 0):
+    if mix.longest > _MIX_STEPS or (_few_and_long(mix, n, cx, cout) and chunk_of(n, dx, 1, mix.n_out, cx, 0, cout) > 0):
         return None
     n_groups = mix.groups_for(n, -(-cout // 64))
     walk = kernels.cached(_anchor(table), ("uvl_walk", transposed, str(x.device)), lambda: _MixWalk(mix, x.device))

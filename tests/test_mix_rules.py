@@ -24,3 +24,31 @@ def test_by_rows_work_and_type(kind, l, c, n, widened, fits):
     if x.data_ptr() % 16:
         pytest.skip("the allocation is not on a 16-byte boundary")
     assert N.mix_fits(x, w, table, kind == "so2", widened) == fits
+
+
+def _mix(kind, irreps):
+    from test_uv_mix import _table
+
+    from equitorch_amd import nn as enn
+    from equitorch_amd.nn.functional import _irreps_gemm as G
+    from equitorch_amd.nn.functional import _uv_native as N
+    if kind == "so2":
+        mod = enn.SO2Linear(irreps, irreps, 4, 4, feature_mode="uv")
+        plan = G.plan_of_product_info(mod.info_forward, mod.irreps_in.dim, mod.num_weights)
+    else:
+        mod = enn.IrrepsLinear(irreps, irreps, 4, 4)
+        plan = G.plan_of_linear_info(mod.forward_info)
+    return N._MixTable(_table([(p.o0 + j, p.i0 + j, p.w, p.scale) for p in plan.paths for j in range(p.k)], mod.irreps_in.dim, plan.out_size,
+                              plan.n_paths).coo, False)
+
+
+@pytest.mark.parametrize("kind,irreps,cin,cout,n,fp32", [
+    ("so2", "0e+1o", 64, 64, 4096, True), ("so2", "0e+1o", 64, 64, 5000, False), ("so2", "0e+1o", 64, 68, 4096, False),
+    ("so2", "0e+1o", 64, 32, 4096, False), ("so2", "0e+1o", 96, 32, 4096, True), ("so2", "0e+1o", 32, 64, 4096, False),
+    ("so2", "0e+1o+2e", 64, 16, 4096, True), ("so2", "0e+1o+2e", 128, 16, 9999, True), ("so2", "0e+1o+2e", 128, 16, 10000, False),
+    ("so2", "0e+1o+2e", 128, 20, 4096, False), ("so2", "0e+1o+2e+3o", 128, 16, 500, False),
+    ("lin", "0e+0e", 128, 128, 500, True), ("lin", "0e+0e+0e", 128, 64, 500, False), ("lin", "0e+1o", 128, 64, 500, False),
+    ("lin", "0e+1o", 256, 256, 2047, True), ("lin", "0e+1o", 256, 256, 2048, False)])
+def test_small_results_of_two_rows_stay_on_the_fp32_kernels(kind, irreps, cin, cout, n, fp32):
+    from equitorch_amd.nn.functional import _uv_native as N
+    assert N._few_and_long(_mix(kind, irreps), n, cin, cout) == fp32
