@@ -515,11 +515,14 @@ __global__ void __launch_bounds__(256, 2) uvl_gw_kernel(const UvlGwDev a) {
   }
 }
 
-// Samples per wavefront: 32 or more, at most 8192 wavefronts and 512 partial results (the rule of uvt_grad_w_small_kernel).
+// Samples per wavefront: 32 or more, at most 8192 wavefronts and as many partial results as the fp32 kernels have: 512 up to 64
+// channels, 128 past 64 on both sides (128 x 128, lmax 1, 16000 samples 53 us with 512, 42 with 256, 36 with 128; 65536: 129, 119, 111),
+// with 64 on one side 256 (64 x 128: 37, 28 and 34 us; 65536: 73, 64, 103).
 static int64_t uvl_gw_chunk(const cgtp_uvl_gw_args* a) {
   const int64_t blocks = (int64_t)((a->cx + 63) / 64) * ((a->cout + 63) / 64) * a->n_paths;
+  const int64_t partials = (a->cx > 64 ? 1 : 2) * (a->cout > 64 ? 1 : 2) * 128;
   int64_t chunk = 32;
-  while ((a->n_rows + chunk - 1) / chunk > 512 || (a->n_rows + chunk - 1) / chunk * blocks > 8192) {
+  while ((a->n_rows + chunk - 1) / chunk > partials || (a->n_rows + chunk - 1) / chunk * blocks > 8192) {
     chunk *= 2;
     if (chunk >= a->n_rows) break;
   }

@@ -52,3 +52,19 @@ def _mix(kind, irreps):
 def test_small_results_of_two_rows_stay_on_the_fp32_kernels(kind, irreps, cin, cout, n, fp32):
     from equitorch_amd.nn.functional import _uv_native as N
     assert N._few_and_long(_mix(kind, irreps), n, cin, cout) == fp32
+
+
+@pytest.mark.parametrize("n", [1, 500, 4097, 32768, 1 << 20])
+@pytest.mark.parametrize("cin,cout,paths", [(64, 64, 3), (128, 128, 2), (128, 128, 16), (96, 68, 85), (64, 128, 4), (16, 100, 1)])
+def test_the_weight_gradient_takes_no_more_memory(n, cin, cout, paths):
+    """Partial results of the weight gradient: as many as the fp32 kernels have, twice as many with 64 channels on one side only."""
+    import ctypes as C
+
+    from equitorch_amd import _lib
+    a = _lib.UvlGwArgs(4096, 4096, 4096, 4096, 4096, 4096, n, paths, 3, 16, 16, cin, cout)
+    one_side = (cin > 64) != (cout > 64)
+    most = 512 if max(cin, cout) <= 64 else 256 if one_side else 128
+    size = _lib.lib.cgtp_uvl_grad_w_workspace_bytes(C.byref(a))
+    assert 0 < size <= most * paths * cin * cout * 4
+    if n >= 4097:
+        assert size <= (2 if one_side else 1) * _lib.lib.cgtp_uvt_grad_w_workspace_bytes(n, paths, cin, cout, _lib.dtype_code(torch.float32))
