@@ -31,7 +31,7 @@ def test_struct_layouts_match_the_ctypes_mirror():
     from equitorch_amd import _lib
     for which, cls in enumerate((_lib.Operand, _lib.TriArgs, _lib.GenOperand, _lib.GenArgs, _lib.UvuArgs, _lib.UvtItem,
                                 _lib.UvtArgs, _lib.UvtGwArgs, _lib.UvtGyArgs, _lib.UvuTab, _lib.PswTable,
-                                _lib.PswArgs)):
+                                _lib.PswArgs, _lib.UvuMx, _lib.UvlArgs, _lib.UvgArgs, _lib.UvlGwArgs)):
         n = _lib.lib.cgtp_abi_layout(which, None, 0)
         assert n == 1 + len(cls._fields_), f"{cls.__name__}: {n - 1} fields in the library, {len(cls._fields_)} here"
         buf = (C.c_int64 * n)()
@@ -39,7 +39,7 @@ def test_struct_layouts_match_the_ctypes_mirror():
         assert buf[0] == C.sizeof(cls), f"sizeof {cls.__name__}"
         for k, (name, _) in enumerate(cls._fields_):
             assert buf[1 + k] == getattr(cls, name).offset, f"{cls.__name__}.{name}"
-    assert _lib.lib.cgtp_abi_layout(99, None, 0) == -1
+    assert _lib.lib.cgtp_abi_layout(16, None, 0) == _lib.lib.cgtp_abi_layout(99, None, 0) == -1
 
 
 def test_version_and_status_strings():
@@ -428,3 +428,67 @@ def test_torch_extension_loads_and_matches_the_library():
     assert mod.abi_version() == _lib.lib.cgtp_version()
     i = torch.zeros(3, dtype=torch.int64)
     mod.EdgeHandle(0, 9, 0, None, i, None, i, i, None, i, i, i, i, i, torch.zeros(2, dtype=torch.int32), None)
+
+
+def _given(cls, **changed):
+    """Arguments that their entry point accepts, some of them changed; no pointer is read by the host."""
+    a = cls()
+    for name, kind in cls._fields_:
+        if kind is C.c_void_p:
+            setattr(a, name, 4096)
+    for name, v in {**dict(n_rows=100, n_blocks=3, n_groups=2, rows_per_task=2, max_steps=64, dx=9, dout=9, dg=9, cx=32, cout=64,
+                           n_paths=3, max_pairs=64, n_ranges=8, n_wgs=64, n_slots=80, c=96, cy=0), **changed}.items():
+        if name in dict(cls._fields_):
+            setattr(a, name, v)
+    return a
+
+
+NULL, SHAPE, ALIGN, CONFIG = 1, 2, 3, 5
+
+
+@pytest.mark.parametrize("changed,status", [
+    ({}, 0), ({"n_rows": 0}, 0), ({"cx": 4, "cout": 4}, 0), ({"w": 4100}, 0), ({"by_unit": 1}, 0), ({"dx": 1 << 17}, 0),
+    *(({k: None}, NULL) for k in ("x", "packed", "w", "out", "steps", "tasks", "groups", "blocks")),
+    *(({k: v}, SHAPE) for k, v in (("n_rows", -1), ("n_blocks", 0), ("n_blocks", 65536), ("n_groups", 0), ("rows_per_task", 0),
+                                   ("rows_per_task", 3), ("by_unit", 2), ("by_unit", -1), ("max_steps", 65), ("dx", 0), ("dx", (1 << 17) + 1), ("dout", 0), ("cx", 0), ("cx", 30),
+                                   ("cout", 6), ("n_rows", 1 << 40))),
+    *(({k: 4104}, ALIGN) for k in ("x", "packed", "out"))])
+def test_channel_mixing_refuses(changed, status):
+    from equitorch_amd import _lib
+    assert _lib.lib.cgtp_uvl_validate(C.byref(_given(_lib.UvlArgs, **changed))) == status
+    if status:                         # before anything is launched
+        assert _lib.lib.cgtp_uvl_apply(C.byref(_given(_lib.UvlArgs, **changed)), None) == status
+
+
+@pytest.mark.parametrize("changed,status", [
+    ({}, 0), ({"cx": 4, "cout": 4}, 0), ({"dx": 1 << 17}, 0), ({"workspace": None}, 0),
+    *(({k: None}, NULL) for k in ("x", "g", "gw", "pairs", "path_ptr")),
+    *(({k: v}, SHAPE) for k, v in (("n_rows", 0), ("n_paths", 0), ("max_pairs", 65), ("dx", 0), ("dx", (1 << 17) + 1), ("dg", (1 << 16) + 1),
+                                   ("cx", 30), ("cout", 6))),
+    *(({k: 4104}, ALIGN) for k in ("x", "g", "gw", "workspace"))])
+def test_weight_gradient_of_channel_mixing_refuses(changed, status):
+    from equitorch_amd import _lib
+    args = _given(_lib.UvlGwArgs, **changed)
+    assert (_lib.lib.cgtp_uvl_grad_w_workspace_bytes(C.byref(args)) > 0) == (status == 0)
+    if status:
+        assert _lib.lib.cgtp_uvl_grad_w(C.byref(args), None) == status
+
+
+@pytest.mark.parametrize("changed,status", [
+    ({}, 0), ({"c": 128}, 0), ({"y": 4100}, 0), ({"c": 32, "cy": 32}, 0),
+    *(({k: None}, NULL) for k in ("x", "y", "g", "gw", "workspace", "jobs", "job_ptr", "slot_ptr")),
+    ({"cfg": -1}, CONFIG),
+    *(({k: v}, SHAPE) for k, v in (("n_rows", -1), ("n_rows", (1 << 34) + 1), ("c", 0), ("c", 98), ("c", 132), ("cy", 6), ("n_wgs", 0),
+                                   ("n_ranges", 0), ("n_ranges", 65536), ("n_slots", 0))),
+    ({"c": 32, "cy": 36}, SHAPE), ({"c": 36, "cy": 32}, SHAPE), ({"c": 32, "cy": 32, "y": 4104}, ALIGN),
+    *(({k: 4104}, ALIGN) for k in ("x", "g", "gw", "workspace"))])
+def test_weight_gradient_of_the_fully_connected_products_refuses(changed, status):
+    from equitorch_amd import _lib
+    from equitorch_amd.nn import SO3Linear
+    from equitorch_amd.ops import kernels
+    irreps = "0e+1o+2e"
+    cfg = kernels.uv_config_of(SO3Linear(irreps, irreps, irreps, 4, 4, internal_weights=False, feature_mode="uv").tp_info_forward)
+    args = _given(_lib.UvgArgs, **{"cfg": int(cfg), **changed})
+    assert _lib.lib.cgtp_uvg_validate(C.byref(args)) == status
+    if status:
+        assert _lib.lib.cgtp_uvg_apply(C.byref(args), None) == status

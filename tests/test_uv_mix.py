@@ -169,6 +169,71 @@ def test_no_less_precise_than_fp32_matrix_instructions(device, monkeypatch, kind
         assert err(a) <= (1.1 if n >= 300 else 2.0) * err(b) + 3e-8, name
 
 
+def _tile(mod, kind, transposed, n):
+    """What a launch of ``n`` samples is made of: 16 channels and 64 samples so many times, rows of the result at a time; and
+    whether a group has several tasks."""
+    from equitorch_amd.nn.functional import _irreps_gemm as G
+    from equitorch_amd.nn.functional import _uv_native as N
+    plan = G.plan_of_product_info(mod.info_forward, mod.irreps_in.dim, mod.num_weights) if kind == "so2" else G.plan_of_linear_info(mod.forward_info)
+    mix = N._MixTable(_table([(p.o0 + j, p.i0 + j, p.w, p.scale) for p in plan.paths for j in range(p.k)], mod.irreps_in.dim, plan.out_size,
+                             plan.n_paths).coo, transposed)
+    cout = mod.weight.shape[1 if transposed else 2]
+    tw = 4 if cout % 64 == 0 or cout % 64 > 32 else 2
+    groups, nt = mix.groups_for(n, -(-cout // 64)), 4 // mix.rows_per_task
+    while nt > 1 and -(-n // (64 * nt)) * groups * -(-cout // (16 * tw)) < 512:
+        nt //= 2
+    return tw, nt, mix.rows_per_task, groups < len(mix.tasks)
+
+
+LARGE = [("so2", 4, 64, 64, 33001, (4, 2, 2, True), (4, 2, 2, True)), ("so2", 4, 36, 32, 33001, (2, 2, 2, True), (4, 2, 2, True)),
+         ("so2", 6, 48, 32, 4001, (2, 2, 2, True), (4, 2, 2, True)), ("lin", 2, 64, 32, 20003, (2, 2, 1, True), (4, 2, 1, True)),
+         ("lin", 2, 32, 64, 70001, (4, 4, 1, True), (2, 4, 1, True)), ("lin", 3, 64, 32, 8001, (2, 4, 1, False), (4, 4, 1, False)),
+         ("so2", 2, 64, 64, 20003, (4, 1, 2, True), (4, 1, 2, True)), ("so2", 6, 32, 64, 1500, (4, 1, 2, True), (2, 1, 2, True)),
+         ("lin", 4, 128, 32, 3601, (2, 2, 1, False), (4, 2, 1, True)), ("lin", 6, 96, 32, 9001, (2, 2, 1, True), (2, 4, 1, True)),
+         ("lin", 4, 128, 128, 1001, (4, 1, 1, False), (4, 1, 1, False))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n,tile,tile_back", LARGE)
+def test_every_tile_is_no_less_precise(device, monkeypatch, kind, l, cin, cout, n, tile, tile_back):
+    """Sizes that take two and four times 64 samples of either width, several tasks in a group, ragged at the end."""
+    mod = _module(kind, l, cin, cout, "cpu")
+    assert (_tile(mod, kind, False, n), _tile(mod, kind, True, n)) == (tile, tile_back)
+    x, g = _operands(kind, l, cin, cout, n, stable_seed("mix tiles", kind, l, cin, cout, n))
+    new, old, ref = _routes(monkeypatch, kind, l, cin, cout, x, g, device)
+    for name, a, b, want in zip(("out", "grad x"), new, old, ref):
+        def err(t):        # row by row of the result: each against its own size, the last of the samples by themselves too
+            d = t.double() - want
+            return torch.stack([d[s].norm(dim=(0, 2)) / want[s].norm(dim=(0, 2)).clamp_min(1e-30) for s in (slice(None), slice(-41, None))])
+        e_new, e_old = err(a), err(b)
+        print(f"{name} {kind} lmax={l} {cin}->{cout} n={n}: split {e_new.amax(1).tolist()} fp32 {e_old.amax(1).tolist()}")
+        # 41 samples are some thousand draws, a tenth of the error either way at most; 3e-8: half a rounding of the result
+        assert bool((e_new <= 1.1 * e_old + 3e-8).all()), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n", [case[:5] for case in LARGE])
+def test_what_is_not_split_in_every_tile(device, monkeypatch, kind, l, cin, cout, n):
+    """A sample with an infinity and one with a tiny element in every row, spread over the batch: first, middle and last tasks
+    of a group form their results anew, and no other result changes."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    x, g = _operands(kind, l, cin, cout, n, 17)
+    for t in (x, g):
+        rows = t.shape[1]
+        for k in range(rows):
+            t[(k + 1) * n // (rows + 2), k, 3 * k % t.shape[2]] = float("inf")
+            t[n - 1 - k, k, 5 * k % t.shape[2]] = 2.0 ** -120
+    mod = _module(kind, l, cin, cout, device)
+    new = _run(mod, x.to(device), g.to(device))
+    monkeypatch.setattr(N, "_mix_split", lambda *args: None)
+    monkeypatch.setattr(N, "mix_fits", lambda *args: False)
+    for a, b in zip(new, _run(mod, x.to(device), g.to(device))):
+        fin = torch.isfinite(b)
+        assert not fin.all() and torch.equal(fin, torch.isfinite(a)) and torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num())
+        a, b = (t.nan_to_num(0.0, 0.0, 0.0).double() for t in (a, b))
+        assert float(((a - b).norm(dim=(0, 2)) / b.norm(dim=(0, 2)).clamp_min(1e-30)).max()) <= 1e-6
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,l,cin,cout,n", [("so2", 6, 48, 48, 700), ("so2", 5, 64, 96, 500), ("lin", 4, 256, 64, 900), ("so2", 6, 256, 32, 300),
                                                ("copies", 4, 64, 36, 400), ("copies", 2, 128, 128, 600)])
@@ -270,7 +335,8 @@ def _weight_gradients(monkeypatch, kind, l, cin, cout, x, g, device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,l,cin,cout,n", [("lin", 1, 4, 4, 1), ("lin", 2, 12, 20, 65), ("own", 3, 36, 100, 129), ("lin", 2, 64, 64, 70001),
-                                               ("lin", 3, 128, 96, 700), ("so2", 2, 32, 64, 31), ("so2", 4, 64, 32, 2077), ("so2", 6, 48, 48, 257)])
+                                               ("lin", 3, 128, 96, 700), ("so2", 2, 32, 64, 31), ("so2", 4, 64, 32, 2077), ("so2", 6, 48, 48, 257), ("lin", 1, 96, 128, 40001),
+                                               ("own", 2, 128, 64, 33000)])
 @pytest.mark.parametrize("values", ["normal", "wide"])
 def test_the_weight_gradient_is_no_less_precise(device, monkeypatch, kind, l, cin, cout, n, values):
     x, g = _operands(kind, l, cin, cout, n, stable_seed("mix gw", kind, l, cin, cout, n))
@@ -351,6 +417,24 @@ def test_transforms_of_the_library_route_stay(device):
     assert float((tangent - want).detach().norm()) <= 2e-6 * float(want.norm())
     batched = torch.func.vmap(lambda v: mod(v))(x.view(2, 10, *x.shape[1:]))
     assert float((batched.flatten(0, 1) - out).detach().norm()) <= 2e-6 * float(out.detach().norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", ["jvp", "vmap"])
+def test_a_first_call_inside_a_transform(device, first):
+    """The tables that a layer's first call makes from its plan are data, also where that call is inside a transform."""
+    from equitorch_amd.nn.functional import _irreps_gemm as G
+    mod, other = (_module("so2", 6, 64, 64, device) for _ in range(2))
+    G.plan_of_product_info(mod.info_forward, mod.irreps_in.dim, mod.num_weights)     # which no transform lets be read off
+    x, t = (v.to(device) for v in _operands("so2", 6, 64, 64, 20, 10))
+    if first == "jvp":
+        got, tangent = torch.func.jvp(mod, (x,), (t,))
+        assert float((tangent - other(t)).detach().norm()) <= 2e-6 * float(tangent.detach().norm())
+    else:
+        got = torch.func.vmap(lambda v: mod(v))(x.view(2, 10, *x.shape[1:])).flatten(0, 1)
+    want = other(x)
+    for a in (got, mod(x), torch.func.jvp(mod, (x,), (t,))[0]):
+        assert float((a - want).detach().norm()) <= 2e-6 * float(want.detach().norm())
 
 
 @pytest.mark.gpu
