@@ -151,11 +151,16 @@ def _mix_grad_w(x: Tensor, g: Tensor, table) -> Optional[Tensor]:
     samples: 69 us against 78), and for the same reason past 64 with the few single pairs of SO2Linear of lmax 1 (six paths, eight
     pairs; 128 channels, 4096 samples 32.5 us against 29.4, 65536 203 against 180; lmax 2, 19 and 29: 54.9 against 64.6 and 539 against
     620).  IrrepsLinear and SO2Linear, 8 to 128 channels, 500 to 65536 samples: 0.5 to 1.0 of their time (SO2Linear of lmax 2, 64 channels, 2000
-    samples 1.05)."""
+    samples 1.05).  Tables that were products of the library stay here past 128 channels below 512 samples: its sums are more precise there
+    than those of the fp32 instructions (SO2Linear, lmax 6, 256 channels, 300 samples: library 3.1e-7, fp32 instructions 3.8e-7, here 0.9e-7;
+    IrrepsLinear, lmax 4, 256 -> 64, 40 samples 1.2e-7, 2.4e-7, 0.7e-7; from 512 samples on 4.05e-7 and 4.03e-7), for 708 us against 327 in the first and 31
+    against 49 in the second layer, whose steps still take less than the library's."""
     if not (isinstance(table, CooTable) and table.mixing) or x.dtype != torch.float32 or x.shape[0] == 0:
         return None
     (n, dx, cx), (_, dg, cout), n_paths = x.shape, g.shape, table.coo.P
-    if max(cx, cout) > 128 or (min(cx, cout) > 64 and n_paths <= 8 and len(table.coo.p) < 2 * n_paths and n > 2000):
+    if max(cx, cout) > 128 and (n >= 512 or not _was_the_library(n, cx, cout, table)):
+        return None
+    if min(cx, cout) > 64 and n_paths <= 8 and len(table.coo.p) < 2 * n_paths and n > 2000:
         return None
     pairs = kernels.cached(_anchor(table), ("uvl_pairs", str(x.device)), lambda: _MixPairs(table.coo, x.device))
     gw = torch.empty((n_paths, cx, cout), dtype=x.dtype, device=x.device)
@@ -668,6 +673,12 @@ def _few_and_long(mix: _MixTable, n: int, cx: int, cout: int) -> bool:
             and n < (10000 if cx > 64 and cout <= 16 else 5000) and mix.n_out * cout <= (256 if mix.n_out <= 4 else 144))
 
 
+def _was_the_library(n: int, u: int, wc: int, table) -> bool:
+    """Whether the fp32 kernels do not take channel mixing with this table, ``u -> wc`` channels: the products of the library, whose
+    sums are more precise than theirs, served it."""
+    return kernels.cached(_anchor(table), ("uvl_was_library", u, wc), lambda: not u1v_fits(n, u, wc, table, torch.float32))
+
+
 def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor]:
     """Channel mixing in fp32 on the half-precision matrix cores (``cgtp_uvl_apply``), or None where the fp32 matrix
     instructions serve.  Over 1000 launches (IrrepsLinear of lmax 1 to 4 and of copies of an irrep, SO2Linear of lmax 1 to 6, 8 to
@@ -682,9 +693,7 @@ def _mix_split(x: Tensor, w: Tensor, table, transposed: bool) -> Optional[Tensor
         return None
     n_groups = mix.groups_for(n, -(-cout // 64))
     walk = kernels.cached(_anchor(table), ("uvl_walk", transposed, str(x.device)), lambda: _MixWalk(mix, x.device))
-    # tables the fp32 kernels do not take were products of the library, whose sums are more precise than theirs
-    by_unit = kernels.cached(_anchor(table), ("uvl_by_unit", w.shape[1], w.shape[2]),
-                             lambda: int(not u1v_fits(n, w.shape[1], w.shape[2], table, x.dtype)))
+    by_unit = int(_was_the_library(n, w.shape[1], w.shape[2], table))
     packed = torch.empty(int(_lib.lib.cgtp_uvl_packed_bytes(mix.n_blocks, cx, cout)), dtype=torch.uint8, device=x.device)
     out = torch.empty((n, mix.n_out, cout), dtype=x.dtype, device=x.device)
     steps, groups, tasks, blocks = walk.address[n_groups]

@@ -254,6 +254,35 @@ def test_long_rows_are_no_less_precise_than_the_library(device, monkeypatch, kin
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,l,cin,cout,n", [("so2", 6, 48, 48, 300), ("so2", 6, 256, 256, 40), ("so2", 6, 256, 256, 300), ("so2", 6, 256, 256, 511),
+                                               ("so2", 6, 256, 256, 512), ("so2", 6, 132, 96, 300), ("lin", 4, 256, 64, 40), ("lin", 4, 256, 64, 512)])
+@pytest.mark.parametrize("sign", [False, True])
+def test_their_weight_gradient_is_no_less_precise_than_the_library(device, monkeypatch, kind, l, cin, cout, n, sign):
+    """Of the same layers; thousands of sums each, so that the errors are known to a few parts in a hundred."""
+    from equitorch_amd.nn.functional import _uv_native as N
+    mod = _module(kind, l, cin, cout, device)
+    gen = torch.Generator().manual_seed(stable_seed("long gw", kind, l, cin, cout, n))
+    x, g = (torch.randn(n, irreps.dim, c, generator=gen).to(device) for irreps, c in ((mod.irreps_in, cin), (mod.irreps_out, cout)))
+    if sign:
+        x, g = x.abs(), g.abs()
+    taken, fits = [], N.mix_fits
+
+    def spy(*args):
+        taken.append(fits(*args))
+        return taken[-1]
+    monkeypatch.setattr(N, "mix_fits", spy)
+    new, = torch.autograd.grad(mod(x), [mod.weight], g)
+    assert taken == [True]
+    monkeypatch.setattr(N, "mix_fits", lambda *args: False)
+    old, = torch.autograd.grad(mod(x), [mod.weight], g)
+    mod.double()
+    want, = torch.autograd.grad(mod(x.double()), [mod.weight], g.double())
+    e_new, e_old = (float((t.double() - want).norm() / want.norm()) for t in (new, old))
+    print(f"grad W {kind} {l} {cin}->{cout} n={n} sign={sign}: kernel {e_new:.2e} library {e_old:.2e}")
+    assert e_new <= 1.1 * e_old
+
+
+@pytest.mark.gpu
 def test_what_stays_on_the_library(device, monkeypatch):
     """Rows whose sums the library forms more precisely, and products it forms as quickly."""
     from equitorch_amd.nn.functional import _uv_native as N
