@@ -14,11 +14,12 @@
 //
 // What bounds it: matrix instructions, at the clock of 1.6 to 1.8 GHz that the card keeps under them (SO2Linear, lmax = 4, 64
 // channels, 32768 samples: 134 us of the 270 at 1.7 GHz; without them the launch takes 155, L2 and stores).
-// Measured there: 571 us on fp32 matrix instructions (uvt_apply_kernel) -> 273; lmax 2: 32 channels, 4096 samples 12.9 -> 11.0; IrrepsLinear
-// 64 -> 64, lmax 2, 65536 samples 126 -> 75, 128 -> 128, lmax 3, 32768 samples 308 -> 170.  One workgroup per pair of rows, 325 us: a
-// third of its time went into starting; half lines of x from memory straight into the operands, 300; three wavefronts per
-// SIMD (spills), eight in a workgroup, matrix and vector instructions in turn by hand: no change.  Errors of the results
-// against 64 bits: 0.4e-7 to 3.8e-7, of fp32 matrix instructions 0.9e-7 to 4.5e-7 (BY_UNIT below).
+// Measured there, one call at a time with the packing (the kernel alone: 252): 571 us on fp32 matrix instructions (uvt_apply_kernel)
+// -> 273; lmax 2: 32 channels, 4096 samples 12.9 -> 11.0; IrrepsLinear 64 -> 64, lmax 2, 65536 samples 126 -> 75, 128 -> 128, lmax 3,
+// 32768 samples 308 -> 170.  One workgroup per pair of rows, 325 us: a third of its time went into starting; half lines of x from
+// memory straight into the operands, 300; three wavefronts per SIMD (spills), eight in a workgroup, matrix and vector instructions in
+// turn by hand: no change.  Errors of the results against 64 bits: 0.4e-7 to 3.8e-7, of fp32 matrix instructions 0.9e-7 to 4.5e-7
+// (BY_UNIT below).
 //
 // Values: elements that are not finite or overflow as parts show in the results, and elements below 2^-110 (but not zero; their
 // last part could be below the smallest subnormal) are looked for; a wavefront that sees either forms its results

@@ -21,7 +21,8 @@
 //
 // What bounds it: waiting (43 % of the wavefronts' time at two per SIMD: rows from the last-level cache, three quarters of the requests
 // that miss the L1 at lmax = 3; barriers), then vector and matrix instructions in about equal parts (250 vector ones to 24 matrix
-// ones of 32 cycles per product and wavefront).  128 channels, 32768 samples: lmax 3 1253 -> 855 us, lmax 2 444 -> 318; 4096 samples
+// ones of 32 cycles per product and wavefront).  One call at a time with its reduction (the kernel alone, lmax 3 1218 -> 744 us, "uvw"
+// 1336 -> 846), 128 channels, 32768 samples: lmax 3 1253 -> 855 us, lmax 2 444 -> 318; 4096 samples
 // 196 -> 130 and 80 -> 60; "uvw" 32 x 32 -> 32, lmax 2, 32768 samples 1280 -> 855 us, 4096 235 -> 162.  With all sums of one sign, 32 products
 // each: lmax 3 5.4e-7 in 935 us, 64: 7.2e-7.  Tables walked at run time
 // instead of generated: 1390; one wavefront per l with "uvw": 1300.
